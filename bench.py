@@ -39,10 +39,10 @@ Prints one JSON line.  Besides the metric it reports:
   cpu_baseline           the FP64 oracle (a C restatement of the Go
                          reference) on a bounded sample of the same worlds,
                          on all host cores and on one
-  resolver_split         per leg, the split between the one- and the
-                         four-wavefront resolver kernels that the autotuner
+  resolver_split         per leg, the resolver split that the autotuner
                          (cbz_autotune_resolver) picked on the settled state,
-                         with every candidate's ms/step
+                         with every candidate's ms/step (the split has no
+                         effect any more: the times differ by noise)
 """
 import argparse
 import json
@@ -307,13 +307,13 @@ def run_path(World, sc, ck, precision, steps, warmup):
         "contacts_per_step": contacts / sp,
         "contacts_per_s": contacts / sp * steps / wall,
         "iters_per_step": iters / sp,
-        # the resolver's latency measures: one wavefront per world,
-        # worlds_per_cu of them resident per CU
+        # the resolver's latency measures: one workgroup of four wavefronts
+        # per world, worlds_per_cu of them resident per CU
         "resolver": {
             "iterations_per_world_per_step": iters / sp / sc.n_worlds,
             "worlds_per_cu": per_cu,
             "resident_worlds": resident,
-            "waves_per_simd": resident / (4.0 * n_cu),
+            "waves_per_simd": resident / float(n_cu),
             "ns_per_iteration_aggregate": resolve_ns / (iters / sp) if iters else None,
             "ns_per_iteration_per_world": resolve_ns * resident / (iters / sp) if iters else None,
         },
@@ -452,9 +452,8 @@ def main():
     ap.add_argument("--cpu-budget", type=float, default=20.0, help="seconds of oracle wall time")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--resolver-split", default="auto",
-                    help="the resolver's split between its kernels: 'auto' (the autotuner, per leg, from the "
-                         "window's start state), 'default' (the library's), or 'min,max' (the max largest worlds "
-                         "of at least min contacts take the multi-wave kernel; 0,0: none)")
+                    help="the resolver split to set (no effect on results or times): 'auto' (the autotuner, per leg, "
+                         "from the window's start state), 'default' (the library's), or 'min,max'")
     ap.add_argument("--probe-k1", action="store_true",
                     help="for hardware-counter runs: 20 launches of K1 (FP32 and FP64) on the workload, then 20 "
                          "copies of a 256 MiB float32 buffer as the calibration kernel; prints no JSON")
@@ -626,14 +625,14 @@ def main():
     if dom in ("position_phase", "velocity_phase", "resolve"):
         ms = phases[dom] if use_sur else kern32["resolve"]
         ach = res_bytes / (ms / 1000.0) / 1e9
-        roof = {"kernel": {"position_phase": "k_resolve_f32<polish> (adjustPositions from the network's moves, "
+        roof = {"kernel": {"position_phase": "k_resolve_islands_f32<position polish> (adjustPositions from the network's moves, "
                                              "with the exact fallback)",
-                           "velocity_phase": "k_resolve_f32<polish> (adjustVelocities from the network's changes, "
+                           "velocity_phase": "k_resolve_islands_f32<velocity polish> (adjustVelocities from the network's changes, "
                                              "with the exact fallback)",
-                           "resolve": "k_resolve_f32<plain>"}[dom],
+                           "resolve": "k_resolve_islands_f32<plain>"}[dom],
                 "bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": ach / HBM_PEAK_GBS,
                 "traffic": None, "bytes_per_launch": res_bytes, "ms_per_launch": ms,
-                "note": "serial worst-first iterations per world: latency-bound, see exact_*.resolver"}
+                "note": "serial worst-first iterations per island: latency- and issue-bound, see exact_*.resolver"}
     elif dom == "network":
         roof = dict(out["mlp"])
         roof["traffic"] = None

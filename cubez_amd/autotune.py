@@ -1,14 +1,10 @@
-"""The resolver's split between its one-wavefront and multi-wavefront
-kernels, chosen by measurement (cbz_autotune_resolver) and cached on disk.
+"""The resolver split (cbz_set_resolver_split), measured per scene
+(cbz_autotune_resolver) and cached on disk.
 
-The split is a scheduling choice with no effect on results: of the worlds
-of at least `min_contacts` contacts, the `max_worlds` largest resolve on a
-kernel of four wavefronts per world (one per SIMD, with every contact's
-data on chip), the others on the one-wavefront kernel.  Which is fastest
-depends on the distribution of contact counts over the worlds (a few large
-worlds set the step's critical path; many large worlds make the
-multi-wavefront kernel, one world per CU, a throughput limit), so it is
-measured on the scene itself, from its current (settled) state.
+The split named the worlds that a second resolver kernel took.  Every world
+now runs on one kernel, island by island, so the candidates time alike and
+whichever is kept changes nothing; the module serves the programs that call
+it.
 
 The cache key is the scene's shape and the step kind: precision, world and
 body counts, a coarse histogram of per-world contact counts, and whether

@@ -36,8 +36,6 @@ const FieldInfo kFields[CBZ_NUM_FIELDS] = {
 constexpr uint8_t kUserFlags = CBZ_FLAG_AWAKE | CBZ_FLAG_CAN_SLEEP | CBZ_FLAG_STATIC;
 // real planes per contact slot (see cbz_context::c_real)
 constexpr int kContactPlanes = 40;
-// The resolver's multi-wave kernel takes the 32 largest worlds of more than
-// 256 contacts.
 constexpr int32_t kDefaultMwMin = 257;
 constexpr int32_t kDefaultMwMax = 32;
 
@@ -79,13 +77,10 @@ struct cbz_context {
   int64_t cap_cfg = 0;
   hipStream_t stream = nullptr;
   std::string err;
-  // the resolver's multi-wave kernel: the mw_max largest worlds of at
-  // least mw_min contacts run on stream `side` beside the one-wave kernel
-  hipStream_t side = nullptr;
-  hipEvent_t mw_fork = nullptr, mw_sel = nullptr, mw_join = nullptr;
+  // the resolver split a caller set (cbz_set_resolver_split): kept and
+  // returned, no kernel reads it
   int32_t mw_min = kDefaultMwMin;
   int32_t mw_max = kDefaultMwMax;
-  int32_t n_cu = 256;
 
   // scene
   int32_t nw = 0;
@@ -177,9 +172,8 @@ struct cbz_context {
   int32_t* overflow = nullptr;  // [0] this narrowphase, [1] sticky since the host cleared it
   int64_t* world_iters = nullptr;
   int64_t* world_time = nullptr;  // [4 * nw] resolver workgroup start/end ticks (position, velocity launch)
-  int32_t* mw_list = nullptr;     // [nw] worlds of the multi-wave kernel (resolver launch)
-  int32_t* mw_count = nullptr;    // [2] list length, work-queue head
-  uint8_t* mw_flag = nullptr;     // [nw] listed
+  IslandBuffers isl;              // the resolver's island kernel (first resolve), in isl_mem
+  char* isl_mem = nullptr;
   int32_t* order = nullptr;
   bool have_contacts = false;
 
@@ -208,13 +202,10 @@ struct cbz_context {
     uint8_t* mask = nullptr;
     int32_t* nfall = nullptr;
     float* delta = nullptr;  // [6][n_bodies] predicted change per body
-    void* vel0 = nullptr;    // [7][n_bodies] velocity, rotation, motion before it
-    void* cvel0 = nullptr;   // [3][cap] contact velocities as prepare left them
     // the position phase's polish: per-world mask, predicted change per body
-    // [6][n_bodies], snapshot [22][n_bodies] of the sleeping bodies
+    // [6][n_bodies]
     uint8_t* pmask = nullptr;
     float* dpos = nullptr;
-    void* psnap = nullptr;
     // position polish tolerance (m) above positionEpsilon and budget per
     // contact; a negative tolerance gives every world the plain position phase
     double pos_tol = 0.0;
@@ -379,11 +370,8 @@ void free_sur_buffers(cbz_ctx* c) {
   dfree(u.mask);
   dfree(u.nfall);
   dfree(u.delta);
-  dfree(u.vel0);
-  dfree(u.cvel0);
   dfree(u.pmask);
   dfree(u.dpos);
-  dfree(u.psnap);
   u.inf_cap = 0;
   u.lay_cap = 0;
   u.generation += 1;
@@ -451,9 +439,8 @@ void free_scene(cbz_ctx* c) {
   dfree(c->overflow);
   dfree(c->world_iters);
   dfree(c->world_time);
-  dfree(c->mw_list);
-  dfree(c->mw_count);
-  dfree(c->mw_flag);
+  dfree(c->isl_mem);
+  c->isl = IslandBuffers{};
   dfree(c->order);
   dfree(c->d_awake);
   dfree(c->d_prof);
@@ -645,23 +632,72 @@ int do_narrowphase(cbz_ctx* c, int32_t list_tiles, hipEvent_t* ev = nullptr) {
   return CBZ_OK;
 }
 
+// The island kernel's buffers, one allocation made at the scene's first
+// resolve (and before a capture of one): a program that only generates
+// contacts never pays for them.
+int ensure_islands(cbz_ctx* c) {
+  if (c->isl_mem) return CBZ_OK;
+  IslandBuffers u;
+  int32_t most = 1;
+  for (int32_t w = 0; w < c->nw; ++w) {
+    const int32_t n = c->body_off[w + 1] - c->body_off[w];
+    if (n <= kIslBodies) most = std::max(most, n);
+  }
+  u.nb = (most + 15) & ~15;
+  // log pool for the worlds that exceed their iteration budget: a world of
+  // towers in their first step runs 17 iterations per contact, a slot of the
+  // default capacity holds a quarter of a contact there; worlds that find no
+  // room go to the serial kernel
+  u.log_cap = 4 * c->cap + 65536;
+  const size_t rs = real_size(c), nb = (size_t)std::max<int64_t>(c->nb, 1), nw = (size_t)c->nw, cap = (size_t)c->cap;
+  size_t total = 0;
+  auto place = [&](bool assign) {
+    size_t at = 0;
+    auto take = [&](auto*& p, size_t bytes) {
+      if (assign) p = (std::remove_reference_t<decltype(p)>)(c->isl_mem + at);
+      at += (bytes + 255) & ~size_t(255);
+    };
+    take(u.left_count, 2 * sizeof(int32_t));
+    take(u.log_head, sizeof(int64_t));
+    take(u.cls, nw * kIslWords * sizeof(int32_t));
+    const size_t zeroed = at;
+    take(u.left_list, nw * sizeof(int32_t));
+    take(u.off, nb * sizeof(int32_t));
+    take(u.cnt, nb * sizeof(int32_t));
+    take(u.its, nb * sizeof(int32_t));
+    take(u.nrec, nb * sizeof(int32_t));
+    take(u.log, nb * sizeof(int64_t));
+    take(u.flag, nb);
+    take(u.idx, cap * sizeof(int32_t));
+    take(u.save, 5 * cap * rs);
+    take(u.snap, 21 * nb * rs);
+    take(u.log_key, (size_t)u.log_cap * rs);
+    take(u.log_j, (size_t)u.log_cap * sizeof(int32_t));
+    take(u.log_it, (size_t)u.log_cap * sizeof(int32_t));
+    total = at;
+    return zeroed;
+  };
+  const size_t zeroed = place(false);
+  int rc;
+  if ((rc = dalloc(c, &c->isl_mem, total))) return rc;
+  place(true);
+  c->isl = u;
+  HIPCHK(c, hipMemsetAsync(c->isl_mem, 0, zeroed, c->stream));
+  return CBZ_OK;
+}
+
 template <typename R>
 int do_resolve(cbz_ctx* c, double dt, int64_t mult, int64_t fixed, int32_t mode = 3,
                uint8_t* mask = nullptr, float* labels = nullptr, double polish_tol = 0, int64_t polish_mult = 0) {
+  const int rc = ensure_islands(c);
+  if (rc) return rc;
   ResolveLaunch<R> L;
   L.mode = mode;
   if (c->mat_flags & CBZ_MATERIALS_FRICTIONLESS_TWO_BODY) L.mode |= RM_FRICTIONLESS2;
   L.world_mask = mask;
   L.labels = labels;
   if (mode & RM_POLISH) {
-    if (mode & RM_POS) {
-      L.delta = c->sur.dpos;
-      L.vel0 = (R*)c->sur.psnap;
-    } else {
-      L.delta = c->sur.delta;
-      L.vel0 = (R*)c->sur.vel0;
-      L.cvel0 = (R*)c->sur.cvel0;
-    }
+    L.delta = (mode & RM_POS) ? c->sur.dpos : c->sur.delta;
     L.polish_tol = (R)polish_tol;
     L.polish_mult = polish_mult;
   }
@@ -675,23 +711,10 @@ int do_resolve(cbz_ctx* c, double dt, int64_t mult, int64_t fixed, int32_t mode 
   L.body_off = c->d_body_off;
   L.world_iters = c->world_iters;
   L.world_time = c->world_time;
-  L.mw_min = c->mw_min;
-  L.mw_max = c->mw_max;
-  // A launch without iterations (prepareContacts only) gains nothing from the
-  // multi-wave kernel, and leaves the worlds' iteration counts (the next
-  // position launch picks its multi-wave worlds by the last ones) alone.
-  if (mult == 0 && fixed == 0) {
-    L.mw_max = 0;
-    L.world_iters = nullptr;
-  }
-  L.mw_list = c->mw_list;
-  L.mw_count = c->mw_count;
-  L.mw_flag = c->mw_flag;
-  L.side = c->side;
-  L.fork = c->mw_fork;
-  L.sel = c->mw_sel;
-  L.join = c->mw_join;
-  L.n_cu = c->n_cu;
+  // a launch without iterations (prepareContacts only) leaves the worlds'
+  // iteration counts alone
+  if (mult == 0 && fixed == 0) L.world_iters = nullptr;
+  L.isl = c->isl;
   L.n_worlds = c->nw;
   L.dt = (R)dt;
   L.iter_mult = mult;
@@ -1202,11 +1225,8 @@ int sur_ensure_inference(cbz_ctx* c, int64_t rows) {
   if ((rc = dalloc(c, &u.nfall, 1))) return rc;
   const size_t nb = (size_t)std::max<int64_t>(c->nb, 1);
   if ((rc = dalloc(c, &u.delta, 6 * nb))) return rc;
-  if ((rc = dalloc_bytes(c, &u.vel0, 7 * nb * real_size(c)))) return rc;
-  if ((rc = dalloc_bytes(c, &u.cvel0, 3 * (size_t)std::max<int64_t>(c->cap, 1) * real_size(c)))) return rc;
   if ((rc = dalloc(c, &u.pmask, (size_t)std::max(c->nw, 1)))) return rc;
   if ((rc = dalloc(c, &u.dpos, 6 * nb))) return rc;
-  if ((rc = dalloc_bytes(c, &u.psnap, 22 * nb * real_size(c)))) return rc;
   u.inf_cap = Mpad;
   u.generation += 1;  // buffers moved: a captured surrogate step is stale
   return CBZ_OK;
@@ -1373,11 +1393,6 @@ int cbz_create(const cbz_config* cfg, cbz_ctx** out) {
   bool ok = hipSetDevice(c->device) == hipSuccess &&
             hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
   for (auto& e : c->ev) ok = ok && hipEventCreate(&e) == hipSuccess;
-  ok = ok && hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) == hipSuccess &&
-       hipEventCreateWithFlags(&c->mw_fork, hipEventDisableTiming) == hipSuccess &&
-       hipEventCreateWithFlags(&c->mw_sel, hipEventDisableTiming) == hipSuccess &&
-       hipEventCreateWithFlags(&c->mw_join, hipEventDisableTiming) == hipSuccess &&
-       hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, c->device) == hipSuccess;
   ok = ok && scratch_address(c->device, &c->scratch) == hipSuccess;
   if (!ok) {
     cbz_destroy(c);
@@ -1397,11 +1412,6 @@ int cbz_destroy(cbz_ctx* c) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : c->pev)
     if (e) (void)hipEventDestroy(e);
-  if (c->side) (void)hipStreamSynchronize(c->side);
-  if (c->mw_fork) (void)hipEventDestroy(c->mw_fork);
-  if (c->mw_sel) (void)hipEventDestroy(c->mw_sel);
-  if (c->mw_join) (void)hipEventDestroy(c->mw_join);
-  if (c->side) (void)hipStreamDestroy(c->side);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return CBZ_OK;
@@ -1523,9 +1533,6 @@ int cbz_set_scene(cbz_ctx* c, int32_t n_worlds, const int32_t* body_off, const i
   if ((rc = dalloc(c, &c->world_iters, 2 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->world_time, 4 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->order, (size_t)n_worlds))) return rc;
-  if ((rc = dalloc(c, &c->mw_list, (size_t)n_worlds))) return rc;
-  if ((rc = dalloc(c, &c->mw_count, 2))) return rc;
-  if ((rc = dalloc(c, &c->mw_flag, (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->d_awake, kAwakeSlots))) return rc;
   if ((rc = dalloc(c, &c->d_prof, 4))) return rc;
   if ((rc = dalloc_bytes(c, &c->pos0, rs * 3 * (size_t)std::max<int64_t>(nb, 1)))) return rc;
@@ -1968,11 +1975,8 @@ int cbz_set_resolver_split(cbz_ctx* c, int32_t min_contacts, int32_t max_worlds)
   if (!c) return CBZ_ERR_ARG;
   if (min_contacts < 0 || max_worlds < 0)
     return fail(c, CBZ_ERR_ARG, "set_resolver_split: min_contacts and max_worlds must be >= 0");
-  if (min_contacts != c->mw_min || max_worlds != c->mw_max) {
-    drop_graph(c);  // captured launches carry the split
-    c->mw_min = min_contacts;
-    c->mw_max = max_worlds;
-  }
+  c->mw_min = min_contacts;
+  c->mw_max = max_worlds;
   return CBZ_OK;
 }
 
@@ -2094,6 +2098,7 @@ int cbz_step(cbz_ctx* c, double dt, int32_t n_steps, int64_t iter_per_contact, i
     // launches do no host work and read them from device memory.
     rc = refresh_pow(c, dt);
     if (rc == CBZ_OK) rc = refresh_brad(c);
+    if (rc == CBZ_OK) rc = ensure_islands(c);
     if (rc) return rc;
     if (!c->gexec || c->g_dt != dt || c->g_mult != iter_per_contact) {
       drop_graph(c);
@@ -2741,6 +2746,7 @@ int cbz_step_sur(cbz_ctx* c, double dt, int32_t n_steps, int64_t iter_per_contac
     // inputs are refreshed first, and every buffer the step uses exists.
     rc = refresh_pow(c, dt);
     if (rc == CBZ_OK) rc = refresh_brad(c);
+    if (rc == CBZ_OK) rc = ensure_islands(c);
     if (rc) return rc;
     if (n_steps > c->fb_cap) {
       const int64_t cap = std::max<int64_t>(n_steps, 2 * c->fb_cap);

@@ -18,15 +18,11 @@ namespace cbz {
 // per-body velocity changes in `delta`, then run the velocity loop until
 // every contact is within velocityEpsilon + polish_tol, at most
 // polish_mult * C iterations; a world that does not get there is restored
-// (velocities, rotations, motion, awake flags) and re-solved by the plain
-// velocity phase, and its mask byte set to 1.  Worlds whose mask byte is 1
+// and re-solved by the plain velocity phase, and its mask byte set to 1.  Worlds whose mask byte is 1
 // run the plain velocity phase.
 // RM_POLISH with RM_POS: the same for the position phase, from the per-body
 // position and orientation changes in `delta`, to positionEpsilon +
-// polish_tol; the restore covers positions, orientations, the awake flags
-// and the motion, transform and world inverse inertia of the bodies asleep
-// when the phase starts (snapshot in vel0).  A single launch polishes one
-// phase.
+// polish_tol.  A single launch polishes one phase.
 // RM_PREPARED (with RM_POS): prepareContacts already ran, in an earlier
 // launch with RM_POS and an iteration budget of 0; this launch reads the
 // contact internals and prepare-time positions it stored.
@@ -58,6 +54,33 @@ struct NarrowLaunch {
   Materials<R> mat{};  // per-body and per-plane materials (read when c.fric is set)
 };
 
+// The most bodies of a world the island kernel's LDS tables hold.
+constexpr int kIslBodies = 2048;
+// Words per world of IslandBuffers::cls.
+constexpr int kIslWords = 16;
+
+// The island kernel's device buffers (see RS in cbz_resolve.h).
+struct IslandBuffers {
+  int32_t nb = 0;                   // bodies per LDS table: the largest world of at most kIslBodies
+  int32_t* off = nullptr;           // [n_bodies]
+  int32_t* cnt = nullptr;           // [n_bodies]
+  int32_t* its = nullptr;           // [n_bodies]
+  int32_t* nrec = nullptr;          // [n_bodies]
+  int64_t* log = nullptr;           // [n_bodies]
+  int32_t* cls = nullptr;           // [kIslWords * n_worlds]
+  int32_t* idx = nullptr;           // [cap]
+  void* save = nullptr;             // [5][cap] reals
+  void* snap = nullptr;             // [21][n_bodies] reals
+  uint8_t* flag = nullptr;          // [n_bodies]
+  void* log_key = nullptr;          // [log_cap] reals
+  int32_t* log_j = nullptr;         // [log_cap]
+  int32_t* log_it = nullptr;        // [log_cap]
+  int64_t* log_head = nullptr;      // [1]
+  int64_t log_cap = 0;
+  int32_t* left_list = nullptr;     // [n_worlds]
+  int32_t* left_count = nullptr;    // [2], zero between resolves
+};
+
 template <typename R>
 struct ResolveLaunch {
   Bodies<R> b;
@@ -69,18 +92,7 @@ struct ResolveLaunch {
   const int32_t* body_off;
   int64_t* world_iters;
   int64_t* world_time = nullptr;         // [4][n_worlds] wall-clock ticks (see the resolver's RS)
-  // The multi-wave kernel for the mw_max largest worlds of at least mw_min
-  // contacts (either 0: off), on stream `side`, forked from and joined back
-  // into the launch's stream by the events; mw_list [n_worlds], mw_count [2]
-  // and mw_flag [n_worlds] are its work list.
-  int32_t mw_min = 0;
-  int32_t mw_max = 0;
-  int32_t* mw_list = nullptr;
-  int32_t* mw_count = nullptr;
-  uint8_t* mw_flag = nullptr;
-  hipStream_t side = nullptr;
-  hipEvent_t fork = nullptr, sel = nullptr, join = nullptr;
-  int32_t n_cu = 256;
+  IslandBuffers isl;
   int32_t n_worlds;
   R dt;
   int64_t iter_mult;
@@ -90,8 +102,6 @@ struct ResolveLaunch {
   R* pos0 = nullptr;                     // [3][n_bodies] positions at prepare time
   float* labels = nullptr;               // [cap][13] velocity-phase changes, resolved penetration per contact
   const float* delta = nullptr;          // RM_POLISH: [6][n_bodies] velocity, rotation (or position, orientation) changes
-  R* vel0 = nullptr;                     // RM_POLISH: snapshot, [7][n_bodies] (RM_VEL) or [22][n_bodies] (RM_POS)
-  R* cvel0 = nullptr;                    // RM_POLISH with RM_VEL: [3][cap] contact velocities after prepare
   R polish_tol = R(0);
   int64_t polish_mult = 0;
 };

@@ -17,8 +17,8 @@ constexpr int kOutPad = 32;    // padded to the MFMA tile (32)
 constexpr int kLayers = 4;
 constexpr int kSurBodies = 256;     // bodies per world the surrogate takes
 constexpr int kSurContacts = 2048;  // contacts per world the surrogate takes
-// contacts per world the position polish takes (the one-wavefront
-// kernel's widest register class); larger worlds get the plain position phase
+// contacts per world the position polish takes; larger worlds get the plain
+// position phase
 constexpr int kSurPosContacts = 2048;
 
 // layer l maps kIn[l] -> kOutL[l] features (unpadded)

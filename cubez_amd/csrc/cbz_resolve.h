@@ -1,13 +1,14 @@
-// cbz_resolve.h — K3: ResolveContacts (contact.go:208-222), one wavefront
-// per world.  Device code of the resolver kernel; each (precision, kind)
-// instantiation is compiled in a translation unit of its own
+// cbz_resolve.h — K3: ResolveContacts (contact.go:208-222): the pieces both
+// resolver kernels are made of, and the serial one, a wave per world, for the
+// worlds that the island kernel (cbz_islands.h) leaves.  Each (precision,
+// kind) instantiation is compiled in a translation unit of its own
 // (k_resolve_<precision>_<kind>.hip), the launch dispatch is k_resolve.hip.
 //
 // The reference's resolver is sequential: each iteration picks the worst
 // contact (largest penetration, then largest desired velocity change; ties
 // go to the lowest index because the scan uses a strict '>'), applies a
 // correction to its one or two bodies, and updates every contact that
-// shares one of those bodies.  A world therefore runs on one wave: the
+// shares one of those bodies.  Here a world runs on one wave: the
 // argmax is a lane-strided scan plus a butterfly reduction, the correction
 // is computed redundantly by all 64 lanes (lane 0 stores it), and the
 // update scans the world's contacts lane-parallel, each contact applying
@@ -28,6 +29,13 @@
 namespace cbz {
 
 constexpr int kKeyCap = 1280;
+
+// threads of the island kernel's workgroup
+constexpr int kIslThreads = 256;
+// a left world's entry: its position phase is done already
+constexpr int32_t kLeftVelOnly = 1 << 30;
+// RS::left_count: listed worlds, workgroups of the left kernel that are done
+enum : int { LEFT_WORLDS = 0, LEFT_DONE = 1, LEFT_COUNTS = 2 };
 
 // Relative energy slack of the surrogate's acceptance test (rounding); the
 // absolute slack is 1/2 tol^2 per kilogram: the kinetic energy of the
@@ -69,12 +77,33 @@ struct RS {
   // [4 * n_worlds] (or null): wall-clock ticks when the world's workgroup
   // started and ended, for a launch without (0, 1) and with (2, 3) RM_VEL
   int64_t* world_time;
-  // worlds taken by the multi-wave kernel (resolve_mw), chosen by
-  // k_mw_select: mw_list[0 .. mw_count[0]), flagged in mw_flag; mw_count[1]
-  // is the kernel's work-queue head (null mw_list: none)
-  const int32_t* mw_list;
-  int32_t* mw_count;
-  const uint8_t* mw_flag;
+  // the worlds the island kernel leaves: entries (world | kLeftVelOnly);
+  // left_count: LEFT_*, zero between resolves
+  int32_t* left_list;
+  int32_t* left_count;
+  // the island kernel (cbz_islands.h): per island, at its world's
+  // first body + rank: contacts (offset into isl_idx from the world's first
+  // slot, count), iterations, log records and where the log starts; per
+  // world the class counts and, in entry 6, whether its islands were taken
+  int32_t isl_nb;      // bodies the LDS tables hold
+  int32_t* isl_off;    // [n_bodies]
+  int32_t* isl_cnt;    // [n_bodies]
+  int32_t* isl_its;    // [n_bodies]
+  int32_t* isl_nrec;   // [n_bodies]
+  int64_t* isl_log;    // [n_bodies]
+  int32_t* isl_cls;    // [kIslWords * n_worlds]
+  int32_t* isl_idx;    // [cap]
+  R* isl_save;         // [5][cap] contact velocity, desired velocity change, penetration before the phase
+  // [21][n_bodies] position phase: transform and world inverse inertia of
+  // sleeping bodies; velocity phase: the state table at a pause (6), with
+  // its flags in isl_flag [n_bodies]
+  R* isl_snap;
+  uint8_t* isl_flag;
+  R* log_key;          // [log_cap] the log pool: key, contact, iteration
+  int32_t* log_j;
+  int32_t* log_it;
+  int64_t* log_head;
+  int64_t log_cap;
   int32_t n_worlds;
   R dt;
   int64_t iter_mult;
@@ -88,11 +117,6 @@ struct RS {
   // RM_POLISH: [6][n_bodies] velocity and rotation changes (RM_VEL) or
   // position and orientation changes (RM_POS)
   const float* delta;
-  // RM_POLISH snapshot: [7][n_bodies] vel, rot, motion before the changes
-  // (RM_VEL); [22][n_bodies] motion, transform, iit_world of the bodies
-  // asleep when the phase starts (RM_POS)
-  R* vel0;
-  R* cvel0;                    // RM_POLISH with RM_VEL: [3][cap] contact velocities as prepare left them
   R polish_tol;
   int64_t polish_mult;
 };
@@ -445,7 +469,7 @@ __device__ __forceinline__ R frictionless_delta_velocity(const R im[2], bool has
 // unit impulse, :537-578) and its inverse impulseMatrix (:581); they depend
 // only on contactToWorld, the relative contact positions, both bodies'
 // world inverse inertia and inverse masses, none of which the velocity
-// phase changes, so the register-resident resolver computes them once per
+// phase changes, so the island kernel computes them once per
 // phase for every contact.  It keeps the inverse (9) and deltaVelocity's
 // entries 0, 3, 6 (the only ones the friction cone reads).
 template <typename R>
@@ -739,13 +763,12 @@ __device__ __forceinline__ void resolve_world(const RS<R>& a, int w, int C, int6
   }
 }
 
-constexpr int kRegBodies = 256;   // bodies per world for the register-resident kernel
-constexpr int kRegMaxSlots = 32;  // contacts per lane (64 * 32 = 2048 per world)
+// worlds the surrogate's polish takes; beyond them, the plain phases
+constexpr int kPolishBodies = 256;
+constexpr int kPolishContacts = 2048;
 
-__device__ __forceinline__ bool fits_registers(int C, int n) { return C <= 64 * kRegMaxSlots && n <= kRegBodies; }
-
-// HBM-resident path (worlds too large for the register kernel): selection
-// keys and body ids in LDS when the world has at most kKeyCap contacts.
+// One world on one wave, its state in HBM: selection keys and body ids in
+// LDS when the world has at most kKeyCap contacts.
 template <typename R, int KIND>
 __device__ __forceinline__ void resolve_hbm(const RS<R>& a, int w, int C, char* lds, int lane) {
   if (a.world_iters && lane == 0) {
@@ -766,28 +789,9 @@ __device__ __forceinline__ void resolve_hbm(const RS<R>& a, int w, int C, char* 
 }
 
 // ---------------------------------------------------------------------------
-// Register-resident resolver: worlds with at most 64*SLOTS contacts and
-// kRegBodies bodies.  Lane l holds contacts j = 64*s + l (s < SLOTS) in
-// VGPRs: the selection key, the body ids (world-local, packed 16+16 bits)
-// and, in the velocity phase, the contact velocity; the narrow classes
-// (SLOTS <= 8) also hold the normal and the point, and keep the contact
-// basis scale in LDS (contactToWorld is rebuilt from the normal and that
-// scale bit for bit), while the wide classes read the normal,
-// contactToWorld and relative positions as prepare stored them in HBM.
-//
-// LDS holds per body the position at prepare time (relativeContactPosition
-// = point - that position, recomputed bit for bit where the reference
-// stores it), lastFrameAccelleration * dt, the flag byte, and the state the
-// phase changes: position and orientation in the position phase, velocity
-// and rotation in the velocity phase, written back to HBM when the phase
-// ends.  So every value an iteration writes and a later one reads stays in
-// the wave's registers or LDS, whose operations a wave performs in program
-// order, and the serial loop needs no barrier; the selected contact's
-// register data reaches every lane by readlane.  HBM supplies the
-// read-only data: inverse masses, world inverse inertia (in the position
-// phase a sleeping body's new tensor goes to HBM, followed by a barrier),
-// the velocity phase's impulse data (written when the phase starts).
+// pieces of the island kernel (cbz_islands.h)
 // ---------------------------------------------------------------------------
+// A contact's body ids, world-local, packed 16 + 16 bits.
 constexpr uint32_t kNoBody = 0xFFFFu;
 
 // Kinetic energy of a body, 1/2 (m |v|^2 + w . I w) with I the inverse of
@@ -807,43 +811,6 @@ __device__ __forceinline__ double kinetic_energy(const V3<R>& v, const V3<R>& w,
   const V3<double> Iw = m3v(I, wd);
   const double vv = double(v.x) * double(v.x) + double(v.y) * double(v.y) + double(v.z) * double(v.z);
   return 0.5 * (mass * vv + dot(wd, Iw));
-}
-
-template <typename R>
-__device__ __forceinline__ V3<R> lds3(const R* a, int i) {
-  return V3<R>{a[i], a[kRegBodies + i], a[2 * kRegBodies + i]};
-}
-template <typename R>
-__device__ __forceinline__ void lds3_store(R* a, int i, const V3<R>& v) {
-  a[i] = v.x;
-  a[kRegBodies + i] = v.y;
-  a[2 * kRegBodies + i] = v.z;
-}
-
-// calculateDesiredDeltaVelocity (contact.go:87-112) with the awake flags and
-// lastFrameAccelleration*dt from LDS, for a contact of restitution e.
-template <typename R>
-__device__ __forceinline__ R desired_dv_lds(const uint8_t* fl, const R* lad, int l0, int l1, const V3<R>& n,
-                                            R cvx, R e) {
-  R vfa = R(0);
-  if (fl[l0] & F_AWAKE) vfa += dot(lds3(lad, l0), n);
-  if (l1 >= 0 && (fl[l1] & F_AWAKE)) vfa -= dot(lds3(lad, l1), n);
-  R restitution = e;
-  if (dabs(cvx) < R(0.25)) restitution = R(0);
-  return -cvx - restitution * (cvx - vfa);
-}
-
-// calculateLocalVelocity (contact.go:159-182) with lastFrameAccelleration*dt
-// from LDS.
-template <typename R>
-__device__ __forceinline__ V3<R> local_velocity_lds(const Bodies<R>& b, int body, const V3<R>& lad,
-                                                    const V3<R>& rel, const R* c2w) {
-  const int64_t S = b.stride;
-  V3<R> velocity = add(cross(ld3(b.rot, S, body), rel), ld3(b.vel, S, body));
-  V3<R> cv = m3tv(c2w, velocity);
-  V3<R> accv = m3tv(c2w, lad);
-  accv.x = R(0);
-  return add(cv, accv);
 }
 
 __device__ __forceinline__ int id_lo(uint32_t id) { return int(id & 0xFFFFu); }
@@ -909,20 +876,6 @@ __device__ __forceinline__ V3<R> sel3(bool c, const V3<R>& a, const V3<R>& b) {
 }
 
 
-template <typename R, int SLOTS, int KIND>
-struct RegLds {
-  // the wide classes keep only key, ids and contact velocity in VGPRs; the
-  // rest of a contact comes from HBM where an iteration needs it
-  static constexpr bool WIDE = SLOTS >= 12;
-  static constexpr int CAP = 64 * SLOTS;
-  static constexpr size_t pos0 = 0;                                   // R[3][kRegBodies]
-  static constexpr size_t lad = pos0 + 3 * kRegBodies * sizeof(R);    // R[3][kRegBodies]
-  static constexpr size_t st = lad + 3 * kRegBodies * sizeof(R);      // R[7][kRegBodies] pos+quat / vel+rot
-  static constexpr size_t bs = st + 7 * kRegBodies * sizeof(R);       // double[CAP] basis scale (narrow)
-  static constexpr size_t flags = bs + (WIDE ? 0 : CAP * sizeof(double));  // uint8[kRegBodies]
-  static constexpr size_t bytes = flags + kRegBodies;
-};
-
 // Both bodies' world inverse inertia and inverse mass (zeros for an absent
 // second body).
 template <typename R>
@@ -942,1873 +895,55 @@ __device__ __forceinline__ void body_inertia(const Bodies<R>& b, const int kb[2]
   }
 }
 
-// applyPositionChange (contact.go:286-386) with the bodies' position and
-// orientation in LDS (s_st: pos planes 0-2, quat planes 3-6, world-local
-// index kl).  Returns whether a sleeping body's derived data were rewritten
-// (in HBM).
-// The bodies' world inverse inertia iw and inverse masses im are loaded by
-// the caller (with the iteration's other loads, before any store).
+// Entry e of a left list: the world, and the phases it still needs.
 template <typename R>
-__device__ __forceinline__ bool apply_position_change_lds(const RS<R>& a, const int kb[2], const int kl[2],
-                                                          const bool aw[2], const V3<R>& n, const V3<R> rel[2],
-                                                          R penetration, const R (&iw)[2][9], const R im[2],
-                                                          V3<R> lin[2], V3<R> ang[2], R* s_st, int lane) {
-  const Bodies<R>& b = a.b;
-  constexpr int KB = kRegBodies;
-  const R angularLimit = R(0.2);
-  R angI[2] = {R(0), R(0)}, linI[2] = {R(0), R(0)};
-  R total = R(0);
-  bool rederived = false;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    lin[i] = V3<R>{R(0), R(0), R(0)};
-    ang[i] = V3<R>{R(0), R(0), R(0)};
-    if (kb[i] < 0) continue;
-    V3<R> aiw = cross(rel[i], n);
-    aiw = m3v(iw[i], aiw);
-    aiw = cross(aiw, rel[i]);
-    angI[i] = dot(aiw, n);
-    linI[i] = im[i];
-    total += linI[i] + angI[i];
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int bi = kb[i];
-    if (bi < 0) continue;
-    R sign = R(1);
-    if (i != 0) sign = R(-1);
-    R angM = sign * penetration * (angI[i] / total);
-    R linM = sign * penetration * (linI[i] / total);
-    V3<R> projection = add_scaled(rel[i], n, -dot(rel[i], n));
-    R maxMagnitude = angularLimit * mag(projection);
-    if (angM < -maxMagnitude) {
-      R totalMove = angM + linM;
-      angM = -maxMagnitude;
-      linM = totalMove - angM;
-    } else if (angM > maxMagnitude) {
-      R totalMove = angM + linM;
-      angM = maxMagnitude;
-      linM = totalMove - angM;
-    }
-    if (angM == R(0)) {
-      ang[i] = V3<R>{R(0), R(0), R(0)};
-    } else {
-      V3<R> tad = cross(rel[i], n);
-      ang[i] = mul(m3v(iw[i], tad), angM / angI[i]);
-    }
-    lin[i] = mul(n, linM);
-    const int l = kl[i];
-    V3<R> pos = add_scaled(lds3(s_st, l), n, linM);
-    Q4<R> q{s_st[3 * KB + l], s_st[4 * KB + l], s_st[5 * KB + l], s_st[6 * KB + l]};
-    q = q_add_scaled_vector(q, ang[i], R(1));
-    q = q_normalize(q);
-    if (!aw[i]) {
-      rederive(b, bi, pos, q, lane);
-      rederived = true;
-    }
-    if (lane == 0) {
-      lds3_store(s_st, l, pos);
-      s_st[3 * KB + l] = q.w;
-      s_st[4 * KB + l] = q.x;
-      s_st[5 * KB + l] = q.y;
-      s_st[6 * KB + l] = q.z;
-    }
-  }
-  return rederived;
+__device__ __forceinline__ int left_world(RS<R>& a, int32_t e) {
+  if (e & kLeftVelOnly) a.mode &= ~(RM_POS | RM_PREPARED);
+  return e & ~kLeftVelOnly;
 }
 
-// applyVelocityChange (contact.go:448-494) from the contact's impulse data,
-// with the bodies' velocity and rotation in LDS (s_st: vel planes 0-2, rot
-// planes 3-5, world-local index kl).
+// The worlds the island kernel leaves, a wave each.  The last workgroup to
+// finish clears the counters for the next resolve.
 template <typename R, int KIND>
-__device__ __forceinline__ void apply_velocity_change_lds(const int kb[2], const int kl[2], const V3<R> rel[2],
-                                                          const R* c2w, R ddv, const V3<R>& cvel, const R* imp,
-                                                          const R (&iw)[2][9], const R im[2], V3<R> vc[2],
-                                                          V3<R> rc[2], R* s_st, int lane, R friction) {
-  R* s_rot = s_st + 3 * kRegBodies;
-  V3<R> ic;
-  if (KIND == KIND_MAT && friction == R(0))
-    ic = V3<R>{ddv / imp[0], R(0), R(0)};
-  else
-    ic = friction_impulse_from(imp, imp + 9, ddv, cvel, friction);
-  const V3<R> impulse = m3v(c2w, ic);
-  const V3<R> zero{R(0), R(0), R(0)};
-  V3<R> torque = cross(rel[0], impulse);
-  rc[0] = m3v(iw[0], torque);
-  vc[0] = add_scaled(zero, impulse, im[0]);
-  rc[1] = zero;
-  vc[1] = zero;
-  const V3<R> v0 = add(lds3(s_st, kl[0]), vc[0]);
-  const V3<R> w0 = add(lds3(s_rot, kl[0]), rc[0]);
-  V3<R> v1 = zero, w1 = zero;
-  if (kb[1] >= 0) {
-    torque = cross(impulse, rel[1]);
-    rc[1] = m3v(iw[1], torque);
-    vc[1] = add_scaled(zero, impulse, -im[1]);
-    v1 = add(lds3(s_st, kl[1]), vc[1]);
-    w1 = add(lds3(s_rot, kl[1]), rc[1]);
+__device__ __forceinline__ void resolve_left_block(const RS<R>& args) {
+  __shared__ __align__(16) char lds[kKeyCap * (sizeof(R) + 2 * sizeof(int32_t))];
+  const int lane = threadIdx.x;
+  const int left = args.left_count[LEFT_WORLDS];
+  for (int k = blockIdx.x; k < left; k += gridDim.x) {
+    RS<R> a = args;
+    const int w = left_world(a, args.left_list[k]);
+    int64_t* wt = a.world_time ? a.world_time + 4 * int64_t(w) + ((a.mode & RM_VEL) ? 2 : 0) : nullptr;
+    if (wt && lane == 0) wt[0] = int64_t(wall_clock64());
+    resolve_hbm<R, KIND>(a, w, a.world_cnt[w], lds, lane);
+    __syncthreads();
+    if (wt && lane == 0) wt[1] = int64_t(wall_clock64());
   }
   if (lane == 0) {
-    lds3_store(s_st, kl[0], v0);
-    lds3_store(s_rot, kl[0], w0);
-    if (kb[1] >= 0) {
-      lds3_store(s_st, kl[1], v1);
-      lds3_store(s_rot, kl[1], w1);
+    __threadfence();
+    if (atomicAdd(&args.left_count[LEFT_DONE], 1) == int(gridDim.x) - 1) {
+      for (int q = 0; q < LEFT_COUNTS; ++q) args.left_count[q] = 0;
+      *args.log_head = 0;
     }
-  }
-}
-
-template <typename R, int SLOTS, int KIND>
-__device__ __forceinline__ void resolve_reg(const RS<R>& a, int w, int C, int b0w, int n, char* lds, int lane) {
-  using L = RegLds<R, SLOTS, KIND>;
-  constexpr bool WIDE = L::WIDE;
-  constexpr int KB = kRegBodies;
-  R* s_pos0 = (R*)(lds + L::pos0);
-  R* s_lad = (R*)(lds + L::lad);
-  R* s_st = (R*)(lds + L::st);
-  double* s_bs = (double*)(lds + L::bs);  // narrow classes only
-  uint8_t* s_flags = (uint8_t*)(lds + L::flags);
-  const bool do_pos = (a.mode & RM_POS) != 0;
-  const bool do_prep = do_pos && !(a.mode & RM_PREPARED);
-  const bool do_vel = (a.mode & RM_VEL) != 0 && (KIND == KIND_POLISH || !a.world_mask || a.world_mask[w]);
-  if (a.world_iters && lane == 0) {
-    if (do_pos) a.world_iters[2 * w] = 0;
-    if (a.mode & RM_VEL) a.world_iters[2 * w + 1] = 0;
-  }
-  // ResolveContacts' guard, contact.go:210-212
-  if (a.overflow[0] != 0 || C <= 0 || a.dt <= R(0)) return;
-  if (!do_pos && !do_vel) return;
-
-  const Bodies<R>& b = a.b;
-  const Contacts<R>& c = a.c;
-  const int64_t S = b.stride, CS = c.cap;
-  const int64_t base = a.world_coff[w];
-  const int64_t maxIter = a.iter_fixed > 0 ? a.iter_fixed : a.iter_mult * int64_t(C);
-  const V3<R> zero{R(0), R(0), R(0)};
-
-  for (int i = lane; i < n; i += 64) {
-    const int g = b0w + i;
-    // body positions at prepare time: the current ones when this launch
-    // prepares, else the snapshot the preparing launch stored
-    const V3<R> p = ld3(do_prep ? b.pos : a.pos0, S, g);
-    if (do_prep) st3(a.pos0, S, g, p);
-    lds3_store(s_pos0, i, p);
-    lds3_store(s_lad, i, mul(ld3(b.last_acc, S, g), a.dt));
-    s_flags[i] = b.flags[g];
-  }
-  __syncthreads();
-
-  R key[SLOTS];
-  uint32_t ids[SLOTS];
-  V3<R> nrm[WIDE ? 1 : SLOTS];
-  V3<R> ptr[WIDE ? 1 : SLOTS];
-
-  // prepareContacts / calculateInternals, contact.go:225-229, :59-85, over
-  // this lane's contacts (a rolled loop: the body is large), into the
-  // contact arrays
-  if (do_prep) {
-    for (int j = lane; j < C; j += 64) {
-      const int64_t g = base + j;
-      int c0 = c.body0[g], c1 = c.body1[g];
-      V3<R> nn = ld3(c.normal, CS, g);
-      if (c0 < 0) {  // contact.go:61-65
-        nn = mul(nn, R(-1));
-        c0 = c1;
-        c1 = -1;
-        c.body0[g] = c0;
-        c.body1[g] = c1;
-        st3(c.normal, CS, g, nn);
-      }
-      const int l0 = c0 - b0w, l1 = c1 >= 0 ? c1 - b0w : -1;
-      R m[9];
-      const double sc = basis_scale(nn);
-      basis_from_scale(nn, sc, m);
-      const V3<R> p = ld3(c.point, CS, g);
-      const V3<R> r0 = sub(p, lds3(s_pos0, l0));
-      V3<R> cv = local_velocity_lds(b, c0, lds3(s_lad, l0), r0, m);
-      V3<R> r1 = zero;
-      if (c1 >= 0) {
-        r1 = sub(p, lds3(s_pos0, l1));
-        cv = sub(cv, local_velocity_lds(b, c1, lds3(s_lad, l1), r1, m));
-      }
-      const R ddv = desired_dv_lds(s_flags, s_lad, l0, l1, nn, cv.x, restitution_of<R, KIND>(c, g));
-#pragma unroll
-      for (int k = 0; k < 9; ++k) c.c2w[k * CS + g] = m[k];
-      st3(c.rel, CS, g, r0);
-      st3(c.rel + 3 * CS, CS, g, r1);
-      st3(c.cvel, CS, g, cv);
-      c.ddv[g] = ddv;
-      if constexpr (WIDE) store_rec(c.rec + 16 * g, m, r0, r1);
-      if constexpr (!WIDE) s_bs[j] = sc;
-    }
-  } else if constexpr (!WIDE) {  // prepared by an earlier launch: the basis scales of prepare's normals
-    for (int j = lane; j < C; j += 64) s_bs[j] = basis_scale(ld3(c.normal, CS, base + j));
-  }
-  // this lane's contacts into registers (the lane wrote what it reads here)
-#pragma unroll
-  for (int s = 0; s < SLOTS; ++s) {
-    const int j = 64 * s + lane;
-    key[s] = R(0);
-    ids[s] = 0xFFFFFFFFu;
-    if constexpr (!WIDE) nrm[s] = ptr[s] = zero;
-    if (j < C) {
-      const int64_t g = base + j;
-      const int c0 = c.body0[g], c1 = c.body1[g];
-      ids[s] = uint32_t(c0 - b0w) | (uint32_t(c1 >= 0 ? c1 - b0w : int(kNoBody)) << 16);
-      if (do_pos) key[s] = c.pen[g];
-      if constexpr (!WIDE) {
-        nrm[s] = ld3(c.normal, CS, g);
-        ptr[s] = ld3(c.point, CS, g);
-      }
-    }
-  }
-  // the position phase's body state into LDS; the wide classes read what
-  // prepare stored in HBM below
-  if (do_pos) {
-    for (int i = lane; i < n; i += 64) {
-      const int g = b0w + i;
-      lds3_store(s_st, i, ld3(b.pos, S, g));
-#pragma unroll
-      for (int k = 0; k < 4; ++k) s_st[(3 + k) * KB + i] = b.quat[k * S + g];
-    }
-  }
-  __syncthreads();
-
-  // The surrogate's position polish (KIND_PPOLISH, worlds whose mask byte
-  // is 0): snapshot what the loop may write to HBM for the bodies
-  // asleep now (the motion matchAwakeState sets, the derived data a
-  // sleeping body's move recomputes), add the predicted changes to the
-  // awake bodies' positions and orientations, update every contact's
-  // penetration for them by the loop's own formula, then run the loop to
-  // positionEpsilon + polish_tol within polish_mult * C iterations.
-  bool ppolish = false;
-  R sep_floor = R(0);  // the polished world's least penetration the acceptance test allows
-  // the world's least penetration (every lane gets it)
-  auto key_min = [&]() {
-    R kmin = R(0);
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s)
-      if (64 * s + lane < C) kmin = key[s] < kmin ? key[s] : kmin;
-    return dpp::allreduce(kmin, R(0), [](R x, R y) { return y < x ? y : x; });
-  };
-  // Undo a rejected position polish: positions, orientations and awake
-  // flags from HBM (untouched until the phase ends), the sleeping bodies'
-  // motion and derived data from the snapshot, the penetrations from the
-  // contact array; then the plain phase runs.
-  auto restore_positions = [&]() {
-    // lane 0's HBM stores of the loop (motion, a sleeping body's derived
-    // data) complete before the other lanes restore over them
-    __syncthreads();
-    for (int i = lane; i < n; i += 64) {
-      const int g = b0w + i;
-      lds3_store(s_st, i, ld3(b.pos, S, g));
-#pragma unroll
-      for (int k = 0; k < 4; ++k) s_st[(3 + k) * KB + i] = b.quat[k * S + g];
-      const uint8_t f = b.flags[g];
-      s_flags[i] = f;
-      if (!(f & F_AWAKE)) {
-        b.motion[g] = a.vel0[g];
-#pragma unroll
-        for (int k = 0; k < 12; ++k) b.transform[k * S + g] = a.vel0[(1 + k) * S + g];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) b.iit_world[k * S + g] = a.vel0[(13 + k) * S + g];
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) {
-      const int j = 64 * s + lane;
-      key[s] = j < C ? c.pen[base + j] : R(0);
-    }
-    __syncthreads();
-    if (lane == 0) a.world_mask[w] = 1;
-  };
-  if constexpr (KIND == KIND_PPOLISH) {
-    ppolish = do_pos && a.world_mask[w] == 0;
-    if (ppolish) {
-      R pmax = R(0);
-#pragma unroll
-      for (int s = 0; s < SLOTS; ++s) pmax = key[s] > pmax ? key[s] : pmax;
-      pmax = dpp::allreduce(pmax, R(0), [](R x, R y) { return y > x ? y : x; });
-      sep_floor = -(R(kSepFactor) * pmax + a.polish_tol);
-      const float* dl = a.delta;
-      for (int i = lane; i < n; i += 64) {
-        const int g = b0w + i;
-        if (!(s_flags[i] & F_AWAKE)) {
-          a.vel0[g] = b.motion[g];
-#pragma unroll
-          for (int k = 0; k < 12; ++k) a.vel0[(1 + k) * S + g] = b.transform[k * S + g];
-#pragma unroll
-          for (int k = 0; k < 9; ++k) a.vel0[(13 + k) * S + g] = b.iit_world[k * S + g];
-        }
-      }
-      // the predicted moves times `scale`, from the phase's starting state
-      // (positions and orientations in HBM, penetrations in the contact
-      // array): the awake bodies' state, then every contact's penetration
-      // by the loop's own formula
-      auto take_moves = [&](R scale) {
-        for (int i = lane; i < n; i += 64) {
-          const int g = b0w + i;
-          if (!(s_flags[i] & F_AWAKE)) continue;
-          const V3<R> dx = mul(V3<R>{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])}, scale);
-          const V3<R> dq = mul(V3<R>{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])}, scale);
-          if (dx.x == R(0) && dx.y == R(0) && dx.z == R(0) && dq.x == R(0) && dq.y == R(0) && dq.z == R(0)) continue;
-          lds3_store(s_st, i, add(ld3(b.pos, S, g), dx));
-          Q4<R> q{b.quat[g], b.quat[S + g], b.quat[2 * S + g], b.quat[3 * S + g]};
-          q = q_normalize(q_add_scaled_vector(q, dq, R(1)));
-          s_st[3 * KB + i] = q.w;
-          s_st[4 * KB + i] = q.x;
-          s_st[5 * KB + i] = q.y;
-          s_st[6 * KB + i] = q.z;
-        }
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s) {
-          asm volatile("" ::: "memory");
-          if (64 * s + lane >= C) continue;
-          const int64_t gj = base + 64 * s + lane;
-          const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-          V3<R> nj;
-          if constexpr (WIDE)
-            nj = ld3(c.normal, CS, gj);
-          else
-            nj = nrm[s];
-          R pen = c.pen[gj];
-#pragma unroll
-          for (int bb = 0; bb < 2; ++bb) {
-            if (jb[bb] < 0) continue;
-            const int g = b0w + jb[bb];
-            const V3<R> dx = mul(V3<R>{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])}, scale);
-            const V3<R> dq = mul(V3<R>{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])}, scale);
-            if (dx.x == R(0) && dx.y == R(0) && dx.z == R(0) && dq.x == R(0) && dq.y == R(0) && dq.z == R(0)) continue;
-            V3<R> rj;
-            if constexpr (WIDE)
-              rj = ld3(c.rel + 3 * bb * CS, CS, gj);
-            else
-              rj = sub(ptr[s], lds3(s_pos0, jb[bb]));
-            const V3<R> dp = add(cross(dq, rj), dx);
-            R sign = R(1);
-            if (bb == 0) sign = R(-1);
-            pen += dot(dp, nj) * sign;
-          }
-          key[s] = pen;
-        }
-        __syncthreads();
-      };
-      // a prediction that separates a contact beyond the bound is retried
-      // at a fraction of its moves, then rejected, before the loop spends
-      // iterations on it
-      take_moves(R(1));
-      if (!(key_min() >= sep_floor)) {
-        take_moves(R(kPosRetryScale));
-        if (!(key_min() >= sep_floor)) {
-          restore_positions();
-          ppolish = false;
-        }
-      }
-    }
-  }
-
-  // adjustPositions, contact.go:233-283
-  R peps = ppolish ? R(kPositionEpsilon) + a.polish_tol : R(kPositionEpsilon);
-  int64_t pbudget = ppolish ? a.polish_mult * int64_t(C) : maxIter;
-  int64_t used = 0;
-  // A slot past the world's contacts keeps key 0 (never above the epsilon)
-  // and ids 0xFFFFFFFF (never a body of the world), so the loops below need
-  // no bounds test.
-  while (do_pos) {
-    opaque_ids(ids);
-    R best = peps;
-    int bi = INT_MAX;
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) {
-      if (key[s] > best) {
-        best = key[s];
-        bi = 64 * s + lane;
-      }
-    }
-    wave_argmax_dpp(best, bi);
-    bool reject = false;  // the position polish did not give an acceptable result
-    if (bi == INT_MAX) {
-      if constexpr (KIND == KIND_PPOLISH) {
-        // Every contact is within positionEpsilon + tol.  The plain phase
-        // moves bodies only to resolve penetration; a polished world in
-        // which a contact ends separated by more than kSepFactor times the
-        // world's deepest penetration at the start (+ tol) is rejected: that
-        // is the mark of a prediction that pushed bodies apart.
-        if (ppolish) reject = !(key_min() >= sep_floor);
-      }
-      if (!reject) break;
-    } else if (used >= pbudget) {
-      if (KIND != KIND_PPOLISH || !ppolish) break;
-      reject = true;
-    }
-    if constexpr (KIND == KIND_PPOLISH) {
-      if (reject) {
-        restore_positions();
-        ppolish = false;
-        peps = R(kPositionEpsilon);
-        pbudget = maxIter;
-        used = 0;
-        continue;
-      }
-    }
-    if (bi == INT_MAX || used >= pbudget) break;
-    const int ss = bi >> 6, sl = bi & 63;
-    const uint32_t kid = lane_value(pick(ids, ss), sl);
-    const int kl[2] = {id_lo(kid), id_hi(kid)};
-    const int kb[2] = {b0w + kl[0], kl[1] >= 0 ? b0w + kl[1] : -1};
-    V3<R> n, rel[2];
-    if constexpr (WIDE) {
-      rec_normal(c.rec + 16 * (base + bi), n, rel);
-    } else {
-      n = lane_value(pick(nrm, ss), sl);
-      const V3<R> p = lane_value(pick(ptr, ss), sl);
-      rel[0] = sub(p, lds3(s_pos0, kl[0]));
-      rel[1] = kl[1] >= 0 ? sub(p, lds3(s_pos0, kl[1])) : zero;
-    }
-    // both bodies' inertia, loaded before this iteration's first store
-    R iw[2][9], im[2];
-    body_inertia(b, kb, iw, im);
-    // matchAwakeState, contact.go:185-202
-    bool aw[2] = {(s_flags[kl[0]] & F_AWAKE) != 0, kl[1] >= 0 && (s_flags[kl[1]] & F_AWAKE) != 0};
-    if (kl[1] >= 0 && (aw[0] || aw[1]) && !(aw[0] && aw[1])) {
-      const int t = aw[0] ? kl[1] : kl[0];
-      if (lane == 0) {
-        s_flags[t] = uint8_t(s_flags[t] | F_AWAKE);
-        b.motion[b0w + t] = R(kSleepEpsilon * 2.0);
-      }
-      aw[0] = aw[1] = true;
-    }
-    V3<R> lin[2], ang[2];
-    const bool rederived = apply_position_change_lds(a, kb, kl, aw, n, rel, best, iw, im, lin, ang, s_st, lane);
-    if constexpr (KIND == KIND_LABEL)
-      if (lane == 0) add_pos_label(a, base + bi, best);
-    const int ln = opaque_lane(lane);
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) {
-      const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-      bool any = false;
-#pragma unroll
-      for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-        for (int d = 0; d < 2; ++d) any |= (jb[bb] >= 0 && jb[bb] == kl[d]);
-      if (!any) continue;
-      const int64_t gj = base + 64 * s + ln;
-      R pen = key[s];
-      V3<R> nj, rw[2];
-      if constexpr (WIDE)
-        rec_normal(c.rec + 16 * gj, nj, rw);
-      else
-        nj = nrm[s];
-#pragma unroll
-      for (int bb = 0; bb < 2; ++bb) {
-        if (jb[bb] < 0) continue;
-        V3<R> rj;
-        if constexpr (WIDE)
-          rj = rw[bb];
-        else
-          rj = sub(ptr[s], lds3(s_pos0, jb[bb]));
-        // a side is at most one of the two moved bodies: its change is
-        // selected and applied once
-        if (jb[bb] == kl[0] || jb[bb] == kl[1]) {
-          const bool d0 = jb[bb] == kl[0];
-          V3<R> dp = add(cross(sel3(d0, ang[0], ang[1]), rj), sel3(d0, lin[0], lin[1]));
-          R sign = R(1);
-          if (bb == 0) sign = R(-1);
-          pen += dot(dp, nj) * sign;
-        }
-      }
-      key[s] = pen;
-    }
-    // a sleeping body's new world inverse inertia went to HBM; the next
-    // iteration may read it
-    if (rederived) __syncthreads();
-    ++used;
-  }
-  const int64_t pos_iters = used;
-  if (do_pos) {
-    for (int i = lane; i < n; i += 64) {
-      const int g = b0w + i;
-      st3(b.pos, S, g, lds3(s_st, i));
-#pragma unroll
-      for (int k = 0; k < 4; ++k) b.quat[k * S + g] = s_st[(3 + k) * KB + i];
-    }
-  }
-
-  // adjustVelocities, contact.go:390-445.  The bodies' velocity and
-  // rotation live in LDS for the whole phase; the contact velocities in
-  // VGPRs where they fit, else in the contact array, where each slot is
-  // read and written only by the lane that owns it (the selected one reaches
-  // the other lanes by readlane).
-  constexpr bool CV_REG = SLOTS * sizeof(R) <= 64;
-  R* s_rot = s_st + 3 * KB;
-  V3<R> cvr[CV_REG ? SLOTS : 1];
-  // slot s of this lane, contact g = base + 64 s + lane
-  auto cv_get = [&](int s, int64_t g) -> V3<R> {
-    if constexpr (CV_REG)
-      return cvr[s];
-    else
-      return ld3(c.cvel, CS, g);
-  };
-  auto cv_set = [&](int s, int64_t g, const V3<R>& v) {
-    if constexpr (CV_REG)
-      cvr[s] = v;
-    else
-      st3(c.cvel, CS, g, v);
-  };
-#pragma unroll
-  for (int s = 0; s < SLOTS; ++s) {
-    const int j = 64 * s + lane;
-    if constexpr (CV_REG) cvr[s] = zero;
-    if (do_pos && j < C) c.pen[base + j] = key[s];
-    if (do_vel && j < C) {
-      key[s] = c.ddv[base + j];  // selection keys as prepare stored them
-      if constexpr (CV_REG) cvr[s] = ld3(c.cvel, CS, base + j);
-    }
-  }
-  // every contact's impulse data, fixed for the whole phase, from the
-  // contactToWorld and relative positions prepare stored (this lane's own
-  // contacts)
-  if (do_vel) {
-    for (int j = lane; j < C; j += 64) {
-      const int64_t g = base + j;
-      const int jb[2] = {c.body0[g], c.body1[g]};
-      R mj[9], imp[kImpPlanes];
-      V3<R> rj[2];
-      if constexpr (WIDE) {
-        rec_frame(c.rec + 16 * g, mj, rj);
-      } else {
-#pragma unroll
-        for (int k = 0; k < 9; ++k) mj[k] = c.c2w[k * CS + g];
-        rj[0] = ld3(c.rel, CS, g);
-        rj[1] = ld3(c.rel + 3 * CS, CS, g);
-      }
-      impulse_data<R, KIND>(a, jb, rj, mj, friction_of<R, KIND>(c, g), imp);
-#pragma unroll
-      for (int k = 0; k < kImpPlanes; ++k) c.imp[k * CS + g] = imp[k];
-    }
-  }
-  // the impulse data every lane reads below, and LDS reuse
-  __syncthreads();
-  used = 0;
-  if (do_vel) {
-    for (int i = lane; i < n; i += 64) {
-      const int g = b0w + i;
-      lds3_store(s_st, i, ld3(b.vel, S, g));
-      lds3_store(s_rot, i, ld3(b.rot, S, g));
-    }
-    bool polishing = KIND == KIND_POLISH && a.world_mask[w] == 0;
-    double ke_before = 0.0, world_mass = 0.0;
-    if constexpr (KIND == KIND_POLISH) {
-      if (polishing) {
-        // take the predicted changes: snapshot the motion (matchAwakeState
-        // writes it in HBM; velocity and rotation stay in HBM untouched
-        // until the phase ends), then add the changes to the bodies
-        const float* dl = a.delta;
-        if constexpr (!CV_REG)
-          for (int j = lane; j < C; j += 64) st3(a.cvel0, CS, base + j, ld3(c.cvel, CS, base + j));
-        double ke = 0.0, mass = 0.0;
-        for (int i = lane; i < n; i += 64) {
-          const int g = b0w + i;
-          const V3<R> v = lds3(s_st, i), r = lds3(s_rot, i);
-          R iw[9];
-          ld9(b.iit_world, S, g, iw);
-          double mi;
-          ke += kinetic_energy(v, r, b.inv_mass[g], iw, mi);
-          mass += mi;
-          a.vel0[6 * S + g] = b.motion[g];
-          const V3<R> dv{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])};
-          const V3<R> dw{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])};
-          if (dv.x != R(0) || dv.y != R(0) || dv.z != R(0) || dw.x != R(0) || dw.y != R(0) || dw.z != R(0)) {
-            lds3_store(s_st, i, add(v, dv));
-            lds3_store(s_rot, i, add(r, dw));
-          }
-        }
-        // contact velocities after those changes: the update of
-        // contact.go:424-441 applied to each body's summed change (a
-        // compiler fence per slot keeps the slots' loads from being
-        // interleaved, which would need registers for all of them)
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s) {
-          asm volatile("" ::: "memory");
-          if (64 * s + lane >= C) continue;
-          const int64_t gj = base + 64 * s + lane;
-          const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-          R mj[9];
-          V3<R> rw[2];
-          if constexpr (WIDE) {
-            rec_frame(c.rec + 16 * gj, mj, rw);
-          } else {
-            basis_from_scale(nrm[s], s_bs[64 * s + lane], mj);
-          }
-          V3<R> cvj = cv_get(s, gj);
-          bool moved = false;
-#pragma unroll
-          for (int bb = 0; bb < 2; ++bb) {
-            if (jb[bb] < 0) continue;
-            const int g = b0w + jb[bb];
-            const V3<R> dv{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])};
-            const V3<R> dw{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])};
-            if (dv.x == R(0) && dv.y == R(0) && dv.z == R(0) && dw.x == R(0) && dw.y == R(0) && dw.z == R(0)) continue;
-            moved = true;
-            V3<R> rj;
-            if constexpr (WIDE)
-              rj = rw[bb];
-            else
-              rj = sub(ptr[s], lds3(s_pos0, jb[bb]));
-            R sign = R(1);
-            if (bb == 1) sign = R(-1);
-            cvj = add(cvj, mul(m3tv(mj, add(cross(dw, rj), dv)), sign));
-          }
-          // a contact neither of whose bodies changed keeps the key prepare
-          // gave it, as in the plain loop
-          if (moved) {
-            cv_set(s, gj, cvj);
-            key[s] = desired_dv_lds(s_flags, s_lad, jb[0], jb[1], V3<R>{mj[0], mj[1], mj[2]}, cvj.x,
-                                    restitution_of<R, KIND>(c, gj));
-          }
-        }
-        ke_before = wave_sum_f64(ke);
-        world_mass = wave_sum_f64(mass);
-      }
-    }
-    // The reference's loop.  A polished world first runs it to
-    // velocityEpsilon + polish_tol within polish_mult * C iterations; if that
-    // does not get there, everything the prediction and the loop changed is
-    // undone and the same loop runs as the plain phase.
-    R eps = polishing ? R(kVelocityEpsilon) + a.polish_tol : R(kVelocityEpsilon);
-    int64_t budget = polishing ? a.polish_mult * int64_t(C) : maxIter;
-    int64_t it = 0;
-    while (true) {
-      opaque_ids(ids);
-      R best = eps;
-      int bi = INT_MAX;
-#pragma unroll
-      for (int s = 0; s < SLOTS; ++s) {
-        if (key[s] > best) {
-          best = key[s];
-          bi = 64 * s + lane;
-        }
-      }
-      wave_argmax_dpp(best, bi);
-      bool reject = false;  // the polish did not give an acceptable result
-      if (bi == INT_MAX) {
-        if constexpr (KIND == KIND_POLISH) {
-          // Every contact is within velocityEpsilon + tol of closing.  The
-          // plain phase applies only compressive impulses inside the
-          // friction cone with restitution below 1, so it never adds kinetic
-          // energy; a polished world that ends with more than it started
-          // with, beyond a slack of 1/2 tol^2 per kilogram (which also covers
-          // the acceleration term of the restitution target,
-          // contact.go:87-112), is rejected.  This is what stops a wrong
-          // prediction from pushing bodies apart.
-          if (polishing) {
-            double ke = 0.0, mass = 0.0;
-            for (int i = lane; i < n; i += 64) {
-              const int g = b0w + i;
-              R iw[9];
-              ld9(b.iit_world, S, g, iw);
-              ke += kinetic_energy(lds3(s_st, i), lds3(s_rot, i), b.inv_mass[g], iw, mass);
-            }
-            const double ke_after = wave_sum_f64(ke);
-            const double tol = double(a.polish_tol);
-            reject = !(ke_after <= ke_before * (1.0 + kEnergyRel) + 0.5 * tol * tol * world_mass);
-          }
-        }
-        if (!reject) break;
-      } else if (it >= budget) {
-        if (KIND != KIND_POLISH || !polishing) break;
-        reject = true;
-      }
-      if (reject) {
-        // lane 0's motion stores of the loop complete before other lanes
-        // restore the snapshot over them
-        __syncthreads();
-        for (int i = lane; i < n; i += 64) {
-          const int g = b0w + i;
-          lds3_store(s_st, i, ld3(b.vel, S, g));
-          lds3_store(s_rot, i, ld3(b.rot, S, g));
-          b.motion[g] = a.vel0[6 * S + g];
-          s_flags[i] = b.flags[g];
-        }
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s) {
-          const int j = 64 * s + lane;
-          if (j < C) {
-            key[s] = c.ddv[base + j];
-            cv_set(s, base + j, ld3(CV_REG ? c.cvel : a.cvel0, CS, base + j));
-          }
-        }
-        __syncthreads();
-        if (lane == 0) a.world_mask[w] = 1;
-        polishing = false;
-        eps = R(kVelocityEpsilon);
-        budget = maxIter;
-        it = 0;
-        continue;
-      }
-      const int ss = bi >> 6, sl = bi & 63;
-      const uint32_t kid = lane_value(pick(ids, ss), sl);
-      V3<R> cvk;
-      if constexpr (CV_REG) {
-        cvk = lane_value(pick(cvr, ss), sl);
-      } else {  // the owner lane's own slot
-        const int jo = 64 * ss + lane;
-        cvk = lane_value(jo < C ? ld3(c.cvel, CS, base + jo) : zero, sl);
-      }
-      const int kl[2] = {id_lo(kid), id_hi(kid)};
-      const int kb[2] = {b0w + kl[0], kl[1] >= 0 ? b0w + kl[1] : -1};
-      R m[9], imp[kImpPlanes];
-      V3<R> rel[2];
-      if constexpr (WIDE) {
-        rec_frame(c.rec + 16 * (base + bi), m, rel);
-      } else {
-        const V3<R> n = lane_value(pick(nrm, ss), sl);
-        const V3<R> p = lane_value(pick(ptr, ss), sl);
-        basis_from_scale(n, s_bs[bi], m);
-        rel[0] = sub(p, lds3(s_pos0, kl[0]));
-        rel[1] = kl[1] >= 0 ? sub(p, lds3(s_pos0, kl[1])) : zero;
-      }
-#pragma unroll
-      for (int k = 0; k < kImpPlanes; ++k) imp[k] = c.imp[k * CS + base + bi];
-      // both bodies' inertia, loaded with the impulse data before this
-      // iteration's first store
-      R iw[2][9], im[2];
-      body_inertia(b, kb, iw, im);
-      // matchAwakeState, contact.go:185-202
-      const bool aw0 = (s_flags[kl[0]] & F_AWAKE) != 0;
-      const bool aw1 = kl[1] >= 0 && (s_flags[kl[1]] & F_AWAKE) != 0;
-      if (kl[1] >= 0 && (aw0 || aw1) && !(aw0 && aw1)) {
-        const int t = aw0 ? kl[1] : kl[0];
-        if (lane == 0) {
-          s_flags[t] = uint8_t(s_flags[t] | F_AWAKE);
-          b.motion[b0w + t] = R(kSleepEpsilon * 2.0);
-        }
-      }
-      V3<R> vc[2], rc[2];
-      apply_velocity_change_lds<R, KIND>(kb, kl, rel, m, best, cvk, imp, iw, im, vc, rc, s_st, lane,
-                                         friction_of<R, KIND>(c, base + bi));
-      if constexpr (KIND == KIND_LABEL)
-        if (lane == 0) add_label(a, base + bi, vc, rc);
-      const int ln = opaque_lane(lane);
-#pragma unroll
-      for (int s = 0; s < SLOTS; ++s) {
-        const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-        bool any = false;
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-          for (int d = 0; d < 2; ++d) any |= (jb[bb] >= 0 && jb[bb] == kl[d]);
-        if (!any) continue;
-        const int64_t gj = base + 64 * s + ln;
-        R mj[9];
-        V3<R> rw[2];
-        if constexpr (WIDE) {
-          rec_frame(c.rec + 16 * gj, mj, rw);
-        } else {
-          basis_from_scale(nrm[s], s_bs[64 * s + lane], mj);
-        }
-        V3<R> cvj = cv_get(s, gj);
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb) {
-          if (jb[bb] < 0) continue;
-          V3<R> rj;
-          if constexpr (WIDE)
-            rj = rw[bb];
-          else
-            rj = sub(ptr[s], lds3(s_pos0, jb[bb]));
-          // a side is at most one of the two moved bodies: its change is
-          // selected and applied once
-          if (jb[bb] == kl[0] || jb[bb] == kl[1]) {
-            const bool d0 = jb[bb] == kl[0];
-            V3<R> dv = add(cross(sel3(d0, rc[0], rc[1]), rj), sel3(d0, vc[0], vc[1]));
-            R sign = R(1);
-            if (bb == 1) sign = R(-1);
-            cvj = add(cvj, mul(m3tv(mj, dv), sign));
-          }
-        }
-        cv_set(s, gj, cvj);
-        key[s] = desired_dv_lds(s_flags, s_lad, jb[0], jb[1], V3<R>{mj[0], mj[1], mj[2]}, cvj.x,
-                                restitution_of<R, KIND>(c, gj));
-      }
-      ++it;
-      ++used;
-    }
-#pragma unroll
-    for (int s = 0; s < SLOTS; ++s) {
-      const int j = 64 * s + lane;
-      if (j < C) {
-        c.ddv[base + j] = key[s];
-        if constexpr (CV_REG) st3(c.cvel, CS, base + j, cvr[s]);
-      }
-    }
-    for (int i = lane; i < n; i += 64) {
-      const int g = b0w + i;
-      st3(b.vel, S, g, lds3(s_st, i));
-      st3(b.rot, S, g, lds3(s_rot, i));
-    }
-  }
-  for (int i = lane; i < n; i += 64) b.flags[b0w + i] = s_flags[i];
-  if (lane == 0 && a.world_iters) {
-    if (do_pos) a.world_iters[2 * w] = pos_iters;
-    if (do_vel) a.world_iters[2 * w + 1] = used;
-  }
-}
-
-// ----------------------------------------------------------------------
-// The largest worlds: one workgroup of kMwWaves wavefronts per world.
-//
-// In a world of many hundred contacts, an iteration of the one-wave kernel
-// scans up to 32 contacts per lane and reads the selected contact's impulse
-// data, the bodies' inertia and the contact velocities from HBM: a chain
-// of dependent memory round trips.  Here thread t (of kMwThreads, one wave
-// per SIMD) holds contacts j = t + kMwThreads * s (s < SL, SL = 4 or 8):
-// their selection keys, body ids, basis scales, contact velocities and
-// impulse data in registers; their normals and points are in LDS by
-// contact, beside the bodies' state, world inverse inertia, inverse mass
-// and flags.  An iteration:
-//   1. each wave takes its best contact (larger key; equal keys -> lower
-//      index) by DPP, and the lane that holds it offers its register data
-//      in LDS;                                              barrier A
-//   2. wave 0 alone takes the best of the offers, computes the correction
-//      and stores the bodies' new state (lane 0; wave 0 is the only reader
-//      of that state), then publishes the two bodies' changes; barrier C
-//   3. every thread updates its own contacts that share one of the bodies.
-// The arithmetic, its order and the selection are those of resolve_reg, so
-// both give the same bits.
-constexpr int kMwWaves = 4;
-constexpr int kMwThreads = 64 * kMwWaves;
-constexpr int kMwMaxSlots = 8;
-constexpr int kMwMaxContacts = kMwThreads * kMwMaxSlots;  // 2048
-// per-wave offer: contact velocity 3, impulse data 12, friction 1
-constexpr int kMwPay = 16;
-// wave 0's result: state, packed body ids, woken body
-enum : int { MW_APPLY = 0, MW_DONE = 1, MW_BUDGET = 2 };
-
-// A world the multi-wave kernel can take (the selection then keeps the
-// largest of these).
-__device__ __forceinline__ bool mw_fits(int C, int n, int mw_min) {
-  return mw_min > 0 && C >= mw_min && C <= kMwMaxContacts && n <= kRegBodies;
-}
-
-constexpr size_t up8(size_t x) { return (x + 7) & ~size_t(7); }
-
-template <typename R>
-struct MwLds {
-  static constexpr size_t pos0 = 0;                                   // R[3][kRegBodies]
-  static constexpr size_t lad = pos0 + 3 * kRegBodies * sizeof(R);    // R[3][kRegBodies]
-  static constexpr size_t st = lad + 3 * kRegBodies * sizeof(R);      // R[7][kRegBodies]
-  static constexpr size_t iit = st + 7 * kRegBodies * sizeof(R);      // R[9][kRegBodies]
-  static constexpr size_t im = iit + 9 * kRegBodies * sizeof(R);      // R[kRegBodies]
-  static constexpr size_t cn = im + kRegBodies * sizeof(R);           // R[3][kMwMaxContacts] normals
-  static constexpr size_t cp = cn + 3 * kMwMaxContacts * sizeof(R);   // R[3][kMwMaxContacts] points
-  static constexpr size_t pbs = up8(cp + 3 * kMwMaxContacts * sizeof(R));  // double[kMwWaves] offered basis scale
-  static constexpr size_t sum = pbs + kMwWaves * sizeof(double);      // double[kMwWaves]
-  static constexpr size_t pay = sum + kMwWaves * sizeof(double);      // R[kMwWaves][kMwPay]
-  static constexpr size_t res = up8(pay + kMwWaves * kMwPay * sizeof(R));  // R[12] wave 0's result
-  static constexpr size_t pkey = up8(res + 12 * sizeof(R));           // R[kMwWaves]
-  static constexpr size_t pidx = up8(pkey + kMwWaves * sizeof(R));    // int32[kMwWaves]
-  static constexpr size_t pkid = pidx + kMwWaves * sizeof(int32_t);   // uint32[kMwWaves]
-  static constexpr size_t resi = pkid + kMwWaves * sizeof(uint32_t);  // int32[4] state, ids, woken body
-  static constexpr size_t flags = resi + 4 * sizeof(int32_t);         // uint8[kRegBodies]
-  static constexpr size_t bytes = flags + kRegBodies;
-};
-
-// The largest (MAX) or least value over the workgroup; every thread gets it.
-template <bool MAX>
-__device__ __forceinline__ double mw_extreme(double v, double* s_sum, int t) {
-  v = dpp::allreduce(v, MAX ? -__builtin_inf() : __builtin_inf(),
-                     [](double x, double y) { return MAX ? (y > x ? y : x) : (y < x ? y : x); });
-  if ((t & 63) == 0) s_sum[t >> 6] = v;
-  __syncthreads();
-  double r = s_sum[0];
-#pragma unroll
-  for (int k = 1; k < kMwWaves; ++k) r = MAX ? (s_sum[k] > r ? s_sum[k] : r) : (s_sum[k] < r ? s_sum[k] : r);
-  __syncthreads();
-  return r;
-}
-
-// Sum over the workgroup in a fixed order (each wave's butterfly, then the
-// waves in index order); every thread gets the result.
-__device__ __forceinline__ double mw_sum(double v, double* s_sum, int t) {
-  v = wave_sum_f64(v);
-  if ((t & 63) == 0) s_sum[t >> 6] = v;
-  __syncthreads();
-  double r = 0.0;
-#pragma unroll
-  for (int k = 0; k < kMwWaves; ++k) r += s_sum[k];
-  __syncthreads();
-  return r;
-}
-
-// The best of the waves' offers (larger key; equal keys -> lower index);
-// gw = -1 when no wave offered a contact.
-template <typename R>
-__device__ __forceinline__ int mw_best(const R* s_pkey, const int32_t* s_pidx, R& key, int& idx) {
-  int gw = -1;
-#pragma unroll
-  for (int v = 0; v < kMwWaves; ++v) {
-    const int i = s_pidx[v];
-    if (i == INT_MAX) continue;
-    const R k = s_pkey[v];
-    if (k > key || (k == key && i < idx)) {
-      key = k;
-      idx = i;
-      gw = v;
-    }
-  }
-  return gw;
-}
-
-// applyPositionChange (contact.go:286-386) as apply_position_change_lds,
-// from the LDS tables, storing nothing: the bodies' new position and
-// orientation come back in np/nq.  Bit i of the result is set when body i
-// sleeps (its derived data are rewritten from np/nq, whose orientation has
-// then been normalised a second time, as CalculateDerivedData does).
-template <typename R>
-__device__ __forceinline__ int position_change_mw(const int kl[2], const bool aw[2], const V3<R>& n,
-                                                  const V3<R> rel[2], R penetration, V3<R> lin[2], V3<R> ang[2],
-                                                  V3<R> np[2], Q4<R> nq[2], const R* s_st, const R* s_iit,
-                                                  const R* s_im) {
-  constexpr int KB = kRegBodies;
-  const R angularLimit = R(0.2);
-  R angI[2] = {R(0), R(0)}, linI[2] = {R(0), R(0)};
-  R total = R(0);
-  int sleeping = 0;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    lin[i] = V3<R>{R(0), R(0), R(0)};
-    ang[i] = V3<R>{R(0), R(0), R(0)};
-    np[i] = V3<R>{R(0), R(0), R(0)};
-    nq[i] = Q4<R>{R(1), R(0), R(0), R(0)};
-    if (kl[i] < 0) continue;
-    R iw[9];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) iw[k] = s_iit[k * KB + kl[i]];
-    V3<R> aiw = cross(rel[i], n);
-    aiw = m3v(iw, aiw);
-    aiw = cross(aiw, rel[i]);
-    angI[i] = dot(aiw, n);
-    linI[i] = s_im[kl[i]];
-    total += linI[i] + angI[i];
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int l = kl[i];
-    if (l < 0) continue;
-    R sign = R(1);
-    if (i != 0) sign = R(-1);
-    R angM = sign * penetration * (angI[i] / total);
-    R linM = sign * penetration * (linI[i] / total);
-    V3<R> projection = add_scaled(rel[i], n, -dot(rel[i], n));
-    R maxMagnitude = angularLimit * mag(projection);
-    if (angM < -maxMagnitude) {
-      R totalMove = angM + linM;
-      angM = -maxMagnitude;
-      linM = totalMove - angM;
-    } else if (angM > maxMagnitude) {
-      R totalMove = angM + linM;
-      angM = maxMagnitude;
-      linM = totalMove - angM;
-    }
-    if (angM == R(0)) {
-      ang[i] = V3<R>{R(0), R(0), R(0)};
-    } else {
-      V3<R> tad = cross(rel[i], n);
-      R iw[9];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) iw[k] = s_iit[k * KB + l];
-      ang[i] = mul(m3v(iw, tad), angM / angI[i]);
-    }
-    lin[i] = mul(n, linM);
-    np[i] = add_scaled(lds3(s_st, l), n, linM);
-    Q4<R> q{s_st[3 * KB + l], s_st[4 * KB + l], s_st[5 * KB + l], s_st[6 * KB + l]};
-    q = q_add_scaled_vector(q, ang[i], R(1));
-    q = q_normalize(q);
-    if (!aw[i]) {
-      q = q_normalize(q);
-      sleeping |= 1 << i;
-    }
-    nq[i] = q;
-  }
-  return sleeping;
-}
-
-template <typename R, int KIND, int SL>
-__device__ __forceinline__ void resolve_mw(const RS<R>& a, int w, int C, int b0w, int n, char* lds, int t) {
-  using L = MwLds<R>;
-  constexpr int KB = kRegBodies, T = kMwThreads, KC = kMwMaxContacts;
-  constexpr bool MAT = KIND == KIND_MAT;
-  R* s_pos0 = (R*)(lds + L::pos0);
-  R* s_lad = (R*)(lds + L::lad);
-  R* s_st = (R*)(lds + L::st);
-  R* s_rot = s_st + 3 * KB;
-  R* s_iit = (R*)(lds + L::iit);
-  R* s_im = (R*)(lds + L::im);
-  R* s_cn = (R*)(lds + L::cn);
-  R* s_cp = (R*)(lds + L::cp);
-  double* s_pbs = (double*)(lds + L::pbs);
-  double* s_sum = (double*)(lds + L::sum);
-  R* s_pay = (R*)(lds + L::pay);
-  R* s_res = (R*)(lds + L::res);
-  R* s_pkey = (R*)(lds + L::pkey);
-  int32_t* s_pidx = (int32_t*)(lds + L::pidx);
-  uint32_t* s_pkid = (uint32_t*)(lds + L::pkid);
-  int32_t* s_resi = (int32_t*)(lds + L::resi);
-  uint8_t* s_flags = (uint8_t*)(lds + L::flags);
-  auto cnrm = [&](int j) { return V3<R>{s_cn[j], s_cn[KC + j], s_cn[2 * KC + j]}; };
-  auto cpt = [&](int j) { return V3<R>{s_cp[j], s_cp[KC + j], s_cp[2 * KC + j]}; };
-  // wave 0's result: four vectors (the two bodies' linear and angular
-  // changes)
-  auto res_store = [&](int k, const V3<R>& v) {
-    s_res[3 * k] = v.x;
-    s_res[3 * k + 1] = v.y;
-    s_res[3 * k + 2] = v.z;
-  };
-  auto res_load = [&](int k) { return V3<R>{s_res[3 * k], s_res[3 * k + 1], s_res[3 * k + 2]}; };
-  const int lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
-  const bool do_pos = (a.mode & RM_POS) != 0;
-  const bool do_prep = do_pos && !(a.mode & RM_PREPARED);
-  const bool do_vel = (a.mode & RM_VEL) != 0 && (KIND == KIND_POLISH || !a.world_mask || a.world_mask[w]);
-  if (a.world_iters && t == 0) {
-    if (do_pos) a.world_iters[2 * w] = 0;
-    if (a.mode & RM_VEL) a.world_iters[2 * w + 1] = 0;
-  }
-  // ResolveContacts' guard, contact.go:210-212
-  if (a.overflow[0] != 0 || C <= 0 || a.dt <= R(0)) return;
-  if (!do_pos && !do_vel) return;
-
-  const Bodies<R>& b = a.b;
-  const Contacts<R>& c = a.c;
-  const int64_t S = b.stride, CS = c.cap;
-  const int64_t base = a.world_coff[w];
-  const int64_t maxIter = a.iter_fixed > 0 ? a.iter_fixed : a.iter_mult * int64_t(C);
-  const V3<R> zero{R(0), R(0), R(0)};
-
-  for (int i = t; i < n; i += T) {
-    const int g = b0w + i;
-    const V3<R> p = ld3(do_prep ? b.pos : a.pos0, S, g);
-    if (do_prep) st3(a.pos0, S, g, p);
-    lds3_store(s_pos0, i, p);
-    lds3_store(s_lad, i, mul(ld3(b.last_acc, S, g), a.dt));
-    s_flags[i] = b.flags[g];
-#pragma unroll
-    for (int k = 0; k < 9; ++k) s_iit[k * KB + i] = b.iit_world[k * S + g];
-    s_im[i] = b.inv_mass[g];
-  }
-  __syncthreads();
-
-  // prepareContacts / calculateInternals, contact.go:225-229, :59-85, as in
-  // resolve_reg
-  if (do_prep) {
-    for (int j = t; j < C; j += T) {
-      const int64_t g = base + j;
-      int c0 = c.body0[g], c1 = c.body1[g];
-      V3<R> nn = ld3(c.normal, CS, g);
-      if (c0 < 0) {  // contact.go:61-65
-        nn = mul(nn, R(-1));
-        c0 = c1;
-        c1 = -1;
-        c.body0[g] = c0;
-        c.body1[g] = c1;
-        st3(c.normal, CS, g, nn);
-      }
-      const int l0 = c0 - b0w, l1 = c1 >= 0 ? c1 - b0w : -1;
-      R m[9];
-      basis_from_scale(nn, basis_scale(nn), m);
-      const V3<R> p = ld3(c.point, CS, g);
-      const V3<R> r0 = sub(p, lds3(s_pos0, l0));
-      V3<R> cv = local_velocity_lds(b, c0, lds3(s_lad, l0), r0, m);
-      V3<R> r1 = zero;
-      if (c1 >= 0) {
-        r1 = sub(p, lds3(s_pos0, l1));
-        cv = sub(cv, local_velocity_lds(b, c1, lds3(s_lad, l1), r1, m));
-      }
-      const R ddv = desired_dv_lds(s_flags, s_lad, l0, l1, nn, cv.x, restitution_of<R, KIND>(c, g));
-#pragma unroll
-      for (int k = 0; k < 9; ++k) c.c2w[k * CS + g] = m[k];
-      st3(c.rel, CS, g, r0);
-      st3(c.rel + 3 * CS, CS, g, r1);
-      st3(c.cvel, CS, g, cv);
-      c.ddv[g] = ddv;
-    }
-  }
-  // this thread's contacts into registers and LDS (it wrote what it reads
-  // here)
-  R key[SL];
-  uint32_t ids[SL];
-  double bsc[SL];
-  R fr[MAT ? SL : 1], rs[MAT ? SL : 1];
-#pragma unroll
-  for (int s = 0; s < SL; ++s) {
-    const int j = T * s + t;
-    key[s] = R(0);
-    ids[s] = 0xFFFFFFFFu;
-    bsc[s] = 0.0;
-    if constexpr (MAT) fr[s] = rs[s] = R(0);
-    if (j < C) {
-      const int64_t g = base + j;
-      const int c0 = c.body0[g], c1 = c.body1[g];
-      ids[s] = uint32_t(c0 - b0w) | (uint32_t(c1 >= 0 ? c1 - b0w : int(kNoBody)) << 16);
-      if (do_pos) key[s] = c.pen[g];
-      const V3<R> nn = ld3(c.normal, CS, g), p = ld3(c.point, CS, g);
-      s_cn[j] = nn.x; s_cn[KC + j] = nn.y; s_cn[2 * KC + j] = nn.z;
-      s_cp[j] = p.x; s_cp[KC + j] = p.y; s_cp[2 * KC + j] = p.z;
-      bsc[s] = basis_scale(nn);
-      if constexpr (MAT) {
-        fr[s] = c.fric[g];
-        rs[s] = c.rest[g];
-      }
-    }
-  }
-  if (do_pos) {
-    for (int i = t; i < n; i += T) {
-      const int g = b0w + i;
-      lds3_store(s_st, i, ld3(b.pos, S, g));
-#pragma unroll
-      for (int k = 0; k < 4; ++k) s_st[(3 + k) * KB + i] = b.quat[k * S + g];
-    }
-  }
-  __syncthreads();
-
-  // The surrogate's position polish, as in resolve_reg: snapshot the
-  // sleeping bodies' motion and derived data, take the predicted moves, update
-  // the penetrations, reject a world they over-separate, then the loop to
-  // positionEpsilon + polish_tol within polish_mult * C iterations.
-  bool ppolish = KIND == KIND_PPOLISH && do_pos && a.world_mask[w] == 0;
-  R sep_floor = R(0);
-  auto key_min = [&]() {
-    R kmin = R(0);
-#pragma unroll
-    for (int s = 0; s < SL; ++s)
-      if (T * s + t < C) kmin = key[s] < kmin ? key[s] : kmin;
-    return R(mw_extreme<false>(double(kmin), s_sum, t));
-  };
-  auto restore_positions = [&]() {
-    // wave 0's HBM stores of the loop (motion, a sleeping body's derived
-    // data) complete before the other threads restore over them
-    __syncthreads();
-    for (int i = t; i < n; i += T) {
-      const int g = b0w + i;
-      lds3_store(s_st, i, ld3(b.pos, S, g));
-#pragma unroll
-      for (int k = 0; k < 4; ++k) s_st[(3 + k) * KB + i] = b.quat[k * S + g];
-      const uint8_t f = b.flags[g];
-      s_flags[i] = f;
-      if (!(f & F_AWAKE)) {
-        b.motion[g] = a.vel0[g];
-#pragma unroll
-        for (int k = 0; k < 12; ++k) b.transform[k * S + g] = a.vel0[(1 + k) * S + g];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-          const R v = a.vel0[(13 + k) * S + g];
-          b.iit_world[k * S + g] = v;
-          s_iit[k * KB + i] = v;
-        }
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < SL; ++s) {
-      const int j = T * s + t;
-      key[s] = j < C ? c.pen[base + j] : R(0);
-    }
-    __syncthreads();
-    if (t == 0) a.world_mask[w] = 1;
-  };
-  if constexpr (KIND == KIND_PPOLISH) {
-    if (ppolish) {
-      R pmax = R(0);
-#pragma unroll
-      for (int s = 0; s < SL; ++s) pmax = key[s] > pmax ? key[s] : pmax;
-      pmax = R(mw_extreme<true>(double(pmax), s_sum, t));
-      sep_floor = -(R(kSepFactor) * pmax + a.polish_tol);
-      const float* dl = a.delta;
-      for (int i = t; i < n; i += T) {
-        const int g = b0w + i;
-        if (!(s_flags[i] & F_AWAKE)) {
-          a.vel0[g] = b.motion[g];
-#pragma unroll
-          for (int k = 0; k < 12; ++k) a.vel0[(1 + k) * S + g] = b.transform[k * S + g];
-#pragma unroll
-          for (int k = 0; k < 9; ++k) a.vel0[(13 + k) * S + g] = b.iit_world[k * S + g];
-        }
-      }
-      // the predicted moves times `scale` from the phase's starting state,
-      // as in resolve_reg
-      auto take_moves = [&](R scale) {
-        for (int i = t; i < n; i += T) {
-          const int g = b0w + i;
-          if (!(s_flags[i] & F_AWAKE)) continue;
-          const V3<R> dx = mul(V3<R>{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])}, scale);
-          const V3<R> dq = mul(V3<R>{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])}, scale);
-          if (dx.x == R(0) && dx.y == R(0) && dx.z == R(0) && dq.x == R(0) && dq.y == R(0) && dq.z == R(0)) continue;
-          lds3_store(s_st, i, add(ld3(b.pos, S, g), dx));
-          Q4<R> q{b.quat[g], b.quat[S + g], b.quat[2 * S + g], b.quat[3 * S + g]};
-          q = q_normalize(q_add_scaled_vector(q, dq, R(1)));
-          s_st[3 * KB + i] = q.w;
-          s_st[4 * KB + i] = q.x;
-          s_st[5 * KB + i] = q.y;
-          s_st[6 * KB + i] = q.z;
-        }
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-          const int j = T * s + t;
-          if (j >= C) continue;
-          const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-          const V3<R> nj = cnrm(j), ps = cpt(j);
-          R pen = c.pen[base + j];
-#pragma unroll
-          for (int bb = 0; bb < 2; ++bb) {
-            if (jb[bb] < 0) continue;
-            const int g = b0w + jb[bb];
-            const V3<R> dx = mul(V3<R>{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])}, scale);
-            const V3<R> dq = mul(V3<R>{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])}, scale);
-            if (dx.x == R(0) && dx.y == R(0) && dx.z == R(0) && dq.x == R(0) && dq.y == R(0) && dq.z == R(0)) continue;
-            const V3<R> rj = sub(ps, lds3(s_pos0, jb[bb]));
-            const V3<R> dp = add(cross(dq, rj), dx);
-            R sign = R(1);
-            if (bb == 0) sign = R(-1);
-            pen += dot(dp, nj) * sign;
-          }
-          key[s] = pen;
-        }
-        __syncthreads();
-      };
-      take_moves(R(1));
-      if (!(key_min() >= sep_floor)) {
-        take_moves(R(kPosRetryScale));
-        if (!(key_min() >= sep_floor)) {
-          restore_positions();
-          ppolish = false;
-        }
-      }
-    }
-  }
-
-  // adjustPositions, contact.go:233-283.  A slot past the world's contacts
-  // keeps key 0 and ids 0xFFFFFFFF, so the loops need no bounds test.
-  R peps = ppolish ? R(kPositionEpsilon) + a.polish_tol : R(kPositionEpsilon);
-  int64_t pbudget = ppolish ? a.polish_mult * int64_t(C) : maxIter;
-  int64_t used = 0;
-  while (do_pos) {
-    opaque_ids(ids);
-    R best = peps;
-    int bi = INT_MAX;
-#pragma unroll
-    for (int s = 0; s < SL; ++s) {
-      if (key[s] > best) {
-        best = key[s];
-        bi = T * s + t;
-      }
-    }
-    wave_argmax_dpp(best, bi);
-    if (bi == INT_MAX) {
-      if (lane == 0) s_pidx[wv] = INT_MAX;
-    } else if ((bi & (T - 1)) == t) {
-      const int ss = unsigned(bi) / T;
-      s_pkey[wv] = best;
-      s_pidx[wv] = bi;
-#pragma unroll
-      for (int s = 0; s < SL; ++s)
-        if (s == ss) s_pkid[wv] = ids[s];
-    }
-    __syncthreads();  // A
-    if (wv == 0) {
-      R gk = peps;
-      int gi = INT_MAX;
-      const int gw = mw_best(s_pkey, s_pidx, gk, gi);
-      if (gw < 0) {
-        if (lane == 0) s_resi[0] = MW_DONE;
-      } else if (used >= pbudget) {
-        if (lane == 0) s_resi[0] = MW_BUDGET;
-      } else {
-        const uint32_t kid = s_pkid[gw];
-        const int kl[2] = {id_lo(kid), id_hi(kid)};
-        const V3<R> nn = cnrm(gi), p = cpt(gi);
-        V3<R> rel[2];
-        rel[0] = sub(p, lds3(s_pos0, kl[0]));
-        rel[1] = kl[1] >= 0 ? sub(p, lds3(s_pos0, kl[1])) : zero;
-        // matchAwakeState, contact.go:185-202
-        bool aw[2] = {(s_flags[kl[0]] & F_AWAKE) != 0, kl[1] >= 0 && (s_flags[kl[1]] & F_AWAKE) != 0};
-        int woke = -1;
-        if (kl[1] >= 0 && (aw[0] || aw[1]) && !(aw[0] && aw[1])) {
-          woke = aw[0] ? kl[1] : kl[0];
-          aw[0] = aw[1] = true;
-        }
-        V3<R> lin[2], ang[2], np[2];
-        Q4<R> nq[2];
-        const int sleeping = position_change_mw(kl, aw, nn, rel, gk, lin, ang, np, nq, s_st, s_iit, s_im);
-        if (lane == 0) {
-          if (woke >= 0) {  // SetAwake(true), rigidbody.go:183-186
-            s_flags[woke] = uint8_t(s_flags[woke] | F_AWAKE);
-            b.motion[b0w + woke] = R(kSleepEpsilon * 2.0);
-          }
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            const int l = kl[i];
-            if (l < 0) continue;
-            lds3_store(s_st, l, np[i]);
-            s_st[3 * KB + l] = nq[i].w;
-            s_st[4 * KB + l] = nq[i].x;
-            s_st[5 * KB + l] = nq[i].y;
-            s_st[6 * KB + l] = nq[i].z;
-            if (sleeping & (1 << i)) {  // CalculateDerivedData, rigidbody.go:268-272
-              const int g = b0w + l;
-              R Tm[12], IB[9], IW[9];
-              set_as_transform(np[i], nq[i], Tm);
-              ld9(b.iit_body, S, g, IB);
-              transform_inertia(IB, Tm, IW);
-#pragma unroll
-              for (int k = 0; k < 12; ++k) b.transform[k * S + g] = Tm[k];
-#pragma unroll
-              for (int k = 0; k < 9; ++k) {
-                b.iit_world[k * S + g] = IW[k];
-                s_iit[k * KB + l] = IW[k];
-              }
-            }
-          }
-          res_store(0, lin[0]);
-          res_store(1, lin[1]);
-          res_store(2, ang[0]);
-          res_store(3, ang[1]);
-          if constexpr (KIND == KIND_LABEL) add_pos_label(a, base + gi, gk);
-          s_resi[1] = int32_t(kid);
-          s_resi[0] = MW_APPLY;
-        }
-      }
-    }
-    __syncthreads();  // C
-    const int state = s_resi[0];
-    if (state != MW_APPLY) {
-      bool reject = false;
-      if constexpr (KIND == KIND_PPOLISH) {
-        // every contact within positionEpsilon + tol: the separation test;
-        // out of budget: rejected
-        if (ppolish) reject = state == MW_BUDGET || !(key_min() >= sep_floor);
-      }
-      if (!reject) break;
-      restore_positions();
-      ppolish = false;
-      peps = R(kPositionEpsilon);
-      pbudget = maxIter;
-      used = 0;
-      continue;
-    }
-    {
-      const uint32_t kid = uint32_t(s_resi[1]);
-      const int kl[2] = {id_lo(kid), id_hi(kid)};
-      const V3<R> lin[2] = {res_load(0), res_load(1)};
-      const V3<R> ang[2] = {res_load(2), res_load(3)};
-#pragma unroll
-      for (int s = 0; s < SL; ++s) {
-        const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-        bool any = false;
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-          for (int d = 0; d < 2; ++d) any |= (jb[bb] >= 0 && jb[bb] == kl[d]);
-        if (!any) continue;
-        R pen = key[s];
-        const V3<R> ns = cnrm(T * s + t), ps = cpt(T * s + t);
-#pragma unroll
-        for (int bb = 0; bb < 2; ++bb) {
-          if (jb[bb] < 0) continue;
-          const V3<R> rj = sub(ps, lds3(s_pos0, jb[bb]));
-          // a side is at most one of the two moved bodies: its change is
-          // selected and applied once
-          if (jb[bb] == kl[0] || jb[bb] == kl[1]) {
-            const bool d0 = jb[bb] == kl[0];
-            V3<R> dp = add(cross(sel3(d0, ang[0], ang[1]), rj), sel3(d0, lin[0], lin[1]));
-            R sign = R(1);
-            if (bb == 0) sign = R(-1);
-            pen += dot(dp, ns) * sign;
-          }
-        }
-        key[s] = pen;
-      }
-    }
-    ++used;
-  }
-  const int64_t pos_iters = used;
-  __syncthreads();
-  if (do_pos) {
-    for (int i = t; i < n; i += T) {
-      const int g = b0w + i;
-      st3(b.pos, S, g, lds3(s_st, i));
-#pragma unroll
-      for (int k = 0; k < 4; ++k) b.quat[k * S + g] = s_st[(3 + k) * KB + i];
-    }
-  }
-
-  // adjustVelocities, contact.go:390-445
-  V3<R> cv[SL];
-  R imp[SL][kImpPlanes];
-#pragma unroll
-  for (int s = 0; s < SL; ++s) {
-    const int j = T * s + t;
-    cv[s] = zero;
-#pragma unroll
-    for (int k = 0; k < kImpPlanes; ++k) imp[s][k] = R(0);
-    if (do_pos && j < C) c.pen[base + j] = key[s];
-    if (do_vel && j < C) {
-      key[s] = c.ddv[base + j];  // selection keys as prepare stored them
-      cv[s] = ld3(c.cvel, CS, base + j);
-      // the impulse data, fixed for the whole phase (as impulse_data from
-      // the contact arrays prepare stored: same values)
-      const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-      R mj[9], i0[9], i1[9];
-      const V3<R> ps = cpt(j);
-      basis_from_scale(cnrm(j), bsc[s], mj);
-      const V3<R> rj[2] = {sub(ps, lds3(s_pos0, jb[0])), jb[1] >= 0 ? sub(ps, lds3(s_pos0, jb[1])) : zero};
-#pragma unroll
-      for (int k = 0; k < 9; ++k) {
-        i0[k] = s_iit[k * KB + jb[0]];
-        i1[k] = jb[1] >= 0 ? s_iit[k * KB + jb[1]] : R(0);
-      }
-      const R invm[2] = {s_im[jb[0]], jb[1] >= 0 ? s_im[jb[1]] : R(0)};
-      R fj = R(kFriction);
-      if constexpr (MAT) fj = fr[s];
-      impulse_data_from<R, KIND>(a.mode, i0, i1, invm, jb[1] >= 0, rj, mj, fj, imp[s]);
-    }
-  }
-  // the position write-back read the LDS state that the velocity phase
-  // reuses
-  __syncthreads();
-  used = 0;
-  if (do_vel) {
-    for (int i = t; i < n; i += T) {
-      const int g = b0w + i;
-      lds3_store(s_st, i, ld3(b.vel, S, g));
-      lds3_store(s_rot, i, ld3(b.rot, S, g));
-    }
-    bool polishing = KIND == KIND_POLISH && a.world_mask[w] == 0;
-    double ke_before = 0.0, world_mass = 0.0;
-    if constexpr (KIND == KIND_POLISH) {
-      if (polishing) {
-        // take the predicted changes (as resolve_reg)
-        const float* dl = a.delta;
-        double ke = 0.0, mass = 0.0;
-        for (int i = t; i < n; i += T) {
-          const int g = b0w + i;
-          const V3<R> v = lds3(s_st, i), r = lds3(s_rot, i);
-          R iw[9];
-#pragma unroll
-          for (int k = 0; k < 9; ++k) iw[k] = s_iit[k * KB + i];
-          double mi;
-          ke += kinetic_energy(v, r, s_im[i], iw, mi);
-          mass += mi;
-          a.vel0[6 * S + g] = b.motion[g];
-          const V3<R> dv{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])};
-          const V3<R> dw{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])};
-          if (dv.x != R(0) || dv.y != R(0) || dv.z != R(0) || dw.x != R(0) || dw.y != R(0) || dw.z != R(0)) {
-            lds3_store(s_st, i, add(v, dv));
-            lds3_store(s_rot, i, add(r, dw));
-          }
-        }
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-          if (T * s + t >= C) continue;
-          const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-          R mj[9];
-          basis_from_scale(cnrm(T * s + t), bsc[s], mj);
-          const V3<R> ps = cpt(T * s + t);
-          V3<R> cvj = cv[s];
-          bool moved = false;
-#pragma unroll
-          for (int bb = 0; bb < 2; ++bb) {
-            if (jb[bb] < 0) continue;
-            const int g = b0w + jb[bb];
-            const V3<R> dv{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])};
-            const V3<R> dw{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])};
-            if (dv.x == R(0) && dv.y == R(0) && dv.z == R(0) && dw.x == R(0) && dw.y == R(0) && dw.z == R(0)) continue;
-            moved = true;
-            const V3<R> rj = sub(ps, lds3(s_pos0, jb[bb]));
-            R sign = R(1);
-            if (bb == 1) sign = R(-1);
-            cvj = add(cvj, mul(m3tv(mj, add(cross(dw, rj), dv)), sign));
-          }
-          if (moved) {
-            cv[s] = cvj;
-            key[s] = desired_dv_lds(s_flags, s_lad, jb[0], jb[1], V3<R>{mj[0], mj[1], mj[2]}, cvj.x,
-                                    R(kRestitution));
-          }
-        }
-        ke_before = mw_sum(ke, s_sum, t);
-        world_mass = mw_sum(mass, s_sum, t);
-      }
-    }
-    __syncthreads();
-    R eps = polishing ? R(kVelocityEpsilon) + a.polish_tol : R(kVelocityEpsilon);
-    int64_t budget = polishing ? a.polish_mult * int64_t(C) : maxIter;
-    int64_t it = 0;
-    while (true) {
-      opaque_ids(ids);
-      R best = eps;
-      int bi = INT_MAX;
-#pragma unroll
-      for (int s = 0; s < SL; ++s) {
-        if (key[s] > best) {
-          best = key[s];
-          bi = T * s + t;
-        }
-      }
-      wave_argmax_dpp(best, bi);
-      if (bi == INT_MAX) {
-        if (lane == 0) s_pidx[wv] = INT_MAX;
-      } else if ((bi & (T - 1)) == t) {
-        const int ss = unsigned(bi) / T;
-        R* pay = s_pay + wv * kMwPay;
-        s_pkey[wv] = best;
-        s_pidx[wv] = bi;
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-          if (s != ss) continue;
-          s_pkid[wv] = ids[s];
-          s_pbs[wv] = bsc[s];
-          pay[0] = cv[s].x; pay[1] = cv[s].y; pay[2] = cv[s].z;
-#pragma unroll
-          for (int k = 0; k < kImpPlanes; ++k) pay[3 + k] = imp[s][k];
-          if constexpr (MAT) pay[15] = fr[s];
-        }
-      }
-      __syncthreads();  // A
-      if (wv == 0) {
-        R gk = eps;
-        int gi = INT_MAX;
-        const int gw = mw_best(s_pkey, s_pidx, gk, gi);
-        if (gw < 0 || it >= budget) {
-          if (lane == 0) s_resi[0] = gw < 0 ? MW_DONE : MW_BUDGET;
-        } else {
-          const uint32_t kid = s_pkid[gw];
-          const R* pay = s_pay + gw * kMwPay;
-          const int kl[2] = {id_lo(kid), id_hi(kid)};
-          const V3<R> nn = cnrm(gi), p = cpt(gi);
-          const V3<R> cvk{pay[0], pay[1], pay[2]};
-          R m[9], ik[kImpPlanes];
-          basis_from_scale(nn, s_pbs[gw], m);
-#pragma unroll
-          for (int k = 0; k < kImpPlanes; ++k) ik[k] = pay[3 + k];
-          R fk = R(kFriction);
-          if constexpr (MAT) fk = pay[15];
-          V3<R> rel[2];
-          rel[0] = sub(p, lds3(s_pos0, kl[0]));
-          rel[1] = kl[1] >= 0 ? sub(p, lds3(s_pos0, kl[1])) : zero;
-          // matchAwakeState, contact.go:185-202
-          const bool aw0 = (s_flags[kl[0]] & F_AWAKE) != 0;
-          const bool aw1 = kl[1] >= 0 && (s_flags[kl[1]] & F_AWAKE) != 0;
-          int woke = -1;
-          if (kl[1] >= 0 && (aw0 || aw1) && !(aw0 && aw1)) woke = aw0 ? kl[1] : kl[0];
-          // applyVelocityChange, contact.go:448-494 (apply_velocity_change_lds)
-          V3<R> ic;
-          if (MAT && fk == R(0))
-            ic = V3<R>{gk / ik[0], R(0), R(0)};
-          else
-            ic = friction_impulse_from(ik, ik + 9, gk, cvk, fk);
-          const V3<R> impulse = m3v(m, ic);
-          V3<R> vc[2], rc[2];
-          R iw[9];
-#pragma unroll
-          for (int k = 0; k < 9; ++k) iw[k] = s_iit[k * KB + kl[0]];
-          V3<R> torque = cross(rel[0], impulse);
-          rc[0] = m3v(iw, torque);
-          vc[0] = add_scaled(zero, impulse, s_im[kl[0]]);
-          rc[1] = zero;
-          vc[1] = zero;
-          if (kl[1] >= 0) {
-#pragma unroll
-            for (int k = 0; k < 9; ++k) iw[k] = s_iit[k * KB + kl[1]];
-            torque = cross(impulse, rel[1]);
-            rc[1] = m3v(iw, torque);
-            vc[1] = add_scaled(zero, impulse, -s_im[kl[1]]);
-          }
-          if (lane == 0) {
-            if (woke >= 0) {  // SetAwake(true), rigidbody.go:183-186
-              s_flags[woke] = uint8_t(s_flags[woke] | F_AWAKE);
-              b.motion[b0w + woke] = R(kSleepEpsilon * 2.0);
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-              if (kl[i] < 0) continue;
-              lds3_store(s_st, kl[i], add(lds3(s_st, kl[i]), vc[i]));
-              lds3_store(s_rot, kl[i], add(lds3(s_rot, kl[i]), rc[i]));
-            }
-            if constexpr (KIND == KIND_LABEL) add_label(a, base + gi, vc, rc);
-            res_store(0, vc[0]);
-            res_store(1, vc[1]);
-            res_store(2, rc[0]);
-            res_store(3, rc[1]);
-            s_resi[1] = int32_t(kid);
-            s_resi[0] = MW_APPLY;
-          }
-        }
-      }
-      __syncthreads();  // C
-      const int state = s_resi[0];
-      if (state != MW_APPLY) {
-        bool reject = false;  // the polish did not give an acceptable result
-        if (state == MW_DONE) {
-          if constexpr (KIND == KIND_POLISH) {
-            // the acceptance test of resolve_reg
-            if (polishing) {
-              double ke = 0.0, mass = 0.0;
-              for (int i = t; i < n; i += T) {
-                R iw[9];
-#pragma unroll
-                for (int k = 0; k < 9; ++k) iw[k] = s_iit[k * KB + i];
-                ke += kinetic_energy(lds3(s_st, i), lds3(s_rot, i), s_im[i], iw, mass);
-              }
-              const double ke_after = mw_sum(ke, s_sum, t);
-              const double tol = double(a.polish_tol);
-              reject = !(ke_after <= ke_before * (1.0 + kEnergyRel) + 0.5 * tol * tol * world_mass);
-            }
-          }
-          if (!reject) break;
-        } else {  // the iteration budget is used
-          if (KIND != KIND_POLISH || !polishing) break;
-          reject = true;
-        }
-        // undo the prediction and the loop; run the plain phase
-        __syncthreads();
-        for (int i = t; i < n; i += T) {
-          const int g = b0w + i;
-          lds3_store(s_st, i, ld3(b.vel, S, g));
-          lds3_store(s_rot, i, ld3(b.rot, S, g));
-          b.motion[g] = a.vel0[6 * S + g];
-          s_flags[i] = b.flags[g];
-        }
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-          const int j = T * s + t;
-          if (j < C) {
-            key[s] = c.ddv[base + j];
-            cv[s] = ld3(c.cvel, CS, base + j);
-          }
-        }
-        __syncthreads();
-        if (t == 0) a.world_mask[w] = 1;
-        polishing = false;
-        eps = R(kVelocityEpsilon);
-        budget = maxIter;
-        it = 0;
-        continue;
-      }
-      {
-        const uint32_t kid = uint32_t(s_resi[1]);
-        const int kl[2] = {id_lo(kid), id_hi(kid)};
-        const V3<R> vc[2] = {res_load(0), res_load(1)};
-        const V3<R> rc[2] = {res_load(2), res_load(3)};
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-          const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
-          bool any = false;
-#pragma unroll
-          for (int bb = 0; bb < 2; ++bb)
-#pragma unroll
-            for (int d = 0; d < 2; ++d) any |= (jb[bb] >= 0 && jb[bb] == kl[d]);
-          if (!any) continue;
-          R mj[9];
-          basis_from_scale(cnrm(T * s + t), bsc[s], mj);
-          const V3<R> ps = cpt(T * s + t);
-          V3<R> cvj = cv[s];
-#pragma unroll
-          for (int bb = 0; bb < 2; ++bb) {
-            if (jb[bb] < 0) continue;
-            const V3<R> rj = sub(ps, lds3(s_pos0, jb[bb]));
-            // a side is at most one of the two moved bodies: its change is
-            // selected and applied once
-            if (jb[bb] == kl[0] || jb[bb] == kl[1]) {
-              const bool d0 = jb[bb] == kl[0];
-              V3<R> dv = add(cross(sel3(d0, rc[0], rc[1]), rj), sel3(d0, vc[0], vc[1]));
-              R sign = R(1);
-              if (bb == 1) sign = R(-1);
-              cvj = add(cvj, mul(m3tv(mj, dv), sign));
-            }
-          }
-          cv[s] = cvj;
-          R e = R(kRestitution);
-          if constexpr (MAT) e = rs[s];
-          key[s] = desired_dv_lds(s_flags, s_lad, jb[0], jb[1], V3<R>{mj[0], mj[1], mj[2]}, cvj.x, e);
-        }
-      }
-      ++it;
-      ++used;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < SL; ++s) {
-      const int j = T * s + t;
-      if (j < C) {
-        c.ddv[base + j] = key[s];
-        st3(c.cvel, CS, base + j, cv[s]);
-      }
-    }
-    for (int i = t; i < n; i += T) {
-      const int g = b0w + i;
-      st3(b.vel, S, g, lds3(s_st, i));
-      st3(b.rot, S, g, lds3(s_rot, i));
-    }
-  }
-  __syncthreads();
-  for (int i = t; i < n; i += T) b.flags[b0w + i] = s_flags[i];
-  if (t == 0 && a.world_iters) {
-    if (do_pos) a.world_iters[2 * w] = pos_iters;
-    if (do_vel) a.world_iters[2 * w + 1] = used;
   }
 }
 
 template <typename R, int KIND>
-__device__ __forceinline__ void resolve_mw_world(const RS<R>& a, int w, int C, int b0w, int n, char* lds, int t) {
-  if (C <= kMwThreads * 4)
-    resolve_mw<R, KIND, 4>(a, w, C, b0w, n, lds, t);
-  else
-    resolve_mw<R, KIND, kMwMaxSlots>(a, w, C, b0w, n, lds, t);
+__global__ void __launch_bounds__(64) k_resolve_left(RS<R> a) {
+  resolve_left_block<R, KIND>(a);
 }
 
-constexpr size_t cmax(size_t x, size_t y) { return x > y ? x : y; }
+// Workgroups beyond the list end at once.
+constexpr int kLeftGrid = 256;
 template <typename R, int KIND>
-constexpr size_t resolve_lds_bytes() {
-  return cmax(cmax(RegLds<R, 32, KIND>::bytes, RegLds<R, 8, KIND>::bytes),
-              kKeyCap * (sizeof(R) + 2 * sizeof(int32_t)));
-}
-
-// The polish kind carries more state through its loop: its widest
-// register class is 24 slots (1536 contacts).
-template <int KIND>
-constexpr int max_slots() {
-  return KIND == KIND_POLISH ? 24 : kRegMaxSlots;
-}
-
-template <typename R, int KIND>
-__device__ __forceinline__ void resolve_world_kind(const RS<R>& a, int w, int C, int b0w, int n, char* lds, int lane) {
-  if (!fits_registers(C, n) || C > 64 * max_slots<KIND>()) {
-    resolve_hbm<R, KIND>(a, w, C, lds, lane);
-  } else if (C <= 64) {
-    resolve_reg<R, 1, KIND>(a, w, C, b0w, n, lds, lane);
-  } else if (C <= 128) {
-    resolve_reg<R, 2, KIND>(a, w, C, b0w, n, lds, lane);
-  } else if (C <= 256) {
-    resolve_reg<R, 4, KIND>(a, w, C, b0w, n, lds, lane);
-  } else if (C <= 512) {
-    resolve_reg<R, 8, KIND>(a, w, C, b0w, n, lds, lane);
-  } else if (C <= 768) {
-    resolve_reg<R, 12, KIND>(a, w, C, b0w, n, lds, lane);
-  } else if (C <= 1024) {
-    resolve_reg<R, 16, KIND>(a, w, C, b0w, n, lds, lane);
-  } else if (C <= 1536) {
-    resolve_reg<R, 24, KIND>(a, w, C, b0w, n, lds, lane);
-  } else if constexpr (max_slots<KIND>() >= 32) {
-    resolve_reg<R, 32, KIND>(a, w, C, b0w, n, lds, lane);
-  }
-}
-
-// One launch for every world: each workgroup takes the world order[blockIdx]
-// (larger worlds first) and runs the variant for its contact count.
-template <typename R, int KIND>
-__device__ __forceinline__ void resolve_block(const RS<R>& a) {
-  __shared__ __align__(16) char lds[resolve_lds_bytes<R, KIND>()];
-  const int lane = threadIdx.x;
-  const int w = a.order ? a.order[blockIdx.x] : int(blockIdx.x);
-  if (w >= a.n_worlds) return;
-  const int C = a.world_cnt[w];
-  const int b0w = a.body_off[w], n = a.body_off[w + 1] - b0w;
-  if (a.mw_list && a.mw_flag[w]) return;  // the multi-wave kernel's
-  int64_t* wt = a.world_time ? a.world_time + 4 * int64_t(w) + ((a.mode & RM_VEL) ? 2 : 0) : nullptr;
-  if (wt && lane == 0) wt[0] = int64_t(wall_clock64());
-  resolve_world_kind<R, KIND>(a, w, C, b0w, n, lds, lane);
-  if (wt && lane == 0) wt[1] = int64_t(wall_clock64());
-}
-
-// The multi-wave kernel, persistent: each workgroup takes the next listed
-// world (largest first) from the queue until the list is done.
-template <typename R, int KIND>
-__device__ __forceinline__ void resolve_mw_block(const RS<R>& a) {
-  __shared__ __align__(16) char lds[MwLds<R>::bytes];
-  __shared__ int32_t s_next;
-  const int t = threadIdx.x;
-  const int nbig = a.mw_count[0];
-  while (true) {
-    if (t == 0) s_next = atomicAdd(&a.mw_count[1], 1);
-    __syncthreads();
-    const int k = s_next;
-    __syncthreads();
-    if (k >= nbig) break;
-    const int w = a.mw_list[k];
-    const int C = a.world_cnt[w];
-    const int b0w = a.body_off[w], n = a.body_off[w + 1] - b0w;
-    int64_t* wt = a.world_time ? a.world_time + 4 * int64_t(w) + ((a.mode & RM_VEL) ? 2 : 0) : nullptr;
-    if (wt && t == 0) wt[0] = int64_t(wall_clock64());
-    resolve_mw_world<R, KIND>(a, w, C, b0w, n, lds, t);
-    __syncthreads();
-    if (wt && t == 0) wt[1] = int64_t(wall_clock64());
-  }
-}
-
-// The FP64 kernel keeps a full wave's registers (its working set spills
-// heavily below that); its LDS (about 21 KB) lets 4 worlds share a CU.  The
-// FP32 kernel is held to two waves per SIMD: its few spills cost less than
-// the second wave gains.
-template <int KIND>
-__global__ void __launch_bounds__(64) k_resolve_f64(RS<double> a) {
-  resolve_block<double, KIND>(a);
-}
-template <int KIND>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) k_resolve_f32(RS<float> a) {
-  resolve_block<float, KIND>(a);
-}
-
-template <int KIND>
-__global__ void __launch_bounds__(kMwThreads) k_resolve_mw_f64(RS<double> a) {
-  resolve_mw_block<double, KIND>(a);
-}
-template <int KIND>
-__global__ void __launch_bounds__(kMwThreads) k_resolve_mw_f32(RS<float> a) {
-  resolve_mw_block<float, KIND>(a);
-}
-
-template <typename R, int KIND>
-void launch_kind(const RS<R>& a, hipStream_t st) {
-  if constexpr (sizeof(R) == 8)
-    k_resolve_f64<KIND><<<a.n_worlds, 64, 0, st>>>(a);
-  else
-    k_resolve_f32<KIND><<<a.n_worlds, 64, 0, st>>>(a);
-}
-
-// The multi-wave kernel over mw_list: at most one workgroup per CU (each
-// takes a whole CU's registers).
-template <typename R, int KIND>
-void launch_mw_kind(const RS<R>& a, int grid, hipStream_t st) {
-  if constexpr (sizeof(R) == 8)
-    k_resolve_mw_f64<KIND><<<grid, kMwThreads, 0, st>>>(a);
-  else
-    k_resolve_mw_f32<KIND><<<grid, kMwThreads, 0, st>>>(a);
-}
-
-// Worlds (workgroups) of one kind's kernel resident per CU, from its
-// register and LDS use.
-template <typename R, int KIND>
-hipError_t kind_occupancy(int* worlds_per_cu) {
-  if constexpr (sizeof(R) == 8)
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(worlds_per_cu, k_resolve_f64<KIND>, 64, 0);
-  else
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(worlds_per_cu, k_resolve_f32<KIND>, 64, 0);
+void launch_left_kind(const RS<R>& a, hipStream_t st) {
+  k_resolve_left<R, KIND><<<a.n_worlds < kLeftGrid ? a.n_worlds : kLeftGrid, 64, 0, st>>>(a);
 }
 
 // Every instantiation lives in one translation unit of its own
 // (k_resolve_<precision>_<kind>.hip); other units only declare them.
 #define CBZ_RESOLVE_KIND(EXT, R, KIND)                                          \
-  EXT template void launch_kind<R, KIND>(const RS<R>&, hipStream_t);           \
-  EXT template void launch_mw_kind<R, KIND>(const RS<R>&, int, hipStream_t);   \
-  EXT template hipError_t kind_occupancy<R, KIND>(int*);
-#ifndef CBZ_RESOLVE_INSTANTIATE
-CBZ_RESOLVE_KIND(extern, double, KIND_PLAIN)
-CBZ_RESOLVE_KIND(extern, double, KIND_LABEL)
-CBZ_RESOLVE_KIND(extern, double, KIND_POLISH)
-CBZ_RESOLVE_KIND(extern, double, KIND_MAT)
-CBZ_RESOLVE_KIND(extern, double, KIND_PPOLISH)
-CBZ_RESOLVE_KIND(extern, float, KIND_PLAIN)
-CBZ_RESOLVE_KIND(extern, float, KIND_LABEL)
-CBZ_RESOLVE_KIND(extern, float, KIND_POLISH)
-CBZ_RESOLVE_KIND(extern, float, KIND_MAT)
-CBZ_RESOLVE_KIND(extern, float, KIND_PPOLISH)
-#endif
+  EXT template void launch_left_kind<R, KIND>(const RS<R>&, hipStream_t);      \
+  EXT template hipError_t launch_islands_kind<R, KIND>(const RS<R>&, hipStream_t); \
+  EXT template hipError_t islands_occupancy<R, KIND>(int, int*);
 
 }  // namespace cbz

@@ -78,13 +78,12 @@ struct Contacts {
   R* fric;         // [cap]
   R* rest;         // [cap]
   // resolver scratch: per contact the impulse data of the velocity phase
-  // (impulseMatrix 9, deltaVelocity entries 0, 3, 6), written when the
-  // phase starts
-  R* imp;          // [12][cap]
+  // (impulseMatrix 9, deltaVelocity entries 0, 3, 6), written when an island
+  // of more than 256 contacts is loaded
+  R* imp;          // [cap][12]
   // per contact one 16-value record, contactToWorld 9,
   // relativeContactPosition[0] 3, [1] 3, 1 unused: a copy of c2w and rel
-  // that the one-wavefront resolver's wide classes write in prepare and read
-  // in their loops from one address
+  // that prepare writes and the resolver reads from one address
   R* rec;          // [cap][16]
 };
 

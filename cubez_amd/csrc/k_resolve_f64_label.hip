@@ -1,6 +1,6 @@
-// k_resolve_f64_label.hip — the FP64 resolver kernel, kind KIND_LABEL (cbz_resolve.h).
+// k_resolve_f64_label.hip — the FP64 resolver kernel, kind KIND_LABEL (cbz_islands.h, cbz_resolve.h).
 #define CBZ_RESOLVE_INSTANTIATE
-#include "cbz_resolve.h"
+#include "cbz_islands.h"
 
 namespace cbz {
 CBZ_RESOLVE_KIND(, double, KIND_LABEL)

@@ -199,10 +199,8 @@ class World:
         return a.value, b.value
 
     def set_resolver_split(self, min_contacts, max_worlds=32):
-        """Of the worlds of at least min_contacts contacts (at most 2048, and
-        256 bodies), the max_worlds largest resolve on the kernel of four
-        wavefronts per world; either 0: none (cbz_set_resolver_split; the
-        same results either way)."""
+        """A split between two resolver kernels (cbz_set_resolver_split): kept
+        and returned, without effect; every world runs on one kernel."""
         self._chk(self._lib.cbz_set_resolver_split(self._h, int(min_contacts), int(max_worlds)))
 
     def resolver_split(self):

@@ -249,19 +249,13 @@ int cbz_resolver_iterations(cbz_ctx *ctx, int64_t *iters);
  * counterpart in the reference (a measurement of this implementation). */
 int cbz_resolver_world_times(cbz_ctx *ctx, double *us);
 /* Worlds the resolver keeps resident per CU (the plain kernel of the
- * context's precision: one wavefront per world, bounded by its registers
- * and LDS) and the device's CU count; the bench derives the time per
- * serial iteration from them. */
+ * context's precision: one workgroup per world, bounded by its registers
+ * and its LDS tables for 256 bodies) and the device's CU count. */
 int cbz_resolver_occupancy(cbz_ctx *ctx, int32_t *worlds_per_cu, int32_t *n_cu);
-/* The resolver's split between its two kernels.  Of the worlds of at least
- * min_contacts contacts (and at most 2048 contacts and 256 bodies), the
- * max_worlds largest resolve on a persistent kernel of four wavefronts per
- * world, on a second stream beside the one-wavefront kernel that takes the
- * others; both give the same bits.  Either value 0 sends every world to the
- * one-wavefront kernel; the defaults are 257 and 32 (cbz_autotune_resolver
- * picks it by measurement).  A scheduling choice of this implementation, with
- * no counterpart in the reference (ResolveContacts, contact.go:208-222, is
- * the same loop either way). */
+/* A split of the worlds between two resolver kernels, by contact count and
+ * number of worlds (defaults 257 and 32).  Every world now runs on one kernel,
+ * island by island: the values are kept and returned for the programs that
+ * set them, and change neither results nor times. */
 int cbz_set_resolver_split(cbz_ctx *ctx, int32_t min_contacts, int32_t max_worlds);
 int cbz_get_resolver_split(cbz_ctx *ctx, int32_t *min_contacts, int32_t *max_worlds);
 /* The autotuner of that split: from the current state, times n_steps of
@@ -269,7 +263,8 @@ int cbz_get_resolver_split(cbz_ctx *ctx, int32_t *min_contacts, int32_t *max_wor
  * polish_per_contact) for each candidate split (cand_min[i], cand_max[i]),
  * restoring the body state before each run and at the end, then keeps the
  * fastest: its index in *best, the times in ms_per_step[n_cand] (may be
- * NULL).  Profiling must be off.  No counterpart in the reference. */
+ * NULL).  The split has no effect, so the times differ by noise alone.
+ * Profiling must be off.  No counterpart in the reference. */
 int cbz_autotune_resolver(cbz_ctx *ctx, double dt, int64_t iter_per_contact, int32_t n_steps, int32_t surrogate,
                           double tol, int64_t polish_per_contact, int32_t n_cand, const int32_t *cand_min,
                           const int32_t *cand_max, double *ms_per_step, int32_t *best);
@@ -389,8 +384,9 @@ int cbz_sur_check_gemms(int32_t rows, char *msg, int32_t msg_len);
  * (cbz_sur_set_position), for at most its budget per contact * C
  * iterations; the polished world is accepted only if, besides, no contact
  * ends separated by more than the world's deepest penetration at the start
- * plus that tolerance.  Worlds of more than 1536 contacts, and every world
- * when the position tolerance is negative, take the plain position phase.
+ * plus that tolerance.  Worlds of more than 256 bodies or 2048 contacts,
+ * and every world when the position tolerance is negative, take the plain
+ * position phase.
  * Velocity phase: likewise from the predicted changes, to velocityEpsilon +
  * tol (tol in m/s) within polish_per_contact * C iterations, accepted only
  * if the world's kinetic energy did not grow (beyond 1/2 tol^2 per kg).
