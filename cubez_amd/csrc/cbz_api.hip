@@ -185,8 +185,8 @@ struct cbz_context {
     float* adam_m = nullptr;
     float* adam_v = nullptr;
     int64_t adam_t = 0;
-    __bf16* Wnk[cbz::kLayers] = {};  // [Npad x Kpad] forward operand
-    __bf16* Wkn[cbz::kLayers] = {};  // [Kpad x Npad] backward operand
+    __bf16* Wf[cbz::kLayers] = {};  // [Npad x Kpad] forward operand
+    __bf16* Wb[cbz::kLayers] = {};  // [Kpad x Npad] backward operand (not of layer 0)
     float* norm = nullptr;  // in_mean 40, in_inv_std 40, out_mean 13, out_std 13, out_inv_std 13
     // dataset of (raw features, labels)
     float* dsX = nullptr;
@@ -213,17 +213,13 @@ struct cbz_context {
     bool last_pos = false;  // the last surrogate resolve polished positions (pmask is valid)
     // training buffers
     int batch_cap = 0;
-    int64_t* idx = nullptr;
-    __bf16* bX = nullptr;
-    float* bT = nullptr;
-    float* Z[cbz::kLayers] = {};
-    __bf16* Hb[cbz::kLayers - 1] = {};
-    __bf16* At[cbz::kLayers] = {};  // transposed layer inputs: X^T, H0^T, H1^T, H2^T
-    float* Yout = nullptr;
-    __bf16* dZ[cbz::kLayers] = {};
-    __bf16* dZt[cbz::kLayers] = {};
-    float* dA = nullptr;
+    __bf16* At[cbz::kLayers] = {};   // layer inputs, transposed
+    __bf16* dZt[cbz::kLayers] = {};  // dL/dZ, transposed
     float* row_loss = nullptr;
+    // rows a caller hands over (cbz_sur_grad, cbz_sur_predict)
+    float* sx = nullptr;
+    float* sy = nullptr;
+    int64_t stage_cap = 0;
     float* losses = nullptr;
     int losses_cap = 0;
   } sur;
@@ -940,22 +936,10 @@ int64_t round32(int64_t n) { return (n + 31) / 32 * 32; }
 // the allocator and the shape check (cbz_sur_check_gemms) share this list.
 template <typename F>
 void sur_batch_buffers(cbz_context::Sur& u, int64_t Mpad, F&& f) {
-  f(u.idx, Mpad);
-  f(u.bX, Mpad * kFeatPad);
-  f(u.bT, Mpad * kOut);
-  f(u.At[0], Mpad * kFeatPad);
   for (int l = 0; l < kLayers; ++l) {
-    const int64_t w = Mpad * layer_out_pad(l);
-    f(u.Z[l], w);
-    f(u.dZ[l], w);
-    f(u.dZt[l], w);
-    if (l < kLayers - 1) {
-      f(u.Hb[l], w);
-      f(u.At[l + 1], w);
-    }
+    f(u.At[l], Mpad * layer_in_frag(l));
+    f(u.dZt[l], Mpad * layer_out_pad(l));
   }
-  f(u.Yout, Mpad * kOut);
-  f(u.dA, Mpad * kHidden);
   f(u.row_loss, Mpad);
 }
 
@@ -970,8 +954,8 @@ void sur_model_buffers(cbz_context::Sur& u, F&& f) {
   f(u.adam_v, total);
   f(u.norm, int64_t(kNorm));
   for (int l = 0; l < kLayers; ++l) {
-    f(u.Wnk[l], int64_t(layer_out_pad(l)) * layer_in_pad(l));
-    f(u.Wkn[l], int64_t(layer_out_pad(l)) * layer_in_pad(l));
+    f(u.Wf[l], int64_t(layer_out_pad(l)) * layer_in_pad(l));
+    if (l > 0) f(u.Wb[l], int64_t(layer_out_pad(l)) * layer_in_pad(l));
   }
 }
 
@@ -1012,22 +996,16 @@ void sur_free_model(cbz_ctx* c) {
   dfree(u.adam_v);
   dfree(u.norm);
   for (int l = 0; l < kLayers; ++l) {
-    dfree(u.Wnk[l]);
-    dfree(u.Wkn[l]);
+    dfree(u.Wf[l]);
+    dfree(u.Wb[l]);
   }
   dfree(u.dsX);
   dfree(u.dsY);
-  dfree(u.idx);
-  dfree(u.bX);
-  dfree(u.bT);
-  for (auto& p : u.Z) dfree(p);
-  for (auto& p : u.Hb) dfree(p);
   for (auto& p : u.At) dfree(p);
-  for (auto& p : u.dZ) dfree(p);
   for (auto& p : u.dZt) dfree(p);
-  dfree(u.Yout);
-  dfree(u.dA);
   dfree(u.row_loss);
+  dfree(u.sx);
+  dfree(u.sy);
   dfree(u.losses);
   u = cbz_context::Sur{};
 }
@@ -1036,7 +1014,7 @@ int sur_pack(cbz_ctx* c) {
   auto& u = c->sur;
   const LayerOff o = layer_offsets();
   for (int l = 0; l < kLayers; ++l)
-    HIPCHK(c, launch_pack_weights(u.params + o.w[l], layer_out(l), layer_in(l), u.Wnk[l], layer_in_pad(l), u.Wkn[l],
+    HIPCHK(c, launch_pack_weights(u.params + o.w[l], layer_out(l), layer_in(l), u.Wf[l], layer_in_pad(l), u.Wb[l],
                                   layer_out_pad(l), c->stream));
   return CBZ_OK;
 }
@@ -1050,9 +1028,9 @@ bool dry_inside(const cbz_ctx* c, const void* p, int64_t bytes) {
 }
 
 // One GEMM of the surrogate: launched, or in the shape check compared with
-// the extents of the buffers it reads and writes (k_gemm reads rows < M of A
-// and rows < N of Bt, K elements each; writes Z/Y where row < m_valid and
-// col < n_valid, H/Ht where row < M and col < N).
+// the extents of the buffers it reads and writes (k_gemm reads rows < M of A,
+// K elements each, and the fragments of Bt; writes Y where row < m_valid and
+// col < n_valid, H where row < M and col < N).
 int run_gemm(cbz_ctx* c, const GemmArgs& g, const char* what) {
   if (!c->dry_regions) {
     HIPCHK(c, launch_gemm(g, c->stream));
@@ -1064,27 +1042,23 @@ int run_gemm(cbz_ctx* c, const GemmArgs& g, const char* what) {
                                       std::to_string(g.K) + ")");
   };
   if (g.M <= 0 || g.N <= 0) return CBZ_OK;
-  if (g.K <= 0 || g.K % 16 || g.lda < g.K || g.ldb < g.K) return bad("K");
+  if (g.K <= 0 || g.K % 16 || g.N % 32 || g.lda < g.K) return bad("K");
   const int64_t b2 = 2, b4 = 4;
   if (!dry_inside(c, g.A, ((g.M - 1) * g.lda + g.K) * b2)) return bad("A");
-  if (!dry_inside(c, g.Bt, ((g.N - 1) * g.ldb + g.K) * b2)) return bad("Bt");
+  if (!dry_inside(c, g.Bt, (frag_at(g.N - 1, g.K - 1, g.K) + 1) * b2)) return bad("Bt");
   const int64_t mv = std::min(g.M, g.m_valid), nv = std::min(g.N, g.n_valid);
   if (g.bias && nv > 0 && !dry_inside(c, g.bias, nv * b4)) return bad("bias");
   if (mv > 0 && nv > 0) {
-    if (g.Z && !dry_inside(c, g.Z, ((mv - 1) * g.ldz + nv) * b4)) return bad("Z");
     if (g.Y && !dry_inside(c, g.Y, ((mv - 1) * g.ldy + nv) * b4)) return bad("Y");
     if (g.y_scale && (!dry_inside(c, g.y_scale, nv * b4) || !dry_inside(c, g.y_shift, nv * b4))) return bad("y_scale");
   }
   if (g.H && !dry_inside(c, g.H, ((g.M - 1) * g.ldh + g.N) * b2)) return bad("H");
-  if (g.Ht && !dry_inside(c, g.Ht, ((g.N - 1) * g.ldht + g.M) * b2)) return bad("Ht");
   return CBZ_OK;
 }
 
-// Forward pass over M rows (Mpad = M rounded up to 32) of BF16 inputs X.
-// train: keep pre-activations, activations and their transposes for the
-// backward pass and write normalised outputs to Yout; else write
-// denormalised predictions to Yp.
-int sur_forward(cbz_ctx* c, const __bf16* X, int64_t M, int64_t Mpad, bool train) {
+// Forward pass over M rows (Mpad = M rounded up to 32) of BF16 inputs X,
+// layer by layer: denormalised predictions to Yp.
+int sur_forward(cbz_ctx* c, const __bf16* X, int64_t M, int64_t Mpad) {
   auto& u = c->sur;
   const LayerOff o = layer_offsets();
   const __bf16* in = X;
@@ -1095,33 +1069,22 @@ int sur_forward(cbz_ctx* c, const __bf16* X, int64_t M, int64_t Mpad, bool train
     g.K = layer_in_pad(l);
     g.A = in;
     g.lda = layer_in_pad(l);
-    g.Bt = u.Wnk[l];
-    g.ldb = layer_in_pad(l);
+    g.Bt = u.Wf[l];
     g.bias = u.params + o.b[l];
     g.act = l < kLayers - 1;
     g.m_valid = (int)M;
     g.n_valid = layer_out(l);
     if (l < kLayers - 1) {
-      __bf16* out = train ? u.Hb[l] : u.H[l % 2];
-      g.H = out;
+      g.H = u.H[l % 2];
       g.ldh = layer_out_pad(l);
-      if (train) {
-        g.Z = u.Z[l];
-        g.ldz = layer_out_pad(l);
-        g.Ht = u.At[l + 1];
-        g.ldht = Mpad;
-      }
-      in = out;
-    } else if (train) {
-      g.Y = u.Yout;
-      g.ldy = kOut;
+      in = g.H;
     } else {
       g.Y = u.Yp;
       g.ldy = kOut;
       g.y_scale = u.norm + 2 * kFeat + kOut;  // out_std
       g.y_shift = u.norm + 2 * kFeat;         // out_mean
     }
-    int rc = run_gemm(c, g, train ? "forward (training)" : "forward");
+    int rc = run_gemm(c, g, "forward");
     if (rc) return rc;
   }
   return CBZ_OK;
@@ -1138,7 +1101,7 @@ int sur_infer(cbz_ctx* c, const __bf16* X, int64_t M, const int64_t* M_dev = nul
   f.M_dev = M_dev;
   f.X = X;
   for (int l = 0; l < kLayers; ++l) {
-    f.W[l] = u.Wnk[l];
+    f.W[l] = u.Wf[l];
     f.bias[l] = u.params + o.b[l];
   }
   f.y_scale = u.norm + 2 * kFeat + kOut;  // out_std
@@ -1148,52 +1111,57 @@ int sur_infer(cbz_ctx* c, const __bf16* X, int64_t M, const int64_t* M_dev = nul
   return CBZ_OK;
 }
 
-// Backward pass of the mean-squared error against bT; gradients into grad.
-int sur_backward(cbz_ctx* c, int64_t M, int64_t Mpad) {
+// Forward, backward and, with `update`, Adam on a batch of M rows: sampled
+// from the dataset (step `step` of `seed`), or the staged rows.  The gradient
+// into grad, the loss into *loss (device).
+int sur_train_step(cbz_ctx* c, int64_t M, bool sample, uint64_t seed, uint64_t step, bool update, float lr,
+                   float* loss) {
   auto& u = c->sur;
   const LayerOff o = layer_offsets();
-  const bool dry = c->dry_regions != nullptr;
-  int rc;
-  if (!dry)
-    HIPCHK(c, launch_mse(u.Yout, u.bT, (int)Mpad, (int)M, u.row_loss, u.dZ[kLayers - 1], u.dZt[kLayers - 1],
-                         (int)Mpad, c->stream));
-  for (int l = kLayers - 1; l >= 0; --l) {
-    const int N = layer_out(l), K = layer_in(l), Np = layer_out_pad(l), Kp = layer_in_pad(l);
-    // dW = dZ^T * A_in : [Np x Mpad] * [Mpad x Kp]
-    GemmArgs g{};
-    g.M = Np;
-    g.N = Kp;
-    g.K = (int)Mpad;
-    g.A = u.dZt[l];
-    g.lda = Mpad;
-    g.Bt = u.At[l];
-    g.ldb = Mpad;
-    g.Y = u.grad + o.w[l];
-    g.ldy = K;
-    g.m_valid = N;
-    g.n_valid = K;
-    if ((rc = run_gemm(c, g, "weight gradient"))) return rc;
-    if (!dry) HIPCHK(c, launch_colsum(u.dZ[l], (int)Mpad, N, Np, u.grad + o.b[l], c->stream));
-    if (l > 0) {
-      // dA_in = dZ * W : [Mpad x Np] * [Np x Kp], B given as Wkn [Kp x Np]
-      GemmArgs h{};
-      h.M = (int)Mpad;
-      h.N = Kp;
-      h.K = Np;
-      h.A = u.dZ[l];
-      h.lda = Np;
-      h.Bt = u.Wkn[l];
-      h.ldb = Np;
-      h.Y = u.dA;
-      h.ldy = Kp;
-      h.m_valid = (int)M;
-      h.n_valid = Kp;
-      if ((rc = run_gemm(c, h, "input gradient"))) return rc;
-      if (!dry)
-        HIPCHK(c, launch_silu_bwd(u.dA, u.Z[l - 1], (int)Mpad, (int)M, Kp, Kp, u.dZ[l - 1], u.dZt[l - 1], (int)Mpad,
-                                c->stream));
-    }
+  const int64_t Mpad = round32(M);
+  TrainArgs r{};
+  r.M = (int)M;
+  r.Mpad = (int)Mpad;
+  r.Xraw = sample ? u.dsX : u.sx;
+  r.Yraw = sample ? u.dsY : u.sy;
+  r.rows = sample ? u.ds_rows : M;
+  r.sample = sample;
+  r.seed = seed;
+  r.step = step;
+  r.in_mean = u.norm;
+  r.in_inv_std = u.norm + kFeat;
+  r.out_mean = u.norm + 2 * kFeat;
+  r.out_inv_std = u.norm + 2 * kFeat + 2 * kOut;
+  UpdateArgs a{};
+  a.Mpad = (int)Mpad;
+  a.update = update;
+  for (int l = 0; l < kLayers; ++l) {
+    r.Wf[l] = a.Wf[l] = u.Wf[l];
+    r.Wb[l] = a.Wb[l] = u.Wb[l];
+    r.bias[l] = u.params + o.b[l];
+    a.At[l] = r.At[l] = u.At[l];
+    a.dZt[l] = r.dZt[l] = u.dZt[l];
+    a.off_w[l] = o.w[l];
+    a.off_b[l] = o.b[l];
   }
+  r.row_loss = u.row_loss;
+  a.row_loss = u.row_loss;
+  a.loss = loss;
+  a.grad = u.grad;
+  a.p = u.params;
+  a.m = u.adam_m;
+  a.v = u.adam_v;
+  if (update) {
+    u.adam_t += 1;
+    a.lr = lr;
+    a.b1 = 0.9f;
+    a.b2 = 0.999f;
+    a.eps = 1e-8f;
+    a.c1 = 1.0f / (1.0f - std::pow(a.b1, (float)u.adam_t));
+    a.c2 = 1.0f / (1.0f - std::pow(a.b2, (float)u.adam_t));
+  }
+  HIPCHK(c, launch_train_rows(r, c->stream));
+  HIPCHK(c, launch_train_update(a, c->stream));
   return CBZ_OK;
 }
 
@@ -1201,6 +1169,7 @@ int sur_ensure_batch(cbz_ctx* c, int rows) {
   auto& u = c->sur;
   const int Mpad = (int)round32(rows);
   if (Mpad <= u.batch_cap) return CBZ_OK;
+  u.batch_cap = 0;  // until every buffer is there
   int rc = CBZ_OK;
   sur_batch_buffers(u, Mpad, [&](auto*& p, int64_t n) {
     if (rc == CBZ_OK) rc = dalloc(c, &p, (size_t)n);
@@ -2519,23 +2488,8 @@ int cbz_sur_train(cbz_ctx* c, int32_t steps, int32_t batch, float lr, uint64_t s
     if ((rc = dalloc(c, &u.losses, (size_t)steps))) return rc;
     u.losses_cap = steps;
   }
-  const int64_t Mpad = round32(batch);
-  const LayerOff o = layer_offsets();
-  const float* nm = u.norm;
-  for (int32_t s = 0; s < steps; ++s) {
-    HIPCHK(c, launch_sample_idx(u.idx, batch, seed, (uint64_t)s, u.ds_rows, c->stream));
-    HIPCHK(c, launch_gather_batch(u.dsX, u.dsY, u.idx, (int)Mpad, batch, nm, nm + kFeat, nm + 2 * kFeat,
-                                  nm + 2 * kFeat + 2 * kOut, u.bX, u.At[0], u.bT, c->stream));
-    if ((rc = sur_forward(c, u.bX, batch, Mpad, true))) return rc;
-    if ((rc = sur_backward(c, batch, Mpad))) return rc;
-    HIPCHK(c, launch_sum_f32(u.row_loss, (int)Mpad, u.losses + s, c->stream));
-    u.adam_t += 1;
-    const float b1 = 0.9f, b2 = 0.999f;
-    const float c1 = 1.0f / (1.0f - std::pow(b1, (float)u.adam_t));
-    const float c2 = 1.0f / (1.0f - std::pow(b2, (float)u.adam_t));
-    HIPCHK(c, launch_adam(u.params, u.grad, u.adam_m, u.adam_v, o.total, lr, b1, b2, 1e-8f, c1, c2, c->stream));
-    if ((rc = sur_pack(c))) return rc;
-  }
+  for (int32_t s = 0; s < steps; ++s)
+    if ((rc = sur_train_step(c, batch, true, seed, (uint64_t)s, true, lr, u.losses + s))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (losses && steps > 0) HIPCHK(c, hipMemcpy(losses, u.losses, steps * sizeof(float), hipMemcpyDeviceToHost));
   return CBZ_OK;
@@ -2563,9 +2517,21 @@ int cbz_sur_check_gemms(int32_t rows, char* msg, int32_t msg_len) {
   sur_infer_buffers(fake.sur, Mpad, place);
   sur_layered_buffers(fake.sur, Mpad, place);
   fake.dry_regions = &regions;
-  int rc = sur_forward(&fake, fake.sur.bX, rows, Mpad, true);
-  if (!rc) rc = sur_backward(&fake, rows, Mpad);
-  if (!rc) rc = sur_forward(&fake, fake.sur.bX, rows, Mpad, false);
+  // the weight gradients of a training step: every fragment of both operands
+  // and the sums they give
+  int rc = CBZ_OK;
+  const LayerOff o = layer_offsets();
+  for (int l = 0; l < kLayers && !rc; ++l) {
+    const auto& u = fake.sur;
+    const int64_t a = batch_at(layer_out_pad(l) - 1, Mpad - 1, layer_out_pad(l)) + 1;
+    const int64_t b = batch_at(layer_in_frag(l) - 1, Mpad - 1, layer_in_frag(l)) + 1;
+    if (!dry_inside(&fake, u.dZt[l], a * (int64_t)sizeof(__bf16)) ||
+        !dry_inside(&fake, u.At[l], b * (int64_t)sizeof(__bf16)) ||
+        !dry_inside(&fake, u.grad + o.w[l], int64_t(layer_out(l)) * layer_in(l) * (int64_t)sizeof(float)) ||
+        !dry_inside(&fake, u.grad + o.b[l], layer_out(l) * (int64_t)sizeof(float)))
+      rc = fail(&fake, CBZ_ERR_STATE, "weight gradient of layer " + std::to_string(l) + " outside its buffers");
+  }
+  if (!rc) rc = sur_forward(&fake, fake.sur.X, rows, Mpad);
   if (msg && msg_len > 0) {
     std::snprintf(msg, (size_t)msg_len, "%s", rc ? fake.err.c_str() : "");
   }
@@ -2575,25 +2541,15 @@ int cbz_sur_check_gemms(int32_t rows, char* msg, int32_t msg_len) {
 // rows of raw features (and raw labels) -> the staging batch
 static int sur_stage_rows(cbz_ctx* c, int32_t rows, const float* X, const float* Y) {
   auto& u = c->sur;
-  int rc = sur_ensure_batch(c, rows);
-  if (rc) return rc;
-  const int64_t Mpad = round32(rows);
-  float *dx = nullptr, *dy = nullptr;
-  HIPCHK(c, hipMalloc((void**)&dx, (size_t)rows * kFeat * sizeof(float)));
-  HIPCHK(c, hipMalloc((void**)&dy, (size_t)rows * kOut * sizeof(float)));
-  std::vector<int64_t> idx((size_t)rows);
-  for (int i = 0; i < rows; ++i) idx[i] = i;
-  hipError_t e = hipMemcpy(dx, X, rows * kFeat * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess && Y) e = hipMemcpy(dy, Y, rows * kOut * sizeof(float), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(u.idx, idx.data(), rows * sizeof(int64_t), hipMemcpyHostToDevice);
-  const float* nm = u.norm;
-  if (e == hipSuccess)
-    e = launch_gather_batch(dx, Y ? dy : nullptr, u.idx, (int)Mpad, rows, nm, nm + kFeat, nm + 2 * kFeat,
-                            nm + 2 * kFeat + 2 * kOut, u.bX, u.At[0], u.bT, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  (void)hipFree(dx);
-  (void)hipFree(dy);
-  if (e != hipSuccess) return fail(c, CBZ_ERR_HIP, std::string("sur: staging: ") + hipGetErrorString(e));
+  if (rows > u.stage_cap) {
+    int rc;
+    u.stage_cap = 0;
+    if ((rc = dalloc(c, &u.sx, (size_t)rows * kFeat)) || (rc = dalloc(c, &u.sy, (size_t)rows * kOut))) return rc;
+    u.stage_cap = rows;
+  }
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, hipMemcpy(u.sx, X, (size_t)rows * kFeat * sizeof(float), hipMemcpyHostToDevice));
+  if (Y) HIPCHK(c, hipMemcpy(u.sy, Y, (size_t)rows * kOut * sizeof(float), hipMemcpyHostToDevice));
   return CBZ_OK;
 }
 
@@ -2601,18 +2557,17 @@ int cbz_sur_grad(cbz_ctx* c, int32_t rows, const float* X, const float* Y, float
   if (!c || rows <= 0 || !X || !Y) return fail(c, CBZ_ERR_ARG, "sur_grad: bad arguments");
   if (!c->sur.have_model) return fail(c, CBZ_ERR_STATE, "sur_grad: no model");
   HIPCHK(c, hipSetDevice(c->device));
-  int rc = sur_stage_rows(c, rows, X, Y);
+  int rc = sur_ensure_batch(c, rows);
   if (rc) return rc;
+  if ((rc = sur_stage_rows(c, rows, X, Y))) return rc;
   auto& u = c->sur;
-  const int64_t Mpad = round32(rows);
-  if ((rc = sur_forward(c, u.bX, rows, Mpad, true))) return rc;
-  if ((rc = sur_backward(c, rows, Mpad))) return rc;
-  float* dl = nullptr;
-  HIPCHK(c, hipMalloc((void**)&dl, sizeof(float)));
-  HIPCHK(c, launch_sum_f32(u.row_loss, (int)Mpad, dl, c->stream));
+  if (!u.losses) {
+    if ((rc = dalloc(c, &u.losses, 1))) return rc;
+    u.losses_cap = 1;
+  }
+  if ((rc = sur_train_step(c, rows, false, 0, 0, false, 0.f, u.losses))) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (loss) HIPCHK(c, hipMemcpy(loss, dl, sizeof(float), hipMemcpyDeviceToHost));
-  (void)hipFree(dl);
+  if (loss) HIPCHK(c, hipMemcpy(loss, u.losses, sizeof(float), hipMemcpyDeviceToHost));
   if (grad) HIPCHK(c, hipMemcpy(grad, u.grad, layer_offsets().total * sizeof(float), hipMemcpyDeviceToHost));
   return CBZ_OK;
 }
@@ -2621,16 +2576,17 @@ int cbz_sur_predict(cbz_ctx* c, int32_t rows, const float* X, float* Y, int32_t 
   if (!c || rows <= 0 || !X || !Y) return fail(c, CBZ_ERR_ARG, "sur_predict: bad arguments");
   if (!c->sur.have_model) return fail(c, CBZ_ERR_STATE, "sur_predict: no model");
   HIPCHK(c, hipSetDevice(c->device));
-  int rc = sur_stage_rows(c, rows, X, nullptr);
+  int rc = sur_ensure_inference(c, rows);
   if (rc) return rc;
+  if ((rc = sur_stage_rows(c, rows, X, nullptr))) return rc;
   auto& u = c->sur;
-  if ((rc = sur_ensure_inference(c, rows))) return rc;
   const int64_t Mpad = round32(rows);
+  HIPCHK(c, launch_normalise_rows(u.sx, (int)Mpad, rows, u.norm, u.norm + kFeat, u.X, c->stream));
   if (flags & CBZ_SUR_PREDICT_LAYERED) {
     if ((rc = sur_ensure_layered(c, rows))) return rc;
-    rc = sur_forward(c, u.bX, rows, Mpad, false);
+    rc = sur_forward(c, u.X, rows, Mpad);
   } else
-    rc = sur_infer(c, u.bX, rows);
+    rc = sur_infer(c, u.X, rows);
   if (rc) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   HIPCHK(c, hipMemcpy(Y, u.Yp, (size_t)rows * kOut * sizeof(float), hipMemcpyDeviceToHost));
@@ -2650,14 +2606,13 @@ int cbz_sur_predict_device(cbz_ctx* c, int32_t rows, const float* features, floa
   auto& u = c->sur;
   const float* nm = u.norm;
   __bf16* X = (__bf16*)c->scratch;  // every row the network reads is written here first
-  HIPCHK(c, launch_gather_batch(features, nullptr, nullptr, rows, rows, nm, nm + kFeat, nm + 2 * kFeat,
-                                nm + 2 * kFeat + 2 * kOut, X, nullptr, nullptr, c->stream));
+  HIPCHK(c, launch_normalise_rows(features, rows, rows, nm, nm + kFeat, X, c->stream));
   const LayerOff o = layer_offsets();
   MlpArgs f{};
   f.M = rows;
   f.X = X;
   for (int l = 0; l < kLayers; ++l) {
-    f.W[l] = u.Wnk[l];
+    f.W[l] = u.Wf[l];
     f.bias[l] = u.params + o.b[l];
   }
   f.y_scale = u.norm + 2 * kFeat + kOut;  // out_std

@@ -11,35 +11,25 @@
 //   k_degree      contacts per body (an input feature)
 //   k_features    the 40 input features of every contact, normalised, BF16
 //   k_gemm        C = A * B (+bias, SiLU) on MFMA 32x32x16, FP32 accumulate
-//   k_silu_bwd, k_mse, k_colsum, k_adam   backward pass and optimiser
+//   k_mlp_forward all four layers per block of rows
 //   k_sur_scatter per world: sum the predicted changes per body (the
 //                 resolver then polishes or re-solves the world)
+// Training is in k_train.hip.
 #include <algorithm>
 #include <climits>
 
 #include "cbz_devmath.h"
 #include "cbz_launch.h"
+#include "cbz_mfma.h"
 #include "cbz_mlp.h"
 #include "cbz_types.h"
 #include "cbz_wave.h"
 
 namespace cbz {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
 template <typename R>
 __device__ __forceinline__ V3<R> ld3c(const R* a, int64_t s, int64_t i) {
   return V3<R>{a[i], a[s + i], a[2 * s + i]};
-}
-
-// SiLU with the hardware reciprocal (about 1 ulp): its result is rounded to
-// BF16 for the next layer
-__device__ __forceinline__ float silu(float z) { return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z)); }
-__device__ __forceinline__ float silu_grad(float z) {
-  const float s = 1.0f / (1.0f + __expf(-z));
-  return s * (1.0f + z * (1.0f - s));
 }
 
 // ---------------------------------------------------------------------------
@@ -155,36 +145,16 @@ __global__ void __launch_bounds__(256) k_features_world(Bodies<R> b, Contacts<R>
   }
 }
 
-// Batch sampling on the device: row i of training step `step` is
-// SplitMix64(seed, step * n + i) mod rows (uniform with replacement).
-__global__ void k_sample_idx(int64_t* idx, int n, uint64_t seed, uint64_t step, int64_t rows) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint64_t z = seed * 0xD1B54A32D192ED03ull + (step * uint64_t(n) + uint64_t(i) + 1ull) * 0x9E3779B97F4A7C15ull;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  z ^= z >> 31;
-  idx[i] = int64_t(z % uint64_t(rows));
-}
-
-// raw features / labels of a sampled batch -> normalised BF16 inputs and
-// FP32 targets (training).  idx null takes rows 0..valid_rows-1 in order;
-// Xt (the transposed copy) and T (the targets) may be null.
-__global__ void k_gather_batch(const float* Xraw, const float* Yraw, const int64_t* idx, int rows, int valid_rows,
-                               const float* in_mean, const float* in_inv_std, const float* out_mean,
-                               const float* out_inv_std, __bf16* X, __bf16* Xt, float* T) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows) return;
-  const bool v = i < valid_rows;
-  const int64_t s = v ? (idx ? idx[i] : int64_t(i)) : 0;  // idx null: row i itself
-  for (int k = 0; k < kFeatPad; ++k) {
-    const __bf16 x = __bf16(v && k < kFeat ? (Xraw[s * kFeat + k] - in_mean[k]) * in_inv_std[k] : 0.f);
-    X[int64_t(i) * kFeatPad + k] = x;
-    if (Xt) Xt[int64_t(k) * rows + i] = x;
-  }
-  if (T)
-    for (int k = 0; k < kOut; ++k)
-      T[int64_t(i) * kOut + k] = v && Yraw ? (Yraw[s * kOut + k] - out_mean[k]) * out_inv_std[k] : 0.f;
+// Raw feature rows -> normalised BF16 rows (zeros from valid_rows on).  Four
+// rows of 48 values per 192 threads: consecutive threads read consecutive
+// features and write consecutive values.
+__global__ void __launch_bounds__(192) k_normalise_rows(const float* Xraw, int rows, int valid_rows,
+                                                        const float* in_mean, const float* in_inv_std, __bf16* X) {
+  const int k = threadIdx.x % kFeatPad;
+  const bool feat = k < kFeat;
+  const float mean = feat ? in_mean[k] : 0.f, inv = feat ? in_inv_std[k] : 0.f;
+  for (int64_t i = int64_t(blockIdx.x) * 4 + threadIdx.x / kFeatPad; i < rows; i += int64_t(gridDim.x) * 4)
+    X[i * kFeatPad + k] = __bf16(feat && i < valid_rows ? (Xraw[i * kFeat + k] - mean) * inv : 0.f);
 }
 
 // column mean and standard deviation of a row-major FP32 table (one block
@@ -247,13 +217,12 @@ __global__ void k_fill_f32(float* p, int64_t n, float v) {
 // GEMM on the matrix cores
 // ---------------------------------------------------------------------------
 // C[M x N] = A[M x K] * B[K x N] with A row-major (K contiguous) and B given
-// as Bt = [N x K] row-major (K contiguous): both operands load their MFMA
-// fragments as 16-byte vectors.  Fragment layout of v_mfma_f32_32x32x16_bf16
-// for lane l (r = l % 32, h = l / 32): A[r][8h .. 8h+7], B[8h .. 8h+7][r],
+// as Bt = [N x K] in fragments (frag_at).  Fragment layout of
+// v_mfma_f32_32x32x16_bf16 for lane l (r = l % 32, h = l / 32): A[r][8h .. 8h+7], B[8h .. 8h+7][r],
 // and accumulator j holds D[8 (j/4) + 4h + j%4][r].  Each wave computes one
-// 32x32 tile; a block holds WM x WN waves.  K is a multiple of 16.  A tile
-// that extends past row M of A or row N of Bt reads zeros there and writes
-// nothing there, so an operand needs only M (N) rows.
+// 32x32 tile; a block holds WM x WN waves.  K is a multiple of 16, N of 32.
+// A tile that extends past row M of A reads zeros there and writes nothing
+// there, so A needs only M rows.
 template <int WM, int WN>
 __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -261,18 +230,17 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
   const int n0 = (blockIdx.y * WN + wave / WM) * 32;
   if (m0 >= g.M || n0 >= g.N) return;
   const int r = lane & 31, h = lane >> 5;
-  const bool a_in = m0 + r < g.M, b_in = n0 + r < g.N;
+  const bool a_in = m0 + r < g.M;
   const __bf16* ap = g.A + int64_t(a_in ? m0 + r : 0) * g.lda + 8 * h;
-  const __bf16* bp = g.Bt + int64_t(b_in ? n0 + r : 0) * g.ldb + 8 * h;
+  const __bf16* bp = g.Bt + frag_at(n0 + r, 8 * h, g.K);
   f32x16 acc = {};
   const bf16x8 zero = {};
   for (int k = 0; k < g.K; k += 16) {
     const bf16x8 a = a_in ? *(const bf16x8*)(ap + k) : zero;
-    const bf16x8 bb = b_in ? *(const bf16x8*)(bp + k) : zero;
+    const bf16x8 bb = *(const bf16x8*)(bp + k * 32);
     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bb, acc, 0, 0, 0);
   }
   const int col = n0 + r;
-  if (col >= g.N) return;
   // bias has n_valid entries (padding columns produce zeros)
   const float bias = g.bias && col < g.n_valid ? g.bias[col] : 0.f;
 #pragma unroll
@@ -282,90 +250,24 @@ __global__ void __launch_bounds__(64 * WM * WN) k_gemm(GemmArgs g) {
     const float z = acc[j] + bias;
     const float y = g.act ? silu(z) : z;
     if (row < g.m_valid && col < g.n_valid) {
-      if (g.Z) g.Z[int64_t(row) * g.ldz + col] = z;
       if (g.Y) g.Y[int64_t(row) * g.ldy + col] = g.y_scale ? y * g.y_scale[col] + g.y_shift[col] : y;
     }
     // BF16 activations keep their zero padding (rows >= m_valid, cols >= n_valid)
     const float yv = (row < g.m_valid && col < g.n_valid) ? y : 0.f;
     if (g.H) g.H[int64_t(row) * g.ldh + col] = __bf16(yv);
-    if (g.Ht) g.Ht[int64_t(col) * g.ldht + row] = __bf16(yv);
   }
 }
 
-// dZ = dA * SiLU'(Z), written as BF16 row-major and transposed.
-__global__ void k_silu_bwd(const float* dA, const float* Z, int rows, int valid_rows, int cols, int ld, __bf16* dZ,
-                           __bf16* dZt, int ldt) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= int64_t(rows) * cols) return;
-  const int r = int(i / cols), c = int(i % cols);
-  const float v = r < valid_rows ? dA[int64_t(r) * ld + c] * silu_grad(Z[int64_t(r) * ld + c]) : 0.f;
-  dZ[int64_t(r) * ld + c] = __bf16(v);
-  dZt[int64_t(c) * ldt + r] = __bf16(v);
-}
-
-// Mean-squared error over rows x kOut; writes dL/dY as BF16 (row-major,
-// width kOutPad, and transposed) and the per-row squared error.
-__global__ void k_mse(const float* Y, const float* T, int rows, int valid_rows, float* row_loss, __bf16* dY,
-                      __bf16* dYt, int ldt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows) return;
-  float acc = 0.f;
-  for (int k = 0; k < kOutPad; ++k) {
-    float d = 0.f;
-    if (k < kOut && i < valid_rows) {
-      const float e = Y[int64_t(i) * kOut + k] - T[int64_t(i) * kOut + k];
-      acc += e * e;
-      d = 2.0f * e / float(valid_rows * kOut);
-    }
-    dY[int64_t(i) * kOutPad + k] = __bf16(d);
-    dYt[int64_t(k) * ldt + i] = __bf16(d);
-  }
-  row_loss[i] = i < valid_rows ? acc / float(valid_rows * kOut) : 0.f;
-}
-
-// column sums of a row-major BF16 matrix: bias gradient, and (FP32 input)
-// the loss.  One thread per column, rows summed in order.
-__global__ void k_colsum(const __bf16* A, int rows, int cols, int ld, float* out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
-  float s = 0.f;
-  for (int r = 0; r < rows; ++r) s += float(A[int64_t(r) * ld + c]);
-  out[c] = s;
-}
-__global__ void k_sum_f32(const float* a, int n, float* out) {
-  __shared__ float part[256];
-  float s = 0.f;
-  for (int i = threadIdx.x; i < n; i += 256) s += a[i];
-  part[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = part[0];
-}
-
-// Adam on the FP32 master parameters, then refresh the BF16 copies of one
-// layer's weights: Wnk [N x Kpad] (forward B-operand layout) and Wkn
-// [K x Npad] (backward), padding left at zero.
-__global__ void k_adam(float* p, const float* grad, float* m, float* v, int64_t n, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gr = grad[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gr;
-  const float vi = b2 * v[i] + (1.f - b2) * gr * gr;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
-}
-__global__ void k_pack_weights(const float* W, int N, int K, __bf16* Wnk, int kpad, __bf16* Wkn, int npad) {
+// The BF16 copies of one layer's weights in fragments: Wf [Npad x Kpad] for
+// the forward pass and Wb [Kpad x Npad] for the backward (null: none), padding
+// left at zero.
+__global__ void k_pack_weights(const float* W, int N, int K, __bf16* Wf, int kpad, __bf16* Wb, int npad) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N * K) return;
   const int n = i / K, k = i % K;
   const __bf16 w = __bf16(W[i]);
-  Wnk[int64_t(n) * kpad + k] = w;
-  Wkn[int64_t(k) * npad + n] = w;
+  Wf[frag_at(n, k, kpad)] = w;
+  if (Wb) Wb[frag_at(k, n, npad)] = w;
 }
 
 // ---------------------------------------------------------------------------
@@ -374,7 +276,9 @@ __global__ void k_pack_weights(const float* W, int N, int K, __bf16* Wnk, int kp
 // One workgroup (4 waves) per block of kFuseRows rows runs all four layers:
 // the block's activations stay in LDS (one 128 x 256 BF16 tile, updated in
 // place), so HBM sees only the BF16 features in and the 13 outputs out; the
-// weights stream from the L2, once per 128 rows.  Each wave computes a
+// weights stream from the L2, once per 128 rows, as contiguous 1 KB fragments
+// (57 us for 100003 rows; 61 from row-major weights, whose fragments are 32
+// pieces of 32 bytes).  Each wave computes a
 // 128-row x 64-column slab of a hidden layer as 4 x 2 MFMA 32x32x16 tiles
 // (eight independent accumulators).  The k order of every dot product is
 // that of k_gemm, so the results are the same bits.  LDS element (row, k) sits at
@@ -384,8 +288,6 @@ constexpr int kFuseRows = 128;
 constexpr int kRowTiles = kFuseRows / 32;  // 32-row MFMA tiles per block (one per wave in layer 3)
 constexpr int kFuseWaves = 4;
 constexpr int kColTiles = kHidden / 32 / kFuseWaves;  // 32-column tiles per wave
-
-__device__ __forceinline__ int fswz(int row, int k) { return row * kHidden + ((((k >> 3) ^ (row & 31))) << 3) + (k & 7); }
 
 // One block of kFuseRows rows starting at m0 (of M rows), all four layers.
 __device__ __forceinline__ void mlp_block(const MlpArgs& f, int64_t M, int64_t m0, __bf16* H) {
@@ -431,7 +333,7 @@ __device__ __forceinline__ void mlp_block(const MlpArgs& f, int64_t M, int64_t m
       a[t] = row < M ? *(const bf16x8*)(f.X + row * kFeatPad + k + 8 * h) : bf16x8{};
     }
 #pragma unroll
-    for (int u = 0; u < kColTiles; ++u) b[u] = *(const bf16x8*)(f.W[0] + (wave * 32 * kColTiles + 32 * u + r) * kFeatPad + k + 8 * h);
+    for (int u = 0; u < kColTiles; ++u) b[u] = *(const bf16x8*)(f.W[0] + frag_at((wave * kColTiles + u) * 32, k, kFeatPad) + lane * 8);
 #pragma unroll
     for (int t = 0; t < kRowTiles; ++t)
 #pragma unroll
@@ -452,7 +354,7 @@ __device__ __forceinline__ void mlp_block(const MlpArgs& f, int64_t M, int64_t m
 #pragma unroll
       for (int t = 0; t < kRowTiles; ++t) a[t] = *(const bf16x8*)(H + fswz(32 * t + r, k + 8 * h));
 #pragma unroll
-      for (int u = 0; u < kColTiles; ++u) b[u] = *(const bf16x8*)(W + (wave * 32 * kColTiles + 32 * u + r) * kHidden + k + 8 * h);
+      for (int u = 0; u < kColTiles; ++u) b[u] = *(const bf16x8*)(W + frag_at((wave * kColTiles + u) * 32, k, kHidden) + lane * 8);
 #pragma unroll
       for (int t = 0; t < kRowTiles; ++t)
 #pragma unroll
@@ -470,7 +372,7 @@ __device__ __forceinline__ void mlp_block(const MlpArgs& f, int64_t M, int64_t m
 #pragma unroll 4
     for (int k = 0; k < kHidden; k += 16) {
       const bf16x8 a = *(const bf16x8*)(H + fswz(32 * wave + r, k + 8 * h));
-      const bf16x8 b = *(const bf16x8*)(W + r * kHidden + k + 8 * h);
+      const bf16x8 b = *(const bf16x8*)(W + frag_at(0, k, kHidden) + lane * 8);
       y = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, y, 0, 0, 0);
     }
     const int64_t row = m0 + 32 * wave + r;
@@ -649,8 +551,8 @@ __global__ void __launch_bounds__(256) k_sur_scatter(SurApply<R> a) {
 // ---------------------------------------------------------------------------
 hipError_t launch_gemm(const GemmArgs& g, hipStream_t st) {
   if (g.M <= 0 || g.N <= 0) return hipSuccess;
-  // the fragment loads step K by 16 and read K contiguous elements per row
-  if (g.K <= 0 || g.K % 16 != 0 || g.lda < g.K || g.ldb < g.K) return hipErrorInvalidValue;
+  // the fragment loads step K by 16 and read K elements per row
+  if (g.K <= 0 || g.K % 16 != 0 || g.N % 32 != 0 || g.lda < g.K) return hipErrorInvalidValue;
   if (g.N >= 128) {
     dim3 grid((g.M + 63) / 64, (g.N + 63) / 64);
     k_gemm<2, 2><<<grid, 256, 0, st>>>(g);
@@ -693,16 +595,10 @@ hipError_t launch_sur_scatter(const SurApply<R>& a, int n_worlds, hipStream_t st
   return hipGetLastError();
 }
 
-hipError_t launch_gather_batch(const float* Xraw, const float* Yraw, const int64_t* idx, int rows, int valid_rows,
-                               const float* in_mean, const float* in_inv_std, const float* out_mean,
-                               const float* out_inv_std, __bf16* X, __bf16* Xt, float* T, hipStream_t st) {
-  k_gather_batch<<<(rows + 255) / 256, 256, 0, st>>>(Xraw, Yraw, idx, rows, valid_rows, in_mean, in_inv_std,
-                                                   out_mean, out_inv_std, X, Xt, T);
-  return hipGetLastError();
-}
-hipError_t launch_sample_idx(int64_t* idx, int n, uint64_t seed, uint64_t step, int64_t rows, hipStream_t st) {
-  if (n <= 0 || rows <= 0) return hipSuccess;
-  k_sample_idx<<<(n + 255) / 256, 256, 0, st>>>(idx, n, seed, step, rows);
+hipError_t launch_normalise_rows(const float* Xraw, int rows, int valid_rows, const float* in_mean,
+                                 const float* in_inv_std, __bf16* X, hipStream_t st) {
+  if (rows <= 0) return hipSuccess;
+  k_normalise_rows<<<std::min((rows + 3) / 4, 4096), 192, 0, st>>>(Xraw, rows, valid_rows, in_mean, in_inv_std, X);
   return hipGetLastError();
 }
 hipError_t launch_col_stats(const float* A, int64_t rows, int cols, float* mean, float* stdv, hipStream_t st) {
@@ -722,33 +618,9 @@ hipError_t launch_fill_f32(float* p, int64_t n, float v, hipStream_t st) {
   k_fill_f32<<<int((n + 255) / 256), 256, 0, st>>>(p, n, v);
   return hipGetLastError();
 }
-hipError_t launch_silu_bwd(const float* dA, const float* Z, int rows, int valid_rows, int cols, int ld, __bf16* dZ,
-                           __bf16* dZt, int ldt, hipStream_t st) {
-  const int64_t n = int64_t(rows) * cols;
-  k_silu_bwd<<<int((n + 255) / 256), 256, 0, st>>>(dA, Z, rows, valid_rows, cols, ld, dZ, dZt, ldt);
-  return hipGetLastError();
-}
-hipError_t launch_mse(const float* Y, const float* T, int rows, int valid_rows, float* row_loss, __bf16* dY,
-                      __bf16* dYt, int ldt, hipStream_t st) {
-  k_mse<<<(rows + 255) / 256, 256, 0, st>>>(Y, T, rows, valid_rows, row_loss, dY, dYt, ldt);
-  return hipGetLastError();
-}
-hipError_t launch_colsum(const __bf16* A, int rows, int cols, int ld, float* out, hipStream_t st) {
-  k_colsum<<<(cols + 63) / 64, 64, 0, st>>>(A, rows, cols, ld, out);
-  return hipGetLastError();
-}
-hipError_t launch_sum_f32(const float* a, int n, float* out, hipStream_t st) {
-  k_sum_f32<<<1, 256, 0, st>>>(a, n, out);
-  return hipGetLastError();
-}
-hipError_t launch_adam(float* p, const float* grad, float* m, float* v, int64_t n, float lr, float b1, float b2,
-                       float eps, float c1, float c2, hipStream_t st) {
-  k_adam<<<int((n + 255) / 256), 256, 0, st>>>(p, grad, m, v, n, lr, b1, b2, eps, c1, c2);
-  return hipGetLastError();
-}
-hipError_t launch_pack_weights(const float* W, int N, int K, __bf16* Wnk, int kpad, __bf16* Wkn, int npad,
+hipError_t launch_pack_weights(const float* W, int N, int K, __bf16* Wf, int kpad, __bf16* Wb, int npad,
                                hipStream_t st) {
-  k_pack_weights<<<(N * K + 255) / 256, 256, 0, st>>>(W, N, K, Wnk, kpad, Wkn, npad);
+  k_pack_weights<<<(N * K + 255) / 256, 256, 0, st>>>(W, N, K, Wf, kpad, Wb, npad);
   return hipGetLastError();
 }
 
