@@ -123,6 +123,7 @@ struct cbz_context {
   int64_t cand_cap = 0;
   // explicit-list pair space (grown on demand)
   int32_t l_tiles_cap = 0, l_pairs_cap = 0;
+  int32_t l_max_tiles = 0;  // the most tiles of one world in the last pair list
   int32_t* l_tile_world = nullptr;
   int32_t* l_world_tile0 = nullptr;
   int32_t* l_world_q = nullptr;
@@ -135,16 +136,15 @@ struct cbz_context {
   struct Broad {
     bool ready = false;
     int32_t* body_world = nullptr;     // [nb]
-    double* lo = nullptr;              // [2][nb]
-    double* hi = nullptr;              // [2][nb]
+    BroadBox* box = nullptr;           // [nb]
     float* hix = nullptr;              // [nb]
-    uint8_t* wild = nullptr;           // [nb]
     uint64_t* key_in = nullptr;        // [nb]
     uint64_t* key_out = nullptr;
     int32_t* val_in = nullptr;
     int32_t* val_out = nullptr;
     int64_t* plane_base = nullptr;     // [nw]
     int64_t plane_pairs = 0;
+    int64_t slots = 0;                 // the most planes and bodies of one world
     uint64_t* pkey_in = nullptr;       // [pcap]
     uint64_t* pkey = nullptr;
     int64_t pcap = 0;
@@ -400,10 +400,8 @@ void free_scene(cbz_ctx* c) {
   {
     auto& bp = c->bp;
     dfree(bp.body_world);
-    dfree(bp.lo);
-    dfree(bp.hi);
+    dfree(bp.box);
     dfree(bp.hix);
-    dfree(bp.wild);
     dfree(bp.key_in);
     dfree(bp.key_out);
     dfree(bp.val_in);
@@ -591,7 +589,7 @@ int do_narrowphase(cbz_ctx* c, int32_t list_tiles, hipEvent_t* ev = nullptr) {
     L.ps.list_two = nullptr;
   } else {
     L.ps.n_tiles = list_tiles;
-    L.ps.max_world_tiles = 0;  // list worlds are short: the one-wave scan
+    L.ps.max_world_tiles = c->l_max_tiles;
     L.ps.tile_world = c->l_tile_world;
     L.ps.world_tile0 = c->l_world_tile0;
     L.ps.world_q = c->l_world_q;
@@ -743,9 +741,11 @@ int check_overflow(cbz_ctx* c);
 int run_list_narrowphase(cbz_ctx* c, const std::vector<int32_t>& wq, int64_t* total) {
   std::vector<int32_t> wt0(c->nw + 1), tw;
   int64_t nt = 0;
+  c->l_max_tiles = 0;
   for (int32_t w = 0; w < c->nw; ++w) {
     wt0[w] = (int32_t)nt;
     nt += (wq[w] + 63) / 64;
+    c->l_max_tiles = std::max(c->l_max_tiles, (wq[w] + 63) / 64);
   }
   wt0[c->nw] = (int32_t)nt;
   if (nt > INT32_MAX / 64) return fail(c, CBZ_ERR_ARG, "narrowphase: pair list too long");
@@ -778,16 +778,17 @@ int bp_ensure(cbz_ctx* c, int64_t pcap) {
     std::vector<int32_t> bw(nb, 0);
     std::vector<int64_t> base((size_t)c->nw, 0);
     int64_t acc = 0;
+    bp.slots = 0;
     for (int32_t w = 0; w < c->nw; ++w) {
       for (int32_t i = c->body_off[w]; i < c->body_off[w + 1]; ++i) bw[i] = w;
       base[w] = acc;
-      acc += (int64_t)(c->body_off[w + 1] - c->body_off[w]) * (c->plane_off[w + 1] - c->plane_off[w]);
+      const int64_t n = c->body_off[w + 1] - c->body_off[w], np = c->plane_off[w + 1] - c->plane_off[w];
+      acc += n * np;
+      bp.slots = std::max(bp.slots, n + np);
     }
     if ((rc = dalloc(c, &bp.body_world, nb))) return rc;
-    if ((rc = dalloc(c, &bp.lo, 2 * nb))) return rc;
-    if ((rc = dalloc(c, &bp.hi, 2 * nb))) return rc;
+    if ((rc = dalloc(c, &bp.box, nb))) return rc;
     if ((rc = dalloc(c, &bp.hix, nb))) return rc;
-    if ((rc = dalloc(c, &bp.wild, nb))) return rc;
     if ((rc = dalloc(c, &bp.key_in, nb))) return rc;
     if ((rc = dalloc(c, &bp.key_out, nb))) return rc;
     if ((rc = dalloc(c, &bp.val_in, nb))) return rc;
@@ -819,16 +820,15 @@ BroadArgs<R> bp_args(cbz_ctx* c) {
   auto& bp = c->bp;
   BroadArgs<R> a;
   a.nb = (int32_t)c->nb;
+  a.nw = c->nw;
   a.stride = c->nb;
   a.ctransform = (const R*)c->field[CBZ_CTRANSFORM];
   a.brad = c->brad;
   a.body_world = bp.body_world;
   a.body_off = c->d_body_off;
   a.plane_off = c->d_plane_off;
-  a.lo = bp.lo;
-  a.hi = bp.hi;
+  a.box = bp.box;
   a.hix = bp.hix;
-  a.wild = bp.wild;
   a.key_in = bp.key_in;
   a.key_out = bp.key_out;
   a.val_in = bp.val_in;
@@ -866,7 +866,7 @@ int do_broadphase(cbz_ctx* c, int64_t* n_pairs) {
   }
   const int64_t n = bp.plane_pairs + found;
   if ((rc = ensure_list(c, n))) return rc;
-  BroadList L{n, c->nw, bp.pkey_in, bp.pkey, bp.body_world, c->d_body_off, c->d_plane_off, c->l_one, c->l_two,
+  BroadList L{n, c->nw, c->nb, bp.slots, bp.pkey_in, bp.pkey, bp.body_world, c->d_body_off, c->d_plane_off, c->l_one, c->l_two,
               c->l_off};
   HIPCHK(c, launch_bp_list(L, bp.tmp, bp.tmp_bytes, c->stream));
   *n_pairs = n;

@@ -5,19 +5,21 @@
 
 namespace cbz {
 
+struct alignas(32) BroadBox {
+  double lo_y, lo_z, hi_y, hi_z;
+};
+
 template <typename R>
 struct BroadArgs {
-  int32_t nb;
+  int32_t nb, nw;
   int64_t stride;
   const R* ctransform;       // [12][stride]: collider centre in planes 9..11
   const double* brad;        // [nb] bounding radius
   const int32_t* body_world; // [nb]
   const int32_t* body_off;   // [nw + 1]
   const int32_t* plane_off;  // [nw + 1]
-  double* lo;                // [2][nb] lower y, z bounds
-  double* hi;                // [2][nb] upper y, z bounds
+  BroadBox* box;             // [nb] y, z bounds (a body that is not finite: everything)
   float* hix;                // [nb] upper x bound, rounded up
-  uint8_t* wild;             // [nb] centre or radius not finite
   uint64_t* key_in;          // [nb] world << 32 | ordered lower x bound (rounded down)
   uint64_t* key_out;         // [nb] sorted
   int32_t* val_in;           // [nb] body index
@@ -40,6 +42,7 @@ struct BroadPlanes {
 struct BroadList {
   int64_t n;                 // pair keys
   int32_t nw;
+  int64_t nb, slots;         // bodies, and the most planes and bodies of one world: the keys' ranges
   const uint64_t* pkey_in;   // unsorted keys
   uint64_t* pkey;            // sorted keys
   const int32_t* body_world;

@@ -45,6 +45,13 @@ __device__ __forceinline__ float f32_unorder(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
+// bits of the numbers 0 .. n-1
+static int bits_for(int64_t n) {
+  int b = 0;
+  while ((int64_t(1) << b) < n) ++b;
+  return b;
+}
+
 // Boxes and the sort keys (world << 32 | ordered lower x bound, rounded down).
 template <typename R>
 __global__ void __launch_bounds__(256) k_bp_bounds(BroadArgs<R> a) {
@@ -55,19 +62,17 @@ __global__ void __launch_bounds__(256) k_bp_bounds(BroadArgs<R> a) {
   const double cy = double(a.ctransform[10 * S + i]);
   const double cz = double(a.ctransform[11 * S + i]);
   const double r = kBroadGrow * a.brad[i];
-  const bool wild = !(isfinite(cx) && isfinite(cy) && isfinite(cz) && isfinite(r));
-  float hx = INFINITY;  // a body that is not finite spans the whole axis
+  // a body that is not finite spans every axis
+  BroadBox box{-INFINITY, -INFINITY, INFINITY, INFINITY};
+  float hx = INFINITY;
   uint32_t kx = f32_order(-INFINITY);
-  if (!wild) {
-    a.lo[i] = cy - r;
-    a.lo[a.nb + i] = cz - r;
-    a.hi[i] = cy + r;
-    a.hi[a.nb + i] = cz + r;
+  if (isfinite(cx) && isfinite(cy) && isfinite(cz) && isfinite(r)) {
+    box = BroadBox{cy - r, cz - r, cy + r, cz + r};
     hx = f32_up(cx + r);
     kx = f32_order(f32_down(cx - r));
   }
+  a.box[i] = box;
   a.hix[i] = hx;
-  a.wild[i] = wild ? 1 : 0;
   a.key_in[i] = (uint64_t(uint32_t(a.body_world[i])) << 32) | kx;
   a.val_in[i] = i;
 }
@@ -82,61 +87,78 @@ __global__ void __launch_bounds__(256) k_bp_planes(BroadPlanes p) {
   for (int k = 0; k < np; ++k) p.pkey[at + k] = (uint64_t(uint32_t(i)) << 32) | uint32_t(k);
 }
 
-// Sweep along x over each world's sorted boxes: thread p scans forward from
-// sorted position p while the next lower bound is within its upper bound,
-// tests y and z, and appends both ordered pairs of every overlap.  Run once
-// to count (block-aggregated, one atomic per block) and write; entries past
-// the capacity are counted and dropped.
+// Sweep along x over each world's sorted boxes: position p meets the
+// positions after it up to the first lower bound past its upper bound, y and z
+// are tested, and both ordered pairs of every overlap are appended; entries
+// past the capacity are counted and dropped.
+//
+// A workgroup takes 64 positions, one per lane of each of its 4 waves, and
+// passes over what follows them in tiles of 128 boxes in LDS, a wave every
+// fourth box: a box is one broadcast read for 64 tests.  Overlaps are collected
+// in LDS, so that one atomic per workgroup reserves their places (a workgroup
+// with more of them appends the rest one by one).  40000 bodies with about 300
+// boxes each in reach along x take 36 us; with a thread per position walking them
+// by itself, twice (to count, then to write), they took 1063.
+constexpr int kSweepTile = 128;
+constexpr int kSweepHits = 2048;
+
 template <typename R>
 __global__ void __launch_bounds__(256) k_bp_sweep(BroadArgs<R> a) {
-  __shared__ int s_wtot[4];
+  __shared__ BroadBox s_box[kSweepTile];
+  __shared__ float s_lo[kSweepTile];
+  __shared__ int s_j[kSweepTile];
+  __shared__ int2 s_hit[kSweepHits];
+  __shared__ int s_n;
   __shared__ long long s_base;
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  int mine = 0;
-  int i = -1, w = 0, end = 0;
-  float hx = 0.0f;
-  if (p < a.nb) {
-    i = a.val_out[p];
-    w = int(a.key_out[p] >> 32);
-    end = a.body_off[w + 1];
-    hx = a.hix[i];
-    for (int q = p + 1; q < end; ++q) {
-      if (f32_unorder(uint32_t(a.key_out[q])) > hx) break;
-      const int j = a.val_out[q];
-      const bool keep = a.wild[i] || a.wild[j] ||
-                        (a.lo[j] <= a.hi[i] && a.lo[i] <= a.hi[j] && a.lo[a.nb + j] <= a.hi[a.nb + i] &&
-                         a.lo[a.nb + i] <= a.hi[a.nb + j]);
-      mine += keep ? 2 : 0;
-    }
-  }
-  // block-wide reservation (all 4 waves take part)
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int incl = wave_incl_scan_i32(mine);
-  if (lane == 63) s_wtot[wv] = incl;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int tot = 0;
-    for (int u = 0; u < 4; ++u) tot += s_wtot[u];
-    s_base = tot > 0 ? (long long)atomicAdd((unsigned long long*)a.pcount, (unsigned long long)tot) : 0;
-  }
-  __syncthreads();
-  int64_t at = int64_t(a.plane_pairs) + s_base;
-  for (int u = 0; u < wv; ++u) at += s_wtot[u];
-  at += incl - mine;
-  if (mine == 0) return;
-  const int b0 = a.body_off[w];
-  const int np = a.plane_off[w + 1] - a.plane_off[w];
-  for (int q = p + 1; q < end; ++q) {
-    if (f32_unorder(uint32_t(a.key_out[q])) > hx) break;
-    const int j = a.val_out[q];
-    const bool keep = a.wild[i] || a.wild[j] ||
-                      (a.lo[j] <= a.hi[i] && a.lo[i] <= a.hi[j] && a.lo[a.nb + j] <= a.hi[a.nb + i] &&
-                       a.lo[a.nb + i] <= a.hi[a.nb + j]);
-    if (!keep) continue;
+  const int t = threadIdx.x, wv = t >> 6;
+  const int first = blockIdx.x * 64, p = first + (t & 63);
+  if (t == 0) s_n = 0;
+  // both keys of a pair, i's row first
+  auto append = [&](int64_t at, int i, int j) {
+    const int w = a.body_world[i], b0 = a.body_off[w];
+    const int np = a.plane_off[w + 1] - a.plane_off[w];
     if (at < a.pcap) a.pkey[at] = (uint64_t(uint32_t(i)) << 32) | uint32_t(np + (j - b0));
     if (at + 1 < a.pcap) a.pkey[at + 1] = (uint64_t(uint32_t(j)) << 32) | uint32_t(np + (i - b0));
-    at += 2;
+  };
+  int i = 0, end = 0;
+  float hx = 0.f;
+  BroadBox b{};
+  if (p < a.nb) {
+    i = a.val_out[p];
+    end = a.body_off[int(a.key_out[p] >> 32) + 1];
+    hx = a.hix[i];
+    b = a.box[i];
   }
+  for (int q0 = first + 1;; q0 += kSweepTile) {
+    __syncthreads();  // every wave is done with the last tile
+    if (t < kSweepTile && q0 + t < a.nb) {
+      const int j = a.val_out[q0 + t];
+      s_j[t] = j;
+      s_lo[t] = f32_unorder(uint32_t(a.key_out[q0 + t]));
+      s_box[t] = a.box[j];
+    }
+    __syncthreads();
+    // the same in every wave; false for all once q0 is past the last world
+    if (!__any(p < a.nb && (p >= q0 || (q0 < end && s_lo[0] <= hx)))) break;
+#pragma unroll 4
+    for (int k = wv; k < kSweepTile; k += 4) {
+      const BroadBox c = s_box[k];
+      const int q = q0 + k;
+      const bool keep = (q > p) & (q < end) & (s_lo[k] <= hx) & (c.lo_y <= b.hi_y) & (b.lo_y <= c.hi_y) &
+                        (c.lo_z <= b.hi_z) & (b.lo_z <= c.hi_z);
+      if (keep) {
+        const int n = atomicAdd(&s_n, 1);
+        if (n < kSweepHits)
+          s_hit[n] = int2{i, s_j[k]};
+        else
+          append(a.plane_pairs + int64_t(atomicAdd((unsigned long long*)a.pcount, 2ull)), i, s_j[k]);
+      }
+    }
+  }
+  const int n = min(s_n, kSweepHits);
+  if (t == 0 && n > 0) s_base = (long long)atomicAdd((unsigned long long*)a.pcount, 2ull * (unsigned long long)n);
+  __syncthreads();
+  for (int h = t; h < n; h += 256) append(a.plane_pairs + s_base + 2 * h, s_hit[h].x, s_hit[h].y);
 }
 
 // Sorted pair keys -> the explicit list (one, two); a plane is -(k+1).
@@ -174,7 +196,7 @@ hipError_t launch_bp_bounds_sort(const BroadArgs<R>& a, void* tmp, size_t tmp_by
   k_bp_bounds<R><<<(a.nb + 255) / 256, 256, 0, st>>>(a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  return radix_sort_u64(a.key_in, a.key_out, a.val_in, a.val_out, a.nb, tmp, tmp_bytes, st);
+  return radix_sort_u64(a.key_in, a.key_out, a.val_in, a.val_out, a.nb, tmp, tmp_bytes, st, 32, bits_for(a.nw));
 }
 
 template <typename R>
@@ -183,14 +205,14 @@ hipError_t launch_bp_sweep(const BroadArgs<R>& a, const BroadPlanes& p, hipStrea
   hipError_t e = launch_fill_i32((int32_t*)a.pcount, 2, 0, st);
   if (e != hipSuccess) return e;
   k_bp_planes<<<(p.nb + 255) / 256, 256, 0, st>>>(p);
-  k_bp_sweep<R><<<(a.nb + 255) / 256, 256, 0, st>>>(a);
+  k_bp_sweep<R><<<(a.nb + 63) / 64, 256, 0, st>>>(a);
   return hipGetLastError();
 }
 
 hipError_t launch_bp_list(const BroadList& L, void* tmp, size_t tmp_bytes, hipStream_t st) {
   hipError_t e = hipSuccess;
   if (L.n > 0) {
-    e = radix_sort_u64(L.pkey_in, L.pkey, nullptr, nullptr, L.n, tmp, tmp_bytes, st);
+    e = radix_sort_u64(L.pkey_in, L.pkey, nullptr, nullptr, L.n, tmp, tmp_bytes, st, bits_for(L.slots), bits_for(L.nb));
     if (e != hipSuccess) return e;
     k_bp_unpack<<<int((L.n + 255) / 256), 256, 0, st>>>(L);
   }

@@ -609,8 +609,13 @@ __global__ void __launch_bounds__(256) k_np_count(NP<R> a) {
   }
 }
 
-// above this many tiles in one world the 16-wave tile scan is launched
+// The 16-wave tile scan is launched above this many tiles in one world, or
+// from a quarter of a thousand on where every world can have a CU: one wave
+// takes 64 tiles per dependent step, 25 us for the 4000 of 40000 listed bodies
+// where 16 waves take 5 us; with more worlds than CUs the chip is full
+// either way and 16 waves per world would mostly wait.
 constexpr int kWideScanTiles = 4096;
+constexpr int kWideScanFew = 256;  // tiles, and worlds
 
 template <typename R>
 __global__ void __launch_bounds__(64) k_np_scan_tiles(NP<R> a) {
@@ -764,7 +769,7 @@ hipError_t launch_narrowphase(const NarrowLaunch<R>& L, hipStream_t st, hipEvent
     k_np_eval<R><<<int(want < 8192 ? (want > 0 ? want : 1) : 8192), 256, 0, st>>>(a);
   }
   if (ev) (void)hipEventRecord(ev[1], st);
-  if (a.ps.max_world_tiles > kWideScanTiles)
+  if (a.ps.max_world_tiles > kWideScanTiles || (a.ps.max_world_tiles > kWideScanFew && a.n_worlds <= kWideScanFew))
     k_np_scan_tiles_wide<R><<<a.n_worlds, 1024, 0, st>>>(a);
   else
     k_np_scan_tiles<R><<<a.n_worlds, 64, 0, st>>>(a);
