@@ -120,6 +120,10 @@ struct cbz_context {
   int32_t* n_hits = nullptr;
   uint32_t* cand = nullptr;  // [cand_cap] candidate pairs of the last cull
   int32_t* n_cand = nullptr;
+  int32_t* n_pairs = nullptr;
+  int32_t* d_body_world = nullptr;  // [nb]
+  int64_t plane_pairs = 0;          // body-plane pairs of the scene
+  int32_t max_planes = 0;           // of one world
   int64_t cand_cap = 0;
   // explicit-list pair space (grown on demand)
   int32_t l_tiles_cap = 0, l_pairs_cap = 0;
@@ -430,7 +434,8 @@ void free_scene(cbz_ctx* c) {
   dfree(c->world_cnt);
   dfree(c->world_coff);
   dfree(c->total);
-  dfree(c->overflow);
+  c->n_pairs = c->overflow = nullptr;  // in n_hits
+  dfree(c->d_body_world);
   dfree(c->world_iters);
   dfree(c->world_time);
   dfree(c->isl_mem);
@@ -553,17 +558,19 @@ int refresh_pow(cbz_ctx* c, double dt) {
 }
 
 
+// clear: the narrowphase's counters too (see do_narrowphase; not without bodies).
 template <typename R>
-int do_integrate(cbz_ctx* c, double dt) {
+int do_integrate(cbz_ctx* c, double dt, bool clear = false) {
   int rc = refresh_pow(c, dt);
   if (rc) return rc;
-  HIPCHK(c, launch_integrate<R>(bodies_view<R>(c), (R)dt, (R)c->sleep_bias, c->stream));
+  HIPCHK(c, launch_integrate<R>(bodies_view<R>(c), (R)dt, (R)c->sleep_bias, clear ? c->n_hits : nullptr, c->stream));
   return CBZ_OK;
 }
 
 // list_tiles < 0 selects the all-pairs space.
+// cleared: the integrate launch before it cleared the counters.
 template <typename R>
-int do_narrowphase(cbz_ctx* c, int32_t list_tiles, hipEvent_t* ev = nullptr) {
+int do_narrowphase(cbz_ctx* c, int32_t list_tiles, hipEvent_t* ev = nullptr, bool cleared = false) {
   int rc = refresh_brad(c);
   if (rc) return rc;
   if (list_tiles < 0) c->l_last = -1;  // no pair list: no per-pair counts
@@ -613,14 +620,18 @@ int do_narrowphase(cbz_ctx* c, int32_t list_tiles, hipEvent_t* ev = nullptr) {
   L.hits = c->hits;
   L.n_hits = c->n_hits;
   L.cand = c->cand;
+  L.n_pairs = c->n_pairs;
   L.n_cand = c->n_cand;
   L.cand_cap = c->cand_cap;
+  L.plane_pairs = c->plane_pairs;
+  L.body_world = c->d_body_world;
+  L.max_planes = c->max_planes;
   L.n_worlds = c->nw;
   L.mat.body_fric = (const R*)c->field[CBZ_FRICTION];
   L.mat.body_rest = (const R*)c->field[CBZ_RESTITUTION];
   L.mat.plane_fric = (const R*)c->plane_fric;
   L.mat.plane_rest = (const R*)c->plane_rest;
-  HIPCHK(c, launch_fill_i32(c->overflow, 1, 0, c->stream));
+  if (!cleared) HIPCHK(c, launch_fill_i32(c->n_hits, kNarrowCounters, 0, c->stream));
   HIPCHK(c, launch_narrowphase<R>(L, c->stream, ev));
   c->have_contacts = true;
   return CBZ_OK;
@@ -1484,21 +1495,32 @@ int cbz_set_scene(cbz_ctx* c, int32_t n_worlds, const int32_t* body_off, const i
   if ((rc = dalloc_bytes(c, &c->c_real, rs * kContactPlanes * (size_t)c->cap))) return rc;
   if ((rc = dalloc_bytes(c, &c->c_rec, rs * 16 * (size_t)c->cap))) return rc;
   if ((rc = dalloc(c, &c->hits, (size_t)c->cap))) return rc;
-  if ((rc = dalloc(c, &c->n_hits, 1))) return rc;
+  // n_hits, n_pairs, overflow[0..1]: the narrowphase's counters side by side
+  if ((rc = dalloc(c, &c->n_hits, 4))) return rc;
+  static_assert(kNarrowCounters == 3, "hits, pairs, overflow[0]");
+  c->n_pairs = c->n_hits + 1;
+  c->overflow = c->n_hits + 2;
   // candidate pairs of the cull: 4 per contact slot plus the scene's ordered
   // pairs up to 32 M (a dense pile keeps many pairs inside the cull's bound)
   int64_t pairs_total = 0;
+  std::vector<int32_t> bw((size_t)std::max<int64_t>(nb, 1), 0);
+  c->plane_pairs = 0;
+  c->max_planes = 0;
   for (int32_t w = 0; w < n_worlds; ++w) {
     const int64_t n = body_off[w + 1] - body_off[w], npw = plane_off[w + 1] - plane_off[w];
     pairs_total += n * (n - 1 + npw);
+    c->plane_pairs += n * npw;
+    if (n > 0) c->max_planes = std::max<int32_t>(c->max_planes, (int32_t)npw);
+    std::fill(bw.begin() + body_off[w], bw.begin() + body_off[w + 1], w);
   }
+  if ((rc = dalloc(c, &c->d_body_world, bw.size()))) return rc;
+  HIPCHK(c, hipMemcpy(c->d_body_world, bw.data(), bw.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   c->cand_cap = std::min<int64_t>(4 * c->cap + std::min<int64_t>(pairs_total, int64_t(32) << 20), INT32_MAX);
   if ((rc = dalloc(c, &c->cand, (size_t)c->cand_cap))) return rc;
   if ((rc = dalloc(c, &c->n_cand, 1))) return rc;
   if ((rc = dalloc(c, &c->world_cnt, (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->world_coff, (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->total, 1))) return rc;
-  if ((rc = dalloc(c, &c->overflow, 2))) return rc;
   if ((rc = dalloc(c, &c->world_iters, 2 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->world_time, 4 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->order, (size_t)n_worlds))) return rc;
@@ -2072,9 +2094,10 @@ int cbz_step(cbz_ctx* c, double dt, int32_t n_steps, int64_t iter_per_contact, i
     if (!c->gexec || c->g_dt != dt || c->g_mult != iter_per_contact) {
       drop_graph(c);
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      int crc = c->precision == CBZ_F64 ? do_integrate<double>(c, dt) : do_integrate<float>(c, dt);
+      int crc = c->precision == CBZ_F64 ? do_integrate<double>(c, dt, true) : do_integrate<float>(c, dt, true);
       if (crc == CBZ_OK)
-        crc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, -1) : do_narrowphase<float>(c, -1);
+        crc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, -1, nullptr, c->nb > 0)
+                          : do_narrowphase<float>(c, -1, nullptr, c->nb > 0);
       if (crc == CBZ_OK)
         crc = c->precision == CBZ_F64 ? do_resolve<double>(c, dt, iter_per_contact, 0)
                                       : do_resolve<float>(c, dt, iter_per_contact, 0);
@@ -2121,11 +2144,11 @@ int cbz_step(cbz_ctx* c, double dt, int32_t n_steps, int64_t iter_per_contact, i
   for (int32_t s = 0; s < n_steps && rc == CBZ_OK; ++s) {
     hipEvent_t* e = E ? E + 8 * (size_t)s : nullptr;
     if (e) HIPCHK(c, hipEventRecord(e[0], c->stream));
-    rc = c->precision == CBZ_F64 ? do_integrate<double>(c, dt) : do_integrate<float>(c, dt);
+    rc = c->precision == CBZ_F64 ? do_integrate<double>(c, dt, true) : do_integrate<float>(c, dt, true);
     if (rc) break;
     if (e) HIPCHK(c, hipEventRecord(e[7], c->stream));
-    rc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, -1, e ? e + 1 : nullptr)
-                                 : do_narrowphase<float>(c, -1, e ? e + 1 : nullptr);
+    rc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, -1, e ? e + 1 : nullptr, c->nb > 0)
+                                 : do_narrowphase<float>(c, -1, e ? e + 1 : nullptr, c->nb > 0);
     if (rc) break;
     if (hist)
       HIPCHK(c, hipMemcpyAsync(hist + (size_t)s * c->nw, c->world_cnt, c->nw * sizeof(int32_t),
@@ -2716,8 +2739,9 @@ int cbz_step_sur(cbz_ctx* c, double dt, int32_t n_steps, int64_t iter_per_contac
       if (c->sgexec) (void)hipGraphExecDestroy(c->sgexec);
       c->sgexec = nullptr;
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-      int crc = f64 ? do_integrate<double>(c, dt) : do_integrate<float>(c, dt);
-      if (crc == CBZ_OK) crc = f64 ? do_narrowphase<double>(c, -1) : do_narrowphase<float>(c, -1);
+      int crc = f64 ? do_integrate<double>(c, dt, true) : do_integrate<float>(c, dt, true);
+      if (crc == CBZ_OK) crc = f64 ? do_narrowphase<double>(c, -1, nullptr, c->nb > 0)
+                          : do_narrowphase<float>(c, -1, nullptr, c->nb > 0);
       if (crc == CBZ_OK)
         crc = f64 ? sur_resolve<double>(c, dt, iter_per_contact, tol, polish_per_contact, flags, c->sur.nfall)
                   : sur_resolve<float>(c, dt, iter_per_contact, tol, polish_per_contact, flags, c->sur.nfall);
@@ -2763,9 +2787,10 @@ int cbz_step_sur(cbz_ctx* c, double dt, int32_t n_steps, int64_t iter_per_contac
   }
   HIPCHK(c, launch_fill_i32(c->overflow, 2, 0, c->stream));
   for (int32_t s = 0; s < n_steps && rc == CBZ_OK; ++s) {
-    rc = f64 ? do_integrate<double>(c, dt) : do_integrate<float>(c, dt);
+    rc = f64 ? do_integrate<double>(c, dt, true) : do_integrate<float>(c, dt, true);
     if (rc) break;
-    rc = f64 ? do_narrowphase<double>(c, -1) : do_narrowphase<float>(c, -1);
+    rc = f64 ? do_narrowphase<double>(c, -1, nullptr, c->nb > 0)
+                          : do_narrowphase<float>(c, -1, nullptr, c->nb > 0);
     if (rc) break;
     if (hist)
       HIPCHK(c, hipMemcpyAsync(hist + (size_t)s * c->nw, c->world_cnt, c->nw * sizeof(int32_t),

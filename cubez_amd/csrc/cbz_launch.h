@@ -47,9 +47,13 @@ struct NarrowLaunch {
   int32_t* overflow;
   uint32_t* hits;     // [cap] hit pairs as tile * 64 + lane (all-pairs)
   int32_t* n_hits;
-  uint32_t* cand;     // [cand_cap] candidate pairs, same coding
-  int32_t* n_cand;
-  int64_t cand_cap;
+  uint32_t* cand;     // [cand_cap] candidate body pairs (i, j), i < j, same coding
+  int32_t* n_pairs;   // how many; n_hits and n_pairs are cleared by the caller
+  int32_t* n_cand;    // out: the candidates in both orders and the body-plane pairs
+  int64_t cand_cap;   // most n_cand
+  int64_t plane_pairs;        // body-plane pairs
+  const int32_t* body_world;  // [n_bodies]
+  int32_t max_planes;         // of one world
   int32_t n_worlds;
   Materials<R> mat{};  // per-body and per-plane materials (read when c.fric is set)
 };
@@ -109,7 +113,7 @@ struct ResolveLaunch {
 template <typename R>
 hipError_t launch_calculate_derived(const Bodies<R>& b, hipStream_t st);
 template <typename R>
-hipError_t launch_integrate(const Bodies<R>& b, R dt, R bias, hipStream_t st);
+hipError_t launch_integrate(const Bodies<R>& b, R dt, R bias, int32_t* clear, hipStream_t st);
 template <typename R>
 hipError_t launch_narrowphase(const NarrowLaunch<R>& L, hipStream_t st, hipEvent_t* ev = nullptr);
 template <typename R>

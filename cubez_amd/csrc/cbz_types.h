@@ -109,6 +109,10 @@ struct Materials {
 // per tile instead.
 constexpr int kRowBlock = 16;
 
+// Counters that start at zero in every narrowphase: hits, candidate pairs and
+// the overflow flag, side by side in this order.
+constexpr int kNarrowCounters = 3;
+
 // counters of awake bodies the integrate kernel fills when asked (summed by
 // the reader)
 constexpr int kAwakeSlots = 256;

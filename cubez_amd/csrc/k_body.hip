@@ -78,8 +78,10 @@ __global__ void __launch_bounds__(256) k_calculate_derived(Bodies<R> b) {
 // API adds to them), so lastFrameAccelleration = Acceleration + 0*invMass
 // and the angular acceleration is iitWorld * 0.
 template <typename R>
-__global__ void __launch_bounds__(256) k_integrate(Bodies<R> b, R dt, R bias) {
+__global__ void __launch_bounds__(256) k_integrate(Bodies<R> b, R dt, R bias, int32_t* clear) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  // the counters of the narrowphase that follows, so that it needs no launch for them
+  if (clear && i < kNarrowCounters) clear[i] = 0;
   uint8_t f = i < b.n ? b.flags[i] : uint8_t(F_STATIC);
   if (b.n_awake) {  // kAwakeSlots counters, so the waves' atomics do not queue on one address
     const uint64_t m = __ballot(!(f & F_STATIC) && (f & F_AWAKE));
@@ -157,15 +159,15 @@ hipError_t launch_calculate_derived(const Bodies<R>& b, hipStream_t st) {
 }
 
 template <typename R>
-hipError_t launch_integrate(const Bodies<R>& b, R dt, R bias, hipStream_t st) {
+hipError_t launch_integrate(const Bodies<R>& b, R dt, R bias, int32_t* clear, hipStream_t st) {
   if (b.n <= 0) return hipSuccess;
-  k_integrate<R><<<(b.n + 255) / 256, 256, 0, st>>>(b, dt, bias);
+  k_integrate<R><<<(b.n + 255) / 256, 256, 0, st>>>(b, dt, bias, clear);
   return hipGetLastError();
 }
 
 template hipError_t launch_calculate_derived<double>(const Bodies<double>&, hipStream_t);
 template hipError_t launch_calculate_derived<float>(const Bodies<float>&, hipStream_t);
-template hipError_t launch_integrate<double>(const Bodies<double>&, double, double, hipStream_t);
-template hipError_t launch_integrate<float>(const Bodies<float>&, float, float, hipStream_t);
+template hipError_t launch_integrate<double>(const Bodies<double>&, double, double, int32_t*, hipStream_t);
+template hipError_t launch_integrate<float>(const Bodies<float>&, float, float, int32_t*, hipStream_t);
 
 }  // namespace cbz

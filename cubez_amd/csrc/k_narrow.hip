@@ -13,19 +13,26 @@
 //
 // Launches (all-pairs):
 //   cull        — one wave per (column tile, 16 rows): clears the tiles and
-//                 lists the candidate pairs.  Cube-cube and cube-sphere
-//                 pairs whose bounding spheres are far apart are rejected:
-//                 the bound guarantees that the reference's own test reports
-//                 no contact (see far_apart below), so the result is
-//                 unchanged.
-//   eval        — one thread per candidate: the reference's test; per tile
-//                 a hit bitmask and contact total, and the hit list.
+//                 lists the candidate body pairs (i, j), i < j.  Cube-cube
+//                 and cube-sphere pairs whose bounding spheres are far apart
+//                 are rejected: the bound guarantees that the reference's own
+//                 test reports no contact (see far_apart below), so the
+//                 result is unchanged.
+//   eval        — one thread per body (its planes) and per candidate: the
+//                 reference's test; per tile a hit bitmask and contact total,
+//                 and the hit list.  A pair is tested once for both orders:
+//                 swapping the bodies negates the centre offset and the cross
+//                 products and swaps the terms of sums, so every comparison
+//                 of the test (colliders.go:216-254, 369-441, 445-477) comes
+//                 out the same, NaNs included.
 //   scan_tiles  — one wave per world: exclusive scan of tile totals.
 //   scan_worlds — one block: exclusive scan of world totals.
 //   emit_hits   — one thread per hit pair: recompute it and write its
 //                 contacts at world offset + tile offset + in-tile prefix.
 // (The explicit-list form counts and emits one wave per tile.)
 // All geometry is evaluated in FP64 whatever the storage type R.
+#include <algorithm>
+
 #include "cbz_devmath.h"
 #include "cbz_launch.h"
 #include "cbz_types.h"
@@ -69,8 +76,11 @@ struct NP {
   uint32_t* hits;
   int32_t* n_hits;
   uint32_t* cand;
+  int32_t* n_pairs;
   int32_t* n_cand;
-  int64_t cand_cap;
+  int64_t cand_cap, plane_pairs;
+  const int32_t* body_world;
+  int32_t max_planes;
   int32_t n_worlds;
   Materials<R> mat;  // read when c.fric is set
 };
@@ -385,6 +395,13 @@ __device__ __forceinline__ void pair_of(const PairSpace& ps, int w, int q, int& 
   two = ps.list_two[p];
 }
 
+// Orders a wave's LDS writes before its later reads, and the other way.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------
 // all-pairs space
 // ---------------------------------------------------------------------------
@@ -409,29 +426,46 @@ __device__ __forceinline__ int64_t block_reserve(int mine, int32_t* counter, int
   return base + incl - mine;
 }
 
-// tasks per wave of the cull: their candidates share one block reservation
-constexpr int kCullTasks = 4;
+// Cull: each wave takes TASKS consecutive tasks (world w, column tile c,
+// rows r0 .. r0+15).  Lane l owns column 64c + l for the whole task: a plane,
+// or body j whose centre, bounding radius and shape stay in registers; the 16
+// row bodies are put in LDS once and read as broadcasts.  Each tile is
+// cleared here; the body pairs with j > r that pass the conservative bound
+// (see far_apart) go to the candidate list.
+//
+// The 16 tests of a lane run in FP32 on positions relative to the first row's
+// body, with a margin that covers the rounding: for s = sqrt(kf) rr and an
+// error e of the distance, (s + e)^2 <= 1.004 s^2 + 251 e^2, and with the
+// coordinates' and the difference's rounding e <= 2^-23 (|a| + |b|) in the
+// 1-norms of a and b, so 251 e^2 is below 4e-12 (|a| + |b|)^2.  What they leave (a NaN or an infinity passes) is
+// tested again as far_apart does it, once per pair that is left instead of once
+// per pair: the list is the same.  4096 worlds of 8 to 256 cubes take
+// 99 us (183 with every ordered pair tested in FP64, rows shuffled from lane to
+// lane), bound by the tests' instructions and the clearing of 1.4 million tiles.
+constexpr int kCullSmall = 8192;  // tasks up to which a wave takes one: every task has its wave
+                                  // on the chip, and a launch is one task long (one world of 64 cubes: 22 to 5 us)
 
-// Cull: each wave takes kCullTasks consecutive tasks (world w, column tile
-// c, rows r0 .. r0+15).  Lane l owns column 64c + l for the whole task: a plane, or body j whose centre,
-// bounding radius and shape stay in registers; the 16 row bodies are loaded
-// once (lane k holds row r0 + k) and broadcast.  Each tile is cleared here;
-// its plane pairs and the body pairs that pass the conservative bound (see
-// far_apart) go to the candidate list.
-template <typename R>
+struct CullRow {
+  float x, y, z, r;    // relative to the first row's body
+  double dx, dy, dz, dr;
+  float norm;          // |x| + |y| + |z|
+  int shape;
+};
+
+template <typename R, int TASKS>
 __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
+  __shared__ CullRow s_row[4][kRowBlock];
   __shared__ int s_wtot[4];
   __shared__ int s_base;
-  const int lane = threadIdx.x & 63;
-  const int task0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kCullTasks;
-  // bit 16(q%4) + k of word q/4: row r0(q) + k of the wave's task q is a
-  // candidate for this lane
-  uint64_t cm[(kCullTasks + 3) / 4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int task0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + wv) * TASKS);
+  CullRow* row = s_row[wv];
+  // bit k of cm[q]: row r0(q) + k of the wave's task q is a candidate for this lane
+  uint32_t cm[TASKS];
+  int t0[TASKS], r0[TASKS], nch[TASKS], cc[TASKS];
 #pragma unroll
-  for (int u = 0; u < (kCullTasks + 3) / 4; ++u) cm[u] = 0;
-  int t0[kCullTasks], r0[kCullTasks], nch[kCullTasks], cc[kCullTasks];
-#pragma unroll
-  for (int q = 0; q < kCullTasks; ++q) {
+  for (int q = 0; q < TASKS; ++q) {
+    cm[q] = 0;
     t0[q] = 0;
     r0[q] = 0;
     nch[q] = 1;
@@ -440,17 +474,22 @@ __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
     if (task >= a.ps.n_tasks) continue;  // the wave still joins the block's reservation
     const int w = a.ps.task_world[task];
     const int b0 = a.ps.body_off[w], n = a.ps.body_off[w + 1] - b0;
-    const int p0 = a.ps.plane_off[w], np = a.ps.plane_off[w + 1] - p0;
+    const int np = a.ps.plane_off[w + 1] - a.ps.plane_off[w];
     nch[q] = (np + n + 63) >> 6;
     const int k = task - a.ps.world_task0[w];
     const int c = k % nch[q];
     cc[q] = c;
     r0[q] = (k / nch[q]) * kRowBlock;
-    const int r1 = min(n, r0[q] + kRowBlock);
-    const int col = 64 * c + lane;
-    const bool is_plane = col < np;
-    const int j = col - np;
-    const bool is_body = !is_plane && j < n;
+    t0[q] = a.ps.world_tile0[w];
+    const int rows = min(n - r0[q], kRowBlock);
+    if (lane < rows) {
+      const int t = t0[q] + (r0[q] + lane) * nch[q] + c;
+      a.tile_cnt[t] = 0;
+      a.tile_mask[t] = 0ull;
+    }
+    if (64 * c + 63 - np <= r0[q]) continue;  // no column with j > r
+    const int j = 64 * c + lane - np;
+    const bool is_body = j >= 0 && j < n;
     const int64_t S = a.b.stride;
     double tj[3] = {0, 0, 0}, rj = 0;
     int sj = 0;
@@ -462,10 +501,9 @@ __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
       rj = a.brad[g];
       sj = a.b.shape[g];
     }
-    // row bodies r0 .. r1-1: lane k < 16 loads row r0 + k
     double ti[3] = {0, 0, 0}, ri = 0;
     int si = 0;
-    if (lane < r1 - r0[q]) {
+    if (lane < rows) {  // lane k holds row r0 + k
       const int g = b0 + r0[q] + lane;
       ti[0] = double(a.b.ctransform[9 * S + g]);
       ti[1] = double(a.b.ctransform[10 * S + g]);
@@ -473,51 +511,79 @@ __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
       ri = a.brad[g];
       si = a.b.shape[g];
     }
-    t0[q] = a.ps.world_tile0[w];
-    for (int r = r0[q]; r < r1; ++r) {
-      const int src = r - r0[q];
-      const double x = __shfl(ti[0], src, 64), y = __shfl(ti[1], src, 64), z = __shfl(ti[2], src, 64);
-      const double rr = __shfl(ri, src, 64) + rj;
-      const int s_i = __shfl(si, src, 64);
-      bool cand = is_plane;
-      if (is_body && j != r) {
-        const double dx = tj[0] - x, dy = tj[1] - y, dz = tj[2] - z;
-        const double d2 = dx * dx + dy * dy + dz * dz;
-        const bool spheres = s_i == SHAPE_SPHERE && sj == SHAPE_SPHERE;
-        const double kf = (s_i == SHAPE_CUBE && sj == SHAPE_CUBE) ? 3.003 : 1.001;
-        cand = spheres || !(d2 > kf * rr * rr);
-      }
-      if (cand) cm[q >> 2] |= 1ull << (16 * (q & 3) + src);
-      if (lane == 0) {
-        const int t = t0[q] + r * nch[q] + c;
-        a.tile_cnt[t] = 0;
-        a.tile_mask[t] = 0ull;
-      }
+    const double ox = __shfl(ti[0], 0, 64), oy = __shfl(ti[1], 0, 64), oz = __shfl(ti[2], 0, 64);
+    const float xj = float(tj[0] - ox), yj = float(tj[1] - oy), zj = float(tj[2] - oz), fj = float(rj);
+    const float normj = fabsf(xj) + fabsf(yj) + fabsf(zj);
+    wave_lds_fence();  // the last task's rows have been read
+    if (lane < kRowBlock) {
+      CullRow v;
+      v.x = float(ti[0] - ox), v.y = float(ti[1] - oy), v.z = float(ti[2] - oz), v.r = float(ri);
+      v.dx = ti[0], v.dy = ti[1], v.dz = ti[2], v.dr = ri;
+      v.norm = fabsf(v.x) + fabsf(v.y) + fabsf(v.z);
+      v.shape = si;
+      row[lane] = v;
     }
+    wave_lds_fence();
+    // kf with its margin, for a row that is a cube and one that is not
+    // (two spheres are always a candidate)
+    const bool cj = sj == SHAPE_CUBE;
+    const float kc = (cj ? 3.003f : 1.001f) * 1.0042f;
+    const float ks = sj == SHAPE_SPHERE ? INFINITY : 1.001f * 1.0042f;
+    uint32_t m = 0;
+#pragma unroll
+    for (int k2 = 0; k2 < kRowBlock; ++k2) {
+      const CullRow& v = row[k2];
+      const float dx = xj - v.x, dy = yj - v.y, dz = zj - v.z;
+      const float d2 = dx * dx + dy * dy + dz * dz;
+      const float rr = v.r + fj, nn = v.norm + normj;
+      const float lim = (v.shape == SHAPE_CUBE ? kc : (v.shape == SHAPE_SPHERE ? ks : 1.001f * 1.0042f)) * (rr * rr);
+      if (!(d2 > lim + 1e-10f * (nn * nn))) m |= 1u << k2;
+    }
+    // rows below the column's body only
+    const int up = min(max(j - r0[q], 0), rows);
+    m = is_body ? m & ((1u << up) - 1u) : 0u;
+    uint32_t keep = 0;
+    for (; m; m &= m - 1u) {
+      const int k2 = __ffs(m) - 1;
+      const CullRow& v = row[k2];
+      const double dx = tj[0] - v.dx, dy = tj[1] - v.dy, dz = tj[2] - v.dz;
+      const double d2 = dx * dx + dy * dy + dz * dz;
+      const double rr = v.dr + rj;
+      const bool spheres = v.shape == SHAPE_SPHERE && sj == SHAPE_SPHERE;
+      const double kf = (v.shape == SHAPE_CUBE && cj) ? 3.003 : 1.001;
+      if (spheres || !(d2 > kf * rr * rr)) keep |= 1u << k2;
+    }
+    cm[q] = keep;
   }
   // one reservation per block for all of its waves' tasks
-  int ncand = 0;
+  int npair = 0;
 #pragma unroll
-  for (int u = 0; u < (kCullTasks + 3) / 4; ++u) ncand += __popcll(cm[u]);
-  int64_t pos = block_reserve(ncand, a.n_cand, s_wtot, &s_base);
+  for (int q = 0; q < TASKS; ++q) npair += __popc(cm[q]);
+  int64_t pos = block_reserve(npair, a.n_pairs, s_wtot, &s_base);
 #pragma unroll
-  for (int q = 0; q < kCullTasks; ++q) {
-    for (uint32_t m = uint32_t(cm[q >> 2] >> (16 * (q & 3))) & 0xFFFFu; m; m &= m - 1u, ++pos) {
+  for (int q = 0; q < TASKS; ++q)
+    for (uint32_t m = cm[q]; m; m &= m - 1u, ++pos) {
       const int r = r0[q] + __ffs(m) - 1;
       if (pos < a.cand_cap) a.cand[pos] = uint32_t(t0[q] + r * nch[q] + cc[q]) * 64u + uint32_t(lane);
     }
-  }
 }
 
-// Eval: one thread per candidate pair: the reference's test (contact count
-// only); hits add to their tile's total and mask (integer atomics: the sums
-// do not depend on the order) and join the hit list.  Too many candidates
-// for the list raise the overflow flags (the step reports a capacity error).
+// Eval: the first workgroups take a body per thread, against its world's
+// planes, the others a candidate pair per thread: the reference's test
+// (contact count only); hits add to their tile's total and mask (integer
+// atomics: the sums do not depend on the order) and join the hit list.  Too
+// many candidates (in both orders, the planes' pairs among them) for the list
+// raise the overflow flags (the step reports a capacity error).  The planes
+// apart from the pairs: a wave that holds both runs both tests.
+// 4096 worlds of 8 to 256 cubes take 110 us (166 with both orders tested and the
+// planes among the pairs), bound by the gathers of two bodies per thread and the
+// longest axis search of each wave.
 template <typename R>
-__global__ void __launch_bounds__(256) k_np_eval(NP<R> a) {
+__global__ void __launch_bounds__(256) k_np_eval(NP<R> a, int plane_blocks) {
   __shared__ int s_wtot[4];
   __shared__ int s_base;
-  const int64_t nc = a.n_cand[0];
+  const int64_t np2 = a.n_pairs[0], nc = 2 * np2 + a.plane_pairs;
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.n_cand[0] = int32_t(min(nc, int64_t(INT32_MAX)));
   if (nc > a.cand_cap) {
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       a.overflow[0] = 1;
@@ -525,29 +591,58 @@ __global__ void __launch_bounds__(256) k_np_eval(NP<R> a) {
     }
     return;  // uniform over the grid
   }
-  for (int64_t e0 = int64_t(blockIdx.x) * blockDim.x; e0 < nc; e0 += int64_t(gridDim.x) * blockDim.x) {
+  auto hit = [&](int t, int l, int cnt) {
+    atomicAdd(&a.tile_cnt[t], cnt);
+    atomicOr((unsigned long long*)&a.tile_mask[t], 1ull << l);
+  };
+  if (int(blockIdx.x) < plane_blocks) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    int r = 0, p0 = 0, np = 0, nch = 0, t0 = 0;
+    if (i < a.b.n) {
+      const int w = a.body_world[i];
+      const int b0 = a.ps.body_off[w], n = a.ps.body_off[w + 1] - b0;
+      r = i - b0;
+      p0 = a.ps.plane_off[w], np = a.ps.plane_off[w + 1] - p0;
+      nch = (np + n + 63) >> 6;
+      t0 = a.ps.world_tile0[w];
+    }
+    for (int k = 0; k < a.max_planes; ++k) {
+      const int t = t0 + r * nch + (k >> 6), l = k & 63;
+      const int cnt = k < np ? pair_eval<R, false>(a, i, -(p0 + k) - 1, 0) : 0;
+      if (cnt > 0) hit(t, l, cnt);
+      const int64_t idx = block_reserve(cnt > 0 ? 1 : 0, a.n_hits, s_wtot, &s_base);
+      if (cnt > 0 && idx < a.c.cap) a.hits[idx] = uint32_t(t) * 64u + uint32_t(l);
+    }
+    return;
+  }
+  const int64_t stride = int64_t(gridDim.x - plane_blocks) * blockDim.x;
+  for (int64_t e0 = int64_t(blockIdx.x - plane_blocks) * blockDim.x; e0 < np2; e0 += stride) {
     const int64_t e = e0 + threadIdx.x;
     int cnt = 0;
-    uint32_t code = 0;
-    if (e < nc) {
+    uint32_t code = 0, back = 0;
+    if (e < np2) {
       code = a.cand[e];
       const int t = int(code >> 6), l = int(code & 63u);
       const int w = a.ps.tile_world[t];
       const int b0 = a.ps.body_off[w], n = a.ps.body_off[w + 1] - b0;
-      const int p0 = a.ps.plane_off[w], np = a.ps.plane_off[w + 1] - p0;
-      const int nch = (np + n + 63) >> 6;
-      const int k = t - a.ps.world_tile0[w];
+      const int np = a.ps.plane_off[w + 1] - a.ps.plane_off[w];
+      const int nch = (np + n + 63) >> 6, t0 = a.ps.world_tile0[w];
+      const int k = t - t0;
       const int r = k / nch, c = k - r * nch;
-      const int col = 64 * c + l;
-      const int i = b0 + r;
-      cnt = col < np ? pair_eval<R, false>(a, i, -(p0 + col) - 1, 0) : pair_eval<R, false>(a, i, b0 + (col - np), 0);
+      const int j = 64 * c + l - np;
+      cnt = pair_eval<R, false>(a, b0 + r, b0 + j, 0);  // one contact or none
       if (cnt > 0) {
-        atomicAdd(&a.tile_cnt[t], cnt);
-        atomicOr((unsigned long long*)&a.tile_mask[t], 1ull << l);
+        const int tb = t0 + j * nch + ((np + r) >> 6), lb = (np + r) & 63;
+        back = uint32_t(tb) * 64u + uint32_t(lb);
+        hit(t, l, cnt);
+        hit(tb, lb, cnt);
       }
     }
-    const int64_t idx = block_reserve(cnt > 0 ? 1 : 0, a.n_hits, s_wtot, &s_base);
-    if (cnt > 0 && idx < a.c.cap) a.hits[idx] = code;
+    const int64_t idx = block_reserve(cnt > 0 ? 2 : 0, a.n_hits, s_wtot, &s_base);
+    if (cnt > 0) {
+      if (idx < a.c.cap) a.hits[idx] = code;
+      if (idx + 1 < a.c.cap) a.hits[idx + 1] = back;
+    }
   }
 }
 
@@ -617,6 +712,27 @@ __global__ void __launch_bounds__(256) k_np_count(NP<R> a) {
 constexpr int kWideScanTiles = 4096;
 constexpr int kWideScanFew = 256;  // tiles, and worlds
 
+// The totals over all worlds, by one thread: the sum, and the flags when it
+// exceeds the capacity.
+template <typename R>
+__device__ __forceinline__ void put_total(const NP<R>& a, int64_t total) {
+  a.total[0] = total;
+  if (total > a.c.cap) {
+    a.overflow[0] = 1;  // this narrowphase (read by emit and the resolver)
+    a.overflow[1] = 1;  // sticky until the host clears it
+  }
+}
+
+// With one world its tile scan is all there is to scan.
+template <typename R>
+__device__ __forceinline__ void put_world(const NP<R>& a, int w, int cnt) {
+  a.world_cnt[w] = cnt;
+  if (a.n_worlds == 1) {
+    a.world_coff[0] = 0;
+    put_total(a, cnt);
+  }
+}
+
 template <typename R>
 __global__ void __launch_bounds__(64) k_np_scan_tiles(NP<R> a) {
   const int w = blockIdx.x;
@@ -630,7 +746,7 @@ __global__ void __launch_bounds__(64) k_np_scan_tiles(NP<R> a) {
     if (k < nt) a.tile_off[t0 + k] = carry + inc - v;
     carry += __shfl(inc, 63, 64);
   }
-  if (lane == 0) a.world_cnt[w] = carry;
+  if (lane == 0) put_world(a, w, carry);
 }
 
 // The same scan for worlds of many tiles (thousands of bodies): 16 waves,
@@ -671,7 +787,7 @@ __global__ void __launch_bounds__(1024) k_np_scan_tiles_wide(NP<R> a) {
     if (tid == 1023) s_carry = carry + before + inc;
     __syncthreads();
   }
-  if (tid == 0) a.world_cnt[w] = s_carry;
+  if (tid == 0) put_world(a, w, s_carry);
 }
 
 template <typename R>
@@ -695,13 +811,7 @@ __global__ void __launch_bounds__(1024) k_np_scan_worlds(NP<R> a) {
     if (tid == 1023) s_carry = carry + before + inc;
     __syncthreads();
   }
-  if (tid == 0) {
-    a.total[0] = s_carry;
-    if (s_carry > a.c.cap) {
-      a.overflow[0] = 1;  // this narrowphase (read by emit and the resolver)
-      a.overflow[1] = 1;  // sticky until the host clears it
-    }
-  }
+  if (tid == 0) put_total(a, s_carry);
 }
 
 template <typename R>
@@ -744,15 +854,19 @@ hipError_t launch_narrowphase(const NarrowLaunch<R>& L, hipStream_t st, hipEvent
   a.hits = L.hits;
   a.n_hits = L.n_hits;
   a.cand = L.cand;
+  a.n_pairs = L.n_pairs;
   a.n_cand = L.n_cand;
   a.cand_cap = L.cand_cap;
+  a.plane_pairs = L.plane_pairs;
+  a.body_world = L.body_world;
+  a.max_planes = L.max_planes;
   a.n_worlds = L.n_worlds;
   a.mat = L.mat;
   if (a.n_worlds <= 0) return hipSuccess;
   if (a.c.fric && (!a.c.rest || !a.mat.body_fric || !a.mat.body_rest || !a.mat.plane_fric || !a.mat.plane_rest))
     return hipErrorInvalidValue;
   const bool list = a.ps.list_one != nullptr;
-  if (!list && (!a.hits || !a.n_hits || !a.cand || !a.n_cand)) return hipErrorInvalidValue;
+  if (!list && (!a.hits || !a.n_hits || !a.cand || !a.n_cand || !a.n_pairs || !a.body_world)) return hipErrorInvalidValue;
   // ev (optional): recorded before the count, after it, after the scans
   // and after the emit, for per-kernel timing on this stream.
   const int nb = (a.ps.n_tiles + 3) / 4;
@@ -760,20 +874,21 @@ hipError_t launch_narrowphase(const NarrowLaunch<R>& L, hipStream_t st, hipEvent
   if (list) {
     if (nb > 0) k_np_count<R><<<nb, 256, 0, st>>>(a);
   } else {
-    hipError_t e = launch_fill_i32(a.n_hits, 1, 0, st);
-    if (e == hipSuccess) e = launch_fill_i32(a.n_cand, 1, 0, st);
-    if (e != hipSuccess) return e;
-    const int nbt = (a.ps.n_tasks + 4 * kCullTasks - 1) / (4 * kCullTasks);
-    if (nbt > 0) k_np_cull<R><<<nbt, 256, 0, st>>>(a);
-    const int64_t want = (a.cand_cap + 255) / 256;
-    k_np_eval<R><<<int(want < 8192 ? (want > 0 ? want : 1) : 8192), 256, 0, st>>>(a);
+    if (a.ps.n_tasks > kCullSmall) {
+      k_np_cull<R, 4><<<(a.ps.n_tasks + 15) / 16, 256, 0, st>>>(a);
+    } else if (a.ps.n_tasks > 0) {
+      k_np_cull<R, 1><<<(a.ps.n_tasks + 3) / 4, 256, 0, st>>>(a);
+    }
+    const int64_t want = std::min<int64_t>(std::max<int64_t>((a.cand_cap + 511) / 512, 1), 8192);
+    const int planes = a.max_planes > 0 ? (a.b.n + 255) / 256 : 0;
+    k_np_eval<R><<<planes + int(want), 256, 0, st>>>(a, planes);
   }
   if (ev) (void)hipEventRecord(ev[1], st);
   if (a.ps.max_world_tiles > kWideScanTiles || (a.ps.max_world_tiles > kWideScanFew && a.n_worlds <= kWideScanFew))
     k_np_scan_tiles_wide<R><<<a.n_worlds, 1024, 0, st>>>(a);
   else
     k_np_scan_tiles<R><<<a.n_worlds, 64, 0, st>>>(a);
-  k_np_scan_worlds<R><<<1, 1024, 0, st>>>(a);
+  if (a.n_worlds > 1) k_np_scan_worlds<R><<<1, 1024, 0, st>>>(a);
   if (ev) (void)hipEventRecord(ev[2], st);
   if (list) {
     if (nb > 0) k_np_emit<R><<<nb, 256, 0, st>>>(a);
