@@ -179,6 +179,7 @@ struct cbz_context {
   IslandBuffers isl;              // the resolver's island kernel (first resolve), in isl_mem
   char* isl_mem = nullptr;
   int32_t* order = nullptr;
+  int32_t* cost = nullptr;  // [2 * nw] worlds' costs and the order by them
   bool have_contacts = false;
 
   // resolver surrogate (see cbz_sur_*)
@@ -441,6 +442,7 @@ void free_scene(cbz_ctx* c) {
   dfree(c->isl_mem);
   c->isl = IslandBuffers{};
   dfree(c->order);
+  dfree(c->cost);
   dfree(c->d_awake);
   dfree(c->d_prof);
   dfree(c->pos0);
@@ -713,6 +715,7 @@ int do_resolve(cbz_ctx* c, double dt, int64_t mult, int64_t fixed, int32_t mode 
   L.world_coff = c->world_coff;
   L.overflow = c->overflow;
   L.order = c->order;
+  L.cost = c->cost;
   L.body_off = c->d_body_off;
   L.world_iters = c->world_iters;
   L.world_time = c->world_time;
@@ -1524,6 +1527,7 @@ int cbz_set_scene(cbz_ctx* c, int32_t n_worlds, const int32_t* body_off, const i
   if ((rc = dalloc(c, &c->world_iters, 2 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->world_time, 4 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->order, (size_t)n_worlds))) return rc;
+  if ((rc = dalloc(c, &c->cost, 2 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->d_awake, kAwakeSlots))) return rc;
   if ((rc = dalloc(c, &c->d_prof, 4))) return rc;
   if ((rc = dalloc_bytes(c, &c->pos0, rs * 3 * (size_t)std::max<int64_t>(nb, 1)))) return rc;
@@ -1531,6 +1535,7 @@ int cbz_set_scene(cbz_ctx* c, int32_t n_worlds, const int32_t* body_off, const i
   HIPCHK(c, hipMemset(c->world_coff, 0, n_worlds * sizeof(int64_t)));
   HIPCHK(c, hipMemset(c->world_iters, 0, 2 * n_worlds * sizeof(int64_t)));
   HIPCHK(c, hipMemset(c->world_time, 0xFF, 4 * n_worlds * sizeof(int64_t)));  // -1: no launch yet
+  HIPCHK(c, hipMemset(c->cost, 0, 2 * n_worlds * sizeof(int32_t)));
   HIPCHK(c, hipMemset(c->overflow, 0, 2 * sizeof(int32_t)));
   HIPCHK(c, hipMemset(c->total, 0, sizeof(int64_t)));
   std::vector<int32_t> ord;

@@ -82,9 +82,9 @@ struct IslFixed {
   double sum[kIslWaves];
   // each wave's best contact of a big island (two iterations' worth), with
   // what its correction would change: the two bodies' changes 12, their new
-  // velocity and rotation 12
+  // velocity and rotation 12 (position and orientation 14)
   IslBest<R> best[2][kIslWaves];
-  R bx[2][kIslWaves][24];
+  R bx[2][kIslWaves][28];
   unsigned long long total;       // the phase's iterations
   int32_t cls[kIslWords];         // class counts, then cursors
   int32_t next, over, bad, off, ok;
@@ -135,6 +135,21 @@ __device__ __forceinline__ T group_reduce(T v, int lg, OP op) {
     v = lg > 5 ? op(lo, hi) : (threadIdx.x & 32) ? hi : lo;
   }
   return v;
+}
+
+// The lane of each group whose key is the group's greatest (m); among equal keys
+// the lowest index j.  gm: the group's lanes.  The second reduction is made
+// only when some group has equal keys.
+template <typename R>
+__device__ __forceinline__ bool group_owner(bool top, int j, int lg, uint64_t gm) {
+  const uint64_t g = __ballot(top) & gm;
+  if (!__any(__popcll(g) > 1)) return top;
+  const int jm = group_reduce(top ? j : INT_MAX, lg, [](int p, int q) { return q < p ? q : p; });
+  return top && j == jm;
+}
+__device__ __forceinline__ uint64_t group_lanes(int lg) {
+  const int lane = int(threadIdx.x & 63);
+  return lg == 6 ? ~uint64_t(0) : ((uint64_t(1) << (1 << lg)) - 1) << (lane >> lg << lg);
 }
 
 // Body i's entry in the state table: 8 reals, position 0-2 and orientation
@@ -348,40 +363,67 @@ __device__ __forceinline__ void isl_log(const RS<R>& a, int64_t at, R key, int j
   a.log_it[at] = it;
 }
 
-// applyPositionChange (contact.go:286-386) by the one lane that owns the
-// selected contact, the bodies' position and orientation in the tables.
-// Returns bit i for a sleeping body i whose derived data went to HBM.
+// What applyPositionChange (contact.go:286-386) computes of a contact that
+// does not depend on its penetration: the shares of the angular and linear
+// move, the angular limit, and the rotation per unit of angular inertia.  It
+// changes only with a body's world inverse inertia (a sleeping body's derived
+// data).  Kept per contact it takes three divisions, a square root and three
+// matrix products out of every iteration, and fewer registers than the two
+// tensors.  With it, with the sides of a touched contact side by side and with
+// one barrier per iteration of a big island, 301 cubes in one world (FP32) take
+// 10% less per step, 1000 worlds (FP64) 5%.
 template <typename R>
-__device__ __forceinline__ uint32_t isl_position_change(const Bodies<R>& b, const IslWorld<R>& W, const int kl[2],
-                                                        const bool aw[2], const V3<R>& n, const V3<R> rel[2],
-                                                        R penetration, const R (&iw)[2][9], const R im[2],
-                                                        V3<R> lin[2], V3<R> ang[2]) {
+struct IslMove {
+  R ai[2], ra[2], rl[2], mm[2];  // angular inertia, shares, limit
+  V3<R> td[2];
+};
+template <typename R>
+__device__ __forceinline__ void isl_move_of(bool has1, const V3<R>& n, const V3<R> rel[2], const R (&iw)[2][9],
+                                            const R im[2], IslMove<R>& mv) {
   const R angularLimit = R(0.2);
-  R angI[2] = {R(0), R(0)}, linI[2] = {R(0), R(0)};
-  R total = R(0);
-  uint32_t rederived = 0;
+  R linI[2] = {R(0), R(0)}, total = R(0);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    mv.ai[i] = R(0);
+    if (i == 1 && !has1) continue;
+    V3<R> aiw = cross(rel[i], n);
+    aiw = m3v(iw[i], aiw);
+    aiw = cross(aiw, rel[i]);
+    mv.ai[i] = dot(aiw, n);
+    linI[i] = im[i];
+    total += linI[i] + mv.ai[i];
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    mv.ra[i] = mv.ai[i] / total;
+    mv.rl[i] = linI[i] / total;
+    V3<R> projection = add_scaled(rel[i], n, -dot(rel[i], n));
+    mv.mm[i] = angularLimit * mag(projection);
+    mv.td[i] = m3v(iw[i], cross(rel[i], n));
+  }
+}
+
+// The rest of it: the moves of the two bodies for a penetration, and their new
+// position and orientation from the tables (st: 7 reals per body).
+template <typename R>
+__device__ __forceinline__ void isl_position_change(const IslWorld<R>& W, const int kl[2], const V3<R>& n,
+                                                    R penetration, const IslMove<R>& mv, V3<R> lin[2], V3<R> ang[2],
+                                                    R (&st)[2][7]) {
+  const int l1 = kl[1] >= 0 ? kl[1] : kl[0];
+#pragma unroll
+  for (int q = 0; q < 7; ++q) st[0][q] = W.st[kIslSt * kl[0] + q];
+#pragma unroll
+  for (int q = 0; q < 7; ++q) st[1][q] = W.st[kIslSt * l1 + q];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     lin[i] = V3<R>{R(0), R(0), R(0)};
     ang[i] = V3<R>{R(0), R(0), R(0)};
-    if (kl[i] < 0) continue;
-    V3<R> aiw = cross(rel[i], n);
-    aiw = m3v(iw[i], aiw);
-    aiw = cross(aiw, rel[i]);
-    angI[i] = dot(aiw, n);
-    linI[i] = im[i];
-    total += linI[i] + angI[i];
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int l = kl[i];
-    if (l < 0) continue;
+    if (i == 1 && kl[1] < 0) continue;
     R sign = R(1);
     if (i != 0) sign = R(-1);
-    R angM = sign * penetration * (angI[i] / total);
-    R linM = sign * penetration * (linI[i] / total);
-    V3<R> projection = add_scaled(rel[i], n, -dot(rel[i], n));
-    R maxMagnitude = angularLimit * mag(projection);
+    R angM = sign * penetration * mv.ra[i];
+    R linM = sign * penetration * mv.rl[i];
+    const R maxMagnitude = mv.mm[i];
     if (angM < -maxMagnitude) {
       R totalMove = angM + linM;
       angM = -maxMagnitude;
@@ -391,98 +433,114 @@ __device__ __forceinline__ uint32_t isl_position_change(const Bodies<R>& b, cons
       angM = maxMagnitude;
       linM = totalMove - angM;
     }
-    if (angM == R(0)) {
-      ang[i] = V3<R>{R(0), R(0), R(0)};
-    } else {
-      V3<R> tad = cross(rel[i], n);
-      ang[i] = mul(m3v(iw[i], tad), angM / angI[i]);
-    }
+    if (angM != R(0)) ang[i] = mul(mv.td[i], angM / mv.ai[i]);
     lin[i] = mul(n, linM);
-    R* e = W.st + kIslSt * l;
-    const V3<R> pos = add_scaled(tab3(e), n, linM);
-    Q4<R> q{e[3], e[4], e[5], e[6]};
+    if (i == 1 && kl[1] == kl[0])  // a body against itself: from what the first side left
+#pragma unroll
+      for (int q = 0; q < 7; ++q) st[1][q] = st[0][q];
+    const V3<R> pos = add_scaled(V3<R>{st[i][0], st[i][1], st[i][2]}, n, linM);
+    Q4<R> q{st[i][3], st[i][4], st[i][5], st[i][6]};
     q = q_add_scaled_vector(q, ang[i], R(1));
     q = q_normalize(q);
-    tab3_store(e, pos);
-    e[3] = q.w;
-    e[4] = q.x;
-    e[5] = q.y;
-    e[6] = q.z;
-    if (!aw[i]) rederived |= 1u << i;
+    st[i][0] = pos.x; st[i][1] = pos.y; st[i][2] = pos.z;
+    st[i][3] = q.w; st[i][4] = q.x; st[i][5] = q.y; st[i][6] = q.z;
   }
-  // a sleeping body's derived data, from the state just stored (rare, and
-  // large: one copy of the code)
+}
+
+// World inverse inertia and inverse mass of a contact's bodies, from the LDS
+// table where the launch has one.
+template <typename R>
+__device__ __forceinline__ void isl_inertia(const Bodies<R>& b, const IslWorld<R>& W, const int kl[2], R (&iw)[2][9],
+                                            R im[2]) {
+  if (W.iw) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const R* e = W.iw + kIslIw * (kl[i] >= 0 ? kl[i] : kl[0]);
+#pragma unroll
+      for (int q = 0; q < 9; ++q) iw[i][q] = e[q];
+      im[i] = e[9];
+    }
+  } else {
+    const int kb[2] = {W.b0w + kl[0], kl[1] >= 0 ? W.b0w + kl[1] : -1};
+    body_inertia(b, kb, iw, im);
+  }
+}
+
+// The derived data of the sleeping bodies of `red` (bit i: kl[i]), from the
+// state just stored, to HBM and to the table (rare, and large: one copy of the
+// code).
+template <typename R>
+__device__ __forceinline__ void isl_rederive(const Bodies<R>& b, const IslWorld<R>& W, const int kl[2], uint32_t red) {
 #pragma unroll 1
-  for (int i = 0; i < 2 && rederived; ++i) {
-    if (!(rederived >> i & 1u)) continue;
+  for (int i = 0; i < 2 && red; ++i) {
+    if (!(red >> i & 1u)) continue;
     const int l = i == 0 ? kl[0] : kl[1];
     R* e = W.st + kIslSt * l;
     Q4<R> q{e[3], e[4], e[5], e[6]};
-    rederive(b, W.b0w + l, tab3(e), q, 0);
+    R iw[9];
+    rederive(b, W.b0w + l, tab3(e), q, 0, iw);
     e[3] = q.w;
     e[4] = q.x;
     e[5] = q.y;
     e[6] = q.z;
+    if (W.iw) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k) W.iw[kIslIw * l + k] = iw[k];
+    }
   }
-  return rederived;
+}
+// Contacts of a body whose derived data changed take their part of it again.
+// Out of the table that is a few LDS reads; from HBM, where the store has to be
+// waited for as well, such an iteration takes three times as long (3.6 us).
+template <typename R>
+__device__ __forceinline__ void isl_move_again(const Bodies<R>& b, const IslWorld<R>& W, const int jb[2],
+                                               const V3<R>& n, const V3<R> rel[2], IslMove<R>& mv) {
+  R iw[2][9], im[2];
+  if (W.iw) {
+    isl_inertia(b, W, jb, iw, im);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int l = W.b0w + opaque_lane(jb[i] >= 0 ? jb[i] : jb[0]);
+      const volatile R* src = b.iit_world + l;
+#pragma unroll
+      for (int q = 0; q < 9; ++q) iw[i][q] = src[q * b.stride];
+      im[i] = b.inv_mass[l];
+    }
+  }
+  isl_move_of(jb[1] >= 0, n, rel, iw, im, mv);
 }
 
-// matchAwakeState (contact.go:185-202) on the flag table; the motion a woken
-// body gets is written when the phase ends (isl_commit).
+// matchAwakeState (contact.go:185-202) on the flag table, in two parts: the
+// flags of a contact's bodies, read with the rest of what a correction needs,
+// and the store.  The motion a woken body gets is written when the phase ends
+// (isl_commit).  The result has bit i for a body i that stays asleep.
+struct IslAwake {
+  uint8_t f0, f1;
+};
 template <typename R>
-__device__ __forceinline__ void isl_match_awake(const IslWorld<R>& W, const int kl[2], bool aw[2]) {
-  aw[0] = (W.fl[kl[0]] & F_AWAKE) != 0;
-  aw[1] = kl[1] >= 0 && (W.fl[kl[1]] & F_AWAKE) != 0;
-  if (kl[1] >= 0 && (aw[0] || aw[1]) && !(aw[0] && aw[1])) {
-    const int t = aw[0] ? kl[1] : kl[0];
-    W.fl[t] = uint8_t(W.fl[t] | F_AWAKE);
-    aw[0] = aw[1] = true;
-  }
+__device__ __forceinline__ IslAwake isl_awake_of(const IslWorld<R>& W, const int kl[2]) {
+  return IslAwake{W.fl[kl[0]], W.fl[kl[1] >= 0 ? kl[1] : kl[0]]};
+}
+template <typename R>
+__device__ __forceinline__ uint32_t isl_match_awake(const IslWorld<R>& W, const int kl[2], IslAwake f, bool store) {
+  const bool a0 = (f.f0 & F_AWAKE) != 0, a1 = (f.f1 & F_AWAKE) != 0;
+  if (kl[1] < 0) return a0 ? 0u : 1u;
+  if (a0 != a1 && store) W.fl[a0 ? kl[1] : kl[0]] = uint8_t((a0 ? f.f1 : f.f0) | F_AWAKE);
+  return a0 || a1 ? 0u : 3u;
 }
 
 // calculateDesiredDeltaVelocity (contact.go:87-112) from the products of
 // lastFrameAccelleration * dt with the normal (d0, d1), which the phase does
 // not change, and the flags, which it does.
 template <typename R>
-__device__ __forceinline__ R isl_desired_dv(const uint8_t* fl, int l0, int l1, R d0, R d1, R cvx, R e) {
+__device__ __forceinline__ R isl_desired_dv(IslAwake f, bool has1, R d0, R d1, R cvx, R e) {
   R vfa = R(0);
-  if (fl[l0] & F_AWAKE) vfa += d0;
-  if (l1 >= 0 && (fl[l1] & F_AWAKE)) vfa -= d1;
+  if (f.f0 & F_AWAKE) vfa += d0;
+  if (has1 && (f.f1 & F_AWAKE)) vfa -= d1;
   R restitution = e;
   if (dabs(cvx) < R(0.25)) restitution = R(0);
   return -cvx - restitution * (cvx - vfa);
-}
-
-// applyVelocityChange (contact.go:448-494) by the lane that owns the
-// selected contact, the bodies' velocity and rotation in the tables; their
-// new velocity and rotation come back in nv, nw.
-template <typename R, int KIND>
-__device__ __forceinline__ void isl_velocity_change(const IslWorld<R>& W, const int kl[2], const V3<R> rel[2],
-                                                    const R* c2w, R ddv, const V3<R>& cvel, const R* imp,
-                                                    const R (&iw)[2][9], const R im[2], V3<R> vc[2], V3<R> rc[2],
-                                                    V3<R> nv[2], V3<R> nw[2], R friction) {
-  V3<R> ic;
-  if (KIND == KIND_MAT && friction == R(0))
-    ic = V3<R>{ddv / imp[0], R(0), R(0)};
-  else
-    ic = friction_impulse_from(imp, imp + 9, ddv, cvel, friction);
-  const V3<R> impulse = m3v(c2w, ic);
-  const V3<R> zero{R(0), R(0), R(0)};
-  V3<R> torque = cross(rel[0], impulse);
-  rc[0] = m3v(iw[0], torque);
-  vc[0] = add_scaled(zero, impulse, im[0]);
-  rc[1] = vc[1] = nv[1] = nw[1] = zero;
-  const R* e0 = W.st + kIslSt * kl[0];
-  nv[0] = add(tab3(e0), vc[0]);
-  nw[0] = add(tab3(e0 + 3), rc[0]);
-  if (kl[1] >= 0) {
-    torque = cross(impulse, rel[1]);
-    rc[1] = m3v(iw[1], torque);
-    vc[1] = add_scaled(zero, impulse, -im[1]);
-    const R* e1 = W.st + kIslSt * kl[1];
-    nv[1] = add(tab3(e1), vc[1]);
-    nw[1] = add(tab3(e1 + 3), rc[1]);
-  }
 }
 
 // The two bodies' changes through LDS: written by the owner, read by the
@@ -498,6 +556,74 @@ __device__ __forceinline__ void isl_get(const R* x, int d, V3<R>& v, V3<R>& u) {
   x += 6 * d;
   v = V3<R>{x[0], x[1], x[2]};
   u = V3<R>{x[3], x[4], x[5]};
+}
+
+// What a correction of the bodies kl (their changes at x: velocity and
+// rotation) does to the closing velocity of a contact of the bodies jb: side 0,
+// then side 1.  Both terms are computed whatever the sides are: they overlap,
+// where under conditions each would wait for its own reads.  Returns whether
+// the contact is touched.
+template <typename R>
+__device__ __forceinline__ bool isl_touch_velocity(const R* x, const int jb[2], const int kl[2], const R* m9,
+                                                   const V3<R> rel[2], V3<R>& cv) {
+  const bool h0 = jb[0] >= 0 && (jb[0] == kl[0] || jb[0] == kl[1]);
+  const bool h1 = jb[1] >= 0 && (jb[1] == kl[0] || jb[1] == kl[1]);
+  V3<R> v0, u0, v1, u1;
+  isl_get(x, jb[0] == kl[0] ? 0 : 1, v0, u0);
+  isl_get(x, jb[1] == kl[0] ? 0 : 1, v1, u1);
+  const V3<R> t0 = m3tv(m9, add(cross(u0, rel[0]), v0));
+  const V3<R> t1 = mul(m3tv(m9, add(cross(u1, rel[1]), v1)), R(-1));
+  cv = sel3(h0, add(cv, t0), cv);
+  cv = sel3(h1, add(cv, t1), cv);
+  return h0 || h1;
+}
+// The same for a penetration (changes: linear and angular moves).
+template <typename R>
+__device__ __forceinline__ void isl_touch_position(const R* x, const int jb[2], const int kl[2], const V3<R>& n,
+                                                   const V3<R> rel[2], R& key) {
+  const bool h0 = jb[0] >= 0 && (jb[0] == kl[0] || jb[0] == kl[1]);
+  const bool h1 = jb[1] >= 0 && (jb[1] == kl[0] || jb[1] == kl[1]);
+  V3<R> v0, u0, v1, u1;
+  isl_get(x, jb[0] == kl[0] ? 0 : 1, v0, u0);
+  isl_get(x, jb[1] == kl[0] ? 0 : 1, v1, u1);
+  const R t0 = dot(add(cross(u0, rel[0]), v0), n) * R(-1);
+  const R t1 = dot(add(cross(u1, rel[1]), v1), n);
+  key = h0 ? key + t0 : key;
+  key = h1 ? key + t1 : key;
+}
+
+// applyVelocityChange (contact.go:448-494) by the lane that owns the
+// selected contact, the bodies' velocity and rotation in the tables; their
+// new velocity and rotation come back in nv, nw.
+template <typename R, int KIND>
+__device__ __forceinline__ void isl_velocity_change(const IslWorld<R>& W, const int kl[2], const V3<R> rel[2],
+                                                    const R* c2w, R ddv, const V3<R>& cvel, const R* imp,
+                                                    const R (&iw)[2][9], const R im[2], V3<R> vc[2], V3<R> rc[2],
+                                                    V3<R> nv[2], V3<R> nw[2], R friction) {
+  // the bodies' state first: its reads overlap with what follows
+  const R* e0 = W.st + kIslSt * kl[0];
+  const R* e1 = W.st + kIslSt * (kl[1] >= 0 ? kl[1] : kl[0]);
+  const V3<R> v0 = tab3(e0), w0 = tab3(e0 + 3), v1 = tab3(e1), w1 = tab3(e1 + 3);
+  V3<R> ic;
+  if (KIND == KIND_MAT && friction == R(0))
+    ic = V3<R>{ddv / imp[0], R(0), R(0)};
+  else
+    ic = friction_impulse_from(imp, imp + 9, ddv, cvel, friction);
+  const V3<R> impulse = m3v(c2w, ic);
+  const V3<R> zero{R(0), R(0), R(0)};
+  V3<R> torque = cross(rel[0], impulse);
+  rc[0] = m3v(iw[0], torque);
+  vc[0] = add_scaled(zero, impulse, im[0]);
+  rc[1] = vc[1] = nv[1] = nw[1] = zero;
+  nv[0] = add(v0, vc[0]);
+  nw[0] = add(w0, rc[0]);
+  if (kl[1] >= 0) {
+    torque = cross(impulse, rel[1]);
+    rc[1] = m3v(iw[1], torque);
+    vc[1] = add_scaled(zero, impulse, -im[1]);
+    nv[1] = add(v1, vc[1]);
+    nw[1] = add(w1, rc[1]);
+  }
 }
 
 __device__ __forceinline__ uint32_t isl_ids(int c0, int c1, int b0w) {
@@ -520,18 +646,17 @@ __device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R>&
   R key = R(0);
   uint32_t id = 0xFFFFFFFFu;
   V3<R> n{R(0), R(0), R(0)}, rel[2] = {n, n};
-  R iw[2][9], im[2];
-#pragma unroll
-  for (int q = 0; q < 9; ++q) iw[0][q] = iw[1][q] = R(0);
-  im[0] = im[1] = R(0);
+  IslMove<R> mv{};
   if (has) {
     j = a.isl_idx[W.base + a.isl_off[W.b0w + k] + li];
     const int64_t g = W.base + j;
     const int c0 = c.body0[g], c1 = c.body1[g];
     id = isl_ids(c0, c1, W.b0w);
     rec_normal(c.rec + 16 * g, n, rel);
-    const int kb[2] = {c0, c1};
-    body_inertia(a.b, kb, iw, im);
+    const int kl[2] = {id_lo(id), id_hi(id)};
+    R iw[2][9], im[2];
+    isl_inertia(a.b, W, kl, iw, im);
+    isl_move_of(c1 >= 0, n, rel, iw, im, mv);
     if (P.pass == ISL_FREE) {
       key = c.pen[g];
       if (!P.saved) a.isl_save[4 * CS + g] = key;
@@ -543,6 +668,7 @@ __device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R>&
   int64_t logat = P.pass == ISL_LOG && live ? a.isl_log[W.b0w + k] : 0;
   R* x = W.f->x[wave][grp];
   volatile uint32_t* xi = W.f->xi[wave][grp];
+  const uint64_t gm = group_lanes(lg);
   const int jb[2] = {id_lo(id), id_hi(id)};
   int it = 0, nrec = 0;
   R runmin = R(__builtin_inf());
@@ -551,28 +677,39 @@ __device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R>&
     const R kk = (has && live && key > eps) ? key : R(-__builtin_inf());
     const R m = group_reduce(kk, lg, [](R p, R q) { return q > p ? q : p; });
     const bool any = m > R(-__builtin_inf());
-    const int jm = group_reduce((any && kk == m) ? j : INT_MAX, lg, [](int p, int q) { return q < p ? q : p; });
+    const bool top = group_owner<R>(any && kk == m, j, lg, gm);
     live = live && any;
     if (live && it >= lim) {
       over = true;
       live = false;
     }
     if (!__any(live)) break;
-    const bool owner = live && j == jm;
+    const bool owner = live && top;
     if (P.pass == ISL_LOG && live && (nrec == 0 || m <= runmin)) {
       runmin = m;
       if (owner) isl_log(a, logat + nrec, m, j, it);
       ++nrec;
     }
     if (owner) {
-      // opaque: the addresses of the rare sleeping body's data are computed
-      // here and not kept for the whole loop
-      const int kl[2] = {opaque_lane(jb[0]), opaque_lane(jb[1])};
-      bool aw[2];
-      isl_match_awake(W, kl, aw);
+      const int kl[2] = {jb[0], jb[1]};
+      const IslAwake f = isl_awake_of(W, kl);
       V3<R> lin[2], ang[2];
-      const uint32_t red = isl_position_change(a.b, W, kl, aw, n, rel, key, iw, im, lin, ang);
+      R st[2][7];
+      isl_position_change(W, kl, n, key, mv, lin, ang, st);
       isl_put(x, lin, ang);
+      const uint32_t red = isl_match_awake(W, kl, f, true);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (kl[i] < 0) continue;
+#pragma unroll
+        for (int q = 0; q < 7; ++q) W.st[kIslSt * kl[i] + q] = st[i][q];
+      }
+      if (red) {
+        // opaque: the addresses of the rare sleeping body's data are computed
+        // here and not kept for the whole loop
+        const int ko[2] = {opaque_lane(kl[0]), opaque_lane(kl[1])};
+        isl_rederive(a.b, W, ko, red);
+      }
       xi[0] = id;
       xi[1] = red;
       if constexpr (KIND == KIND_LABEL)
@@ -580,37 +717,19 @@ __device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R>&
     }
     wave_fence();
     const uint32_t kid = xi[0], red = xi[1];
-    if (live) {
-      const int kl[2] = {id_lo(kid), id_hi(kid)};
-      R p = key;
-#pragma unroll
-      for (int bb = 0; bb < 2; ++bb) {
-        if (jb[bb] < 0 || !has) continue;
-        if (jb[bb] == kl[0] || jb[bb] == kl[1]) {
-          V3<R> lv, av;
-          isl_get(x, jb[bb] == kl[0] ? 0 : 1, lv, av);
-          const V3<R> dp = add(cross(av, rel[bb]), lv);
-          R sign = R(1);
-          if (bb == 0) sign = R(-1);
-          p += dot(dp, n) * sign;
-        }
-      }
-      key = p;
-      ++it;
-    }
-    // a sleeping body's new world inverse inertia went to HBM
+    const int kl[2] = {id_lo(kid), id_hi(kid)};
+    R p = key;
+    isl_touch_position(x, jb, kl, n, rel, p);
+    key = live ? p : key;
+    it += live ? 1 : 0;
+    // a sleeping body's new world inverse inertia
     if (__any(live && red != 0)) {
-      __threadfence_block();
+      if (!W.iw) __threadfence_block();
+      bool hit = false;
 #pragma unroll
-      for (int bb = 0; bb < 2; ++bb) {
-        const bool hit = live && has && jb[bb] >= 0 &&
-                         ((jb[bb] == id_lo(kid) && (red & 1)) || (jb[bb] == id_hi(kid) && (red & 2)));
-        if (hit) {
-          const volatile R* src = a.b.iit_world + W.b0w + opaque_lane(jb[bb]);
-#pragma unroll
-          for (int q = 0; q < 9; ++q) iw[bb][q] = src[q * a.b.stride];
-        }
-      }
+      for (int bb = 0; bb < 2; ++bb)
+        hit |= jb[bb] >= 0 && ((jb[bb] == kl[0] && (red & 1)) || (jb[bb] == kl[1] && (red & 2)));
+      if (live && has && hit) isl_move_again(a.b, W, jb, n, rel, mv);
     }
     wave_fence();
   }
@@ -677,6 +796,7 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
   const int64_t logat = P.pass == ISL_LOG && live ? a.isl_log[W.b0w + k] : 0;
   R* x = W.f->x[wave][grp];
   volatile uint32_t* xi = W.f->xi[wave][grp];
+  const uint64_t gm = group_lanes(lg);
   const int jb[2] = {id_lo(id), id_hi(id)};
   int it = 0, nrec = 0;
   R runmin = R(__builtin_inf());
@@ -685,14 +805,14 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
     const R kk = (has && live && key > eps) ? key : R(-__builtin_inf());
     const R m = group_reduce(kk, lg, [](R p, R q) { return q > p ? q : p; });
     const bool any = m > R(-__builtin_inf());
-    const int jm = group_reduce((any && kk == m) ? j : INT_MAX, lg, [](int p, int q) { return q < p ? q : p; });
+    const bool top = group_owner<R>(any && kk == m, j, lg, gm);
     live = live && any;
     if (live && it >= lim) {
       over = true;
       live = false;
     }
     if (!__any(live)) break;
-    const bool owner = live && j == jm;
+    const bool owner = live && top;
     if (P.pass == ISL_LOG && live && (nrec == 0 || m <= runmin)) {
       runmin = m;
       if (owner) isl_log(a, logat + nrec, m, j, it);
@@ -700,8 +820,7 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
     }
     if (owner) {
       const int kl[2] = {jb[0], jb[1]};
-      bool aw[2];
-      isl_match_awake(W, kl, aw);
+      const IslAwake f = isl_awake_of(W, kl);
       V3<R> vc[2], rc[2], nv[2], nw[2];
       isl_velocity_change<R, KIND>(W, kl, rel, m9, key, cv, imp, iw, im, vc, rc, nv, nw, fr);
 #pragma unroll
@@ -710,6 +829,7 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
         tab3_store(W.st + kIslSt * kl[i], nv[i]);
         tab3_store(W.st + kIslSt * kl[i] + 3, nw[i]);
       }
+      isl_match_awake(W, kl, f, true);
       isl_put(x, vc, rc);
       xi[0] = id;
       if constexpr (KIND == KIND_LABEL)
@@ -717,25 +837,14 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
     }
     wave_fence();
     const uint32_t kid = xi[0];
-    if (live) {
-      const int kl[2] = {id_lo(kid), id_hi(kid)};
-      bool touched = false;
-#pragma unroll
-      for (int bb = 0; bb < 2; ++bb) {
-        if (jb[bb] < 0 || !has) continue;
-        if (jb[bb] == kl[0] || jb[bb] == kl[1]) {
-          V3<R> vv, rv;
-          isl_get(x, jb[bb] == kl[0] ? 0 : 1, vv, rv);
-          const V3<R> dv = add(cross(rv, rel[bb]), vv);
-          R sign = R(1);
-          if (bb == 1) sign = R(-1);
-          cv = add(cv, mul(m3tv(m9, dv), sign));
-          touched = true;
-        }
-      }
-      if (touched) key = isl_desired_dv(W.fl, jb[0], jb[1], d0, d1, cv.x, rs);
-      ++it;
+    const int kl[2] = {id_lo(kid), id_hi(kid)}, jo[2] = {jb[0] >= 0 ? jb[0] : 0, jb[1]};
+    const IslAwake f = isl_awake_of(W, jo);
+    V3<R> cn = cv;
+    if (isl_touch_velocity(x, jb, kl, m9, rel, cn) && live) {
+      cv = cn;
+      key = isl_desired_dv(f, jb[1] >= 0, d0, d1, cn.x, rs);
     }
+    it += live ? 1 : 0;
     wave_fence();
   }
   if (has && P.pass != ISL_LOG) {
@@ -786,9 +895,9 @@ __device__ __forceinline__ void isl_imp_load(const R* q, R (&v)[kImpPlanes]) {
 // contact per thread everything is in registers, as in the batches; with two,
 // the impulse data come from HBM (written when the island is loaded) and the
 // bodies' inertia from an LDS table where the launch has one; with eight, the
-// records from HBM too.  A velocity iteration has one barrier, after the waves'
-// best contacts and the corrections these would make; a position iteration
-// two, the second after the correction.
+// records from HBM too.  An iteration has one barrier, after the waves' best
+// contacts and the corrections these would make (two more where a sleeping
+// body's derived data change).
 template <typename R, int KIND, bool VEL, int SL>
 __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, const IslPass& P, int k, bool last, R eps,
                                         R& kmin) {
@@ -801,6 +910,8 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
   const int32_t* idx = a.isl_idx + W.base + a.isl_off[W.b0w + k];
   const V3<R> zero{R(0), R(0), R(0)};
   constexpr bool REG = SL == 1;
+  constexpr bool MOVE = !VEL && SL <= 2;  // what a position change keeps is in registers
+  IslMove<R> mv[MOVE ? SL : 1];
   const bool resume = VEL && k == P.resume;
   if (P.pass == ISL_LIMIT && a.isl_its[W.b0w + k] < 0) return;
   R rimp[kImpPlanes], riw[2][9], rim[2];  // REG
@@ -837,7 +948,13 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
       fr[s] = c.fric[g];
       rs[s] = c.rest[g];
     }
-    if constexpr (!VEL && REC) rec_frame(c.rec + 16 * g, rm[s], rrel[s]);
+    if constexpr (MOVE) {
+      rec_frame(c.rec + 16 * g, rm[s], rrel[s]);
+      const int kl[2] = {id_lo(ids[s]), id_hi(ids[s])};
+      R iw[2][9], im[2];
+      isl_inertia(b, W, kl, iw, im);
+      isl_move_of(c1 >= 0, V3<R>{rm[s][0], rm[s][1], rm[s][2]}, rrel[s], iw, im, mv[s]);
+    }
     if constexpr (VEL) {
       R mj[9];
       V3<R> rj[2];
@@ -934,21 +1051,10 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
         if constexpr (REG) {
           isl_velocity_change<R, KIND>(W, kl, rrel[0], rm[0], wm, cv[0], rimp, riw, rim, v, u, nv, nw, fk);
         } else {
-          const int kb[2] = {W.b0w + kl[0], kl[1] >= 0 ? W.b0w + kl[1] : -1};
           R iw[2][9], im[2], mj[9], imp[kImpPlanes];
           V3<R> rel[2];
           isl_imp_load(c.imp + kImpPlanes * g, imp);
-          if (W.iw) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-              const R* e = W.iw + kIslIw * (kl[i] >= 0 ? kl[i] : 0);
-#pragma unroll
-              for (int q = 0; q < 9; ++q) iw[i][q] = e[q];
-              im[i] = e[9];
-            }
-          } else {
-            body_inertia(b, kb, iw, im);
-          }
+          isl_inertia(b, W, kl, iw, im);
           if constexpr (REC) {
 #pragma unroll
             for (int q = 0; q < 9; ++q) mj[q] = bs ? rm[SL - 1][q] : rm[0][q];
@@ -961,6 +1067,38 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
         }
         isl_put(W.f->bx[par][wave], v, u);
         isl_put(W.f->bx[par][wave] + 12, nv, nw);
+      }
+    } else if (tie && bj == wj) {
+      const uint32_t id = pick(ids, bs);
+      const int kl[2] = {id_lo(id), id_hi(id)};
+      V3<R> v[2], u[2], nj;
+      R st[2][7];
+      IslMove<R> mj;
+      if constexpr (MOVE) {
+        nj = sel3(bs != 0, V3<R>{rm[SL - 1][0], rm[SL - 1][1], rm[SL - 1][2]}, V3<R>{rm[0][0], rm[0][1], rm[0][2]});
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          mj.ai[i] = bs ? mv[SL - 1].ai[i] : mv[0].ai[i];
+          mj.ra[i] = bs ? mv[SL - 1].ra[i] : mv[0].ra[i];
+          mj.rl[i] = bs ? mv[SL - 1].rl[i] : mv[0].rl[i];
+          mj.mm[i] = bs ? mv[SL - 1].mm[i] : mv[0].mm[i];
+          mj.td[i] = sel3(bs != 0, mv[SL - 1].td[i], mv[0].td[i]);
+        }
+      } else {
+        R iw[2][9], im[2], m9[9];
+        V3<R> rel[2];
+        rec_frame(c.rec + 16 * (W.base + wj), m9, rel);
+        isl_inertia(b, W, kl, iw, im);
+        nj = V3<R>{m9[0], m9[1], m9[2]};
+        isl_move_of(kl[1] >= 0, nj, rel, iw, im, mj);
+      }
+      isl_position_change(W, kl, nj, pick(key, bs), mj, v, u, st);
+      R* o = W.f->bx[par][wave];
+      isl_put(o, v, u);
+#pragma unroll
+      for (int q = 0; q < 7; ++q) {
+        o[12 + q] = st[0][q];
+        o[19 + q] = st[1][q];
       }
     }
     __syncthreads();
@@ -988,54 +1126,51 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
       if (owner) isl_log(a, logat + nrec, runmin, runj, it);
       ++nrec;
     }
-    const R* x = W.f->x[0][0];
-    if constexpr (VEL) {
-      // Every wave stores the bodies' new state and the woken body's flag (the
-      // same values), so each reads its own stores in the next iteration and
-      // one barrier per iteration is enough; the offers alternate between two
-      // sets.
-      x = W.f->bx[par][bw];
-      const int l = t & 63;
-      if (l < 6) {
-        if (kl[0] != kl[1]) W.st[kIslSt * kl[0] + l] = x[12 + l];
-      } else if (l < 12 && kl[1] >= 0) {
-        W.st[kIslSt * kl[1] + l - 6] = x[12 + l];
-      }
-      if (l == 0) {
-        bool aw[2];
-        isl_match_awake(W, kl, aw);
-      }
-      if constexpr (KIND == KIND_LABEL) {
-        if (owner && P.pass != ISL_LOG) {
+    // Every wave stores the bodies' new state and the woken body's flag (the
+    // same values), so each reads its own stores in the next iteration and
+    // one barrier per iteration is enough; the offers alternate between two
+    // sets.
+    const R* x = W.f->bx[par][bw];
+    constexpr int NS = VEL ? 6 : 7;
+    const int l = t & 63;
+    const IslAwake fa = isl_awake_of(W, kl);
+    if (l < NS) {
+      if (kl[0] != kl[1]) W.st[kIslSt * kl[0] + l] = x[12 + l];
+    } else if (l < 2 * NS && kl[1] >= 0) {
+      W.st[kIslSt * kl[1] + l - NS] = x[12 + l];
+    }
+    const uint32_t red = isl_match_awake(W, kl, fa, l == 0);
+    if constexpr (KIND == KIND_LABEL) {
+      if (owner && P.pass != ISL_LOG) {
+        if constexpr (VEL) {
           const V3<R> v[2] = {V3<R>{x[0], x[1], x[2]}, V3<R>{x[6], x[7], x[8]}};
           const V3<R> u[2] = {V3<R>{x[3], x[4], x[5]}, V3<R>{x[9], x[10], x[11]}};
           add_label(a, W.base + jm, v, u);
-        }
-      }
-      wave_fence();
-    } else {
-      if (owner) {
-        const int kb[2] = {W.b0w + kl[0], kl[1] >= 0 ? W.b0w + kl[1] : -1};
-        V3<R> v[2], u[2];
-        bool aw[2];
-        isl_match_awake(W, kl, aw);
-        R iw[2][9], im[2], mj[9];
-        V3<R> rel[2];
-        if constexpr (REC) {
-#pragma unroll
-          for (int q = 0; q < 9; ++q) mj[q] = bs ? rm[SL - 1][q] : rm[0][q];
-          rel[0] = sel3(bs != 0, rrel[SL - 1][0], rrel[0][0]);
-          rel[1] = sel3(bs != 0, rrel[SL - 1][1], rrel[0][1]);
         } else {
-          rec_frame(c.rec + 16 * (W.base + jm), mj, rel);
+          add_pos_label(a, W.base + jm, m);
         }
-        body_inertia(b, kb, iw, im);
-        isl_position_change(b, W, kl, aw, V3<R>{mj[0], mj[1], mj[2]}, rel, m, iw, im, v, u);
-        if constexpr (KIND == KIND_LABEL)
-          if (P.pass != ISL_LOG) add_pos_label(a, W.base + jm, m);
-        isl_put(W.f->x[0][0], v, u);
       }
-      __syncthreads();  // also: a sleeping body's new tensor, before the next iteration reads it
+    }
+    wave_fence();
+    if constexpr (!VEL) {
+      // Another wave may have stored a woken body's flag before this one read
+      // it; asleep it stays only if no wave wakes it, so all agree.
+      if (__any(red != 0)) {
+        __syncthreads();  // every wave has stored the state the owner now corrects
+        if (owner) isl_rederive(b, W, kl, red);
+        __syncthreads();
+        if constexpr (MOVE) {
+#pragma unroll
+          for (int s = 0; s < SL; ++s) {
+            const int jb[2] = {id_lo(ids[s]), id_hi(ids[s])};
+            bool hit = false;
+#pragma unroll
+            for (int bb = 0; bb < 2; ++bb)
+              hit |= jb[bb] >= 0 && ((jb[bb] == kl[0] && (red & 1)) || (jb[bb] == kl[1] && (red & 2)));
+            if (hit) isl_move_again(b, W, jb, V3<R>{rm[s][0], rm[s][1], rm[s][2]}, rrel[s], mv[s]);
+          }
+        }
+      }
     }
     par ^= 1;
 #pragma unroll
@@ -1057,21 +1192,10 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
         rec_frame(c.rec + 16 * (W.base + int(js[s])), mj, rj);
       }
       const V3<R> nj{mj[0], mj[1], mj[2]};
-#pragma unroll
-      for (int bb = 0; bb < 2; ++bb) {
-        if (jb[bb] < 0 || !(jb[bb] == kl[0] || jb[bb] == kl[1])) continue;
-        V3<R> v, u;
-        isl_get(x, jb[bb] == kl[0] ? 0 : 1, v, u);
-        const V3<R> d = add(cross(u, rj[bb]), v);
-        R sign = R(1);
-        if constexpr (VEL) {
-          if (bb == 1) sign = R(-1);
-          cv[s] = add(cv[s], mul(m3tv(mj, d), sign));
-        } else {
-          if (bb == 0) sign = R(-1);
-          key[s] += dot(d, nj) * sign;
-        }
-      }
+      if constexpr (VEL)
+        isl_touch_velocity(x, jb, kl, mj, rj, cv[s]);
+      else
+        isl_touch_position(x, jb, kl, nj, rj, key[s]);
       if constexpr (VEL) {
         R d0, d1 = R(0);
         if constexpr (DN) {
@@ -1086,7 +1210,7 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
           e = rs[s];
         else
           e = restitution_of<R, KIND>(c, W.base + int(js[s]));
-        key[s] = isl_desired_dv(W.fl, jb[0], jb[1], d0, d1, cv[s].x, e);
+        key[s] = isl_desired_dv(isl_awake_of(W, jb), jb[1] >= 0, d0, d1, cv[s].x, e);
       }
     }
     ++it;
@@ -1132,7 +1256,7 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
   __syncthreads();
   const int32_t* cls = W.f->cls;
   const int n0 = cls[0], n1 = cls[1], nbig = n0 + n1 + cls[2];
-  if (VEL && W.iw && n0 + n1 > 0) {
+  if (W.iw && (!VEL || n0 + n1 > 0)) {
     for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
       R iw[9];
       ld9(a.b.iit_world, a.b.stride, W.b0w + i, iw);
@@ -1141,6 +1265,7 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
       W.iw[kIslIw * i + 9] = a.b.inv_mass[W.b0w + i];
     }
   }
+  if constexpr (!VEL) __syncthreads();
   while (!P.only) {
     // every lane adds one (one LDS operation for the wave); under a branch on
     // the lane, the compiler makes the other lanes a loop of their own, which
@@ -1573,8 +1698,8 @@ __device__ __forceinline__ void isl_take_changes(const RS<R>& a, const IslWorld<
       const R d0 = dot(mul(ld3(b.last_acc, S, kb[0]), a.dt), nj);
       const R d1 = kb[1] >= 0 ? dot(mul(ld3(b.last_acc, S, kb[1]), a.dt), nj) : R(0);
       st3(c.cvel, CS, gj, cvj);
-      c.ddv[gj] = isl_desired_dv(W.fl, kb[0] - W.b0w, kb[1] >= 0 ? kb[1] - W.b0w : -1, d0, d1, cvj.x,
-                                 restitution_of<R, KIND_POLISH>(c, gj));
+      const int jl[2] = {kb[0] - W.b0w, kb[1] >= 0 ? kb[1] - W.b0w : -1};
+      c.ddv[gj] = isl_desired_dv(isl_awake_of(W, jl), kb[1] >= 0, d0, d1, cvj.x, restitution_of<R, KIND_POLISH>(c, gj));
     }
   }
   __syncthreads();

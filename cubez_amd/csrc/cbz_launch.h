@@ -93,6 +93,7 @@ struct ResolveLaunch {
   const int64_t* world_coff;
   const int32_t* overflow;
   const int32_t* order;
+  int32_t* cost = nullptr;  // [2][n_worlds] what the worlds take, and the order by it (or null)
   const int32_t* body_off;
   int64_t* world_iters;
   int64_t* world_time = nullptr;         // [4][n_worlds] wall-clock ticks (see the resolver's RS)

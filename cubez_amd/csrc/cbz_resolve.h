@@ -344,12 +344,12 @@ __device__ __forceinline__ void match_awake(const RS<R>& a, int k0, int k1, bool
 }
 
 // CalculateDerivedData (rigidbody.go:268-272) for a sleeping body moved by
-// applyPositionChange (contact.go:380-382).
+// applyPositionChange (contact.go:380-382); IW: its world inverse inertia.
 template <typename R>
-__device__ __forceinline__ void rederive(const Bodies<R>& b, int i, const V3<R>& pos, Q4<R>& q, int lane) {
+__device__ __forceinline__ void rederive(const Bodies<R>& b, int i, const V3<R>& pos, Q4<R>& q, int lane, R (&IW)[9]) {
   const int64_t S = b.stride;
   q = q_normalize(q);
-  R T[12], IB[9], IW[9];
+  R T[12], IB[9];
   set_as_transform(pos, q, T);
   ld9(b.iit_body, S, i, IB);
   transform_inertia(IB, T, IW);
@@ -416,7 +416,8 @@ __device__ __forceinline__ void apply_position_change(const RS<R>& a, const int 
     Q4<R> q{b.quat[bi], b.quat[S + bi], b.quat[2 * S + bi], b.quat[3 * S + bi]};
     q = q_add_scaled_vector(q, ang[i], R(1));
     q = q_normalize(q);
-    if (!aw[i]) rederive(b, bi, pos, q, lane);
+    R iwn[9];
+    if (!aw[i]) rederive(b, bi, pos, q, lane, iwn);
     if (lane == 0) {
       st3(b.pos, S, bi, pos);
       b.quat[bi] = q.w;
