@@ -125,8 +125,15 @@ struct cbz_context {
   int64_t plane_pairs = 0;          // body-plane pairs of the scene
   int32_t max_planes = 0;           // of one world
   int64_t cand_cap = 0;
-  // explicit-list pair space (grown on demand)
-  int32_t l_tiles_cap = 0, l_pairs_cap = 0;
+  // pinned host memory for what the host reads and writes in every step
+  // (kStageBytes, then kStatusBytes for the status words), and whether an
+  // upload out of it may be in flight
+  char* stage = nullptr;
+  bool stage_busy = false;
+  // explicit-list pair space: one allocation, grown on demand; the pointers
+  // below are places in it
+  int32_t* l_mem = nullptr;
+  int64_t l_mem_cap = 0, l_pairs_cap = 0;
   int32_t l_max_tiles = 0;  // the most tiles of one world in the last pair list
   int32_t* l_tile_world = nullptr;
   int32_t* l_world_tile0 = nullptr;
@@ -331,25 +338,85 @@ int upload_real(cbz_ctx* c, void* dst, const double* src, int64_t n, int k) {
   return CBZ_OK;
 }
 
-// Device [k][stride] (from element `first`, n elements) -> host [n][k] doubles.
-int download_real(cbz_ctx* c, const void* srcbase, int64_t stride, int64_t first, int64_t n, int k, double* dst) {
-  if (n == 0) return CBZ_OK;
-  if (c->precision == CBZ_F64) {
-    std::vector<double> t((size_t)n);
-    for (int j = 0; j < k; ++j) {
-      const double* s = (const double*)srcbase + (size_t)j * stride + first;
-      HIPCHK(c, hipMemcpy(t.data(), s, n * sizeof(double), hipMemcpyDeviceToHost));
-      for (int64_t i = 0; i < n; ++i) dst[(size_t)i * k + j] = t[i];
+// The stage: copies between it and the device are queued behind the kernels
+// and waited for once, where a copy from or to pageable memory is waited for by
+// itself: some 12 us each, a dozen of them in a frame of a program that hands over
+// its pair list, 237 us a frame where one upload and one download make it 66.
+// It is a megabyte; whoever needs more does so in pieces, and lists larger
+// than it are uploaded as before.
+constexpr size_t kStageBytes = size_t(1) << 20, kStatusBytes = 256;
+constexpr int kStatusWords = 7;
+int stage_ready(cbz_ctx* c) {
+  if (!c->stage) HIPCHK(c, hipHostMalloc((void**)&c->stage, kStageBytes + kStatusBytes, hipHostMallocDefault));
+  if (c->stage_busy) {
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->stage_busy = false;
+  }
+  return CBZ_OK;
+}
+int stage_wait(cbz_ctx* c) {
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->stage_busy = false;
+  return CBZ_OK;
+}
+
+// One plane of n elements for the host: `size` bytes each as they are, or
+// (k > 0) reals into component j of dst[n][k] doubles.
+struct Plane {
+  const void* src;
+  size_t size;
+  void* dst;
+  int k = 0, j = 0;
+};
+// Planes -> host, through the stage, when the stream's work is done.
+int fetch_planes(cbz_ctx* c, const Plane* planes, int count, int64_t n) {
+  int rc = stage_ready(c);
+  if (rc || n <= 0 || count <= 0) return rc;
+  size_t per = 0;
+  for (int q = 0; q < count; ++q) per += planes[q].size;
+  const int64_t most = int64_t(kStageBytes / per) & ~int64_t(7);  // planes start at 8-byte places
+  for (int64_t at = 0; at < n; at += most) {
+    const int64_t m = std::min(n - at, most), room = (m + 7) & ~int64_t(7);
+    size_t off = 0;
+    for (int q = 0; q < count; ++q) {
+      HIPCHK(c, hipMemcpyAsync(c->stage + off, (const char*)planes[q].src + at * planes[q].size, m * planes[q].size,
+                               hipMemcpyDeviceToHost, c->stream));
+      off += room * planes[q].size;
     }
-  } else {
-    std::vector<float> t((size_t)n);
-    for (int j = 0; j < k; ++j) {
-      const float* s = (const float*)srcbase + (size_t)j * stride + first;
-      HIPCHK(c, hipMemcpy(t.data(), s, n * sizeof(float), hipMemcpyDeviceToHost));
-      for (int64_t i = 0; i < n; ++i) dst[(size_t)i * k + j] = (double)t[i];
+    if ((rc = stage_wait(c))) return rc;
+    off = 0;
+    for (int q = 0; q < count; ++q) {
+      const Plane& P = planes[q];
+      const char* p = c->stage + off;
+      off += room * P.size;
+      if (P.k == 0) {
+        std::memcpy((char*)P.dst + at * P.size, p, m * P.size);
+        continue;
+      }
+      double* d = (double*)P.dst + at * P.k + P.j;
+      if (P.size == sizeof(double))
+        for (int64_t i = 0; i < m; ++i) d[i * P.k] = ((const double*)p)[i];
+      else
+        for (int64_t i = 0; i < m; ++i) d[i * P.k] = (double)((const float*)p)[i];
     }
   }
   return CBZ_OK;
+}
+int fetch(cbz_ctx* c, void* dst, const void* src, size_t size, int64_t n) {
+  const Plane p{src, size, dst};
+  return fetch_planes(c, &p, 1, n);
+}
+// The planes of device [k][stride] (from element `first`) for host [n][k] doubles.
+void real_planes(cbz_ctx* c, std::vector<Plane>& out, const void* srcbase, int64_t stride, int64_t first, int k,
+                 double* dst) {
+  const size_t rs = real_size(c);
+  for (int j = 0; j < k; ++j) out.push_back(Plane{(const char*)srcbase + ((size_t)j * stride + first) * rs, rs, dst, k, j});
+}
+// Device [k][stride] (from element `first`, n elements) -> host [n][k] doubles.
+int download_real(cbz_ctx* c, const void* srcbase, int64_t stride, int64_t first, int64_t n, int k, double* dst) {
+  std::vector<Plane> p;
+  real_planes(c, p, srcbase, stride, first, k, dst);
+  return fetch_planes(c, p.data(), (int)p.size(), n);
 }
 
 void drop_graph(cbz_ctx* c) {
@@ -399,9 +466,8 @@ void free_scene(cbz_ctx* c) {
   dfree(c->d_task_world);
   dfree(c->d_world_task0);
   dfree(c->hits);
-  dfree(c->n_hits);
   dfree(c->cand);
-  dfree(c->n_cand);
+  c->n_hits = c->n_cand = nullptr;  // in total
   {
     auto& bp = c->bp;
     dfree(bp.body_world);
@@ -418,12 +484,8 @@ void free_scene(cbz_ctx* c) {
     dfree(bp.tmp);
     bp = cbz_context::Broad{};
   }
-  dfree(c->l_tile_world);
-  dfree(c->l_world_tile0);
-  dfree(c->l_world_q);
-  dfree(c->l_off);
-  dfree(c->l_one);
-  dfree(c->l_two);
+  dfree(c->l_mem);
+  c->l_one = c->l_two = c->l_off = c->l_world_tile0 = c->l_world_q = c->l_tile_world = nullptr;
   dfree(c->l_cnt);
   dfree(c->tile_cnt);
   dfree(c->tile_off);
@@ -435,7 +497,7 @@ void free_scene(cbz_ctx* c) {
   dfree(c->world_cnt);
   dfree(c->world_coff);
   dfree(c->total);
-  c->n_pairs = c->overflow = nullptr;  // in n_hits
+  c->n_pairs = c->overflow = nullptr;
   dfree(c->d_body_world);
   dfree(c->world_iters);
   dfree(c->world_time);
@@ -446,7 +508,7 @@ void free_scene(cbz_ctx* c) {
   dfree(c->d_awake);
   dfree(c->d_prof);
   dfree(c->pos0);
-  c->l_tiles_cap = c->l_pairs_cap = c->tiles_cap = 0;
+  c->l_mem_cap = c->l_pairs_cap = c->tiles_cap = 0;
   c->have_contacts = false;
 }
 
@@ -732,55 +794,84 @@ int do_resolve(cbz_ctx* c, double dt, int64_t mult, int64_t fixed, int32_t mode 
 }
 
 // List buffers for n_pairs explicit pairs.
+// Places for a list of n_pairs: one, two and the first pair of every world
+// (uploaded, or made by the broadphase), then what every list is uploaded with.
 int ensure_list(cbz_ctx* c, int64_t n_pairs) {
   int rc;
-  if (n_pairs > c->l_pairs_cap) {
-    if ((rc = dalloc(c, &c->l_one, (size_t)n_pairs))) return rc;
-    if ((rc = dalloc(c, &c->l_two, (size_t)n_pairs))) return rc;
+  if (n_pairs > c->l_pairs_cap || !c->l_cnt) {
     if ((rc = dalloc(c, &c->l_cnt, (size_t)n_pairs))) return rc;
-    c->l_pairs_cap = (int32_t)n_pairs;
+    c->l_pairs_cap = n_pairs;
   }
-  if (!c->l_world_tile0) {
-    if ((rc = dalloc(c, &c->l_world_tile0, (size_t)c->nw + 1))) return rc;
-    if ((rc = dalloc(c, &c->l_world_q, (size_t)c->nw))) return rc;
-    if ((rc = dalloc(c, &c->l_off, (size_t)c->nw + 1))) return rc;
+  const int64_t nw = c->nw, need = 2 * n_pairs + (nw + 1) + (nw + 1) + nw + n_pairs / 64 + nw;
+  if (need > c->l_mem_cap) {
+    c->l_mem_cap = 0;
+    if ((rc = dalloc(c, &c->l_mem, (size_t)need))) return rc;
+    c->l_mem_cap = need;
   }
+  c->l_one = c->l_mem;
+  c->l_two = c->l_one + n_pairs;
+  c->l_off = c->l_two + n_pairs;
+  c->l_world_tile0 = c->l_off + nw + 1;
+  c->l_world_q = c->l_world_tile0 + nw + 1;
+  c->l_tile_world = c->l_world_q + nw;
   return CBZ_OK;
 }
 
-int check_overflow(cbz_ctx* c);
+int check_overflow(cbz_ctx* c, int64_t* total = nullptr);
 
 // The explicit-list narrowphase over l_one/l_two (world w's pairs from
-// l_off[w], wq[w] of them): tiles of 64 consecutive pairs per world.
-int run_list_narrowphase(cbz_ctx* c, const std::vector<int32_t>& wq, int64_t* total) {
-  std::vector<int32_t> wt0(c->nw + 1), tw;
+// l_off[w], wq[w] of them): tiles of 64 consecutive pairs per world.  With
+// `one` the list is the caller's, uploaded with the rest in one copy.
+int run_list_narrowphase(cbz_ctx* c, const std::vector<int32_t>& wq, int64_t* total, int64_t n_pairs = 0,
+                         const int32_t* one = nullptr, const int32_t* two = nullptr) {
+  const int64_t nw = c->nw;
   int64_t nt = 0;
   c->l_max_tiles = 0;
   for (int32_t w = 0; w < c->nw; ++w) {
-    wt0[w] = (int32_t)nt;
     nt += (wq[w] + 63) / 64;
     c->l_max_tiles = std::max(c->l_max_tiles, (wq[w] + 63) / 64);
   }
-  wt0[c->nw] = (int32_t)nt;
   if (nt > INT32_MAX / 64) return fail(c, CBZ_ERR_ARG, "narrowphase: pair list too long");
-  tw.resize((size_t)nt);
-  for (int32_t w = 0; w < c->nw; ++w)
-    for (int32_t t = wt0[w]; t < wt0[w + 1]; ++t) tw[t] = w;
   int rc;
-  if (nt > c->l_tiles_cap) {
-    if ((rc = dalloc(c, &c->l_tile_world, (size_t)nt))) return rc;
-    c->l_tiles_cap = (int32_t)nt;
-  }
   if ((rc = ensure_tiles(c, (int32_t)std::max<int64_t>(nt, 1)))) return rc;
-  if (nt > 0) HIPCHK(c, hipMemcpy(c->l_tile_world, tw.data(), nt * sizeof(int32_t), hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->l_world_tile0, wt0.data(), wt0.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->l_world_q, wq.data(), wq.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-  HIPCHK(c, launch_fill_i32(c->overflow, 2, 0, c->stream));
-  rc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, (int32_t)nt) : do_narrowphase<float>(c, (int32_t)nt);
+  if ((rc = stage_ready(c))) return rc;
+  // the order of ensure_list's places
+  int32_t* dst = one ? c->l_one : c->l_world_tile0;
+  const size_t words = (size_t)((one ? 2 * n_pairs + nw + 1 : 0) + (nw + 1) + nw + nt);
+  std::vector<int32_t> large;
+  int32_t* p = (int32_t*)c->stage;
+  if (words * sizeof(int32_t) > kStageBytes) {
+    large.resize(words);
+    p = large.data();
+  }
+  int32_t* const from = p;
+  if (one) {
+    std::memcpy(p, one, n_pairs * sizeof(int32_t));
+    std::memcpy(p + n_pairs, two, n_pairs * sizeof(int32_t));
+    p += 2 * n_pairs;
+    *p = 0;
+    for (int32_t w = 0; w < c->nw; ++w) p[w + 1] = p[w] + wq[w];
+    p += nw + 1;
+  }
+  *p = 0;
+  for (int32_t w = 0; w < c->nw; ++w) p[w + 1] = p[w] + (wq[w] + 63) / 64;
+  const int32_t* wt0 = p;
+  p += nw + 1;
+  std::copy(wq.begin(), wq.end(), p);
+  p += nw;
+  for (int32_t w = 0; w < c->nw; ++w) std::fill(p + wt0[w], p + wt0[w + 1], w);
+  if (large.empty()) {
+    HIPCHK(c, hipMemcpyAsync(dst, from, words * sizeof(int32_t), hipMemcpyHostToDevice, c->stream));
+    c->stage_busy = true;
+  } else {
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, hipMemcpy(dst, from, words * sizeof(int32_t), hipMemcpyHostToDevice));
+  }
+  HIPCHK(c, launch_fill_i32(c->n_hits, kNarrowCounters + 1, 0, c->stream));  // the sticky flag too
+  rc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, (int32_t)nt, nullptr, true)
+                               : do_narrowphase<float>(c, (int32_t)nt, nullptr, true);
   if (rc) return rc;
-  if ((rc = check_overflow(c))) return rc;
-  if (total) HIPCHK(c, hipMemcpy(total, c->total, sizeof(int64_t), hipMemcpyDeviceToHost));
-  return CBZ_OK;
+  return check_overflow(c, total);
 }
 
 // Broadphase buffers sized for the scene (and pair keys for pcap pairs).
@@ -870,8 +961,7 @@ int do_broadphase(cbz_ctx* c, int64_t* n_pairs) {
   for (int round = 0; round < 2; ++round) {
     pp.pkey = bp.pkey_in;
     HIPCHK(c, launch_bp_sweep<R>(bp_args<R>(c), pp, c->stream));
-    HIPCHK(c, hipMemcpyAsync(&found, bp.pcount, sizeof found, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if ((rc = fetch(c, &found, bp.pcount, sizeof found, 1))) return rc;
     if (bp.plane_pairs + found > INT32_MAX / 2)
       return fail(c, CBZ_ERR_CAPACITY, "broadphase: more than 2^30 candidate pairs");
     if (bp.plane_pairs + found <= bp.pcap) break;
@@ -887,13 +977,22 @@ int do_broadphase(cbz_ctx* c, int64_t* n_pairs) {
   return CBZ_OK;
 }
 
-int check_overflow(cbz_ctx* c) {
-  int32_t of = 0, nc = 0;
+int check_overflow(cbz_ctx* c, int64_t* total) {
+  // the status words (see set_scene) in one copy; an upload may still be on
+  // its way out of the rest of the stage
+  if (!c->stage) {
+    const int rc = stage_ready(c);
+    if (rc) return rc;
+  }
+  const int32_t* st = (const int32_t*)(c->stage + kStageBytes);
+  HIPCHK(c, hipMemcpyAsync(c->stage + kStageBytes, c->total, kStatusWords * sizeof(int32_t), hipMemcpyDeviceToHost,
+                           c->stream));
+  const int rc = stage_wait(c);
+  if (rc) return rc;
   int64_t tot = 0;
-  HIPCHK(c, hipMemcpyAsync(&of, c->overflow + 1, sizeof of, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(&tot, c->total, sizeof tot, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipMemcpyAsync(&nc, c->n_cand, sizeof nc, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  std::memcpy(&tot, st, sizeof tot);
+  const int32_t of = st[(c->overflow + 1) - (int32_t*)c->total], nc = st[c->n_cand - (int32_t*)c->total];
+  if (total) *total = tot;
   if (of && nc > c->cand_cap)
     return fail(c, CBZ_ERR_CAPACITY,
                 "narrowphase candidate list exceeded: " + std::to_string(nc) + " candidate pairs for " +
@@ -1395,6 +1494,7 @@ int cbz_destroy(cbz_ctx* c) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : c->pev)
     if (e) (void)hipEventDestroy(e);
+  if (c->stage) (void)hipHostFree(c->stage);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
   return CBZ_OK;
@@ -1498,11 +1598,14 @@ int cbz_set_scene(cbz_ctx* c, int32_t n_worlds, const int32_t* body_off, const i
   if ((rc = dalloc_bytes(c, &c->c_real, rs * kContactPlanes * (size_t)c->cap))) return rc;
   if ((rc = dalloc_bytes(c, &c->c_rec, rs * 16 * (size_t)c->cap))) return rc;
   if ((rc = dalloc(c, &c->hits, (size_t)c->cap))) return rc;
-  // n_hits, n_pairs, overflow[0..1]: the narrowphase's counters side by side
-  if ((rc = dalloc(c, &c->n_hits, 4))) return rc;
-  static_assert(kNarrowCounters == 3, "hits, pairs, overflow[0]");
+  // the status words: the total (2 words), the narrowphase's counters n_hits,
+  // n_pairs, overflow[0..1] side by side, n_cand
+  if ((rc = dalloc(c, (int32_t**)&c->total, kStatusWords))) return rc;
+  static_assert(kNarrowCounters == 3 && kStatusWords == 7, "hits, pairs, overflow[0]");
+  c->n_hits = (int32_t*)c->total + 2;
   c->n_pairs = c->n_hits + 1;
   c->overflow = c->n_hits + 2;
+  c->n_cand = c->n_hits + 4;
   // candidate pairs of the cull: 4 per contact slot plus the scene's ordered
   // pairs up to 32 M (a dense pile keeps many pairs inside the cull's bound)
   int64_t pairs_total = 0;
@@ -1520,10 +1623,8 @@ int cbz_set_scene(cbz_ctx* c, int32_t n_worlds, const int32_t* body_off, const i
   HIPCHK(c, hipMemcpy(c->d_body_world, bw.data(), bw.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   c->cand_cap = std::min<int64_t>(4 * c->cap + std::min<int64_t>(pairs_total, int64_t(32) << 20), INT32_MAX);
   if ((rc = dalloc(c, &c->cand, (size_t)c->cand_cap))) return rc;
-  if ((rc = dalloc(c, &c->n_cand, 1))) return rc;
   if ((rc = dalloc(c, &c->world_cnt, (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->world_coff, (size_t)n_worlds))) return rc;
-  if ((rc = dalloc(c, &c->total, 1))) return rc;
   if ((rc = dalloc(c, &c->world_iters, 2 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->world_time, 4 * (size_t)n_worlds))) return rc;
   if ((rc = dalloc(c, &c->order, (size_t)n_worlds))) return rc;
@@ -1650,7 +1751,6 @@ int cbz_get_field(cbz_ctx* c, int32_t field, void* host) {
   if (rc) return rc;
   if (field < 0 || field >= CBZ_NUM_FIELDS || !host) return fail(c, CBZ_ERR_ARG, "get_field: bad field");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   const FieldInfo& fi = kFields[field];
   const int64_t nb = c->nb;
   if (field == CBZ_LIN_DAMP || field == CBZ_ANG_DAMP) {
@@ -1659,11 +1759,10 @@ int cbz_get_field(cbz_ctx* c, int32_t field, void* host) {
     return CBZ_OK;
   }
   if (fi.kind == 1) {
-    if (nb > 0) HIPCHK(c, hipMemcpy(host, c->field[field], nb * sizeof(int32_t), hipMemcpyDeviceToHost));
-    return CBZ_OK;
+    return fetch(c, host, c->field[field], sizeof(int32_t), nb);
   }
   if (fi.kind == 2) {
-    if (nb > 0) HIPCHK(c, hipMemcpy(host, c->field[field], nb, hipMemcpyDeviceToHost));
+    if ((rc = fetch(c, host, c->field[field], 1, nb))) return rc;
     uint8_t* h = (uint8_t*)host;
     for (int64_t i = 0; i < nb; ++i) h[i] &= kUserFlags;
     return CBZ_OK;
@@ -1693,12 +1792,11 @@ int cbz_narrowphase(cbz_ctx* c, int64_t* total) {
   int rc = need_scene(c);
   if (rc) return rc;
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, launch_fill_i32(c->overflow, 2, 0, c->stream));
-  rc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, -1) : do_narrowphase<float>(c, -1);
+  HIPCHK(c, launch_fill_i32(c->n_hits, kNarrowCounters + 1, 0, c->stream));  // the sticky flag too
+  rc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, -1, nullptr, true)
+                               : do_narrowphase<float>(c, -1, nullptr, true);
   if (rc) return rc;
-  if ((rc = check_overflow(c))) return rc;
-  if (total) HIPCHK(c, hipMemcpy(total, c->total, sizeof(int64_t), hipMemcpyDeviceToHost));
-  return CBZ_OK;
+  return check_overflow(c, total);
 }
 
 int cbz_narrowphase_pairs(cbz_ctx* c, int64_t n_pairs, const int32_t* one, const int32_t* two, int64_t* total) {
@@ -1716,7 +1814,7 @@ int cbz_narrowphase_pairs(cbz_ctx* c, int64_t n_pairs, const int32_t* one, const
     auto it = std::upper_bound(c->plane_off.begin(), c->plane_off.end(), p);
     return (int32_t)(it - c->plane_off.begin()) - 1;
   };
-  std::vector<int32_t> loff(c->nw + 1, 0), wq(c->nw, 0);
+  std::vector<int32_t> wq(c->nw, 0);
   int32_t prev = 0;
   for (int64_t k = 0; k < n_pairs; ++k) {
     int32_t wa = -1, wb = -1;
@@ -1739,16 +1837,9 @@ int cbz_narrowphase_pairs(cbz_ctx* c, int64_t n_pairs, const int32_t* one, const
     prev = wa;
     wq[wa]++;
   }
-  for (int32_t w = 0; w < c->nw; ++w) loff[w + 1] = loff[w] + wq[w];
   if ((rc = ensure_list(c, n_pairs))) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (n_pairs > 0) {
-    HIPCHK(c, hipMemcpy(c->l_one, one, n_pairs * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->l_two, two, n_pairs * sizeof(int32_t), hipMemcpyHostToDevice));
-  }
-  HIPCHK(c, hipMemcpy(c->l_off, loff.data(), loff.size() * sizeof(int32_t), hipMemcpyHostToDevice));
   c->l_last = -1;
-  if ((rc = run_list_narrowphase(c, wq, total))) return rc;
+  if ((rc = run_list_narrowphase(c, wq, total, n_pairs, one ? one : &prev, two ? two : &prev))) return rc;
   c->l_last = n_pairs;
   return CBZ_OK;
 }
@@ -1759,9 +1850,7 @@ int cbz_pair_contact_counts(cbz_ctx* c, int64_t n_pairs, int32_t* counts) {
   if (n_pairs != c->l_last)
     return fail(c, CBZ_ERR_ARG, "pair_contact_counts: n_pairs differs from the last cbz_narrowphase_pairs");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  if (n_pairs > 0) HIPCHK(c, hipMemcpy(counts, c->l_cnt, n_pairs * sizeof(int32_t), hipMemcpyDeviceToHost));
-  return CBZ_OK;
+  return fetch(c, counts, c->l_cnt, sizeof(int32_t), n_pairs);
 }
 
 int cbz_narrowphase_broad(cbz_ctx* c, int64_t* total, int64_t* pairs_checked) {
@@ -1772,8 +1861,7 @@ int cbz_narrowphase_broad(cbz_ctx* c, int64_t* total, int64_t* pairs_checked) {
   rc = c->precision == CBZ_F64 ? do_broadphase<double>(c, &n) : do_broadphase<float>(c, &n);
   if (rc) return rc;
   std::vector<int32_t> loff((size_t)c->nw + 1), wq((size_t)c->nw);
-  HIPCHK(c, hipMemcpyAsync(loff.data(), c->l_off, loff.size() * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  if ((rc = fetch(c, loff.data(), c->l_off, sizeof(int32_t), (int64_t)loff.size()))) return rc;
   for (int32_t w = 0; w < c->nw; ++w) wq[w] = loff[w + 1] - loff[w];
   if (pairs_checked) *pairs_checked = n;
   return run_list_narrowphase(c, wq, total);
@@ -1784,9 +1872,8 @@ int cbz_contact_counts(cbz_ctx* c, int64_t* counts) {
   if (rc) return rc;
   if (!counts) return fail(c, CBZ_ERR_ARG, "contact_counts: null output");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   std::vector<int32_t> t((size_t)c->nw);
-  HIPCHK(c, hipMemcpy(t.data(), c->world_cnt, c->nw * sizeof(int32_t), hipMemcpyDeviceToHost));
+  if ((rc = fetch(c, t.data(), c->world_cnt, sizeof(int32_t), c->nw))) return rc;
   for (int32_t w = 0; w < c->nw; ++w) counts[w] = t[w];
   return CBZ_OK;
 }
@@ -1796,16 +1883,15 @@ int cbz_get_contacts(cbz_ctx* c, int32_t world, cbz_contact_view* out) {
   if (rc) return rc;
   if (!out || world < -1 || world >= c->nw) return fail(c, CBZ_ERR_ARG, "get_contacts: bad arguments");
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   int64_t n = 0, off = 0;
   if (world < 0) {  // every world: the lists are packed in world order from slot 0
     if (!c->have_contacts) return CBZ_OK;
-    HIPCHK(c, hipMemcpy(&n, c->total, sizeof n, hipMemcpyDeviceToHost));
+    if ((rc = fetch(c, &n, c->total, sizeof n, 1))) return rc;
     n = std::min(n, c->cap);
   } else {
     int32_t nw = 0;
-    HIPCHK(c, hipMemcpy(&nw, c->world_cnt + world, sizeof nw, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(&off, c->world_coff + world, sizeof off, hipMemcpyDeviceToHost));
+    const Plane p[] = {{c->world_cnt + world, sizeof nw, &nw}, {c->world_coff + world, sizeof off, &off}};
+    if ((rc = fetch_planes(c, p, 2, 1))) return rc;
     n = nw;
   }
   if (n == 0) return CBZ_OK;
@@ -1813,8 +1899,9 @@ int cbz_get_contacts(cbz_ctx* c, int32_t world, cbz_contact_view* out) {
   const size_t rs = real_size(c);
   const char* base = (const char*)c->c_real;
   const int64_t S = c->cap;
-  if (out->body0) HIPCHK(c, hipMemcpy(out->body0, (int32_t*)c->c_body0 + off, n * sizeof(int32_t), hipMemcpyDeviceToHost));
-  if (out->body1) HIPCHK(c, hipMemcpy(out->body1, (int32_t*)c->c_body1 + off, n * sizeof(int32_t), hipMemcpyDeviceToHost));
+  std::vector<Plane> planes;
+  if (out->body0) planes.push_back(Plane{(int32_t*)c->c_body0 + off, sizeof(int32_t), out->body0});
+  if (out->body1) planes.push_back(Plane{(int32_t*)c->c_body1 + off, sizeof(int32_t), out->body1});
   struct Part {
     double* dst;
     int plane0;
@@ -1822,8 +1909,7 @@ int cbz_get_contacts(cbz_ctx* c, int32_t world, cbz_contact_view* out) {
   } parts[] = {{out->point, 0, 3}, {out->normal, 3, 3}, {out->pen, 6, 1}, {out->c2w, 7, 9},
                {out->rel, 16, 6},  {out->cvel, 22, 3},  {out->ddv, 25, 1}};
   for (const Part& p : parts) {
-    if (!p.dst) continue;
-    if ((rc = download_real(c, base + (size_t)p.plane0 * S * rs, S, off, n, p.k, p.dst))) return rc;
+    if (p.dst) real_planes(c, planes, base + (size_t)p.plane0 * S * rs, S, off, p.k, p.dst);
   }
   // Contact.Friction / Contact.Restitution: per contact with materials on,
   // else the constants every contact carries
@@ -1833,12 +1919,12 @@ int cbz_get_contacts(cbz_ctx* c, int32_t world, cbz_contact_view* out) {
   for (int m = 0; m < 2; ++m) {
     if (!mats[m].dst) continue;
     if (mat) {
-      if ((rc = download_real(c, base + (size_t)mats[m].plane0 * S * rs, S, off, n, 1, mats[m].dst))) return rc;
+      real_planes(c, planes, base + (size_t)mats[m].plane0 * S * rs, S, off, 1, mats[m].dst);
     } else {
       for (int64_t k = 0; k < n; ++k) mats[m].dst[k] = consts[m];
     }
   }
-  return CBZ_OK;
+  return fetch_planes(c, planes.data(), (int)planes.size(), n);
 }
 
 int cbz_set_contacts(cbz_ctx* c, const int64_t* counts, const int32_t* body0, const int32_t* body1,

@@ -1,0 +1,43 @@
+"""Downloads in pieces of the one-megabyte stage: fields and contacts around
+the sizes at which a second piece starts."""
+import numpy as np
+import pytest
+
+from cubez_amd import World, scenes
+from tests.test_gpu_parity import same
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("worlds", [5460, 5461, 5462, 10923])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_fields_come_back_as_they_went(worlds, precision):
+    """8 bodies per world: three planes of reals fill the stage at 43688
+    (FP64: 5461 worlds) and 87376 bodies (FP32: 10922)."""
+    sc = scenes.batched(0, worlds, 8, 8)
+    rng = np.random.default_rng(worlds)
+    with World(sc, precision=precision) as w:
+        for name in ("pos", "quat", "vel", "inv_mass"):
+            x = rng.normal(0, 1, w.get(name).shape).astype(np.float32).astype(np.float64)
+            w.set(name, x)
+            assert same(w.get(name), x), name
+        fl = rng.integers(0, 2, sc.n_bodies).astype(np.uint8)
+        w.set("flags", fl)
+        assert np.array_equal(w.get("flags"), fl)
+        assert np.array_equal(w.get("shape"), sc.fields["shape"])
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_contacts_of_all_worlds_equal_each_world_s(precision):
+    """More contacts than one piece holds (5 KB per 24 contacts with every
+    internal), worlds one by one against all at once."""
+    sc = scenes.batched(6, 300, 8, 120)
+    with World(sc, precision=precision) as w:
+        w.step(sc.dt, 120, 4)
+        w.integrate(sc.dt)
+        assert w.narrowphase() > 12_000
+        w.resolve(sc.dt, 4)
+        every = w.contacts(-1)
+        each = [w.contacts(k) for k in range(sc.n_worlds)]
+        for name, x in every.items():
+            assert same(x, np.concatenate([e[name] for e in each])), name
