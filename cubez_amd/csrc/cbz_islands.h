@@ -16,13 +16,14 @@
 // islands, most of them one cube with its four ground contacts (3-5
 // iterations), the largest of 10-60 contacts (50-300 iterations).  A step of
 // the exact path, before and after (ms):
-//   1000 batched worlds FP64            7.3 -> 1.1
-//   2048 batched worlds FP32            7.2 -> 1.4
-//   1 world of 301 cubes landing FP32   1.2 -> 0.22
-//   1024 bodies, spheres and cubes      1.1 -> 0.29
+//   1000 batched worlds FP64            7.4 -> 1.0
+//   2048 batched worlds FP32            7.4 -> 1.05
+//   1 world of 301 cubes landing FP32   1.3 -> 0.18
+//   1024 bodies, spheres and cubes      0.82 -> 0.18
 //   1024 worlds of towers, standing     1.5 -> 0.56; collapsed into piles of
-//     200-500 contacts, half of the worlds over their budget, 5.3 -> 5.2
-// and of the surrogate over 4096 worlds 4.4 -> 2.8.
+//     200-500 contacts, half of the worlds over their budget, 4.6 -> 4.3
+// and of the surrogate over 4096 worlds 4.5 -> 2.4 (narrowphase and order of
+// the worlds included).
 //
 // The work of an island: a power-of-two group of lanes, one contact per
 // lane, all of a contact's data in its lane's registers; several groups share
