@@ -395,6 +395,64 @@ __device__ __forceinline__ void pair_of(const PairSpace& ps, int w, int q, int& 
   two = ps.list_two[p];
 }
 
+// A list that a block collects in LDS and appends to a global one at its end
+// with a single atomic: the atomics of a grid on one counter come one after
+// another.  What does not
+// fit in LDS is appended at once.  Entries past the capacity are counted and
+// dropped.
+template <int N>
+struct BlockList {
+  uint32_t item[N];
+  int n, base;
+
+  __device__ __forceinline__ void clear() {
+    if (threadIdx.x == 0) n = 0;
+    __syncthreads();
+  }
+  __device__ __forceinline__ void put(uint32_t v, uint32_t* list, int32_t* counter, int64_t cap) {
+    const int at = atomicAdd(&n, 1);
+    if (at < N) {
+      item[at] = v;
+    } else {
+      const int64_t g = atomicAdd(counter, 1);
+      if (g < cap) list[g] = v;
+    }
+  }
+  // One entry per set bit of every lane of a wave (first + k * step for bit k),
+  // reserved together; all lanes call it.
+  __device__ __forceinline__ void put_bits(uint32_t bits, uint32_t first, uint32_t step, uint32_t* list,
+                                           int32_t* counter, int64_t cap) {
+    const int lane = threadIdx.x & 63;
+    const int mine = __popc(bits), incl = wave_incl_scan_i32(mine), total = __shfl(incl, 63, 64);
+    if (total == 0) return;
+    int at = 0;
+    if (lane == 63) at = atomicAdd(&n, total);
+    at = __shfl(at, 63, 64);
+    const int fit = min(max(N - at, 0), total);  // the first of them go to LDS
+    int64_t g = 0;
+    if (fit < total) {
+      int b = 0;
+      if (lane == 63) b = atomicAdd(counter, total - fit);
+      g = __shfl(b, 63, 64);
+    }
+    for (int k = incl - mine; bits; bits &= bits - 1u, ++k) {
+      const uint32_t v = first + uint32_t(__ffs(bits) - 1) * step;
+      if (k < fit)
+        item[at + k] = v;
+      else if (g + (k - fit) < cap)
+        list[g + (k - fit)] = v;
+    }
+  }
+  __device__ __forceinline__ void flush(uint32_t* list, int32_t* counter, int64_t cap) {
+    __syncthreads();
+    const int m = min(n, N);
+    if (threadIdx.x == 0 && m > 0) base = atomicAdd(counter, m);
+    __syncthreads();
+    for (int k = threadIdx.x; k < m; k += blockDim.x)
+      if (base + int64_t(k) < cap) list[base + int64_t(k)] = item[k];
+  }
+};
+
 // Orders a wave's LDS writes before its later reads, and the other way.
 __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -405,30 +463,9 @@ __device__ __forceinline__ void wave_lds_fence() {
 // ---------------------------------------------------------------------------
 // all-pairs space
 // ---------------------------------------------------------------------------
-// Block-wide append to a global list: every thread of the block calls it
-// with its entry count; returns the list index of the thread's first entry.
-// One atomic per block (a single shared counter hit by every wave of the
-// grid would serialise in the L2).
-__device__ __forceinline__ int64_t block_reserve(int mine, int32_t* counter, int* s_wtot, int* s_base) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const int incl = wave_incl_scan_i32(mine);
-  if (lane == 63) s_wtot[wv] = incl;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int tot = 0;
-    for (int u = 0; u < nw; ++u) tot += s_wtot[u];
-    *s_base = tot > 0 ? atomicAdd(counter, tot) : 0;
-  }
-  __syncthreads();
-  int64_t base = *s_base;
-  for (int u = 0; u < wv; ++u) base += s_wtot[u];
-  __syncthreads();  // s_wtot / s_base are reused by the next call
-  return base + incl - mine;
-}
-
-// Cull: each wave takes TASKS consecutive tasks (world w, column tile c,
-// rows r0 .. r0+15).  Lane l owns column 64c + l for the whole task: a plane,
-// or body j whose centre, bounding radius and shape stay in registers; the 16
+// Cull: each wave takes `per` consecutive tasks (world w, column tile c, rows
+// r0 .. r0+15).  Lane l owns column 64c + l for the whole task: a plane, or
+// body j whose centre, bounding radius and shape stay in registers; the 16
 // row bodies are put in LDS once and read as broadcasts.  Each tile is
 // cleared here; the body pairs with j > r that pass the conservative bound
 // (see far_apart) go to the candidate list.
@@ -440,10 +477,13 @@ __device__ __forceinline__ int64_t block_reserve(int mine, int32_t* counter, int
 // 1-norms of a and b, so 251 e^2 is below 4e-12 (|a| + |b|)^2.  What they leave (a NaN or an infinity passes) is
 // tested again as far_apart does it, once per pair that is left instead of once
 // per pair: the list is the same.  4096 worlds of 8 to 256 cubes take
-// 99 us (183 with every ordered pair tested in FP64, rows shuffled from lane to
+// 97 us (183 with every ordered pair tested in FP64, rows shuffled from lane to
 // lane), bound by the tests' instructions and the clearing of 1.4 million tiles.
-constexpr int kCullSmall = 8192;  // tasks up to which a wave takes one: every task has its wave
-                                  // on the chip, and a launch is one task long (one world of 64 cubes: 22 to 5 us)
+// Tasks per wave: one while every task's wave fits the chip at once (a launch is
+// then one task long: 22 to 5 us for one world of 64 cubes), up to 16 beyond, so
+// that there are few blocks and with them few reservations.
+constexpr int kCullWaves = 8192, kCullPer = 16;
+constexpr int kCullList = 4096;  // every pair of four tasks
 
 struct CullRow {
   float x, y, z, r;    // relative to the first row's body
@@ -452,42 +492,30 @@ struct CullRow {
   int shape;
 };
 
-template <typename R, int TASKS>
-__global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
+template <typename R>
+__global__ void __launch_bounds__(256) k_np_cull(NP<R> a, int per) {
   __shared__ CullRow s_row[4][kRowBlock];
-  __shared__ int s_wtot[4];
-  __shared__ int s_base;
+  __shared__ BlockList<kCullList> s_list;
+  s_list.clear();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int task0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + wv) * TASKS);
+  const int task0 = __builtin_amdgcn_readfirstlane((blockIdx.x * 4 + wv) * per);
   CullRow* row = s_row[wv];
-  // bit k of cm[q]: row r0(q) + k of the wave's task q is a candidate for this lane
-  uint32_t cm[TASKS];
-  int t0[TASKS], r0[TASKS], nch[TASKS], cc[TASKS];
-#pragma unroll
-  for (int q = 0; q < TASKS; ++q) {
-    cm[q] = 0;
-    t0[q] = 0;
-    r0[q] = 0;
-    nch[q] = 1;
-    cc[q] = 0;
-    const int task = task0 + q;
-    if (task >= a.ps.n_tasks) continue;  // the wave still joins the block's reservation
+  for (int task = task0; task < min(task0 + per, a.ps.n_tasks); ++task) {
     const int w = a.ps.task_world[task];
     const int b0 = a.ps.body_off[w], n = a.ps.body_off[w + 1] - b0;
     const int np = a.ps.plane_off[w + 1] - a.ps.plane_off[w];
-    nch[q] = (np + n + 63) >> 6;
+    const int nch = (np + n + 63) >> 6;
     const int k = task - a.ps.world_task0[w];
-    const int c = k % nch[q];
-    cc[q] = c;
-    r0[q] = (k / nch[q]) * kRowBlock;
-    t0[q] = a.ps.world_tile0[w];
-    const int rows = min(n - r0[q], kRowBlock);
+    const int c = k % nch;
+    const int r0 = (k / nch) * kRowBlock;
+    const int t0 = a.ps.world_tile0[w];
+    const int rows = min(n - r0, kRowBlock);
     if (lane < rows) {
-      const int t = t0[q] + (r0[q] + lane) * nch[q] + c;
+      const int t = t0 + (r0 + lane) * nch + c;
       a.tile_cnt[t] = 0;
       a.tile_mask[t] = 0ull;
     }
-    if (64 * c + 63 - np <= r0[q]) continue;  // no column with j > r
+    if (64 * c + 63 - np <= r0) continue;  // no column with j > r
     const int j = 64 * c + lane - np;
     const bool is_body = j >= 0 && j < n;
     const int64_t S = a.b.stride;
@@ -504,7 +532,7 @@ __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
     double ti[3] = {0, 0, 0}, ri = 0;
     int si = 0;
     if (lane < rows) {  // lane k holds row r0 + k
-      const int g = b0 + r0[q] + lane;
+      const int g = b0 + r0 + lane;
       ti[0] = double(a.b.ctransform[9 * S + g]);
       ti[1] = double(a.b.ctransform[10 * S + g]);
       ti[2] = double(a.b.ctransform[11 * S + g]);
@@ -540,7 +568,7 @@ __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
       if (!(d2 > lim + 1e-10f * (nn * nn))) m |= 1u << k2;
     }
     // rows below the column's body only
-    const int up = min(max(j - r0[q], 0), rows);
+    const int up = min(max(j - r0, 0), rows);
     m = is_body ? m & ((1u << up) - 1u) : 0u;
     uint32_t keep = 0;
     for (; m; m &= m - 1u) {
@@ -553,19 +581,10 @@ __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
       const double kf = (v.shape == SHAPE_CUBE && cj) ? 3.003 : 1.001;
       if (spheres || !(d2 > kf * rr * rr)) keep |= 1u << k2;
     }
-    cm[q] = keep;
+    s_list.put_bits(keep, uint32_t(t0 + r0 * nch + c) * 64u + uint32_t(lane), uint32_t(nch) * 64u, a.cand, a.n_pairs,
+                    a.cand_cap);
   }
-  // one reservation per block for all of its waves' tasks
-  int npair = 0;
-#pragma unroll
-  for (int q = 0; q < TASKS; ++q) npair += __popc(cm[q]);
-  int64_t pos = block_reserve(npair, a.n_pairs, s_wtot, &s_base);
-#pragma unroll
-  for (int q = 0; q < TASKS; ++q)
-    for (uint32_t m = cm[q]; m; m &= m - 1u, ++pos) {
-      const int r = r0[q] + __ffs(m) - 1;
-      if (pos < a.cand_cap) a.cand[pos] = uint32_t(t0[q] + r * nch[q] + cc[q]) * 64u + uint32_t(lane);
-    }
+  s_list.flush(a.cand, a.n_pairs, a.cand_cap);
 }
 
 // Eval: the first workgroups take a body per thread, against its world's
@@ -575,13 +594,13 @@ __global__ void __launch_bounds__(256) k_np_cull(NP<R> a) {
 // many candidates (in both orders, the planes' pairs among them) for the list
 // raise the overflow flags (the step reports a capacity error).  The planes
 // apart from the pairs: a wave that holds both runs both tests.
-// 4096 worlds of 8 to 256 cubes take 110 us (166 with both orders tested and the
-// planes among the pairs), bound by the gathers of two bodies per thread and the
+// 4096 worlds of 8 to 256 cubes take 88 us (166 with both orders tested and the
+// planes among the pairs, 110 with a reservation per 256 bodies or pairs), bound by the gathers of two bodies per thread and the
 // longest axis search of each wave.
+constexpr int kEvalList = 2048;
 template <typename R>
 __global__ void __launch_bounds__(256) k_np_eval(NP<R> a, int plane_blocks) {
-  __shared__ int s_wtot[4];
-  __shared__ int s_base;
+  __shared__ BlockList<kEvalList> s_list;
   const int64_t np2 = a.n_pairs[0], nc = 2 * np2 + a.plane_pairs;
   if (blockIdx.x == 0 && threadIdx.x == 0) a.n_cand[0] = int32_t(min(nc, int64_t(INT32_MAX)));
   if (nc > a.cand_cap) {
@@ -595,55 +614,47 @@ __global__ void __launch_bounds__(256) k_np_eval(NP<R> a, int plane_blocks) {
     atomicAdd(&a.tile_cnt[t], cnt);
     atomicOr((unsigned long long*)&a.tile_mask[t], 1ull << l);
   };
+  const int64_t hcap = min(a.c.cap, int64_t(INT32_MAX));
+  s_list.clear();
   if (int(blockIdx.x) < plane_blocks) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    int r = 0, p0 = 0, np = 0, nch = 0, t0 = 0;
-    if (i < a.b.n) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < a.b.n; i += plane_blocks * 256) {
       const int w = a.body_world[i];
       const int b0 = a.ps.body_off[w], n = a.ps.body_off[w + 1] - b0;
-      r = i - b0;
-      p0 = a.ps.plane_off[w], np = a.ps.plane_off[w + 1] - p0;
-      nch = (np + n + 63) >> 6;
-      t0 = a.ps.world_tile0[w];
+      const int p0 = a.ps.plane_off[w], np = a.ps.plane_off[w + 1] - p0;
+      const int nch = (np + n + 63) >> 6, t0 = a.ps.world_tile0[w];
+      for (int k = 0; k < np; ++k) {
+        const int cnt = pair_eval<R, false>(a, i, -(p0 + k) - 1, 0);
+        if (cnt <= 0) continue;
+        const int t = t0 + (i - b0) * nch + (k >> 6), l = k & 63;
+        hit(t, l, cnt);
+        s_list.put(uint32_t(t) * 64u + uint32_t(l), a.hits, a.n_hits, hcap);
+      }
     }
-    for (int k = 0; k < a.max_planes; ++k) {
-      const int t = t0 + r * nch + (k >> 6), l = k & 63;
-      const int cnt = k < np ? pair_eval<R, false>(a, i, -(p0 + k) - 1, 0) : 0;
-      if (cnt > 0) hit(t, l, cnt);
-      const int64_t idx = block_reserve(cnt > 0 ? 1 : 0, a.n_hits, s_wtot, &s_base);
-      if (cnt > 0 && idx < a.c.cap) a.hits[idx] = uint32_t(t) * 64u + uint32_t(l);
-    }
+    s_list.flush(a.hits, a.n_hits, hcap);
     return;
   }
   const int64_t stride = int64_t(gridDim.x - plane_blocks) * blockDim.x;
   for (int64_t e0 = int64_t(blockIdx.x - plane_blocks) * blockDim.x; e0 < np2; e0 += stride) {
     const int64_t e = e0 + threadIdx.x;
-    int cnt = 0;
-    uint32_t code = 0, back = 0;
-    if (e < np2) {
-      code = a.cand[e];
-      const int t = int(code >> 6), l = int(code & 63u);
-      const int w = a.ps.tile_world[t];
-      const int b0 = a.ps.body_off[w], n = a.ps.body_off[w + 1] - b0;
-      const int np = a.ps.plane_off[w + 1] - a.ps.plane_off[w];
-      const int nch = (np + n + 63) >> 6, t0 = a.ps.world_tile0[w];
-      const int k = t - t0;
-      const int r = k / nch, c = k - r * nch;
-      const int j = 64 * c + l - np;
-      cnt = pair_eval<R, false>(a, b0 + r, b0 + j, 0);  // one contact or none
-      if (cnt > 0) {
-        const int tb = t0 + j * nch + ((np + r) >> 6), lb = (np + r) & 63;
-        back = uint32_t(tb) * 64u + uint32_t(lb);
-        hit(t, l, cnt);
-        hit(tb, lb, cnt);
-      }
-    }
-    const int64_t idx = block_reserve(cnt > 0 ? 2 : 0, a.n_hits, s_wtot, &s_base);
-    if (cnt > 0) {
-      if (idx < a.c.cap) a.hits[idx] = code;
-      if (idx + 1 < a.c.cap) a.hits[idx + 1] = back;
-    }
+    if (e >= np2) continue;
+    const uint32_t code = a.cand[e];
+    const int t = int(code >> 6), l = int(code & 63u);
+    const int w = a.ps.tile_world[t];
+    const int b0 = a.ps.body_off[w], n = a.ps.body_off[w + 1] - b0;
+    const int np = a.ps.plane_off[w + 1] - a.ps.plane_off[w];
+    const int nch = (np + n + 63) >> 6, t0 = a.ps.world_tile0[w];
+    const int k = t - t0;
+    const int r = k / nch, c = k - r * nch;
+    const int j = 64 * c + l - np;
+    const int cnt = pair_eval<R, false>(a, b0 + r, b0 + j, 0);  // one contact or none
+    if (cnt <= 0) continue;
+    const int tb = t0 + j * nch + ((np + r) >> 6), lb = (np + r) & 63;
+    hit(t, l, cnt);
+    hit(tb, lb, cnt);
+    s_list.put(code, a.hits, a.n_hits, hcap);
+    s_list.put(uint32_t(tb) * 64u + uint32_t(lb), a.hits, a.n_hits, hcap);
   }
+  s_list.flush(a.hits, a.n_hits, hcap);
 }
 
 // Emit: one thread per hit pair.  Its first contact goes to world offset +
@@ -874,13 +885,14 @@ hipError_t launch_narrowphase(const NarrowLaunch<R>& L, hipStream_t st, hipEvent
   if (list) {
     if (nb > 0) k_np_count<R><<<nb, 256, 0, st>>>(a);
   } else {
-    if (a.ps.n_tasks > kCullSmall) {
-      k_np_cull<R, 4><<<(a.ps.n_tasks + 15) / 16, 256, 0, st>>>(a);
-    } else if (a.ps.n_tasks > 0) {
-      k_np_cull<R, 1><<<(a.ps.n_tasks + 3) / 4, 256, 0, st>>>(a);
+    if (a.ps.n_tasks > 0) {
+      const int per = std::min(std::max(a.ps.n_tasks / kCullWaves, 1), kCullPer);
+      k_np_cull<R><<<(a.ps.n_tasks + 4 * per - 1) / (4 * per), 256, 0, st>>>(a, per);
     }
     const int64_t want = std::min<int64_t>(std::max<int64_t>((a.cand_cap + 511) / 512, 1), 8192);
-    const int planes = a.max_planes > 0 ? (a.b.n + 255) / 256 : 0;
+    // the planes' blocks: a body per thread while they are few, four beyond
+    const int bodies = (a.b.n + 255) / 256;
+    const int planes = a.max_planes > 0 ? (bodies > 512 ? (bodies + 3) / 4 : bodies) : 0;
     k_np_eval<R><<<planes + int(want), 256, 0, st>>>(a, planes);
   }
   if (ev) (void)hipEventRecord(ev[1], st);
