@@ -397,9 +397,8 @@ __device__ __forceinline__ void pair_of(const PairSpace& ps, int w, int q, int& 
 
 // A list that a block collects in LDS and appends to a global one at its end
 // with a single atomic: the atomics of a grid on one counter come one after
-// another.  What does not
-// fit in LDS is appended at once.  Entries past the capacity are counted and
-// dropped.
+// another.  What does not fit in LDS is appended at once.  Entries past the
+// capacity are counted and dropped.
 template <int N>
 struct BlockList {
   uint32_t item[N];

@@ -67,8 +67,8 @@ def test_cull_at_its_bound_and_non_finite():
 
 
 def test_cull_of_small_worlds_and_of_many_tasks():
-    """600 worlds of 1 to 33 bodies (one task per wave), and 480 of 90 to 140:
-    more than the 8192 tasks from which a wave takes four."""
+    """600 worlds of 1 to 33 bodies, and 480 of 90 to 140: more tasks than waves
+    that fit the chip at once."""
     sc = scenes.batched(11, 600, 1, 33)
     pos = sc.fields["pos"].copy()
     pos[:, 1] = 1.0 + (pos[:, 1] % 5.0)
