@@ -838,7 +838,8 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
     }
     wave_fence();
     const uint32_t kid = xi[0];
-    const int kl[2] = {id_lo(kid), id_hi(kid)}, jo[2] = {jb[0] >= 0 ? jb[0] : 0, jb[1]};
+    // a lane without a contact has no bodies: it reads the first one's flags
+    const int kl[2] = {id_lo(kid), id_hi(kid)}, jo[2] = {has ? jb[0] : 0, jb[1]};
     const IslAwake f = isl_awake_of(W, jo);
     V3<R> cn = cv;
     if (isl_touch_velocity(x, jb, kl, m9, rel, cn) && live) {
