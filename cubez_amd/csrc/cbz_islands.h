@@ -1269,11 +1269,13 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
   }
   if constexpr (!VEL) __syncthreads();
   while (!P.only) {
-    // every lane adds one (one LDS operation for the wave); under a branch on
-    // the lane, the compiler makes the other lanes a loop of their own, which
-    // never sees the first lane's value
-    const int q64 = atomicAdd(&W.f->next, 1);
-    int q = __builtin_amdgcn_readfirstlane(q64) >> 6;
+    // One lane takes the wave's ticket.  Its index is opaque: with a branch that
+    // is the same in every turn, the compiler makes the other lanes a loop of
+    // their own, which never sees the first lane's value.
+    int q = 0;
+    if ((opaque_lane(W.t) & 63) == 0) q = atomicAdd(&W.f->next, 1);
+    __builtin_amdgcn_wave_barrier();
+    q = __builtin_amdgcn_readfirstlane(q);
     int at = nbig, k = kIslBigClasses, m = 0, per = 1, lg = 6;
     for (; k < kIslClasses; ++k) {
       m = cls[k];

@@ -34,3 +34,27 @@ def test_no_access_past_the_workgroups_lds(lib, precision):
     o, cs = _at_contacts(sc, 200)
     rc, _, iters, left = emu.resolve(lib, o, cs, sc.dt, precision=precision)
     assert (rc, left) == (0, 0) and min(iters) > 0
+
+
+def _check(lib, o, cs, dt, mult=4, fixed=0, flags=0, **kw):
+    """The emulated resolve against the oracle's, which the world then takes."""
+    rc, got, iters, left = emu.resolve(lib, o, cs, dt, mult, fixed, **kw)
+    assert rc == 0, rc
+    before = dict(o.counters())
+    out = o.resolve(cs, dt, fixed or mult * len(cs), flags)
+    after = o.counters()
+    assert left == 0
+    assert iters == (after["pos_iters"] - before["pos_iters"], after["vel_iters"] - before["vel_iters"])
+    for k in STATE:
+        assert np.array_equal(got[k].T.reshape(-1), o.a[k], equal_nan=True), k
+    for k in INTERNALS:
+        assert np.array_equal(got[k].T.reshape(-1), np.asarray(out[k]).reshape(-1), equal_nan=True), k
+
+
+@pytest.mark.parametrize("across", [False, True])
+def test_batches_are_dealt_out_once(lib, across):
+    """Dozens of small islands of every class: each is run by exactly one wave,
+    also when the waves draw their tickets lane by lane in turn."""
+    sc = _pile(200, 1.0)
+    o, cs = _at_contacts(sc, 200)
+    _check(lib, o, cs, sc.dt, across=across)
