@@ -711,6 +711,7 @@ int ensure_islands(cbz_ctx* c) {
   for (int32_t w = 0; w < c->nw; ++w) {
     const int32_t n = c->body_off[w + 1] - c->body_off[w];
     if (n <= kIslBodies) most = std::max(most, n);
+    if (n > kLeftBodies) u.large += 1;
   }
   u.nb = (most + 15) & ~15;
   // log pool for the worlds that exceed their iteration budget: a world of

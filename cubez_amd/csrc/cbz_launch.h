@@ -60,12 +60,16 @@ struct NarrowLaunch {
 
 // The most bodies of a world the island kernel's LDS tables hold.
 constexpr int kIslBodies = 2048;
+// Worlds of more bodies than this may hold an island that is left to the serial
+// kernel.
+constexpr int kLeftBodies = 256;
 // Words per world of IslandBuffers::cls.
 constexpr int kIslWords = 16;
 
 // The island kernel's device buffers (see RS in cbz_resolve.h).
 struct IslandBuffers {
   int32_t nb = 0;                   // bodies per LDS table: the largest world of at most kIslBodies
+  int32_t large = 0;                // worlds of more than kLeftBodies bodies
   int32_t* off = nullptr;           // [n_bodies]
   int32_t* cnt = nullptr;           // [n_bodies]
   int32_t* its = nullptr;           // [n_bodies]

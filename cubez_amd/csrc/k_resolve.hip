@@ -1,6 +1,8 @@
 // k_resolve.hip — launch dispatch of the resolver (K3): picks the
 // compile-time kind of the kernel for the requested phases and materials.
 // The kernels are in cbz_islands.h and cbz_resolve.h, instantiated by k_resolve_<precision>_<kind>.hip.
+#include <algorithm>
+
 #include "cbz_islands.h"
 
 namespace cbz {
@@ -66,7 +68,8 @@ constexpr int kOrderWorlds = 256;
 // The island kernel, then the kernel for the worlds it leaves (none, as a
 // rule: its workgroups end at once).
 template <typename R, int KIND>
-hipError_t launch_all(const RS<R>& plain, int32_t* cost, hipStream_t st) {
+hipError_t launch_all(const RS<R>& plain, const ResolveLaunch<R>& L, hipStream_t st) {
+  int32_t* cost = L.cost;
   RS<R> a = plain;
   if (a.n_worlds > kOrderWorlds && cost && (a.mode & (RM_POS | RM_VEL | RM_POLISH)) == (RM_POS | RM_VEL)) {
     k_order<<<1, 1024, 0, st>>>(a.world_time + 2, a.body_off, a.n_worlds, cost, cost + a.n_worlds);
@@ -74,7 +77,7 @@ hipError_t launch_all(const RS<R>& plain, int32_t* cost, hipStream_t st) {
   }
   const hipError_t e = launch_islands_kind<R, KIND>(a, st);
   if (e != hipSuccess) return e;
-  launch_left_kind<R, KIND>(a, st);
+  launch_left_kind<R, KIND>(a, std::min(a.n_worlds, std::max(kLeftGrid, L.isl.large)), st);
   return hipGetLastError();
 }
 
@@ -138,11 +141,11 @@ hipError_t launch_resolve(const ResolveLaunch<R>& L, hipStream_t st) {
     kernel<<<a.n_worlds, kIslThreads, lds, st>>>(a);
     return hipGetLastError();
   }
-  if (a.c.fric) return launch_all<R, KIND_MAT>(a, L.cost, st);
+  if (a.c.fric) return launch_all<R, KIND_MAT>(a, L, st);
   if (a.mode & RM_POLISH)
-    return (a.mode & RM_POS) ? launch_all<R, KIND_PPOLISH>(a, L.cost, st) : launch_all<R, KIND_POLISH>(a, L.cost, st);
-  if (a.mode & RM_LABEL) return launch_all<R, KIND_LABEL>(a, L.cost, st);
-  return launch_all<R, KIND_PLAIN>(a, L.cost, st);
+    return (a.mode & RM_POS) ? launch_all<R, KIND_PPOLISH>(a, L, st) : launch_all<R, KIND_POLISH>(a, L, st);
+  if (a.mode & RM_LABEL) return launch_all<R, KIND_LABEL>(a, L, st);
+  return launch_all<R, KIND_PLAIN>(a, L, st);
 }
 
 // Worlds (workgroups) of the plain island kernel resident per CU, from its
