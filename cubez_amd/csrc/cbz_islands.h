@@ -45,9 +45,13 @@
 // between two of those the island's next key is above every other island's,
 // so the serial loop stays in it.
 //
+// A world whose logs find no room is run again as one island of all its
+// contacts, which makes its selections in the serial order up to the budget.
+//
 // Worlds this does not take (more bodies than the LDS tables hold, an island
-// of more than 2048 contacts, contacts that name bodies of another world, a
-// log that finds no room) are left to the serial kernel of cbz_resolve.h.
+// of more than 2048 contacts, contacts that name bodies of another world, more
+// than 2048 contacts and no room for the logs) are left to the serial kernel of
+// cbz_resolve.h.
 #pragma once
 #include "cbz_resolve.h"
 
@@ -340,6 +344,7 @@ struct IslPass {
   bool pause;      // ISL_FREE: the last island stops where the world's budget is spent
   int resume;      // ISL_LOG, ISL_LIMIT: the island that goes on from its pause (-1: none)
   bool only;       // ... alone
+  bool one;        // ISL_FREE: the world's contacts as one island, the serial loop itself
 };
 
 // Ends of a batch: the islands' iteration counts, the world's sum.
@@ -908,8 +913,8 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
   const Contacts<R>& c = a.c;
   const int64_t CS = c.cap, S = b.stride;
   const int t = W.t, wave = t >> 6;
-  const int cnt = a.isl_cnt[W.b0w + k];
-  const int32_t* idx = a.isl_idx + W.base + a.isl_off[W.b0w + k];
+  const int cnt = P.one ? W.C : a.isl_cnt[W.b0w + k];
+  const int32_t* idx = a.isl_idx + W.base + (P.one ? 0 : a.isl_off[W.b0w + k]);
   const V3<R> zero{R(0), R(0), R(0)};
   constexpr bool REG = SL == 1;
   constexpr bool MOVE = !VEL && SL <= 2;  // what a position change keeps is in registers
@@ -942,7 +947,7 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
     }
     if (T * s + t >= cnt) continue;
     asm volatile("" ::: "memory");
-    js[s] = uint32_t(idx[T * s + t]);
+    js[s] = uint32_t(P.one ? T * s + t : idx[T * s + t]);
     const int64_t g = W.base + int(js[s]);
     const int c0 = c.body0[g], c1 = c.body1[g];
     ids[s] = isl_ids(c0, c1, W.b0w);
@@ -1257,7 +1262,13 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
   if (W.t < kIslWords) W.f->cls[W.t] = a.isl_cls[kIslWords * int64_t(W.w) + W.t];
   __syncthreads();
   const int32_t* cls = W.f->cls;
-  const int n0 = cls[0], n1 = cls[1], nbig = n0 + n1 + cls[2];
+  int n0 = cls[0], n1 = cls[1], nbig = n0 + n1 + cls[2];
+  if (P.one) {
+    const int k = isl_class(W.C);
+    n0 = k == 0 ? 1 : 0;
+    n1 = k == 1 ? 1 : 0;
+    nbig = 1;
+  }
   if (W.iw && (!VEL || n0 + n1 > 0)) {
     for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
       R iw[9];
@@ -1268,7 +1279,7 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
     }
   }
   if constexpr (!VEL) __syncthreads();
-  while (!P.only) {
+  while (!P.only && !P.one) {
     // One lane takes the wave's ticket.  Its index is opaque: with a branch that
     // is the same in every turn, the compiler makes the other lanes a loop of
     // their own, which never sees the first lane's value.
@@ -1726,6 +1737,17 @@ __device__ __forceinline__ void isl_contacts_back(const RS<R>& a, const IslWorld
   __syncthreads();
 }
 
+// `need` entries of the log pool: where they start, or -1 (and they stay free
+// for worlds that need less).
+template <typename R>
+__device__ __forceinline__ int64_t isl_reserve(const RS<R>& a, int64_t need) {
+  unsigned long long* head = (unsigned long long*)a.log_head;
+  const int64_t at = int64_t(atomicAdd(head, (unsigned long long)need));
+  if (at + need <= a.log_cap) return at;
+  atomicAdd(head, (unsigned long long)-need);
+  return -1;
+}
+
 // Room in the log pool for the world's logs, an island's being at most the
 // iterations it ran (a paused one's: what it may still run); false when there
 // is none.
@@ -1743,9 +1765,9 @@ __device__ __forceinline__ bool isl_log_room(const RS<R>& a, const IslWorld<R>& 
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) need += __shfl_xor(need, o, 64);
     int64_t at = 0;
-    if (W.t == 0) at = int64_t(atomicAdd((unsigned long long*)a.log_head, (unsigned long long)need));
+    if (W.t == 0) at = isl_reserve(a, need);
     at = __shfl(at, 0, 64);
-    const bool ok = at + need <= a.log_cap;
+    const bool ok = at >= 0;
     if (W.t == 0) W.f->ok = ok ? 1 : 0;
     for (int k0 = 0; ok && k0 < nisl; k0 += 64) {
       const int k = k0 + W.t;
@@ -1762,15 +1784,16 @@ __device__ __forceinline__ bool isl_log_room(const RS<R>& a, const IslWorld<R>& 
 
 // One phase of the world: the tables are loaded, the contacts are as
 // prepared; `polish` first tries the surrogate's polish (its mask byte is
-// set when that is rejected).  Returns false when the world exceeds its
-// budget and the log pool has no room: the phase is undone, for the other
-// kernels to do.
+// set when that is rejected).  A world that exceeds its budget and finds no
+// room in the log pool starts again as one island of all its contacts.
+// Returns false when that has more than kIslMaxContacts of them: the phase is
+// undone, for the serial kernel to do.
 template <typename R, int KIND, bool VEL>
 __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, int64_t budget, bool polish,
                                           int64_t& used) {
   constexpr bool POLISH = VEL ? KIND == KIND_POLISH : KIND == KIND_PPOLISH;
   const R plain_eps = VEL ? R(kVelocityEpsilon) : R(kPositionEpsilon);
-  IslPass P{ISL_FREE, false, budget, true, -1, false};
+  IslPass P{ISL_FREE, false, budget, true, -1, false, false};
   R eps = plain_eps, sep_floor = R(0);
   double ke = 0.0, mass = 0.0;
   bool rejected = false;
@@ -1820,7 +1843,7 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
         isl_load<R, VEL>(a, W);
         if (W.t == 0) a.world_mask[W.w] = 1;
         polish = rejected = false;
-        P = IslPass{ISL_FREE, true, budget, true, -1, false};
+        P = IslPass{ISL_FREE, true, budget, true, -1, false, false};
         eps = plain_eps;
         if (budget <= 0) {
           used = 0;
@@ -1833,7 +1856,7 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
     if (P.pass == ISL_FREE) {
       const int64_t total = int64_t(W.f->total);
       used = total;
-      if (total <= budget && !W.f->over) return true;
+      if (P.one || (total <= budget && !W.f->over)) return true;
       // over the budget: log the selections, merge them, and run each island
       // to its share
       used = budget;
@@ -1849,7 +1872,10 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
       if (!ok) {
         if constexpr (!VEL) isl_sleepers(a, W, true);
         isl_contacts_back<R, VEL>(a, W);
-        return false;
+        if (W.C > kIslMaxContacts) return false;
+        P = IslPass{ISL_FREE, true, budget, false, -1, false, true};
+        isl_load<R, VEL>(a, W);
+        continue;
       }
       P.pass = ISL_LOG;
       P.pause = false;

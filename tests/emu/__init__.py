@@ -28,8 +28,9 @@ class _World(ctypes.Structure):
                 + [(k, ctypes.c_void_p) for k in (*BODY, *CONTACT, "labels", "iters", "left")])
 
 
-def build(out_dir):
-    """The headers without their launches and inline assembly, and the library."""
+def build(out_dir, optimise="-O1"):
+    """The headers without their launches and inline assembly, and the library
+    (with -O0, every access of the source is made)."""
     for name in os.listdir(CSRC):
         if not name.endswith(".h"):
             continue
@@ -41,15 +42,14 @@ def build(out_dir):
         with open(os.path.join(out_dir, name), "w") as f:
             f.write(s)
     lib = os.path.join(out_dir, "libislands.so")
-    # not optimised: every access of the source is made
-    subprocess.run([CLANG, "-O0", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-w", "-I", HERE,
+    subprocess.run([CLANG, optimise, "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-w", "-I", HERE,
                     "-I", out_dir, "-I", os.path.join(ROOT, "include"), os.path.join(HERE, "islands.cpp"), "-o", lib],
                    check=True)
     return ctypes.CDLL(lib)
 
 
 def _planes(x, k, real):
-    return np.ascontiguousarray(np.asarray(x, real).reshape(-1, k).T)
+    return np.array(np.asarray(x).reshape(-1, k).T, real, order="C")
 
 
 def resolve(lib, o, contacts, dt, mult=4, fixed=0, precision="f64", kind=PLAIN, log_cap=200000, across=False):

@@ -3,6 +3,7 @@
 // barriers as the points where the fibers meet.
 #pragma once
 #include <math.h>
+#include <setjmp.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -41,10 +42,13 @@ struct double2 {
 };
 
 namespace emu {
+// entered once through its context, then switched by jumps, which save no
+// signal mask
 struct Fiber {
   ucontext_t ctx;
+  jmp_buf at;
   char* stack = nullptr;
-  bool done = false;
+  bool begun = false, done = false;
 };
 // a meeting point: who has arrived, of how many, and how often all had
 struct Meet {
@@ -57,7 +61,7 @@ struct Meet {
 constexpr int kWaves = 16;
 inline std::vector<Fiber> fibers;
 inline int cur;
-inline ucontext_t scheduler;
+inline jmp_buf scheduler;
 inline Meet wave[kWaves], block;
 inline uint64_t lanes[kWaves][2][64];
 
@@ -65,7 +69,8 @@ inline void meet(Meet& m) {
   const long r = m.round;
   ++m.arrived;
   m.close();
-  while (m.round == r) swapcontext(&fibers[cur].ctx, &scheduler);
+  while (m.round == r)
+    if (!_setjmp(fibers[cur].at)) _longjmp(scheduler, 1);
 }
 inline void wave_sync() { meet(wave[cur >> 6]); }
 // every lane's value of one wave operation

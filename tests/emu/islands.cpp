@@ -2,7 +2,6 @@
 // workgroup's LDS ends at an inaccessible page, so an access past its end is an
 // error here whatever lies there on a device; the fibers' order is the caller's.
 #include <hip/hip_runtime.h>
-#include <setjmp.h>
 #include <signal.h>
 #include <sys/mman.h>
 
@@ -27,7 +26,15 @@ void entry() {
     --m->alive;
     m->close();
   }
-  swapcontext(&emu::fibers[me].ctx, &emu::scheduler);
+  _longjmp(emu::scheduler, 1);
+}
+
+// Runs a fiber to its next meeting point.
+void enter(emu::Fiber& f) {
+  if (_setjmp(emu::scheduler)) return;
+  if (f.begun) _longjmp(f.at, 1);
+  f.begun = true;
+  setcontext(&f.ctx);
 }
 
 // fn(arg) by nt threads; across: a lane of every wave in turn, instead of a
@@ -46,7 +53,7 @@ int run_block(void (*fn)(void*), void* arg, int nt, bool across, long max_steps)
     f.ctx.uc_stack.ss_sp = f.stack;
     f.ctx.uc_stack.ss_size = kStack;
     f.ctx.uc_link = nullptr;
-    f.done = false;
+    f.begun = f.done = false;
     makecontext(&f.ctx, entry, 0);
   }
   if (sigsetjmp(g_back, 1)) return ACCESS;
@@ -58,7 +65,7 @@ int run_block(void (*fn)(void*), void* arg, int nt, bool across, long max_steps)
       if (emu::fibers[i].done) continue;
       emu::cur = i;
       threadIdx.x = i;
-      swapcontext(&emu::scheduler, &emu::fibers[i].ctx);
+      enter(emu::fibers[i]);
       left += !emu::fibers[i].done;
     }
     if (left == 0) return OK;

@@ -14,6 +14,11 @@ def lib(tmp_path_factory):
     return emu.build(str(tmp_path_factory.mktemp("emu")))
 
 
+@pytest.fixture(scope="module")
+def lib_o0(tmp_path_factory):
+    return emu.build(str(tmp_path_factory.mktemp("emu_o0")), "-O0")
+
+
 STATE = ("pos", "quat", "vel", "rot", "iit_world", "transform", "motion", "flags")
 INTERNALS = ("pen", "cvel", "ddv", "c2w", "rel")
 
@@ -27,12 +32,12 @@ def _at_contacts(sc, at, world=0):
 
 
 @pytest.mark.parametrize("precision", ["f64", "f32"])
-def test_no_access_past_the_workgroups_lds(lib, precision):
+def test_no_access_past_the_workgroups_lds(lib_o0, precision):
     """Islands that leave lanes of their group without a contact, in every class
     of one contact per lane."""
     sc = _pile(200, 1.0)
     o, cs = _at_contacts(sc, 200)
-    rc, _, iters, left = emu.resolve(lib, o, cs, sc.dt, precision=precision)
+    rc, _, iters, left = emu.resolve(lib_o0, o, cs, sc.dt, precision=precision)
     assert (rc, left) == (0, 0) and min(iters) > 0
 
 
@@ -58,3 +63,38 @@ def test_batches_are_dealt_out_once(lib, across):
     sc = _pile(200, 1.0)
     o, cs = _at_contacts(sc, 200)
     _check(lib, o, cs, sc.dt, across=across)
+
+
+def _bits(got):
+    return {k: got[k] for k in (*STATE, *INTERNALS, "labels")}
+
+
+@pytest.mark.parametrize("n,squeeze,at", [(64, 1.0, 300), (200, 1.0, 240), (200, 0.5, 200)])
+def test_no_room_for_the_logs(lib, n, squeeze, at):
+    """A world over its budget whose logs find no room runs as one island: the
+    oracle's result, without the serial kernel."""
+    sc = _pile(n, squeeze)
+    o, cs = _at_contacts(sc, at)
+    _check(lib, o, cs, sc.dt, mult=1, log_cap=10)
+
+
+@pytest.mark.parametrize("kind", [emu.PLAIN, emu.LABEL, emu.MAT])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+@pytest.mark.parametrize("mult,fixed", [(1, 0), (2, 0), (4, 33)])
+def test_merged_logs_equal_one_island(lib, kind, precision, mult, fixed):
+    """Two ways to stop a world at its budget, the merged logs of its islands and
+    one island of all of its contacts: the same bits in every kind, labels and
+    iteration counts included."""
+    sc = _pile(120, 0.4)
+    o, cs = _at_contacts(sc, 200)
+    rng = np.random.default_rng(3)
+    cs["friction"] = rng.uniform(0.0, 1.0, len(cs))
+    cs["friction"][::7] = 0.0
+    cs["restitution"] = rng.uniform(0.0, 0.5, len(cs))
+    a = emu.resolve(lib, o, cs, sc.dt, mult, fixed, precision, kind)
+    b = emu.resolve(lib, o, cs, sc.dt, mult, fixed, precision, kind, log_cap=0)
+    budget = fixed or mult * len(cs)
+    assert a[0] == b[0] == 0 and a[3] == b[3] == 0 and a[2] == b[2] and budget in a[2]
+    for k, v in _bits(a[1]).items():
+        assert np.array_equal(v, b[1][k], equal_nan=True), k
+    assert kind != emu.LABEL or np.abs(a[1]["labels"]).max() > 0
