@@ -20,33 +20,45 @@
 //   2048 batched worlds FP32            7.4 -> 1.05
 //   1 world of 301 cubes landing FP32   1.3 -> 0.18
 //   1024 bodies, spheres and cubes      0.82 -> 0.18
-//   1024 worlds of towers, standing     1.5 -> 0.56; collapsed into piles of
-//     200-500 contacts, half of the worlds over their budget, 4.6 -> 4.3
+//   1024 worlds of towers, standing     1.7 -> 0.47; collapsed into piles of
+//     200-500 contacts, up to half of the worlds over their budget, 5.2 -> 5.3
 // and of the surrogate over 4096 worlds 4.5 -> 2.4 (narrowphase and order of
 // the worlds included).
 //
 // The work of an island: a power-of-two group of lanes, one contact per
 // lane, all of a contact's data in its lane's registers; several groups share
-// a wave.  (Islands of more than 64 contacts: the whole workgroup.)  An iteration: the group's argmax by DPP, the lane that owns the
-// selected contact computes the correction alone (the wave would spend the
-// same instructions if every lane did) and puts the two bodies' changes
-// into LDS, from where the group's lanes update their own contacts.  The
-// bodies' state is in LDS for the phase.  Islands are handed out by size,
+// a wave.  (Islands of more than 64 contacts: the whole workgroup.)  An
+// iteration: the group's argmax by DPP, the lane that owns the selected contact
+// computes the correction alone (the wave would spend the same instructions if
+// every lane did) and puts the two bodies' changes into LDS, from where the
+// group's lanes update their own contacts.  The bodies' state is in LDS for the
+// phase.  Islands are handed out by size,
 // the largest first, so that the islands that share a wave run for similar
 // times.
 //
 // The budget.  Each phase first runs every island to its end and counts.  If
 // the world's sum exceeds the budget, the serial loop would have stopped in
-// the middle: the world is put back, run again while each island logs its
-// selections, and the logs are merged as the serial loop orders them
-// (always the island whose next selection has the largest key) up to the
-// budget; a third run stops each island there.  The merge needs only the
+// the middle: the islands' selections are logged, the logs merged as the serial
+// loop orders them (always the island whose next selection has the largest key)
+// up to the budget, and each island runs to its share.  The merge needs only the
 // selections at which an island's running minimum falls (or is met again):
 // between two of those the island's next key is above every other island's,
 // so the serial loop stays in it.
 //
-// A world whose logs find no room is run again as one island of all its
-// contacts, which makes its selections in the serial order up to the budget.
+// What a world over its budget waits for is, as a rule, one island that does not
+// settle.  Three runs of that (to count, to log, to its share) take longer than
+// the serial chain did, so in the velocity phase an island that has run for a
+// quarter of the budget logs from there on and keeps two checkpoints: the second
+// run is of the first quarter, the third starts from the last checkpoint before
+// the share.  1000 landing worlds take 0.40 ms a resolve (0.71 with three whole
+// runs, 0.53 as serial chains), 1000 of 8 to 32 bodies 0.51 (0.75, 0.53).
+//
+// A budget that is small for the world is not worth it: a world whose budget is
+// below half (with more than 512 contacts a quarter) of its contacts, or whose
+// budget of at most 96 is exceeded, runs as one island of all its contacts, which
+// makes its selections in the serial order; so does a world whose logs find no
+// room.  20 iterations of 1000 worlds of 350 contacts take 0.34 ms (0.92 in three
+// runs, 0.32 as serial chains).
 //
 // Worlds this does not take (more bodies than the LDS tables hold, an island
 // of more than 2048 contacts, contacts that name bodies of another world, more
@@ -57,17 +69,20 @@
 
 namespace cbz {
 
-constexpr int kIslWaves = kIslThreads / 64;
-constexpr int kIslMaxContacts = 2048;                   // contacts of the largest island taken
-// Size classes by contact count: 513-2048, 257-512 and 65-256 (the whole
-// workgroup, 8, 2 or 1 contacts per thread), then one contact per lane in
-// groups of 64, 32, 16, 8 and 4 lanes.  RS::isl_cls holds kIslWords words
-// per world: the counts, and at kIslTaken whether the islands were taken.
-constexpr int kIslClasses = 8, kIslBigClasses = 3, kIslTaken = 8;
+// Size classes by contact count: above 4 T, 2 T, T and 64 (the whole workgroup
+// of T threads, 8, 8 or 4, 2 or 1 contacts per thread), then one contact per lane
+// in groups of 64, 32, 16, 8 and 4 lanes.  RS::isl_cls holds kIslWords words per
+// world: the counts, and at kIslTaken the workgroup size the islands were made
+// for (0: not taken).
+constexpr int kIslClasses = 9, kIslBigClasses = 4, kIslTaken = 9;
+// contacts of the largest island taken
+template <int T>
+constexpr int isl_max_contacts() { return 8 * T; }
+template <int T>
 __device__ __forceinline__ int isl_class(int c) {
-  return c > 512 ? 0 : c > 256 ? 1 : c > 64 ? 2 : c > 32 ? 3 : c > 16 ? 4 : c > 8 ? 5 : c > 4 ? 6 : 7;
+  return c > 4 * T ? 0 : c > 2 * T ? 1 : c > T ? 2 : c > 64 ? 3 : c > 32 ? 4 : c > 16 ? 5 : c > 8 ? 6 : c > 4 ? 7 : 8;
 }
-__device__ __forceinline__ int isl_class_lg(int k) { return 9 - k; }  // log2 lanes per island of a small class
+__device__ __forceinline__ int isl_class_lg(int k) { return 10 - k; }  // log2 lanes per island of a small class
 
 enum : int { ISL_FREE = 0, ISL_LOG = 1, ISL_LIMIT = 2 };
 
@@ -80,27 +95,29 @@ struct IslBest {
   int32_t j;
   uint32_t id;
 };
-template <typename R>
+template <typename R, int T>
 struct IslFixed {
-  R x[kIslWaves][16][12];         // the two bodies' changes of each group's iteration
-  uint32_t xi[kIslWaves][16][2];  // packed body ids, rederived bits
-  double sum[kIslWaves];
+  static constexpr int kWaves = T / 64;
+  R x[kWaves][16][12];         // the two bodies' changes of each group's iteration
+  uint32_t xi[kWaves][16][2];  // packed body ids, rederived bits
+  double sum[kWaves];
   // each wave's best contact of a big island (two iterations' worth), with
   // what its correction would change: the two bodies' changes 12, their new
   // velocity and rotation 12 (position and orientation 14)
-  IslBest<R> best[2][kIslWaves];
-  R bx[2][kIslWaves][28];
+  IslBest<R> best[2][kWaves];
+  R bx[2][kWaves][28];
   unsigned long long total;       // the phase's iterations
   int32_t cls[kIslWords];         // class counts, then cursors
   int32_t next, over, bad, off, ok;
   int32_t big, bigs, bigoff;      // contacts and number of the big islands, the next one's place
+  int32_t lates;                  // islands that log late
   int32_t paused, at;             // the big island the budget stopped (-1: none), its iterations there
   int32_t runj;                   // and where its running minimum stood: contact, key
   R runkey;
 };
-template <typename R>
+template <typename R, int T>
 constexpr size_t isl_fixed_bytes() {
-  return (sizeof(IslFixed<R>) + 15) & ~size_t(15);
+  return (sizeof(IslFixed<R, T>) + 15) & ~size_t(15);
 }
 
 // Stores of one lane of a wave before loads of others, through LDS (which a
@@ -177,26 +194,26 @@ __device__ __forceinline__ void tab3_store(R* e, const V3<R>& v) {
 }
 
 // One world as the workgroup sees it.
-template <typename R>
+template <typename R, int T>
 struct IslWorld {
   int w, C, b0w, n, NB, t;
   int64_t base;
-  IslFixed<R>* f;
+  IslFixed<R, T>* f;
   R* st;
   R* iw;  // [n][kIslIw] world inverse inertia 9, inverse mass, or null: no table in this launch
   uint8_t* fl;
 };
 
 // Sum / extreme over the workgroup, in a fixed order.
-template <typename R, typename OP>
-__device__ __forceinline__ double isl_reduce(const IslWorld<R>& W, double v, OP op) {
+template <typename R, typename OP, int T>
+__device__ __forceinline__ double isl_reduce(const IslWorld<R, T>& W, double v, OP op) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = op(v, __shfl_xor(v, o, 64));
   if ((W.t & 63) == 0) W.f->sum[W.t >> 6] = v;
   __syncthreads();
   double r = W.f->sum[0];
 #pragma unroll
-  for (int k = 1; k < kIslWaves; ++k) r = op(r, W.f->sum[k]);
+  for (int k = 1; k < (T / 64); ++k) r = op(r, W.f->sum[k]);
   __syncthreads();
   return r;
 }
@@ -208,9 +225,8 @@ __device__ __forceinline__ double isl_reduce(const IslWorld<R>& W, double v, OP 
 // (any order: ties are broken by the contact's index, which travels with
 // the key).  Writes isl_off / isl_cnt [b0w + rank] with ranks ordered by
 // class, isl_idx [base ..], and the class counts with a "taken" mark.
-template <typename R>
-__device__ __forceinline__ void isl_build(const RS<R>& a, const IslWorld<R>& W) {
-  constexpr int T = kIslThreads;
+template <typename R, int T>
+__device__ __forceinline__ void isl_build(const RS<R>& a, const IslWorld<R, T>& W) {
   int32_t* par = (int32_t*)W.st;
   int32_t* cnt = par + W.NB;
   const Contacts<R>& c = a.c;
@@ -264,24 +280,24 @@ __device__ __forceinline__ void isl_build(const RS<R>& a, const IslWorld<R>& W) 
   for (int j = W.t; j < W.C; j += T) atomicAdd(&cnt[par[c.body0[W.base + j] - W.b0w]], 1);
   __syncthreads();
   for (int i = W.t; i < W.n; i += T) {
-    if (cnt[i] > kIslMaxContacts) W.f->bad = 1;
+    if (cnt[i] > isl_max_contacts<T>()) W.f->bad = 1;
     if (cnt[i] > 64) {
       atomicAdd(&W.f->big, cnt[i]);
       atomicAdd(&W.f->bigs, 1);
     }
-    if (cnt[i] > 0) atomicAdd(&W.f->cls[isl_class(cnt[i])], 1);
+    if (cnt[i] > 0) atomicAdd(&W.f->cls[isl_class<T>(cnt[i])], 1);
   }
   __syncthreads();
   // The big islands run one after another on the whole workgroup; together
   // they run as many iterations as one island of all their contacts, whose
   // loop makes their selections in the serial order.  So they are one, where
   // that is not too large: one island per world can be paused at the budget.
-  const bool one = W.f->bigs > 0 && W.f->big <= kIslMaxContacts;
+  const bool one = W.f->bigs > 0 && W.f->big <= isl_max_contacts<T>();
   if (W.t == 0) {
     if (one) {
 #pragma unroll
       for (int k = 0; k < kIslBigClasses; ++k) W.f->cls[k] = 0;
-      W.f->cls[isl_class(W.f->big)] = 1;
+      W.f->cls[isl_class<T>(W.f->big)] = 1;
       W.f->bigoff = 0;
       W.f->off = W.f->big;
       a.isl_off[W.b0w] = 0;
@@ -295,7 +311,7 @@ __device__ __forceinline__ void isl_build(const RS<R>& a, const IslWorld<R>& W) 
       W.f->cls[k] = at;
       at += m;
     }
-    a.isl_cls[kIslWords * int64_t(W.w) + kIslTaken] = W.f->bad ? 0 : 1;
+    a.isl_cls[kIslWords * int64_t(W.w) + kIslTaken] = W.f->bad ? 0 : T;
   }
   __syncthreads();
   if (W.f->bad) return;
@@ -306,7 +322,7 @@ __device__ __forceinline__ void isl_build(const RS<R>& a, const IslWorld<R>& W) 
       cnt[i] = atomicAdd(&W.f->bigoff, m);
       continue;
     }
-    const int k = atomicAdd(&W.f->cls[isl_class(m)], 1);
+    const int k = atomicAdd(&W.f->cls[isl_class<T>(m)], 1);
     const int o = atomicAdd(&W.f->off, m);
     a.isl_off[W.b0w + k] = o;
     a.isl_cnt[W.b0w + k] = m;
@@ -321,11 +337,11 @@ __device__ __forceinline__ void isl_build(const RS<R>& a, const IslWorld<R>& W) 
 
 // prepareContacts (contact.go:225-229), a thread per contact, with every
 // contact's record, the bodies' prepare-time positions and the islands.
-template <typename R, int KIND>
-__device__ __forceinline__ void isl_prepare(const RS<R>& a, const IslWorld<R>& W, bool islands) {
+template <typename R, int KIND, int T>
+__device__ __forceinline__ void isl_prepare(const RS<R>& a, const IslWorld<R, T>& W, bool islands) {
   const int64_t S = a.b.stride;
-  for (int i = W.t; i < W.n; i += kIslThreads) st3(a.pos0, S, W.b0w + i, ld3(a.b.pos, S, W.b0w + i));
-  for (int j = W.t; j < W.C; j += kIslThreads) prepare_contact<R, KIND, true>(a, W.base + j);
+  for (int i = W.t; i < W.n; i += T) st3(a.pos0, S, W.b0w + i, ld3(a.b.pos, S, W.b0w + i));
+  for (int j = W.t; j < W.C; j += T) prepare_contact<R, KIND, true>(a, W.base + j);
   __syncthreads();
   if (islands) isl_build(a, W);
   __syncthreads();
@@ -345,18 +361,69 @@ struct IslPass {
   int resume;      // ISL_LOG, ISL_LIMIT: the island that goes on from its pause (-1: none)
   bool only;       // ... alone
   bool one;        // ISL_FREE: the world's contacts as one island, the serial loop itself
+  // ISL_FREE: iterations after which an island logs (0: never), with checkpoints at
+  // two and three times as many; ISL_LIMIT: it starts from the last one before its
+  // share
+  int late;
 };
+// isl_nrec: the log was begun in the free pass, after IslPass::late iterations,
+// with room for isl_late_records (a record is a new running minimum, of the log's
+// part here; it takes several iterations to one, as a rule).  Those before them
+// are logged later, in front: entry 0 holds how many, and how many of the later
+// ones are above them, then there is room for `late` of them.  At most kIslLates
+// of a world's islands do so.
+constexpr int kIslLate = 1 << 30, kIslLates = 3;
+__device__ __forceinline__ int isl_late_records(int64_t budget) { return int(budget >> 1); }
+__device__ __forceinline__ bool isl_is_late(int nrec) { return nrec >= kIslLate; }
+
+// An island's log: record r is entry place(r).
+struct IslLog {
+  int64_t at;
+  int n, gap_at, gap;
+  __device__ __forceinline__ int64_t place(int r) const { return at + r + (r >= gap_at ? gap : 0); }
+};
+template <typename R>
+__device__ __forceinline__ IslLog isl_log_of(const RS<R>& a, int g, int late) {
+  const int64_t at = a.isl_log[g];
+  const int n = a.isl_nrec[g];
+  if (!isl_is_late(n)) return IslLog{at, n, INT_MAX, 0};
+  const int before = a.log_it[at], skip = a.log_j[at];
+  return IslLog{at + 1, before + n - kIslLate - skip, before, late - before + skip};
+}
+
+// The first of records lo .. hi of a log whose key is not above tau (hi if there
+// is none).
+template <typename R>
+__device__ __forceinline__ int isl_first(const RS<R>& a, const IslLog& L, int lo, int hi, R tau) {
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (a.log_key[L.place(mid)] > tau)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo;
+}
 
 // Ends of a batch: the islands' iteration counts, the world's sum.
-template <typename R>
-__device__ __forceinline__ void isl_count(const RS<R>& a, const IslWorld<R>& W, const IslPass& P, int k, bool first,
-                                          int it, int nrec, bool over) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_count(const RS<R>& a, const IslWorld<R, T>& W, const IslPass& P, int k, bool first,
+                                          int it, int nrec, bool over, R runmin) {
   if (!first) return;
   if (P.pass == ISL_FREE) {
     a.isl_its[W.b0w + k] = it;
+    a.isl_nrec[W.b0w + k] = nrec < 0 ? -1 : kIslLate + nrec;
     if (it > 0) atomicAdd(&W.f->total, (unsigned long long)it);
     if (over) W.f->over = 1;
   } else if (P.pass == ISL_LOG) {
+    const int n = a.isl_nrec[W.b0w + k];
+    if (P.late > 0 && isl_is_late(n)) {  // the free pass's records from this running minimum on
+      const int64_t at = a.isl_log[W.b0w + k];
+      const int skip = isl_first(a, IslLog{at + 1 + P.late, n - kIslLate, INT_MAX, 0}, 0, n - kIslLate, runmin);
+      a.log_it[at] = nrec;
+      a.log_j[at] = skip;
+      return;
+    }
     a.isl_its[W.b0w + k] = it;
     a.isl_nrec[W.b0w + k] = nrec;
   }
@@ -367,6 +434,17 @@ __device__ __forceinline__ void isl_log(const RS<R>& a, int64_t at, R key, int j
   a.log_key[at] = key;
   a.log_j[at] = j;
   a.log_it[at] = it;
+}
+
+// `need` entries of the log pool: where they start, or -1 (and they stay free
+// for worlds that need less).
+template <typename R>
+__device__ __forceinline__ int64_t isl_reserve(const RS<R>& a, int64_t need) {
+  unsigned long long* head = (unsigned long long*)a.log_head;
+  const int64_t at = int64_t(atomicAdd(head, (unsigned long long)need));
+  if (at + need <= a.log_cap) return at;
+  atomicAdd(head, (unsigned long long)-need);
+  return -1;
 }
 
 // What applyPositionChange (contact.go:286-386) computes of a contact that
@@ -411,8 +489,8 @@ __device__ __forceinline__ void isl_move_of(bool has1, const V3<R>& n, const V3<
 
 // The rest of it: the moves of the two bodies for a penetration, and their new
 // position and orientation from the tables (st: 7 reals per body).
-template <typename R>
-__device__ __forceinline__ void isl_position_change(const IslWorld<R>& W, const int kl[2], const V3<R>& n,
+template <typename R, int T>
+__device__ __forceinline__ void isl_position_change(const IslWorld<R, T>& W, const int kl[2], const V3<R>& n,
                                                     R penetration, const IslMove<R>& mv, V3<R> lin[2], V3<R> ang[2],
                                                     R (&st)[2][7]) {
   const int l1 = kl[1] >= 0 ? kl[1] : kl[0];
@@ -455,8 +533,8 @@ __device__ __forceinline__ void isl_position_change(const IslWorld<R>& W, const 
 
 // World inverse inertia and inverse mass of a contact's bodies, from the LDS
 // table where the launch has one.
-template <typename R>
-__device__ __forceinline__ void isl_inertia(const Bodies<R>& b, const IslWorld<R>& W, const int kl[2], R (&iw)[2][9],
+template <typename R, int T>
+__device__ __forceinline__ void isl_inertia(const Bodies<R>& b, const IslWorld<R, T>& W, const int kl[2], R (&iw)[2][9],
                                             R im[2]) {
   if (W.iw) {
 #pragma unroll
@@ -475,8 +553,8 @@ __device__ __forceinline__ void isl_inertia(const Bodies<R>& b, const IslWorld<R
 // The derived data of the sleeping bodies of `red` (bit i: kl[i]), from the
 // state just stored, to HBM and to the table (rare, and large: one copy of the
 // code).
-template <typename R>
-__device__ __forceinline__ void isl_rederive(const Bodies<R>& b, const IslWorld<R>& W, const int kl[2], uint32_t red) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_rederive(const Bodies<R>& b, const IslWorld<R, T>& W, const int kl[2], uint32_t red) {
 #pragma unroll 1
   for (int i = 0; i < 2 && red; ++i) {
     if (!(red >> i & 1u)) continue;
@@ -498,8 +576,8 @@ __device__ __forceinline__ void isl_rederive(const Bodies<R>& b, const IslWorld<
 // Contacts of a body whose derived data changed take their part of it again.
 // Out of the table that is a few LDS reads; from HBM, where the store has to be
 // waited for as well, such an iteration takes three times as long (3.6 us).
-template <typename R>
-__device__ __forceinline__ void isl_move_again(const Bodies<R>& b, const IslWorld<R>& W, const int jb[2],
+template <typename R, int T>
+__device__ __forceinline__ void isl_move_again(const Bodies<R>& b, const IslWorld<R, T>& W, const int jb[2],
                                                const V3<R>& n, const V3<R> rel[2], IslMove<R>& mv) {
   R iw[2][9], im[2];
   if (W.iw) {
@@ -524,12 +602,12 @@ __device__ __forceinline__ void isl_move_again(const Bodies<R>& b, const IslWorl
 struct IslAwake {
   uint8_t f0, f1;
 };
-template <typename R>
-__device__ __forceinline__ IslAwake isl_awake_of(const IslWorld<R>& W, const int kl[2]) {
+template <typename R, int T>
+__device__ __forceinline__ IslAwake isl_awake_of(const IslWorld<R, T>& W, const int kl[2]) {
   return IslAwake{W.fl[kl[0]], W.fl[kl[1] >= 0 ? kl[1] : kl[0]]};
 }
-template <typename R>
-__device__ __forceinline__ uint32_t isl_match_awake(const IslWorld<R>& W, const int kl[2], IslAwake f, bool store) {
+template <typename R, int T>
+__device__ __forceinline__ uint32_t isl_match_awake(const IslWorld<R, T>& W, const int kl[2], IslAwake f, bool store) {
   const bool a0 = (f.f0 & F_AWAKE) != 0, a1 = (f.f1 & F_AWAKE) != 0;
   if (kl[1] < 0) return a0 ? 0u : 1u;
   if (a0 != a1 && store) W.fl[a0 ? kl[1] : kl[0]] = uint8_t((a0 ? f.f1 : f.f0) | F_AWAKE);
@@ -601,8 +679,8 @@ __device__ __forceinline__ void isl_touch_position(const R* x, const int jb[2], 
 // applyVelocityChange (contact.go:448-494) by the lane that owns the
 // selected contact, the bodies' velocity and rotation in the tables; their
 // new velocity and rotation come back in nv, nw.
-template <typename R, int KIND>
-__device__ __forceinline__ void isl_velocity_change(const IslWorld<R>& W, const int kl[2], const V3<R> rel[2],
+template <typename R, int KIND, int T>
+__device__ __forceinline__ void isl_velocity_change(const IslWorld<R, T>& W, const int kl[2], const V3<R> rel[2],
                                                     const R* c2w, R ddv, const V3<R>& cvel, const R* imp,
                                                     const R (&iw)[2][9], const R im[2], V3<R> vc[2], V3<R> rc[2],
                                                     V3<R> nv[2], V3<R> nw[2], R friction) {
@@ -638,15 +716,15 @@ __device__ __forceinline__ uint32_t isl_ids(int c0, int c1, int b0w) {
 
 // adjustPositions (contact.go:233-283) on islands k0 .. of one class, one
 // contact per lane.
-template <typename R, int KIND>
-__device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R>& W, const IslPass& P, int lg, int k0, int kend, R eps,
+template <typename R, int KIND, int T>
+__device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R, T>& W, const IslPass& P, int lg, int k0, int kend, R eps,
                               R& kmin) {
   const Contacts<R>& c = a.c;
   const int64_t CS = c.cap;
   const int lane = W.t & 63, wave = W.t >> 6, grp = lane >> lg, li = lane & ((1 << lg) - 1);
   const int k = k0 + grp;
-  bool live = k < kend && !(P.pass == ISL_LIMIT && a.isl_its[W.b0w + k] < 0);
-  const int cnt = live ? a.isl_cnt[W.b0w + k] : 0;
+  bool live = k < kend && !(P.pass != ISL_FREE && a.isl_its[W.b0w + k] < 0);
+  const int cnt = !live ? 0 : P.one ? W.C : a.isl_cnt[W.b0w + k];
   const bool has = li < cnt;
   int j = INT_MAX;
   R key = R(0);
@@ -654,7 +732,7 @@ __device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R>&
   V3<R> n{R(0), R(0), R(0)}, rel[2] = {n, n};
   IslMove<R> mv{};
   if (has) {
-    j = a.isl_idx[W.base + a.isl_off[W.b0w + k] + li];
+    j = P.one ? li : a.isl_idx[W.base + a.isl_off[W.b0w + k] + li];
     const int64_t g = W.base + j;
     const int c0 = c.body0[g], c1 = c.body1[g];
     id = isl_ids(c0, c1, W.b0w);
@@ -743,20 +821,55 @@ __device__ __forceinline__ void isl_pos_batch(const RS<R>& a, const IslWorld<R>&
     c.pen[W.base + j] = key;
     kmin = key < kmin ? key : kmin;
   }
-  isl_count(a, W, P, k, k < kend && li == 0, it, nrec, over);
+  isl_count(a, W, P, k, k < kend && li == 0, it, nrec, over, runmin);
+}
+
+// Checkpoint q (2 or 3) of a small island in the velocity phase: the contact's
+// key and closing velocity where a big island's impulse data would be, its
+// bodies' velocity, rotation and flag where the position phase kept the
+// sleepers.  SAVE, or back.
+template <typename R, bool SAVE, int T>
+__device__ __forceinline__ void isl_checkpoint(const RS<R>& a, const IslWorld<R, T>& W, int j, const int jb[2], int q,
+                                               R& key, V3<R>& cv) {
+  const int64_t S = a.b.stride;
+  R* e = a.c.imp + kImpPlanes * (W.base + j) + 4 * (q - 2);
+  if constexpr (SAVE) {
+    e[0] = key, e[1] = cv.x, e[2] = cv.y, e[3] = cv.z;
+  } else {
+    key = e[0];
+    cv = V3<R>{e[1], e[2], e[3]};
+  }
+#pragma unroll 1
+  for (int i = 0; i < 2; ++i) {
+    const int l = opaque_lane(i == 0 ? jb[0] : jb[1]);
+    if (l < 0) continue;
+    R* p = a.isl_snap + W.b0w + l + 7 * (q - 2) * S;
+#pragma unroll 1
+    for (int k = 0; k < 6; ++k) {
+      if constexpr (SAVE)
+        p[k * S] = W.st[kIslSt * l + k];
+      else
+        W.st[kIslSt * l + k] = p[k * S];
+    }
+    if constexpr (SAVE)
+      p[6 * S] = R(W.fl[l]);
+    else
+      W.fl[l] = uint8_t(p[6 * S]);
+  }
 }
 
 // adjustVelocities (contact.go:390-445) on islands k0 .. of one class, one
 // contact per lane.
-template <typename R, int KIND>
-__device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>& W, const IslPass& P, int lg, int k0, int kend, R eps) {
+template <typename R, int KIND, int T>
+__device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R, T>& W, const IslPass& P, int lg, int k0, int kend, R eps) {
   const Bodies<R>& b = a.b;
   const Contacts<R>& c = a.c;
   const int64_t CS = c.cap, S = b.stride;
+  constexpr bool LATE = KIND != KIND_LABEL;
   const int lane = W.t & 63, wave = W.t >> 6, grp = lane >> lg, li = lane & ((1 << lg) - 1);
   const int k = k0 + grp;
-  bool live = k < kend && !(P.pass == ISL_LIMIT && a.isl_its[W.b0w + k] < 0);
-  const int cnt = live ? a.isl_cnt[W.b0w + k] : 0;
+  bool live = k < kend && !(P.pass != ISL_FREE && a.isl_its[W.b0w + k] < 0);
+  const int cnt = !live ? 0 : P.one ? W.C : a.isl_cnt[W.b0w + k];
   const bool has = li < cnt;
   const V3<R> zero{R(0), R(0), R(0)};
   int j = INT_MAX;
@@ -771,7 +884,7 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
   for (int q = 0; q < kImpPlanes; ++q) imp[q] = R(0);
   im[0] = im[1] = R(0);
   if (has) {
-    j = a.isl_idx[W.base + a.isl_off[W.b0w + k] + li];
+    j = P.one ? li : a.isl_idx[W.base + a.isl_off[W.b0w + k] + li];
     const int64_t g = W.base + j;
     const int c0 = c.body0[g], c1 = c.body1[g];
     id = isl_ids(c0, c1, W.b0w);
@@ -798,31 +911,72 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
       cv = ld3(a.isl_save, CS, g);
     }
   }
-  const int64_t lim = P.pass == ISL_LIMIT ? (live ? int64_t(a.isl_its[W.b0w + k]) : 0) : P.budget;
-  const int64_t logat = P.pass == ISL_LOG && live ? a.isl_log[W.b0w + k] : 0;
+  int lim = P.pass == ISL_LIMIT ? (live ? a.isl_its[W.b0w + k] : 0) : int(P.budget);
+  int64_t logat = P.pass == ISL_LOG && live ? a.isl_log[W.b0w + k] : 0;
+  if (LATE && P.pass == ISL_LOG && P.late > 0 && live && isl_is_late(a.isl_nrec[W.b0w + k])) {
+    lim = P.late;  // what the free pass did not log
+    ++logat;
+  }
   R* x = W.f->x[wave][grp];
   volatile uint32_t* xi = W.f->xi[wave][grp];
   const uint64_t gm = group_lanes(lg);
   const int jb[2] = {id_lo(id), id_hi(id)};
-  int it = 0, nrec = 0;
+  bool logs = P.pass == ISL_LOG;  // the wave's islands log
+  int it = 0, nrec = logs ? 0 : -1;  // records: -1 as long as the island does not
   R runmin = R(__builtin_inf());
   bool over = false;
+  if constexpr (LATE) {
+    if (P.pass == ISL_FREE && P.late > 0) lim = P.late;  // where something is kept, and on from there
+    if (P.pass == ISL_LIMIT && P.late > 0) {
+      const int q = live ? min((lim - 1) / P.late, 3) : 0;
+      if (q > 1) {
+        it = q * P.late;
+        if (has) isl_checkpoint<R, false>(a, W, j, jb, q, key, cv);
+      }
+      wave_fence();
+    }
+  }
   while (true) {
     const R kk = (has && live && key > eps) ? key : R(-__builtin_inf());
     const R m = group_reduce(kk, lg, [](R p, R q) { return q > p ? q : p; });
     const bool any = m > R(-__builtin_inf());
     const bool top = group_owner<R>(any && kk == m, j, lg, gm);
     live = live && any;
-    if (live && it >= lim) {
-      over = true;
-      live = false;
+    const bool stop = live && it >= lim;
+    if (__any(stop)) {
+      if (LATE && P.pass == ISL_FREE && P.late > 0 && __any(stop && it < int(P.budget))) {
+        // every live island of the wave has made as many iterations
+        if (stop && it > P.late) {
+          if (has) isl_checkpoint<R, true>(a, W, j, jb, it / P.late, key, cv);
+        } else if (stop) {
+          if (li == 0)
+            logat = atomicAdd(&W.f->lates, 1) < kIslLates ? isl_reserve(a, 1 + P.late + isl_late_records(P.budget)) : -1;
+        }
+        if (!logs) {
+          logs = true;
+          logat = __shfl(logat, grp << lg, 64);
+          if (stop && logat >= 0) {
+            if (li == 0) a.isl_log[W.b0w + k] = logat;
+            logat += 1 + P.late;
+            nrec = 0;
+          }
+        }
+        lim = it < 3 * P.late ? it + P.late : int(P.budget);
+      } else if (stop) {
+        over = true;
+        live = false;
+      }
     }
     if (!__any(live)) break;
     const bool owner = live && top;
-    if (P.pass == ISL_LOG && live && (nrec == 0 || m <= runmin)) {
+    if (logs && live && m <= runmin) {
       runmin = m;
-      if (owner) isl_log(a, logat + nrec, m, j, it);
-      ++nrec;
+      if (LATE && P.pass == ISL_FREE && nrec >= isl_late_records(P.budget)) {
+        nrec = -1;  // no room for more: no log
+      } else if (nrec >= 0) {
+        if (owner) isl_log(a, logat + nrec, m, j, it);
+        ++nrec;
+      }
     }
     if (owner) {
       const int kl[2] = {jb[0], jb[1]};
@@ -858,7 +1012,7 @@ __device__ __forceinline__ void isl_vel_batch(const RS<R>& a, const IslWorld<R>&
     c.ddv[W.base + j] = key;
     st3(c.cvel, CS, W.base + j, cv);
   }
-  isl_count(a, W, P, k, k < kend && li == 0, it, nrec, over);
+  isl_count(a, W, P, k, k < kend && li == 0, it, nrec, over, runmin);
 }
 
 // A contact's impulse data (Contacts::imp), in 16-byte accesses.
@@ -905,10 +1059,9 @@ __device__ __forceinline__ void isl_imp_load(const R* q, R (&v)[kImpPlanes]) {
 // records from HBM too.  An iteration has one barrier, after the waves' best
 // contacts and the corrections these would make (two more where a sleeping
 // body's derived data change).
-template <typename R, int KIND, bool VEL, int SL>
-__device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, const IslPass& P, int k, bool last, R eps,
+template <typename R, int KIND, bool VEL, int SL, int T>
+__device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R, T>& W, const IslPass& P, int k, bool last, R eps,
                                         R& kmin) {
-  constexpr int T = kIslThreads;
   const Bodies<R>& b = a.b;
   const Contacts<R>& c = a.c;
   const int64_t CS = c.cap, S = b.stride;
@@ -920,7 +1073,7 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
   constexpr bool MOVE = !VEL && SL <= 2;  // what a position change keeps is in registers
   IslMove<R> mv[MOVE ? SL : 1];
   const bool resume = VEL && k == P.resume;
-  if (P.pass == ISL_LIMIT && a.isl_its[W.b0w + k] < 0) return;
+  if (P.pass != ISL_FREE && a.isl_its[W.b0w + k] < 0) return;
   R rimp[kImpPlanes], riw[2][9], rim[2];  // REG
   constexpr bool REC = SL <= 2;           // the records are in registers
   R rm[REC ? SL : 1][9];
@@ -1021,7 +1174,7 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
   int it = resume ? W.f->at : 0, nrec = 0;
   R runmin = resume ? W.f->runkey : R(__builtin_inf());
   int runj = resume ? W.f->runj : INT_MAX;
-  bool over = false;
+  int jm = INT_MAX;
   __syncthreads();  // the pause's words are read, the island before is done
   while (true) {
     opaque_ids(ids);
@@ -1042,10 +1195,32 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
     if (tie & (tie - 1)) wj = group_reduce(bj != INT_MAX && best == wm ? bj : INT_MAX, 6, [](int p, int q) { return q < p ? q : p; });
     IslBest<R>* bb4 = W.f->best[par];
     if (tie ? bj == wj : (t & 63) == 0) bb4[wave] = IslBest<R>{wm, tie ? wj : INT_MAX, pick(ids, bs)};
+    // The best of the waves' best, in each quad of lanes: before the corrections
+    // in the launches that fill the chip (narrow workgroups), where those of the
+    // other waves would cost others their turns, and after them else.
+    constexpr bool FULL = T < kIslThreads;
+    int bw = 0;
+    R m = R(0);
+    uint32_t kid = 0;
+    auto winner = [&]() {
+      static_assert(T / 64 <= 4, "a quad holds one offer per wave");
+      const IslBest<R> e = bb4[t & ((T / 64) - 1)];
+      m = group_reduce(e.key, 2, [](R p, R q) { return q > p ? q : p; });
+      jm = __builtin_amdgcn_readfirstlane(
+          group_reduce(e.key == m ? e.j : INT_MAX, 2, [](int p, int q) { return q < p ? q : p; }));
+      bw = __builtin_ctzll(__ballot(e.j == jm)) & ((T / 64) - 1);
+      kid = uint32_t(__builtin_amdgcn_readlane(int(e.id), bw));
+    };
+    if constexpr (FULL) {
+      __syncthreads();
+      winner();
+      if (jm == INT_MAX || it >= lim) break;
+    }
+    const bool mine = FULL ? bj == jm : tie && bj == wj;
     if constexpr (VEL) {
-      // every wave's best contact computes its correction, the winner's is
+      // else every wave's best contact computes its correction, the winner's is
       // taken: the other waves would wait
-      if (tie && bj == wj) {
+      if (mine) {
         const uint32_t id = pick(ids, bs);
         const int64_t g = W.base + wj;
         const int kl[2] = {id_lo(id), id_hi(id)};
@@ -1075,7 +1250,7 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
         isl_put(W.f->bx[par][wave], v, u);
         isl_put(W.f->bx[par][wave] + 12, nv, nw);
       }
-    } else if (tie && bj == wj) {
+    } else if (mine) {
       const uint32_t id = pick(ids, bs);
       const int kl[2] = {id_lo(id), id_hi(id)};
       V3<R> v[2], u[2], nj;
@@ -1109,19 +1284,10 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
       }
     }
     __syncthreads();
-    // the best of the waves' best, in each quad of lanes
-    static_assert(kIslWaves == 4, "a quad holds one offer per wave");
-    const IslBest<R> e = bb4[t & (kIslWaves - 1)];
-    const R m = group_reduce(e.key, 2, [](R p, R q) { return q > p ? q : p; });
-    const int jq = group_reduce(e.key == m ? e.j : INT_MAX, 2, [](int p, int q) { return q < p ? q : p; });
-    const int jm = __builtin_amdgcn_readfirstlane(jq);
-    if (jm == INT_MAX) break;
-    if (it >= lim) {
-      over = true;
-      break;
+    if constexpr (!FULL) {
+      winner();
+      if (jm == INT_MAX || it >= lim) break;
     }
-    const int bw = __builtin_ctzll(__ballot(e.j == jm)) & (kIslWaves - 1);
-    const uint32_t kid = uint32_t(__builtin_amdgcn_readlane(int(e.id), bw));
     const int kl[2] = {id_lo(kid), id_hi(kid)};
     const bool owner = bj == jm;
     const bool low = m <= runmin;
@@ -1222,6 +1388,7 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
     }
     ++it;
   }
+  const bool over = jm != INT_MAX;  // the budget stopped it
   if (P.pass != ISL_LOG) {
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
@@ -1242,35 +1409,39 @@ __device__ __forceinline__ void isl_big(const RS<R>& a, const IslWorld<R>& W, co
     W.f->runkey = runmin;
     W.f->runj = runj;
   }
-  isl_count(a, W, P, k, t == 0, it, nrec, over);
+  isl_count(a, W, P, k, t == 0, it, nrec, over, runmin);
   __syncthreads();  // the waves' best contacts are read, the counts made
 }
 
 // Every island of the world once: the waves take batches of the small ones in
 // class order, then the whole workgroup the big ones, one after another, the
 // one of the largest class last.
-template <typename R, int KIND, bool VEL>
-__device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, const IslPass& P, R eps, R& kmin) {
+template <typename R, int KIND, bool VEL, int T>
+__device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R, T>& W, const IslPass& P, R eps, R& kmin) {
   if (W.t == 0) {
     W.f->next = 0;
     if (P.pass == ISL_FREE) {
       W.f->total = 0;
       W.f->over = 0;
       W.f->paused = -1;
+      W.f->lates = 0;
     }
   }
   if (W.t < kIslWords) W.f->cls[W.t] = a.isl_cls[kIslWords * int64_t(W.w) + W.t];
   __syncthreads();
   const int32_t* cls = W.f->cls;
-  int n0 = cls[0], n1 = cls[1], nbig = n0 + n1 + cls[2];
+  // islands of eight, of four and of two contacts per thread, and all big ones
+  constexpr bool FOUR = T < 256;
+  int n8 = cls[0] + (FOUR ? 0 : cls[1]), n4 = FOUR ? cls[1] : 0, n2 = cls[2], nbig = n8 + n4 + n2 + cls[3];
   if (P.one) {
-    const int k = isl_class(W.C);
-    n0 = k == 0 ? 1 : 0;
-    n1 = k == 1 ? 1 : 0;
-    nbig = 1;
+    const int k = isl_class<T>(W.C);
+    n8 = k == 0 || (!FOUR && k == 1) ? 1 : 0;
+    n4 = FOUR && k == 1 ? 1 : 0;
+    n2 = k == 2 ? 1 : 0;
+    nbig = W.C > 64 ? 1 : 0;
   }
-  if (W.iw && (!VEL || n0 + n1 > 0)) {
-    for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
+  if (W.iw && (!VEL || n8 + n4 + n2 > 0)) {
+    for (int i = opaque_lane(W.t); i < W.n; i += T) {
       R iw[9];
       ld9(a.b.iit_world, a.b.stride, W.b0w + i, iw);
 #pragma unroll
@@ -1279,7 +1450,7 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
     }
   }
   if constexpr (!VEL) __syncthreads();
-  while (!P.only && !P.one) {
+  while (!P.only) {
     // One lane takes the wave's ticket.  Its index is opaque: with a branch that
     // is the same in every turn, the compiler makes the other lanes a loop of
     // their own, which never sees the first lane's value.
@@ -1288,7 +1459,11 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
     __builtin_amdgcn_wave_barrier();
     q = __builtin_amdgcn_readfirstlane(q);
     int at = nbig, k = kIslBigClasses, m = 0, per = 1, lg = 6;
-    for (; k < kIslClasses; ++k) {
+    if (P.one) {
+      if (q > 0 || W.C > 64) break;
+      m = 1;
+    }
+    for (; !P.one && k < kIslClasses; ++k) {
       m = cls[k];
       lg = isl_class_lg(k);
       per = 64 >> lg;
@@ -1308,12 +1483,15 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
   for (int i = nbig - 1; i >= 0; --i) {
     if (P.only ? i != P.resume : P.pass == ISL_LOG && i == P.resume) continue;
     const bool last = i == 0;
-    if (i < n0)
+    if (i < n8) {
       isl_big<R, KIND, VEL, 8>(a, W, P, i, last, eps, kmin);
-    else if (i < n0 + n1)
+    } else if (i < n8 + n4) {
+      if constexpr (FOUR) isl_big<R, KIND, VEL, 4>(a, W, P, i, last, eps, kmin);
+    } else if (i < n8 + n4 + n2) {
       isl_big<R, KIND, VEL, 2>(a, W, P, i, last, eps, kmin);
-    else
+    } else {
       isl_big<R, KIND, VEL, 1>(a, W, P, i, last, eps, kmin);
+    }
   }
 }
 
@@ -1323,11 +1501,11 @@ __device__ __forceinline__ void isl_run(const RS<R>& a, const IslWorld<R>& W, co
 // The body tables as the phase starts.  (Here and below the thread index is
 // opaque, so that the addresses of one loop over the bodies are not kept in
 // registers through a phase for the next.)
-template <typename R, bool VEL>
-__device__ __forceinline__ void isl_load(const RS<R>& a, const IslWorld<R>& W) {
+template <typename R, bool VEL, int T>
+__device__ __forceinline__ void isl_load(const RS<R>& a, const IslWorld<R, T>& W) {
   const Bodies<R>& b = a.b;
   const int64_t S = b.stride;
-  for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
+  for (int i = opaque_lane(W.t); i < W.n; i += T) {
     const int g = W.b0w + i;
     W.fl[i] = b.flags[g];
     if constexpr (VEL) {
@@ -1344,11 +1522,11 @@ __device__ __forceinline__ void isl_load(const RS<R>& a, const IslWorld<R>& W) {
 
 // The position phase writes a sleeping body's derived data in HBM when it
 // moves one (contact.go:380-382): kept, and put back.
-template <typename R>
-__device__ __forceinline__ void isl_sleepers(const RS<R>& a, const IslWorld<R>& W, bool put_back) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_sleepers(const RS<R>& a, const IslWorld<R, T>& W, bool put_back) {
   const Bodies<R>& b = a.b;
   const int64_t S = b.stride;
-  for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
+  for (int i = opaque_lane(W.t); i < W.n; i += T) {
     const int g = W.b0w + i;
     if (b.flags[g] & F_AWAKE) continue;
 #pragma unroll
@@ -1371,11 +1549,11 @@ __device__ __forceinline__ void isl_sleepers(const RS<R>& a, const IslWorld<R>& 
 
 // The phase's result to HBM: the tables, the awake flags and the motion
 // matchAwakeState gives a woken body (SetAwake(true), rigidbody.go:183-186).
-template <typename R, bool VEL>
-__device__ __forceinline__ void isl_commit(const RS<R>& a, const IslWorld<R>& W) {
+template <typename R, bool VEL, int T>
+__device__ __forceinline__ void isl_commit(const RS<R>& a, const IslWorld<R, T>& W) {
   const Bodies<R>& b = a.b;
   const int64_t S = b.stride;
-  for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
+  for (int i = opaque_lane(W.t); i < W.n; i += T) {
     const int g = W.b0w + i;
     if constexpr (VEL) {
       st3(b.vel, S, g, tab3(W.st + kIslSt * i));
@@ -1395,9 +1573,9 @@ __device__ __forceinline__ void isl_commit(const RS<R>& a, const IslWorld<R>& W)
 }
 
 // The world's labels of a phase that is run again.
-template <typename R, bool VEL>
-__device__ __forceinline__ void isl_clear_labels(const RS<R>& a, const IslWorld<R>& W) {
-  for (int j = opaque_lane(W.t); j < W.C; j += kIslThreads) {
+template <typename R, bool VEL, int T>
+__device__ __forceinline__ void isl_clear_labels(const RS<R>& a, const IslWorld<R, T>& W) {
+  for (int j = opaque_lane(W.t); j < W.C; j += T) {
     float* L = a.labels + (W.base + j) * kOut;
     if constexpr (VEL) {
       for (int q = 0; q < 12; ++q) L[q] = 0.f;
@@ -1423,24 +1601,7 @@ struct BitsOf<float> {
   static constexpr type inf = 0x7F800000u;
 };
 
-// The first record of island k whose key is not above tau (their number if
-// there is none), and the iterations before it, from `from` on.
-template <typename R>
-__device__ __forceinline__ int isl_below(const RS<R>& a, int g, R tau, int from, int& its) {
-  const int64_t at = a.isl_log[g];
-  const int nrec = a.isl_nrec[g];
-  int lo = 0, hi = nrec;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (a.log_key[at + mid] > tau)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  its = (lo < nrec ? a.log_it[at + lo] : a.isl_its[g]) - from;
-  return lo;
-}
-
+constexpr double kIslDeal = 16;  // records that are dealt out one by one rather than searched for a level
 // Merges the islands' logs in the serial loop's order up to `budget`
 // iterations; leaves each island's share in isl_its (-1 with `skip` where the
 // island is not cut short).  The serial loop has run every selection above
@@ -1450,41 +1611,74 @@ __device__ __forceinline__ int isl_below(const RS<R>& a, int g, R tau, int from,
 // the largest key.  (A paused island's log starts at its pause, where
 // `at_pause` of its iterations are done.)  The heads are in the state tables'
 // space.
-template <typename R>
-__device__ __forceinline__ void isl_merge(const RS<R>& a, const IslWorld<R>& W, int nisl, int64_t budget, int paused,
-                                          int at_pause, bool skip) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_merge(const RS<R>& a, const IslWorld<R, T>& W, int nisl, int64_t budget, int paused,
+                                          int at_pause, bool skip, int late) {
   typedef typename BitsOf<R>::type U;
   R* hkey = W.st;
   int32_t* hj = (int32_t*)(hkey + W.NB);
   int32_t* hp = hj + W.NB;
-  int64_t rem = budget - at_pause;
   auto plus = [](double p, double q) { return p + q; };
+  auto its = [&](int k, const IslLog& L, int r) {  // of island k before record r of its log
+    return (r < L.n ? a.log_it[L.place(r)] : a.isl_its[W.b0w + k]) - (k == paused ? at_pause : 0);
+  };
   auto above = [&](R tau) {  // iterations above a level
     double n = 0.0;
-    for (int k = W.t; k < nisl; k += kIslThreads) {
-      int its;
-      isl_below(a, W.b0w + k, tau, k == paused ? at_pause : 0, its);
-      n += double(its);
+    for (int k = W.t; k < nisl; k += T) {
+      const IslLog L = isl_log_of(a, W.b0w + k, late);
+      n += double(its(k, L, isl_first(a, L, 0, L.n, tau)));
     }
     return int64_t(isl_reduce(W, n, plus));
   };
+  int64_t rem = budget - at_pause;
   U lo = 0, hi = BitsOf<R>::inf;
-  while (lo < hi) {
-    const U mid = lo + ((hi - lo) >> 1);
-    if (above(real_of_bits(mid)) <= rem)
-      hi = mid;
-    else
-      lo = mid + 1;
+  if (nisl <= T) {
+    // One island per thread (up to 64: per lane, and every wave does the same).
+    // The thread keeps which of its records may be the first at or below the
+    // level, so that a step costs a load or two, and when few are left in the
+    // range they are dealt out below.
+    const bool wave = nisl <= 64;
+    const int k = wave ? W.t & 63 : W.t;
+    const bool has = k < nisl;
+    const IslLog L = has ? isl_log_of(a, W.b0w + k, late) : IslLog{0, 0, INT_MAX, 0};
+    int r0 = 0, r1 = L.n;
+    while (lo < hi) {
+      const U mid = lo + ((hi - lo) >> 1);
+      const int r = isl_first(a, L, r0, r1, real_of_bits(mid));
+      // the iterations above the level, and (times 2^32) the records still in question
+      double sum = has ? double(its(k, L, r)) + double(r1 - r) * 0x1p32 : 0.0;
+      if (wave) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+      } else {
+        sum = isl_reduce(W, sum, plus);
+      }
+      const double records = floor(sum * 0x1p-32);
+      if (int64_t(sum - records * 0x1p32) <= rem) {
+        hi = mid;
+        r0 = r;
+        if (records <= kIslDeal) break;
+      } else {
+        lo = mid + 1;
+        r1 = r;
+      }
+    }
+  } else {
+    while (lo < hi) {
+      const U mid = lo + ((hi - lo) >> 1);
+      if (above(real_of_bits(mid)) <= rem)
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
   }
   const R tau = real_of_bits(hi);
   rem -= above(tau);
-  for (int k = W.t; k < nisl; k += kIslThreads) {
-    int its;
-    const int r = isl_below(a, W.b0w + k, tau, 0, its);
-    const bool some = r < a.isl_nrec[W.b0w + k];
-    const int64_t at = a.isl_log[W.b0w + k] + r;
-    hkey[k] = some ? a.log_key[at] : R(-__builtin_inf());
-    hj[k] = some ? a.log_j[at] : INT_MAX;
+  for (int k = W.t; k < nisl; k += T) {
+    const IslLog L = isl_log_of(a, W.b0w + k, late);
+    const int r = isl_first(a, L, 0, L.n, tau);
+    hkey[k] = r < L.n ? a.log_key[L.place(r)] : R(-__builtin_inf());
+    hj[k] = r < L.n ? a.log_j[L.place(r)] : INT_MAX;
     hp[k] = r;
   }
   __syncthreads();
@@ -1506,18 +1700,18 @@ __device__ __forceinline__ void isl_merge(const RS<R>& a, const IslWorld<R>& W, 
       const int jm = group_reduce(best == m ? bj : INT_MAX, 6, [](int p, int q) { return q < p ? q : p; });
       int run = 0;
       if (bk >= 0 && best == m && bj == jm) {  // this lane's island goes on to its next record
-        const int64_t at = a.isl_log[W.b0w + bk];
-        const int nrec = a.isl_nrec[W.b0w + bk], r = hp[bk];
-        const int end = r + 1 < nrec ? a.log_it[at + r + 1] : a.isl_its[W.b0w + bk];
-        run = end - a.log_it[at + r];
+        const IslLog L = isl_log_of(a, W.b0w + bk, late);
+        const int r = hp[bk], from = a.log_it[L.place(r)];
+        const int end = r + 1 < L.n ? a.log_it[L.place(r + 1)] : a.isl_its[W.b0w + bk];
+        run = end - from;
         if (int64_t(run) >= rem) {
           run = int(rem);
-          hp[bk] = -1 - (a.log_it[at + r] + run);  // settled: its share
+          hp[bk] = -1 - (from + run);  // settled: its share
           hkey[bk] = R(-__builtin_inf());
         } else {
           hp[bk] = r + 1;
-          hkey[bk] = r + 1 < nrec ? a.log_key[at + r + 1] : R(-__builtin_inf());
-          hj[bk] = r + 1 < nrec ? a.log_j[at + r + 1] : INT_MAX;
+          hkey[bk] = r + 1 < L.n ? a.log_key[L.place(r + 1)] : R(-__builtin_inf());
+          hj[bk] = r + 1 < L.n ? a.log_j[L.place(r + 1)] : INT_MAX;
         }
       }
       rem -= group_reduce(run, 6, [](int p, int q) { return q > p ? q : p; });
@@ -1525,26 +1719,27 @@ __device__ __forceinline__ void isl_merge(const RS<R>& a, const IslWorld<R>& W, 
     }
   }
   __syncthreads();
-  for (int k = W.t; k < nisl; k += kIslThreads) {
+  for (int k = W.t; k < nisl; k += T) {
     const int g = W.b0w + k, r = hp[k], all = a.isl_its[g];
-    const int share = r < 0 ? -1 - r : r < a.isl_nrec[g] ? a.log_it[a.isl_log[g] + r] : all;
+    const IslLog L = isl_log_of(a, g, late);
+    const int share = r < 0 ? -1 - r : r < L.n ? a.log_it[L.place(r)] : all;
     a.isl_its[g] = skip && k != paused && share == all ? -1 : share;
   }
   __syncthreads();
 }
 
 // The body tables to HBM scratch, and back.
-template <typename R>
-__device__ __forceinline__ void isl_tables(const RS<R>& a, const IslWorld<R>& W, bool put_back) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_tables(const RS<R>& a, const IslWorld<R, T>& W, bool put_back) {
   const int64_t S = a.b.stride;
-  for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
+  for (int i = opaque_lane(W.t); i < W.n; i += T) {
     const int g = W.b0w + i;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
       if (put_back)
-        W.st[kIslSt * i + k] = a.isl_snap[k * S + g];
+        W.st[kIslSt * i + k] = a.isl_snap[(14 + k) * S + g];
       else
-        a.isl_snap[k * S + g] = W.st[kIslSt * i + k];
+        a.isl_snap[(14 + k) * S + g] = W.st[kIslSt * i + k];
     }
     if (put_back)
       W.fl[i] = a.isl_flag[g];
@@ -1556,11 +1751,11 @@ __device__ __forceinline__ void isl_tables(const RS<R>& a, const IslWorld<R>& W,
 
 // The bodies of the islands that were cut short, as the velocity phase starts
 // (a wave per island; a body of several contacts is written several times).
-template <typename R>
-__device__ __forceinline__ void isl_cut_bodies(const RS<R>& a, const IslWorld<R>& W, int nisl, int paused) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_cut_bodies(const RS<R>& a, const IslWorld<R, T>& W, int nisl, int paused) {
   const Bodies<R>& b = a.b;
   const int64_t S = b.stride;
-  for (int k = W.t >> 6; k < nisl; k += kIslWaves) {
+  for (int k = W.t >> 6; k < nisl; k += (T / 64)) {
     if (k == paused || a.isl_its[W.b0w + k] < 0) continue;
     const int cnt = a.isl_cnt[W.b0w + k];
     const int32_t* idx = a.isl_idx + W.base + a.isl_off[W.b0w + k];
@@ -1587,14 +1782,14 @@ __device__ __forceinline__ void isl_cut_bodies(const RS<R>& a, const IslWorld<R>
 // penetration of separating a contact; a prediction that separates one beyond
 // kSepFactor times it (sep_floor) is tried again at a third of its moves, and
 // given up (false) if that still does.
-template <typename R>
-__device__ __forceinline__ bool isl_take_moves(const RS<R>& a, const IslWorld<R>& W, R& sep_floor) {
+template <typename R, int T>
+__device__ __forceinline__ bool isl_take_moves(const RS<R>& a, const IslWorld<R, T>& W, R& sep_floor) {
   const Bodies<R>& b = a.b;
   const Contacts<R>& c = a.c;
   const int64_t S = b.stride, CS = c.cap;
   const float* dl = a.delta;
   R pmax = R(0);
-  for (int j = W.t; j < W.C; j += kIslThreads) {
+  for (int j = W.t; j < W.C; j += T) {
     const R p = c.pen[W.base + j];
     a.isl_save[4 * CS + W.base + j] = p;
     pmax = p > pmax ? p : pmax;
@@ -1604,7 +1799,7 @@ __device__ __forceinline__ bool isl_take_moves(const RS<R>& a, const IslWorld<R>
   for (int attempt = 0; attempt < 2; ++attempt) {
     // the moves times `scale`, from the phase's starting state
     const R scale = attempt == 0 ? R(1) : R(kPosRetryScale);
-    for (int i = W.t; i < W.n; i += kIslThreads) {
+    for (int i = W.t; i < W.n; i += T) {
       const int g = W.b0w + i;
       if (!(W.fl[i] & F_AWAKE)) continue;
       const V3<R> dx = mul(V3<R>{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])}, scale);
@@ -1620,7 +1815,7 @@ __device__ __forceinline__ bool isl_take_moves(const RS<R>& a, const IslWorld<R>
       e[6] = q.z;
     }
     R kmin = R(0);
-    for (int j = W.t; j < W.C; j += kIslThreads) {
+    for (int j = W.t; j < W.C; j += T) {
       const int64_t gj = W.base + j;
       const int kb[2] = {c.body0[gj], c.body1[gj]};
       V3<R> nj, rj[2];
@@ -1650,10 +1845,10 @@ __device__ __forceinline__ bool isl_take_moves(const RS<R>& a, const IslWorld<R>
 
 // Kinetic energy of the world from the tables (KIND_POLISH); with it the
 // world's mass.
-template <typename R>
-__device__ __forceinline__ double isl_energy(const RS<R>& a, const IslWorld<R>& W, double& mass) {
+template <typename R, int T>
+__device__ __forceinline__ double isl_energy(const RS<R>& a, const IslWorld<R, T>& W, double& mass) {
   double ke = 0.0, m = 0.0;
-  for (int i = opaque_lane(W.t); i < W.n; i += kIslThreads) {
+  for (int i = opaque_lane(W.t); i < W.n; i += T) {
     const int g = W.b0w + i;
     R iw[9];
     ld9(a.b.iit_world, a.b.stride, g, iw);
@@ -1670,13 +1865,13 @@ __device__ __forceinline__ double isl_energy(const RS<R>& a, const IslWorld<R>& 
 // the predicted changes are added to the
 // bodies, and every contact of a changed body gets its contact velocity by
 // the update of contact.go:424-441 and its desired velocity change anew.
-template <typename R>
-__device__ __forceinline__ void isl_take_changes(const RS<R>& a, const IslWorld<R>& W) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_take_changes(const RS<R>& a, const IslWorld<R, T>& W) {
   const Bodies<R>& b = a.b;
   const Contacts<R>& c = a.c;
   const int64_t S = b.stride, CS = c.cap;
   const float* dl = a.delta;
-  for (int i = W.t; i < W.n; i += kIslThreads) {
+  for (int i = W.t; i < W.n; i += T) {
     const int g = W.b0w + i;
     const V3<R> dv{R(dl[g]), R(dl[S + g]), R(dl[2 * S + g])};
     const V3<R> dw{R(dl[3 * S + g]), R(dl[4 * S + g]), R(dl[5 * S + g])};
@@ -1686,7 +1881,7 @@ __device__ __forceinline__ void isl_take_changes(const RS<R>& a, const IslWorld<
       tab3_store(e + 3, add(tab3(e + 3), dw));
     }
   }
-  for (int j = W.t; j < W.C; j += kIslThreads) {
+  for (int j = W.t; j < W.C; j += T) {
     const int64_t gj = W.base + j;
     const int kb[2] = {c.body0[gj], c.body1[gj]};
     V3<R> cvj = ld3(c.cvel, CS, gj);
@@ -1721,11 +1916,11 @@ __device__ __forceinline__ void isl_take_changes(const RS<R>& a, const IslWorld<
 }
 
 // The contacts' values before the phase, put back.
-template <typename R, bool VEL>
-__device__ __forceinline__ void isl_contacts_back(const RS<R>& a, const IslWorld<R>& W) {
+template <typename R, bool VEL, int T>
+__device__ __forceinline__ void isl_contacts_back(const RS<R>& a, const IslWorld<R, T>& W) {
   const Contacts<R>& c = a.c;
   const int64_t CS = c.cap;
-  for (int j = opaque_lane(W.t); j < W.C; j += kIslThreads) {
+  for (int j = opaque_lane(W.t); j < W.C; j += T) {
     const int64_t g = W.base + j;
     if constexpr (VEL) {
       st3(c.cvel, CS, g, ld3(a.isl_save, CS, g));
@@ -1737,29 +1932,18 @@ __device__ __forceinline__ void isl_contacts_back(const RS<R>& a, const IslWorld
   __syncthreads();
 }
 
-// `need` entries of the log pool: where they start, or -1 (and they stay free
-// for worlds that need less).
-template <typename R>
-__device__ __forceinline__ int64_t isl_reserve(const RS<R>& a, int64_t need) {
-  unsigned long long* head = (unsigned long long*)a.log_head;
-  const int64_t at = int64_t(atomicAdd(head, (unsigned long long)need));
-  if (at + need <= a.log_cap) return at;
-  atomicAdd(head, (unsigned long long)-need);
-  return -1;
-}
-
 // Room in the log pool for the world's logs, an island's being at most the
 // iterations it ran (a paused one's: what it may still run); false when there
 // is none.
-template <typename R>
-__device__ __forceinline__ bool isl_log_room(const RS<R>& a, const IslWorld<R>& W, int nisl, int paused,
-                                             int64_t paused_room) {
+template <typename R, int T>
+__device__ __forceinline__ bool isl_log_room(const RS<R>& a, const IslWorld<R, T>& W, int nisl, int paused,
+                                             int64_t paused_room, int late) {
   if (W.t < 64) {
     // an island that is run again whole logs at most its iterations so far,
     // or, stopped by the budget as part of the world's, up to the budget
     int64_t need = 0;
     for (int k = W.t; k < nisl; k += 64) {
-      const int64_t its = a.isl_its[W.b0w + k];
+      const int64_t its = late > 0 && isl_is_late(a.isl_nrec[W.b0w + k]) ? 0 : a.isl_its[W.b0w + k];
       need += k == paused ? its + paused_room : its;
     }
 #pragma unroll
@@ -1771,10 +1955,11 @@ __device__ __forceinline__ bool isl_log_room(const RS<R>& a, const IslWorld<R>& 
     if (W.t == 0) W.f->ok = ok ? 1 : 0;
     for (int k0 = 0; ok && k0 < nisl; k0 += 64) {
       const int k = k0 + W.t;
-      const int64_t its = k < nisl ? int64_t(a.isl_its[W.b0w + k]) : 0;
+      const bool mine = k < nisl && !(late > 0 && isl_is_late(a.isl_nrec[W.b0w + k]));
+      const int64_t its = mine ? a.isl_its[W.b0w + k] : 0;
       const int64_t m = k == paused ? its + paused_room : its;
       const int64_t inc = wave_incl_scan_i64(m);
-      if (k < nisl) a.isl_log[W.b0w + k] = at + inc - m;
+      if (mine) a.isl_log[W.b0w + k] = at + inc - m;
       at += __shfl(inc, 63, 64);
     }
   }
@@ -1782,18 +1967,39 @@ __device__ __forceinline__ bool isl_log_room(const RS<R>& a, const IslWorld<R>& 
   return W.f->ok != 0;
 }
 
+// A budget that is a small part of what the islands would run (below
+// C / kIslSerial) or short altogether, once it is exceeded, is spent on one chain
+// of all the world's contacts: the logs and their merge would cost more.
+constexpr int64_t kIslSerial = 2, kIslShort = 96;
+// After a free pass over the budget: whether every island that ran for more than
+// `late` iterations logged from there on, and there is room for the logs of the
+// rest, which is short.  Not with big islands, which log late only when paused.
+template <typename R, int T>
+__device__ __forceinline__ bool isl_late(const RS<R>& a, const IslWorld<R, T>& W, int nisl, int late) {
+  if (W.f->lates == 0 || W.f->lates > kIslLates || W.f->cls[0] + W.f->cls[1] + W.f->cls[2] + W.f->cls[3] > 0)
+    return false;
+  double bad = 0.0;
+  for (int k = W.t; k < nisl; k += T)
+    if (!isl_is_late(a.isl_nrec[W.b0w + k]) && a.isl_its[W.b0w + k] > late) bad = 1.0;
+  if (isl_reduce(W, bad, [](double p, double q) { return p + q; }) > 0.0) return false;
+  return isl_log_room(a, W, nisl, -1, 0, late);
+}
+
 // One phase of the world: the tables are loaded, the contacts are as
 // prepared; `polish` first tries the surrogate's polish (its mask byte is
 // set when that is rejected).  A world that exceeds its budget and finds no
 // room in the log pool starts again as one island of all its contacts.
-// Returns false when that has more than kIslMaxContacts of them: the phase is
+// Returns false when that has more than isl_max_contacts<T>() of them: the phase is
 // undone, for the serial kernel to do.
-template <typename R, int KIND, bool VEL>
-__device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, int64_t budget, bool polish,
+template <typename R, int KIND, bool VEL, int T>
+__device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R, T>& W, int64_t budget, bool polish,
                                           int64_t& used) {
   constexpr bool POLISH = VEL ? KIND == KIND_POLISH : KIND == KIND_PPOLISH;
   const R plain_eps = VEL ? R(kVelocityEpsilon) : R(kPositionEpsilon);
-  IslPass P{ISL_FREE, false, budget, true, -1, false, false};
+  constexpr bool LATE = VEL && KIND != KIND_LABEL;
+  const int late = LATE && budget >= 16 && budget < kIslLate ? int(budget >> 2) : 0;
+  const bool one = W.C <= isl_max_contacts<T>() && budget * (W.C > 2 * T ? 2 * kIslSerial : kIslSerial) < W.C;
+  IslPass P{ISL_FREE, false, budget, !one, -1, false, one, late};
   R eps = plain_eps, sep_floor = R(0);
   double ke = 0.0, mass = 0.0;
   bool rejected = false;
@@ -1806,7 +2012,8 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
         rejected = !isl_take_moves(a, W, sep_floor);
       }
       P.saved = true;
-      P.pause = false;
+      P.pause = P.one = false;
+      P.late = 0;
       P.budget = isl_budget(a.polish_mult * int64_t(W.C));
       eps = plain_eps + a.polish_tol;
     }
@@ -1843,7 +2050,7 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
         isl_load<R, VEL>(a, W);
         if (W.t == 0) a.world_mask[W.w] = 1;
         polish = rejected = false;
-        P = IslPass{ISL_FREE, true, budget, true, -1, false, false};
+        P = IslPass{ISL_FREE, true, budget, !one, -1, false, one, late};
         eps = plain_eps;
         if (budget <= 0) {
           used = 0;
@@ -1857,14 +2064,22 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
       const int64_t total = int64_t(W.f->total);
       used = total;
       if (P.one || (total <= budget && !W.f->over)) return true;
-      // over the budget: log the selections, merge them, and run each island
-      // to its share
       used = budget;
       for (int k = 0; k < kIslClasses; ++k) nisl += W.f->cls[k];
       paused = W.f->paused;
       at_pause = paused >= 0 ? W.f->at : 0;
-      // a paused island logs what it goes on to run, at most to the budget
-      const bool ok = isl_log_room(a, W, nisl, paused, budget - at_pause);
+      if (LATE && P.late > 0 && budget > kIslShort && isl_late(a, W, nisl, P.late)) {
+        isl_tables(a, W, false);
+        P.pass = ISL_LOG;
+        P.pause = false;
+        isl_load<R, VEL>(a, W);
+        continue;
+      }
+      P.late = 0;
+      // log the selections, merge them, and run each island to its share; a
+      // paused island logs what it goes on to run, at most to the budget
+      const bool large = W.C > isl_max_contacts<T>();
+      const bool ok = (budget > kIslShort || large) && isl_log_room(a, W, nisl, paused, budget - at_pause, 0);
       if constexpr (KIND == KIND_LABEL) {
         isl_clear_labels<R, VEL>(a, W);
         paused = -1;  // its labels would have to be kept
@@ -1872,8 +2087,8 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
       if (!ok) {
         if constexpr (!VEL) isl_sleepers(a, W, true);
         isl_contacts_back<R, VEL>(a, W);
-        if (W.C > kIslMaxContacts) return false;
-        P = IslPass{ISL_FREE, true, budget, false, -1, false, true};
+        if (large) return false;
+        P = IslPass{ISL_FREE, true, budget, false, -1, false, true, 0};
         isl_load<R, VEL>(a, W);
         continue;
       }
@@ -1889,12 +2104,13 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
       P.only = true;
       continue;
     } else {
-      isl_merge(a, W, nisl, budget, paused, VEL && paused >= 0 ? at_pause : 0, VEL && paused >= 0);
+      // islands that ended are as their end left them, the paused one as its
+      // pause did, the others start again
+      const bool keep = VEL && (paused >= 0 || P.late > 0);
+      isl_merge(a, W, nisl, budget, keep ? paused : -1, keep && paused >= 0 ? at_pause : 0, keep, P.late);
       P.pass = ISL_LIMIT;
       P.only = false;
-      if (VEL && paused >= 0) {
-        // the islands that ended are as their end left them, the paused one
-        // as its pause did, the others start again
+      if (keep) {
         isl_tables(a, W, true);
         isl_cut_bodies(a, W, nisl, paused);
         continue;
@@ -1906,13 +2122,13 @@ __device__ __forceinline__ bool isl_phase(const RS<R>& a, const IslWorld<R>& W, 
 }
 
 // Hands the world to the left kernel; vel_only: its position phase is done.
-template <typename R>
-__device__ __forceinline__ void isl_leave(const RS<R>& a, const IslWorld<R>& W, bool vel_only) {
+template <typename R, int T>
+__device__ __forceinline__ void isl_leave(const RS<R>& a, const IslWorld<R, T>& W, bool vel_only) {
   if (W.t == 0) a.left_list[atomicAdd(&a.left_count[LEFT_WORLDS], 1)] = W.w | (vel_only ? kLeftVelOnly : 0);
 }
 
-template <typename R, int KIND>
-__device__ __forceinline__ void isl_world(const RS<R>& a, const IslWorld<R>& W) {
+template <typename R, int KIND, int T>
+__device__ __forceinline__ void isl_world(const RS<R>& a, const IslWorld<R, T>& W) {
   const int w = W.w;
   const bool do_pos = (a.mode & RM_POS) != 0;
   const bool do_prep = do_pos && !(a.mode & RM_PREPARED);
@@ -1930,7 +2146,7 @@ __device__ __forceinline__ void isl_world(const RS<R>& a, const IslWorld<R>& W) 
     return;
   }
   if (do_prep) isl_prepare<R, KIND>(a, W, true);
-  if (a.isl_cls[kIslWords * int64_t(w) + kIslTaken] == 0) {
+  if (a.isl_cls[kIslWords * int64_t(w) + kIslTaken] != T) {
     isl_leave(a, W, false);
     return;
   }
@@ -1964,9 +2180,9 @@ __device__ __forceinline__ void isl_world(const RS<R>& a, const IslWorld<R>& W) 
   }
 }
 
-template <typename R>
-__device__ __forceinline__ IslWorld<R> isl_world_of(const RS<R>& a, char* lds, int w) {
-  IslWorld<R> W;
+template <typename R, int T>
+__device__ __forceinline__ IslWorld<R, T> isl_world_of(const RS<R>& a, char* lds, int w) {
+  IslWorld<R, T> W;
   W.w = w;
   W.t = threadIdx.x;
   W.C = a.world_cnt[w];
@@ -1974,19 +2190,19 @@ __device__ __forceinline__ IslWorld<R> isl_world_of(const RS<R>& a, char* lds, i
   W.n = a.body_off[w + 1] - W.b0w;
   W.base = a.world_coff[w];
   W.NB = a.isl_nb;
-  W.f = (IslFixed<R>*)lds;
-  W.st = (R*)(lds + isl_fixed_bytes<R>());
+  W.f = (IslFixed<R, T>*)lds;
+  W.st = (R*)(lds + isl_fixed_bytes<R, T>());
   R* after = W.st + kIslSt * int64_t(W.NB);
   W.iw = W.NB <= kIslIwBodies ? after : nullptr;
   W.fl = (uint8_t*)(W.NB <= kIslIwBodies ? after + kIslIw * int64_t(W.NB) : after);
   return W;
 }
 
-template <typename R, int KIND>
+template <typename R, int KIND, int T>
 __device__ __forceinline__ void isl_block(const RS<R>& a) {
   extern __shared__ __align__(16) char isl_lds[];
   const int w = a.order ? a.order[blockIdx.x] : int(blockIdx.x);
-  const IslWorld<R> W = isl_world_of(a, isl_lds, w);
+  const IslWorld<R, T> W = isl_world_of<R, T>(a, isl_lds, w);
   int64_t* wt = a.world_time ? a.world_time + 4 * int64_t(w) + ((a.mode & RM_VEL) ? 2 : 0) : nullptr;
   if (wt && W.t == 0) wt[0] = int64_t(wall_clock64());
   isl_world<R, KIND>(a, W);
@@ -1998,26 +2214,26 @@ __device__ __forceinline__ void isl_block(const RS<R>& a) {
 
 // Bound by the longest island's chain of dependent arithmetic in small
 // launches, by instruction issue in large ones.
-template <int KIND>
-__global__ void __launch_bounds__(kIslThreads, 2) k_resolve_islands_f64(RS<double> a) {
-  isl_block<double, KIND>(a);
+template <int KIND, int T>
+__global__ void __launch_bounds__(T, 2) k_resolve_islands_f64(RS<double> a) {
+  isl_block<double, KIND, T>(a);
 }
-template <int KIND>
-__global__ void __launch_bounds__(kIslThreads, 3) k_resolve_islands_f32(RS<float> a) {
-  isl_block<float, KIND>(a);
+template <int KIND, int T>
+__global__ void __launch_bounds__(T, 3) k_resolve_islands_f32(RS<float> a) {
+  isl_block<float, KIND, T>(a);
 }
 
-template <typename R>
+template <typename R, int T>
 size_t isl_lds_bytes(int nb) {
-  return isl_fixed_bytes<R>() + size_t(nb) * ((kIslSt + (nb <= kIslIwBodies ? kIslIw : 0)) * sizeof(R) + 1);
+  return isl_fixed_bytes<R, T>() + size_t(nb) * ((kIslSt + (nb <= kIslIwBodies ? kIslIw : 0)) * sizeof(R) + 1);
 }
 
-template <typename R, int KIND>
+template <typename R, int KIND, int T>
 constexpr void (*isl_kernel())(RS<R>) {
   if constexpr (sizeof(R) == 8)
-    return k_resolve_islands_f64<KIND>;
+    return k_resolve_islands_f64<KIND, T>;
   else
-    return k_resolve_islands_f32<KIND>;
+    return k_resolve_islands_f32<KIND, T>;
 }
 
 // Dynamic LDS beyond the default limit (worlds of more than about 880 bodies
@@ -2028,21 +2244,27 @@ hipError_t isl_allow_lds(void (*kernel)(RS<R>), size_t lds) {
   return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
 }
 
+template <typename R, int KIND, int T>
+hipError_t isl_launch(const RS<R>& a, hipStream_t st) {
+  const size_t lds = isl_lds_bytes<R, T>(a.isl_nb);
+  const hipError_t e = isl_allow_lds<R>(isl_kernel<R, KIND, T>(), lds);
+  if (e != hipSuccess) return e;
+  isl_kernel<R, KIND, T>()<<<a.n_worlds, T, lds, st>>>(a);
+  return hipGetLastError();
+}
+
 template <typename R, int KIND>
 hipError_t launch_islands_kind(const RS<R>& a, hipStream_t st) {
-  const size_t lds = isl_lds_bytes<R>(a.isl_nb);
-  const hipError_t e = isl_allow_lds<R>(isl_kernel<R, KIND>(), lds);
-  if (e != hipSuccess) return e;
-  isl_kernel<R, KIND>()<<<a.n_worlds, kIslThreads, lds, st>>>(a);
-  return hipGetLastError();
+  return isl_launch<R, KIND, kIslThreads>(a, st);
 }
 
 // Worlds (workgroups) of one kind's island kernel resident per CU, from its
 // register and LDS use.
 template <typename R, int KIND>
 hipError_t islands_occupancy(int nb, int* worlds_per_cu) {
-  return hipOccupancyMaxActiveBlocksPerMultiprocessor(worlds_per_cu, (const void*)isl_kernel<R, KIND>(), kIslThreads,
-                                                      isl_lds_bytes<R>(nb));
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(worlds_per_cu,
+                                                      (const void*)isl_kernel<R, KIND, kIslThreads>(), kIslThreads,
+                                                      isl_lds_bytes<R, kIslThreads>(nb));
 }
 
 #ifndef CBZ_RESOLVE_INSTANTIATE

@@ -13,7 +13,7 @@ namespace cbz {
 template <typename R, int KIND>
 __global__ void __launch_bounds__(kIslThreads) k_prepare(RS<R> a) {
   extern __shared__ __align__(16) char isl_lds[];
-  const IslWorld<R> W = isl_world_of(a, isl_lds, int(blockIdx.x));
+  const IslWorld<R, kIslThreads> W = isl_world_of<R, kIslThreads>(a, isl_lds, int(blockIdx.x));
   if (a.overflow[0] != 0 || W.C <= 0) return;  // the resolver's guard
   isl_prepare<R, KIND>(a, W, W.n <= W.NB);
 }
@@ -134,7 +134,7 @@ hipError_t launch_resolve(const ResolveLaunch<R>& L, hipStream_t st) {
   if (a.n_worlds <= 0) return hipSuccess;
   if (a.iter_mult == 0 && a.iter_fixed == 0 && (a.mode & ~RM_FRICTIONLESS2) == RM_POS) {
     if (!a.pos0 || !a.c.rec) return hipErrorInvalidValue;  // k_prepare writes both
-    const size_t lds = isl_lds_bytes<R>(a.isl_nb);
+    const size_t lds = isl_lds_bytes<R, kIslThreads>(a.isl_nb);
     void (*kernel)(RS<R>) = a.c.fric ? k_prepare<R, KIND_MAT> : k_prepare<R, KIND_PLAIN>;
     const hipError_t e = isl_allow_lds<R>(kernel, lds);
     if (e != hipSuccess) return e;

@@ -22,7 +22,7 @@ CONTACT = {"body0": 0, "body1": 0, "point": 3, "normal": 3, "pen": 1, "c2w": 9, 
 
 
 class _World(ctypes.Structure):
-    _fields_ = ([(k, ctypes.c_int32) for k in ("n", "C", "kind", "mode", "f64", "across")]
+    _fields_ = ([(k, ctypes.c_int32) for k in ("n", "C", "kind", "mode", "f64", "across", "threads")]
                 + [(k, ctypes.c_int64) for k in ("mult", "fixed", "log_cap", "max_steps")]
                 + [("dt", ctypes.c_double)]
                 + [(k, ctypes.c_void_p) for k in (*BODY, *CONTACT, "labels", "iters", "left")])
@@ -52,7 +52,7 @@ def _planes(x, k, real):
     return np.array(np.asarray(x).reshape(-1, k).T, real, order="C")
 
 
-def resolve(lib, o, contacts, dt, mult=4, fixed=0, precision="f64", kind=PLAIN, log_cap=200000, across=False):
+def resolve(lib, o, contacts, dt, mult=4, fixed=0, precision="f64", kind=PLAIN, log_cap=200000, across=False, threads=256):
     """ResolveContacts of an oracle world's state and contact list.  Returns the
     status (0), the arrays after it ([plane][n]), the iterations of both phases
     and how many worlds were handed to the serial kernel."""
@@ -69,7 +69,7 @@ def resolve(lib, o, contacts, dt, mult=4, fixed=0, precision="f64", kind=PLAIN, 
             out[k] = _planes(contacts[src.get(k, k)], w, real)
     out["labels"] = np.zeros((C, 13), np.float32)
     iters, left = np.zeros(2, np.int64), np.zeros(1, np.int32)
-    q = _World(n, C, kind, POS_VEL | (4 if kind == LABEL else 0), precision == "f64", across, mult, fixed, log_cap,
+    q = _World(n, C, kind, POS_VEL | (4 if kind == LABEL else 0), precision == "f64", across, threads, mult, fixed, log_cap,
                50_000_000, dt)
     for k in (*BODY, *CONTACT, "labels"):
         setattr(q, k, out[k].ctypes.data)

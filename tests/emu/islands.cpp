@@ -80,13 +80,16 @@ int run_block(void (*fn)(void*), void* arg, int nt, bool across, long max_steps)
 void on_segv(int) { siglongjmp(g_back, 1); }
 
 using namespace cbz;
-template <class R, int KIND>
-void block_of(void* p) {
-  isl_block<R, KIND>(*(RS<R>*)p);
-}
+template <class R, int T>
+struct Block {
+  template <int KIND>
+  static void of(void* p) {
+    isl_block<R, KIND, T>(*(RS<R>*)p);
+  }
+};
 
 struct World {
-  int32_t n, C, kind, mode, f64, across;
+  int32_t n, C, kind, mode, f64, across, threads;
   int64_t mult, fixed, log_cap, max_steps;
   double dt;
   void *pos, *quat, *vel, *rot, *inv_mass, *iit_body, *iit_world, *transform, *last_acc, *motion, *flags;
@@ -95,7 +98,7 @@ struct World {
   int32_t* left;   // worlds handed to the serial kernel
 };
 
-template <class R>
+template <class R, int T>
 int resolve(const World& q) {
   RS<R> a;
   memset((void*)&a, 0, sizeof a);
@@ -135,7 +138,7 @@ int resolve(const World& q) {
   a.pos0 = pos0.data();
   a.labels = (float*)q.labels;
   // LDS, its last byte before the guard
-  const size_t lds = isl_lds_bytes<R>(a.isl_nb), page = 4096, room = (lds + page - 1) / page * page;
+  const size_t lds = isl_lds_bytes<R, T>(a.isl_nb), page = 4096, room = (lds + page - 1) / page * page;
   char* mem = (char*)mmap(nullptr, room + kGuard, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
   mprotect(mem + room, kGuard, PROT_NONE);
   isl_lds = mem + room - lds;
@@ -143,10 +146,11 @@ int resolve(const World& q) {
   struct sigaction on = {}, was;
   on.sa_handler = on_segv;
   sigaction(SIGSEGV, &on, &was);
-  void (*fn)(void*) = q.kind == KIND_MAT     ? block_of<R, KIND_MAT>
-                      : q.kind == KIND_LABEL ? block_of<R, KIND_LABEL>
-                                             : block_of<R, KIND_PLAIN>;
-  const int rc = run_block(fn, &a, kIslThreads, q.across, q.max_steps);
+  typedef Block<R, T> B;
+  void (*fn)(void*) = q.kind == KIND_MAT     ? B::template of<KIND_MAT>
+                      : q.kind == KIND_LABEL ? B::template of<KIND_LABEL>
+                                             : B::template of<KIND_PLAIN>;
+  const int rc = run_block(fn, &a, T, q.across, q.max_steps);
   sigaction(SIGSEGV, &was, nullptr);
   munmap(mem, room + kGuard);
   *q.left = left_count[LEFT_WORLDS];
@@ -154,4 +158,7 @@ int resolve(const World& q) {
 }
 }  // namespace
 
-extern "C" int emu_resolve(const World* q) { return q->f64 ? resolve<double>(*q) : resolve<float>(*q); }
+extern "C" int emu_resolve(const World* q) {
+  if (q->threads == 128) return q->f64 ? resolve<double, 128>(*q) : resolve<float, 128>(*q);
+  return q->f64 ? resolve<double, 256>(*q) : resolve<float, 256>(*q);
+}
