@@ -732,11 +732,12 @@ int ensure_islands(cbz_ctx* c) {
       if (assign) p = (std::remove_reference_t<decltype(p)>)(c->isl_mem + at);
       at += (bytes + 255) & ~size_t(255);
     };
-    take(u.left_count, 2 * sizeof(int32_t));
+    take(u.left_count, 3 * sizeof(int32_t));
     take(u.log_head, sizeof(int64_t));
     take(u.cls, nw * kIslWords * sizeof(int32_t));
     const size_t zeroed = at;
     take(u.left_list, nw * sizeof(int32_t));
+    take(u.wide_list, nw * sizeof(int32_t));
     take(u.off, nb * sizeof(int32_t));
     take(u.cnt, nb * sizeof(int32_t));
     take(u.its, nb * sizeof(int32_t));

@@ -2146,8 +2146,16 @@ __device__ __forceinline__ void isl_world(const RS<R>& a, const IslWorld<R, T>& 
     return;
   }
   if (do_prep) isl_prepare<R, KIND>(a, W, true);
+  if (a.isl_wide && !do_prep) {  // left by the narrow workgroups: its islands are theirs
+    isl_build(a, W);
+    __syncthreads();
+  }
   if (a.isl_cls[kIslWords * int64_t(w) + kIslTaken] != T) {
-    isl_leave(a, W, false);
+    if (T < kIslThreads) {
+      if (W.t == 0) a.wide_list[atomicAdd(&a.left_count[LEFT_WIDE], 1)] = w;
+    } else {
+      isl_leave(a, W, false);
+    }
     return;
   }
   // worlds beyond the polish's reach take the plain phase
@@ -2201,7 +2209,8 @@ __device__ __forceinline__ IslWorld<R, T> isl_world_of(const RS<R>& a, char* lds
 template <typename R, int KIND, int T>
 __device__ __forceinline__ void isl_block(const RS<R>& a) {
   extern __shared__ __align__(16) char isl_lds[];
-  const int w = a.order ? a.order[blockIdx.x] : int(blockIdx.x);
+  if (a.isl_wide && int(blockIdx.x) >= a.left_count[LEFT_WIDE]) return;
+  const int w = a.isl_wide ? a.wide_list[blockIdx.x] : a.order ? a.order[blockIdx.x] : int(blockIdx.x);
   const IslWorld<R, T> W = isl_world_of<R, T>(a, isl_lds, w);
   int64_t* wt = a.world_time ? a.world_time + 4 * int64_t(w) + ((a.mode & RM_VEL) ? 2 : 0) : nullptr;
   if (wt && W.t == 0) wt[0] = int64_t(wall_clock64());
@@ -2253,9 +2262,15 @@ hipError_t isl_launch(const RS<R>& a, hipStream_t st) {
   return hipGetLastError();
 }
 
+// narrow: half the threads per world, and what these leave on whole workgroups.
 template <typename R, int KIND>
-hipError_t launch_islands_kind(const RS<R>& a, hipStream_t st) {
-  return isl_launch<R, KIND, kIslThreads>(a, st);
+hipError_t launch_islands_kind(const RS<R>& a, bool narrow, hipStream_t st) {
+  if (!narrow) return isl_launch<R, KIND, kIslThreads>(a, st);
+  const hipError_t e = isl_launch<R, KIND, kIslThreads / 2>(a, st);
+  if (e != hipSuccess) return e;
+  RS<R> wide = a;
+  wide.isl_wide = 1;
+  return isl_launch<R, KIND, kIslThreads>(wide, st);
 }
 
 // Worlds (workgroups) of one kind's island kernel resident per CU, from its

@@ -86,7 +86,8 @@ struct IslandBuffers {
   int64_t* log_head = nullptr;      // [1]
   int64_t log_cap = 0;
   int32_t* left_list = nullptr;     // [n_worlds]
-  int32_t* left_count = nullptr;    // [2], zero between resolves
+  int32_t* wide_list = nullptr;     // [n_worlds]
+  int32_t* left_count = nullptr;    // [3], zero between resolves
 };
 
 template <typename R>

@@ -30,13 +30,13 @@ namespace cbz {
 
 constexpr int kKeyCap = 1280;
 
-// threads of the island kernel's workgroup
+// threads of the island kernel's workgroup (half of them in large launches)
 constexpr int kIslThreads = 256;
 // a left world's entry: its position phase is done already
 constexpr int32_t kLeftVelOnly = 1 << 30;
 // RS::left_count: listed worlds, workgroups of the left kernel that are done
-// with theirs
-enum : int { LEFT_WORLDS = 0, LEFT_DONE = 1, LEFT_COUNTS = 2 };
+// with theirs, worlds that the narrow workgroups leave to whole ones
+enum : int { LEFT_WORLDS = 0, LEFT_DONE = 1, LEFT_WIDE = 2, LEFT_COUNTS = 3 };
 
 // Relative energy slack of the surrogate's acceptance test (rounding); the
 // absolute slack is 1/2 tol^2 per kilogram: the kinetic energy of the
@@ -81,12 +81,14 @@ struct RS {
   // the worlds the island kernel leaves: entries (world | kLeftVelOnly);
   // left_count: LEFT_*, zero between resolves
   int32_t* left_list;
+  int32_t* wide_list;
   int32_t* left_count;
   // the island kernel (cbz_islands.h): per island, at its world's
   // first body + rank: contacts (offset into isl_idx from the world's first
   // slot, count), iterations, log records and where the log starts; per
   // world the class counts and, in entry 6, whether its islands were taken
   int32_t isl_nb;      // bodies the LDS tables hold
+  int32_t isl_wide;    // the worlds are wide_list
   int32_t* isl_off;    // [n_bodies]
   int32_t* isl_cnt;    // [n_bodies]
   int32_t* isl_its;    // [n_bodies]
@@ -956,7 +958,7 @@ void launch_left_kind(const RS<R>& a, int grid, hipStream_t st) {
 // (k_resolve_<precision>_<kind>.hip); other units only declare them.
 #define CBZ_RESOLVE_KIND(EXT, R, KIND)                                          \
   EXT template void launch_left_kind<R, KIND>(const RS<R>&, int, hipStream_t); \
-  EXT template hipError_t launch_islands_kind<R, KIND>(const RS<R>&, hipStream_t); \
+  EXT template hipError_t launch_islands_kind<R, KIND>(const RS<R>&, bool, hipStream_t); \
   EXT template hipError_t islands_occupancy<R, KIND>(int, int*);
 
 }  // namespace cbz

@@ -10,12 +10,21 @@ namespace cbz {
 // prepareContacts alone (a position launch without iterations): one
 // workgroup per world, a thread per contact, from the bodies' state in HBM,
 // with every contact's record and the world's islands.
-template <typename R, int KIND>
-__global__ void __launch_bounds__(kIslThreads) k_prepare(RS<R> a) {
+template <typename R, int KIND, int T>
+__global__ void __launch_bounds__(T) k_prepare(RS<R> a) {
   extern __shared__ __align__(16) char isl_lds[];
-  const IslWorld<R, kIslThreads> W = isl_world_of<R, kIslThreads>(a, isl_lds, int(blockIdx.x));
+  const IslWorld<R, T> W = isl_world_of<R, T>(a, isl_lds, int(blockIdx.x));
   if (a.overflow[0] != 0 || W.C <= 0) return;  // the resolver's guard
   isl_prepare<R, KIND>(a, W, W.n <= W.NB);
+}
+template <typename R, int T>
+hipError_t launch_prepare(const RS<R>& a, hipStream_t st) {
+  const size_t lds = isl_lds_bytes<R, T>(a.isl_nb);
+  void (*kernel)(RS<R>) = a.c.fric ? k_prepare<R, KIND_MAT, T> : k_prepare<R, KIND_PLAIN, T>;
+  const hipError_t e = isl_allow_lds<R>(kernel, lds);
+  if (e != hipSuccess) return e;
+  kernel<<<a.n_worlds, T, lds, st>>>(a);
+  return hipGetLastError();
 }
 
 // The order in which the worlds start: those that took longest in the last
@@ -65,6 +74,20 @@ __global__ void __launch_bounds__(1024) k_order(const int64_t* time, const int32
 // bodies, and 0.82 against 0.76 in the plain phases).
 constexpr int kOrderWorlds = 256;
 
+// Worlds whose whole workgroups fit the chip (two per CU in FP64, three in FP32).
+template <typename R>
+constexpr int32_t kResident = 256 * (sizeof(R) == 8 ? 2 : 3);
+// Launches of many times that are bound by how many worlds are in flight, not by
+// the longest one's chain: they get workgroups of half the threads, twice as many
+// of them resident, and the few worlds of larger islands whole ones behind.  A
+// step of 4096 worlds of towers, collapsed, takes 9.8 ms in FP64 (13.8 with whole
+// workgroups) and 7.0 in FP32 (8.9), of 16384 in FP32 19 (30); of 2048 batched
+// worlds in FP32 1.13 against 1.02, so the line lies above.
+template <typename R>
+bool isl_narrow(int32_t n_worlds) {
+  return n_worlds > 4 * kResident<R>;
+}
+
 // The island kernel, then the kernel for the worlds it leaves (none, as a
 // rule: its workgroups end at once).
 template <typename R, int KIND>
@@ -75,7 +98,7 @@ hipError_t launch_all(const RS<R>& plain, const ResolveLaunch<R>& L, hipStream_t
     k_order<<<1, 1024, 0, st>>>(a.world_time + 2, a.body_off, a.n_worlds, cost, cost + a.n_worlds);
     a.order = cost + a.n_worlds;
   }
-  const hipError_t e = launch_islands_kind<R, KIND>(a, st);
+  const hipError_t e = launch_islands_kind<R, KIND>(a, isl_narrow<R>(a.n_worlds), st);
   if (e != hipSuccess) return e;
   launch_left_kind<R, KIND>(a, std::min(a.n_worlds, std::max(kLeftGrid, L.isl.large)), st);
   return hipGetLastError();
@@ -94,8 +117,10 @@ hipError_t launch_resolve(const ResolveLaunch<R>& L, hipStream_t st) {
   a.world_iters = L.world_iters;
   a.world_time = L.world_time;
   a.left_list = L.isl.left_list;
+  a.wide_list = L.isl.wide_list;
   a.left_count = L.isl.left_count;
   a.isl_nb = L.isl.nb;
+  a.isl_wide = 0;
   a.isl_off = L.isl.off;
   a.isl_cnt = L.isl.cnt;
   a.isl_its = L.isl.its;
@@ -134,12 +159,7 @@ hipError_t launch_resolve(const ResolveLaunch<R>& L, hipStream_t st) {
   if (a.n_worlds <= 0) return hipSuccess;
   if (a.iter_mult == 0 && a.iter_fixed == 0 && (a.mode & ~RM_FRICTIONLESS2) == RM_POS) {
     if (!a.pos0 || !a.c.rec) return hipErrorInvalidValue;  // k_prepare writes both
-    const size_t lds = isl_lds_bytes<R, kIslThreads>(a.isl_nb);
-    void (*kernel)(RS<R>) = a.c.fric ? k_prepare<R, KIND_MAT> : k_prepare<R, KIND_PLAIN>;
-    const hipError_t e = isl_allow_lds<R>(kernel, lds);
-    if (e != hipSuccess) return e;
-    kernel<<<a.n_worlds, kIslThreads, lds, st>>>(a);
-    return hipGetLastError();
+    return isl_narrow<R>(a.n_worlds) ? launch_prepare<R, kIslThreads / 2>(a, st) : launch_prepare<R, kIslThreads>(a, st);
   }
   if (a.c.fric) return launch_all<R, KIND_MAT>(a, L, st);
   if (a.mode & RM_POLISH)

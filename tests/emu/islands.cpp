@@ -122,10 +122,10 @@ int resolve(const World& q) {
   std::vector<int64_t> log(n);
   std::vector<uint8_t> flag(n);
   const int32_t body_off[2] = {0, n}, overflow = 0;
-  int32_t left_list[1], left_count[LEFT_COUNTS] = {};
+  int32_t left_list[1], wide_list[1], left_count[LEFT_COUNTS] = {};
   int64_t coff = 0, head = 0;
   a.world_cnt = &C, a.world_coff = &coff, a.overflow = &overflow, a.body_off = body_off, a.world_iters = q.iters;
-  a.left_list = left_list, a.left_count = left_count;
+  a.left_list = left_list, a.wide_list = wide_list, a.left_count = left_count;
   a.isl_nb = (n + 15) & ~15;
   a.isl_off = off.data(), a.isl_cnt = cnt.data(), a.isl_its = its.data(), a.isl_nrec = nrec.data();
   a.isl_log = log.data(), a.isl_cls = cls.data(), a.isl_idx = idx.data();
@@ -153,7 +153,7 @@ int resolve(const World& q) {
   const int rc = run_block(fn, &a, T, q.across, q.max_steps);
   sigaction(SIGSEGV, &was, nullptr);
   munmap(mem, room + kGuard);
-  *q.left = left_count[LEFT_WORLDS];
+  *q.left = left_count[LEFT_WORLDS] + left_count[LEFT_WIDE];
   return rc;
 }
 }  // namespace

@@ -100,8 +100,9 @@ def test_merged_logs_equal_one_island(lib, kind, precision, mult, fixed):
     assert kind != emu.LABEL or np.abs(a[1]["labels"]).max() > 0
 
 
+@pytest.mark.parametrize("threads", [256, 128])
 @pytest.mark.parametrize("n,squeeze,at", [(12, 1.0, 60), (64, 1.0, 100), (200, 1.0, 120), (120, 0.4, 200)])
-def test_stopped_at_the_budget(lib, n, squeeze, at):
+def test_stopped_at_the_budget(lib, n, squeeze, at, threads):
     """Budgets around every rule of a world that exceeds its own: one island of
     all contacts (small, or short), logs from the first iteration, logs and
     checkpoints of an island that runs for a quarter of the budget."""
@@ -109,4 +110,4 @@ def test_stopped_at_the_budget(lib, n, squeeze, at):
     for i, budget in enumerate((1, 31, 96, 97, 128, 131, 200, 256, 399, 700, 1500)):
         o, cs = _at_contacts(sc, at)
         if len(cs):
-            _check(lib, o, cs, sc.dt, fixed=budget, log_cap=0 if i % 4 == 3 else 200000)
+            _check(lib, o, cs, sc.dt, fixed=budget, log_cap=0 if i % 4 == 3 else 200000, threads=threads)
