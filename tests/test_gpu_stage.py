@@ -41,3 +41,24 @@ def test_contacts_of_all_worlds_equal_each_world_s(precision):
         each = [w.contacts(k) for k in range(sc.n_worlds)]
         for name, x in every.items():
             assert same(x, np.concatenate([e[name] for e in each])), name
+
+
+# FP64: 4847 contacts fill the stage with every plane; half of it holds 7280 of
+# nine planes, 21840 of three; from 131073 the penetrations and from 262145 the body
+# indices exceed it
+@pytest.mark.parametrize("n", [4847, 4848, 4849, 7281, 14561, 21841, 43681, 131072, 131073, 262145])
+@pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_contacts_come_back_as_they_went(n, precision):
+    sc = scenes.batched(0, 2, 8, 8)
+    rng = np.random.default_rng(n)
+    body = rng.integers(0, 16, (2, n)).astype(np.int32)
+    point, normal, pen = (rng.normal(0, 1, (n, k)).astype(np.float32).astype(np.float64) for k in (3, 3, 1))
+    with World(sc, precision=precision, contact_capacity=n + 3) as w:
+        w.set_contacts([n - 1, 1], body[0], body[1], point, normal, pen[:, 0])
+        got = w.contacts(-1)
+        for name, x in (("body0", body[0]), ("body1", body[1])):
+            assert np.array_equal(got[name], x), name
+        for name, x in (("point", point), ("normal", normal), ("pen", pen[:, 0])):
+            assert same(got[name], x), name
+        one = w.contacts(1)
+        assert same(one["point"], point[n - 1:]) and one["body0"][0] == body[0, -1]
