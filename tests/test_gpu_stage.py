@@ -62,3 +62,25 @@ def test_contacts_come_back_as_they_went(n, precision):
             assert same(got[name], x), name
         one = w.contacts(1)
         assert same(one["point"], point[n - 1:]) and one["body0"][0] == body[0, -1]
+
+
+# a list of 130 053 pairs and its tables are the most the stage holds
+@pytest.mark.parametrize("n", [130_053, 130_054, 200_003])
+def test_pair_lists_around_the_stage(n):
+    sc = scenes.batched(3, 1, 200, 200)
+    sc.fields["pos"][:, 1] *= 0.2
+    rng = np.random.default_rng(n)
+    one = rng.integers(0, 200, n).astype(np.int32)
+    two = ((one + rng.integers(0, 200, n)) % 200).astype(np.int32)
+    two[two == one] = -1
+    with World(sc, contact_capacity=8 * n) as w:
+        w.calculate_derived()
+        total = w.narrowphase_pairs(one, two)
+        got, parts = w.contacts(-1, internals=False), []
+        counts = w.pair_contact_counts(n)
+        assert total == counts.sum() > 0
+        for k in range(0, n, 50_000):
+            assert w.narrowphase_pairs(one[k:k + 50_000], two[k:k + 50_000]) == counts[k:k + 50_000].sum()
+            parts.append(w.contacts(-1, internals=False))
+        for name, x in got.items():
+            assert same(x, np.concatenate([p[name] for p in parts])), name
