@@ -930,7 +930,8 @@ int run_list_narrowphase(cbz_ctx* c, const std::vector<int32_t>& wq, int64_t* to
     HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, hipMemcpy(dst, from, words * sizeof(int32_t), hipMemcpyHostToDevice));
   }
-  HIPCHK(c, launch_fill_i32(c->n_hits, kNarrowCounters + 1, 0, c->stream));  // the sticky flag too
+  // the sticky flag too, and the candidates, which only an all-pairs narrowphase counts
+  HIPCHK(c, launch_fill_i32(c->n_hits, kNarrowCounters + 2, 0, c->stream));
   rc = c->precision == CBZ_F64 ? do_narrowphase<double>(c, (int32_t)nt, nullptr, true)
                                : do_narrowphase<float>(c, (int32_t)nt, nullptr, true);
   if (rc) return rc;
@@ -1700,8 +1701,7 @@ int cbz_set_scene(cbz_ctx* c, int32_t n_worlds, const int32_t* body_off, const i
   HIPCHK(c, hipMemset(c->world_iters, 0, 2 * n_worlds * sizeof(int64_t)));
   HIPCHK(c, hipMemset(c->world_time, 0xFF, 4 * n_worlds * sizeof(int64_t)));  // -1: no launch yet
   HIPCHK(c, hipMemset(c->cost, 0, 2 * n_worlds * sizeof(int32_t)));
-  HIPCHK(c, hipMemset(c->overflow, 0, 2 * sizeof(int32_t)));
-  HIPCHK(c, hipMemset(c->total, 0, sizeof(int64_t)));
+  HIPCHK(c, hipMemset(c->total, 0, kStatusWords * sizeof(int32_t)));
   std::vector<int32_t> ord;
   build_order(c, ord);
   HIPCHK(c, hipMemcpy(c->order, ord.data(), ord.size() * sizeof(int32_t), hipMemcpyHostToDevice));
