@@ -1056,7 +1056,6 @@ int check_overflow(cbz_ctx* c, int64_t* total) {
   int64_t tot = 0;
   std::memcpy(&tot, st, sizeof tot);
   const int32_t of = st[(c->overflow + 1) - (int32_t*)c->total], nc = st[c->n_cand - (int32_t*)c->total];
-  if (total) *total = tot;
   if (of && nc > c->cand_cap)
     return fail(c, CBZ_ERR_CAPACITY,
                 "narrowphase candidate list exceeded: " + std::to_string(nc) + " candidate pairs for " +
@@ -1065,6 +1064,7 @@ int check_overflow(cbz_ctx* c, int64_t* total) {
     return fail(c, CBZ_ERR_CAPACITY,
                 "contact capacity exceeded: " + std::to_string(tot) + " contacts for " + std::to_string(c->cap) +
                     " slots (raise cbz_config.contact_capacity)");
+  if (total) *total = tot;
   return CBZ_OK;
 }
 
