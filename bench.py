@@ -41,8 +41,8 @@ Prints one JSON line.  Besides the metric it reports:
                          on all host cores and on one
   resolver_split         per leg, the resolver split that the autotuner
                          (cbz_autotune_resolver) picked on the settled state,
-                         with every candidate's ms/step (the split has no
-                         effect any more: the times differ by noise)
+                         with the settled step's ms under every candidate
+                         (the split has no effect: one is timed for all)
 """
 import argparse
 import json
@@ -552,9 +552,8 @@ def main():
                                           "exact_f32": exact32["critical_path_last_step"]}
         out["resolver_split"] = {"surrogate": sur["resolver_split"], "exact_f64": exact64["resolver_split"],
                                  "exact_f32": exact32["resolver_split"],
-                                 "what": "(min_contacts, max_worlds): the max_worlds largest worlds of at least "
-                                         "min_contacts contacts resolve on the 4-wavefront kernel (0,0: none); "
-                                         "picked per leg by the autotuner from the window's start state"}
+                                 "what": "(min_contacts, max_worlds), without effect: every world runs on one "
+                                         "kernel; set per leg by the autotuner, which times one candidate for all"}
         out["contacts_per_step"] = sur["contacts_per_step"]
         out["contacts_per_s"] = sur["contacts_per_step"] * sur["value"] / nb
         phases.update(sur["resolver_ms_per_step"])

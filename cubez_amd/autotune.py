@@ -2,9 +2,8 @@
 (cbz_autotune_resolver) and cached on disk.
 
 The split named the worlds that a second resolver kernel took.  Every world
-now runs on one kernel, island by island, so the candidates time alike and
-whichever is kept changes nothing; the module serves the programs that call
-it.
+now runs on one kernel, island by island, so one candidate is timed for all
+and the first is kept; the module serves the programs that call it.
 
 The cache key is the scene's shape and the step kind: precision, world and
 body counts, a coarse histogram of per-world contact counts, and whether
@@ -45,9 +44,9 @@ def _load(path):
 
 def tune(world, dt, iter_per_contact=4, precision="f64", surrogate=False, steps=5, candidates=CANDIDATES,
          tol=0.06, polish=4, use_cache=True):
-    """Set the fastest split for this scene on `world` (from the cache when
-    the scene's key is there, else by measurement from the current state,
-    which is restored) and return {"split", "ms_per_step", "cached", "key"}."""
+    """Set the split for this scene on `world` (from the cache when the scene's
+    key is there, else the first candidate, with the step's time measured from
+    the current state, which is restored) and return {"split", "ms_per_step", "cached", "key"}."""
     world.narrowphase()  # contact counts of the current state for the key
     key = scene_key(world, precision, surrogate)
     path = cache_path()

@@ -2171,26 +2171,20 @@ int cbz_autotune_resolver(cbz_ctx* c, double dt, int64_t iter_per_contact, int32
     return surrogate ? cbz_step_sur(c, dt, steps, iter_per_contact, tol, polish_per_contact, 0, nullptr, fb.data())
                      : cbz_step(c, dt, steps, iter_per_contact, nullptr);
   };
-  int32_t pick = -1;
-  double pick_ms = 0.0;
+  // every world runs on one kernel whatever the split, so one candidate is
+  // timed, for all of them, and the first is kept
   hipError_t e = copy(true);
-  for (int32_t i = 0; e == hipSuccess && !rc && i < n_cand; ++i) {
-    if ((rc = cbz_set_resolver_split(c, cand_min[i], cand_max[i]))) break;
-    // one untimed step captures the step for this split
-    if ((e = copy(false)) != hipSuccess || (rc = run(1))) break;
-    if ((e = copy(false)) != hipSuccess || (e = hipEventRecord(c->ev[0], c->stream)) != hipSuccess) break;
-    if ((rc = run(n_steps))) break;
-    if ((e = hipEventRecord(c->ev[1], c->stream)) != hipSuccess || (e = hipEventSynchronize(c->ev[1])) != hipSuccess)
-      break;
-    float ms = 0.f;
-    if ((e = hipEventElapsedTime(&ms, c->ev[0], c->ev[1])) != hipSuccess) break;
-    const double per = double(ms) / n_steps;
-    if (ms_per_step) ms_per_step[i] = per;
-    if (pick < 0 || per < pick_ms) {
-      pick = i;
-      pick_ms = per;
-    }
-  }
+  if (e == hipSuccess) rc = cbz_set_resolver_split(c, cand_min[0], cand_max[0]);
+  float ms = 0.f;
+  auto timed = [&]() -> hipError_t {
+    hipError_t t = hipSuccess;
+    // one untimed step captures the step
+    if ((rc = run(1)) || (t = copy(false)) != hipSuccess || (t = hipEventRecord(c->ev[0], c->stream)) != hipSuccess) return t;
+    if ((rc = run(n_steps)) || (t = hipEventRecord(c->ev[1], c->stream)) != hipSuccess) return t;
+    if ((t = hipEventSynchronize(c->ev[1])) != hipSuccess) return t;
+    return hipEventElapsedTime(&ms, c->ev[0], c->ev[1]);
+  };
+  if (e == hipSuccess && !rc) e = timed();
   if (e == hipSuccess) e = copy(false);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   dfree(snap);
@@ -2199,8 +2193,9 @@ int cbz_autotune_resolver(cbz_ctx* c, double dt, int64_t iter_per_contact, int32
     cbz_set_resolver_split(c, old_min, old_max);
     return rc;
   }
-  if (best) *best = pick;
-  return cbz_set_resolver_split(c, cand_min[pick], cand_max[pick]);
+  if (ms_per_step) std::fill(ms_per_step, ms_per_step + n_cand, double(ms) / n_steps);
+  if (best) *best = 0;
+  return CBZ_OK;
 }
 
 int cbz_resolver_world_times(cbz_ctx* c, double* us) {

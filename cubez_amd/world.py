@@ -211,9 +211,9 @@ class World:
     def autotune_resolver(self, dt, iter_per_contact=4, steps=5, candidates=((0, 0), (257, 16), (257, 32),
                                                                            (257, 64), (257, 128)),
                           surrogate=False, tol=0.06, polish=4):
-        """Times `steps` steps from the current state for each resolver split
-        (min_contacts, max_worlds), restoring the state around each run,
-        keeps the fastest (cbz_autotune_resolver) and returns
+        """Times `steps` steps from the current state, which it restores, sets
+        the first of the resolver splits (min_contacts, max_worlds), none of
+        which has an effect (cbz_autotune_resolver), and returns
         {"split": (min, max), "ms_per_step": {split: ms}}."""
         cand = np.asarray(candidates, np.int32).reshape(-1, 2)
         lo, hi = np.ascontiguousarray(cand[:, 0]), np.ascontiguousarray(cand[:, 1])

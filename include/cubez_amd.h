@@ -258,13 +258,12 @@ int cbz_resolver_occupancy(cbz_ctx *ctx, int32_t *worlds_per_cu, int32_t *n_cu);
  * set them, and change neither results nor times. */
 int cbz_set_resolver_split(cbz_ctx *ctx, int32_t min_contacts, int32_t max_worlds);
 int cbz_get_resolver_split(cbz_ctx *ctx, int32_t *min_contacts, int32_t *max_worlds);
-/* The autotuner of that split: from the current state, times n_steps of
- * cbz_step (surrogate = 0) or of cbz_step_sur (surrogate = 1, with tol and
- * polish_per_contact) for each candidate split (cand_min[i], cand_max[i]),
- * restoring the body state before each run and at the end, then keeps the
- * fastest: its index in *best, the times in ms_per_step[n_cand] (may be
- * NULL).  The split has no effect, so the times differ by noise alone.
- * Profiling must be off.  No counterpart in the reference. */
+/* The autotuner of that split.  The split has no effect, so one candidate of
+ * (cand_min[i], cand_max[i]) is timed and the first is set: n_steps of cbz_step
+ * (surrogate = 0) or of cbz_step_sur (surrogate = 1, with tol and
+ * polish_per_contact) from the current body state, which is restored at the
+ * end.  Its time is every candidate's in ms_per_step[n_cand] (may be NULL), *best
+ * is 0.  Profiling must be off.  No counterpart in the reference. */
 int cbz_autotune_resolver(cbz_ctx *ctx, double dt, int64_t iter_per_contact, int32_t n_steps, int32_t surrogate,
                           double tol, int64_t polish_per_contact, int32_t n_cand, const int32_t *cand_min,
                           const int32_t *cand_max, double *ms_per_step, int32_t *best);
