@@ -2689,19 +2689,27 @@ int cbz_sur_check_gemms(int32_t rows, char* msg, int32_t msg_len) {
   sur_infer_buffers(fake.sur, Mpad, place);
   sur_layered_buffers(fake.sur, Mpad, place);
   fake.dry_regions = &regions;
-  // the weight gradients of a training step: every fragment of both operands
-  // and the sums they give
+  // A training step: what its forward and backward read of a layer's weights,
+  // biases and normalisation and write per row, every fragment of both operands
+  // of the weight gradients, the sums they give and the parameters these move.
   int rc = CBZ_OK;
   const LayerOff o = layer_offsets();
+  const auto& u = fake.sur;
+  const auto inside = [&](const auto* p, int64_t n) { return dry_inside(&fake, p, n * (int64_t)sizeof(*p)); };
+  // the fragments of K columns of 32 rows at a time, up to row `rows`
+  const auto frags = [](int64_t rows, int64_t K) { return frag_at(rows - 32, K - 16, K) + 512; };
+  const auto batch = [&](int64_t F) { return batch_at(F - 1, Mpad - 1, F) + 1; };
+  if (!inside(u.row_loss, Mpad) || !inside(u.norm, kNorm))
+    rc = fail(&fake, CBZ_ERR_STATE, "training rows' losses or normalisation outside their buffers");
   for (int l = 0; l < kLayers && !rc; ++l) {
-    const auto& u = fake.sur;
-    const int64_t a = batch_at(layer_out_pad(l) - 1, Mpad - 1, layer_out_pad(l)) + 1;
-    const int64_t b = batch_at(layer_in_frag(l) - 1, Mpad - 1, layer_in_frag(l)) + 1;
-    if (!dry_inside(&fake, u.dZt[l], a * (int64_t)sizeof(__bf16)) ||
-        !dry_inside(&fake, u.At[l], b * (int64_t)sizeof(__bf16)) ||
-        !dry_inside(&fake, u.grad + o.w[l], int64_t(layer_out(l)) * layer_in(l) * (int64_t)sizeof(float)) ||
-        !dry_inside(&fake, u.grad + o.b[l], layer_out(l) * (int64_t)sizeof(float)))
-      rc = fail(&fake, CBZ_ERR_STATE, "weight gradient of layer " + std::to_string(l) + " outside its buffers");
+    const int64_t in = layer_in_pad(l), out = layer_out_pad(l), weights = int64_t(layer_out(l)) * layer_in(l);
+    if (!inside(u.Wf[l], frags(out, in)) || (l > 0 && !inside(u.Wb[l], frags(in, out))) ||
+        !inside(u.params + o.b[l], layer_out(l)) || !inside(u.At[l], batch(layer_in_frag(l))) ||
+        !inside(u.dZt[l], batch(out)))
+      rc = fail(&fake, CBZ_ERR_STATE, "training rows of layer " + std::to_string(l) + " outside their buffers");
+    for (const float* p : {u.grad, u.params, u.adam_m, u.adam_v})
+      if (!rc && (!inside(p + o.w[l], weights) || !inside(p + o.b[l], layer_out(l))))
+        rc = fail(&fake, CBZ_ERR_STATE, "weight gradient of layer " + std::to_string(l) + " outside its buffers");
   }
   if (!rc) rc = sur_forward(&fake, fake.sur.X, rows, Mpad);
   if (msg && msg_len > 0) {
