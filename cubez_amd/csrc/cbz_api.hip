@@ -846,7 +846,6 @@ int do_resolve(cbz_ctx* c, double dt, int64_t mult, int64_t fixed, int32_t mode 
   return CBZ_OK;
 }
 
-// List buffers for n_pairs explicit pairs.
 // Places for a list of n_pairs: one, two and the first pair of every world
 // (uploaded, or made by the broadphase), then what every list is uploaded with.
 int ensure_list(cbz_ctx* c, int64_t n_pairs) {

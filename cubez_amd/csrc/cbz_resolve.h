@@ -86,7 +86,7 @@ struct RS {
   // the island kernel (cbz_islands.h): per island, at its world's
   // first body + rank: contacts (offset into isl_idx from the world's first
   // slot, count), iterations, log records and where the log starts; per
-  // world the class counts and, in entry 6, whether its islands were taken
+  // world the class counts and the workgroup size that its islands were made for
   int32_t isl_nb;      // bodies the LDS tables hold
   int32_t isl_wide;    // the worlds are wide_list
   int32_t* isl_off;    // [n_bodies]
@@ -828,9 +828,6 @@ __device__ __forceinline__ int id_lo(uint32_t id) { return int(id & 0xFFFFu); }
 __device__ __forceinline__ int id_hi(uint32_t id) { return (id >> 16) == kNoBody ? -1 : int(id >> 16); }
 
 // Broadcast of lane l's value (l uniform) by readlane.
-__device__ __forceinline__ uint32_t lane_value(uint32_t v, int l) {
-  return uint32_t(__builtin_amdgcn_readlane(int(v), l));
-}
 __device__ __forceinline__ float lane_value(float v, int l) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
@@ -838,24 +835,19 @@ __device__ __forceinline__ double lane_value(double v, int l) {
   return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
                           __builtin_amdgcn_readlane(__double2loint(v), l));
 }
-template <typename R>
-__device__ __forceinline__ V3<R> lane_value(const V3<R>& v, int l) {
-  return V3<R>{lane_value(v.x, l), lane_value(v.y, l), lane_value(v.z, l)};
-}
 // Marks the slots' packed body ids as redefined, so that values derived from
 // them (decoded ids, comparison masks: one 64-bit scalar mask per slot) are
-// recomputed in each serial iteration instead of being hoisted out of the
-// loop, which for 16-32 slots exhausts the register files.
+// recomputed in each iteration instead of being hoisted out of the loop, where
+// they would be spilled.
 template <int N>
 __device__ __forceinline__ void opaque_ids(uint32_t (&ids)[N]) {
 #pragma unroll
   for (int k = 0; k < N; ++k) asm volatile("" : "+v"(ids[k]));
 }
 
-// The lane index as a value redefined at the point of the call: the
-// per-slot addresses computed from it in a serial iteration (hundreds of
-// 64-bit values for the wide classes) are then recomputed there instead of
-// being hoisted out of the loop.
+// A lane's index as a value redefined at the point of the call: the addresses
+// computed from it are then recomputed there instead of being hoisted out of
+// the loop.
 __device__ __forceinline__ int opaque_lane(int lane) {
   asm volatile("" : "+v"(lane));
   return lane;
