@@ -51,7 +51,9 @@
 // quarter of the budget logs from there on and keeps two checkpoints: the second
 // run is of the first quarter, the third starts from the last checkpoint before
 // the share.  1000 landing worlds take 0.40 ms a resolve (0.71 with three whole
-// runs, 0.53 as serial chains), 1000 of 8 to 32 bodies 0.51 (0.75, 0.53).
+// runs, 0.53 as serial chains), 1000 of 8 to 32 bodies 0.51 (0.75, 0.53).  The
+// registers this takes cost every launch 1.4 us (one landing world of 64 bodies:
+// 26.5 instead of 25.0).
 //
 // A budget that is small for the world is not worth it: a world whose budget is
 // below half (with more than 512 contacts a quarter) of its contacts, or whose
